@@ -109,10 +109,9 @@ int ensure_ell(ljgpu_ctx* ctx) {
 // dev_tile_order, which needs positions: a list built on the device gets it
 // at once, a list installed from the caller at its first force evaluation
 // (index order until then). Systems without a periodic box stay in index
-// order. Tiles derived with positions also take the cutoff classes of cl2
-// (cut_partition) when the rows are bank-class ordered; a tiling derived
-// without positions is derived again, once, when positions first come.
-int ensure_tiles(ljgpu_ctx* ctx, const PosIn* q, double box, double cl2) {
+// order. A tiling derived without positions is derived again, once, when
+// positions first come.
+int ensure_tiles(ljgpu_ctx* ctx, const PosIn* q, double box) {
   const int32_t want = ctx->eval_half ? 0 : effective_tile(ctx);
   const bool spatial = ctx->tile_order == LJGPU_TILE_ORDER_SPATIAL && want > 0;
   if (want == ctx->tiles_for && (ctx->tiles_ordered || !q || want == 0)) return LJGPU_OK;
@@ -125,16 +124,8 @@ int ensure_tiles(ljgpu_ctx* ctx, const PosIn* q, double box, double cl2) {
                        ctx->work, &ordered));
   if (ordered) TRY(dev_length_sort(ctx->stream, ctx->eval, want, ctx->rep_off, ctx->work));
   const int32_t* member = ordered ? ctx->work.order.as<int32_t>() : nullptr;
-  CutHint cut;
-  if (q) {
-    cut.q = *q;
-    cut.box = box;
-    cut.rep_box = ctx->rep_box_dev.as<double>();
-    cut.cl2 = cl2;
-  }
   for (int32_t tp = want; tp >= 1 && ctx->eval.n > 0; tp /= 2) {
-    TRY(dev_make_tiles(ctx->stream, ctx->eval, tp, ctx->rep_off, member, ctx->bank_order,
-                       q ? &cut : nullptr, ctx->work, ctx->tiles));
+    TRY(dev_make_tiles(ctx->stream, ctx->eval, tp, ctx->rep_off, member, ctx->work, ctx->tiles));
     if (ctx->tiles.tile_particles > 0) break;
   }
   // The slot-order copies that calls of kSlotMinSteps or more steps run over
@@ -150,21 +141,44 @@ int ensure_tiles(ljgpu_ctx* ctx, const PosIn* q, double box, double cl2) {
   return LJGPU_OK;
 }
 
+const int32_t* tile_row_starts(const ljgpu_ctx* ctx) {
+  return ctx->tiles.order == LJGPU_TILE_ORDER_SPATIAL ? ctx->tiles.slot_ptr.as<int32_t>()
+                                                      : ctx->eval.ptr.as<int32_t>();
+}
+
 // The tiles' offsets sliced for the configured lanes and unroll (built once
-// per tiling and configuration).
-int ensure_sliced(ljgpu_ctx* ctx) {
+// per tiling and configuration), rows in the cutoff classes of the positions
+// a new tiling comes with.
+int ensure_sliced(ljgpu_ctx* ctx, const PosIn* q, double box, double cl2) {
   DevTiles& t = ctx->tiles;
   if (t.blocks <= 0 || (t.sliced_lanes == ctx->lanes && t.sliced_unroll == ctx->unroll))
     return LJGPU_OK;
-  const int32_t* sptr = t.order == LJGPU_TILE_ORDER_SPATIAL ? t.slot_ptr.as<int32_t>()
-                                                            : ctx->eval.ptr.as<int32_t>();
-  return dev_slice_tiles(ctx->stream, sptr, ctx->lanes, ctx->unroll, ctx->work, t);
+  CutHint cut;
+  if (q) {
+    cut.q = *q;
+    cut.box = box;
+    cut.rep_box = ctx->rep_off.empty() ? nullptr : ctx->rep_box_dev.as<double>();
+    cut.cl2 = cl2;
+  }
+  return dev_slice_tiles(ctx->stream, tile_row_starts(ctx), ctx->lanes, ctx->unroll,
+                         ctx->bank_order && !t.bank_done, ctx->eval.n, &cut, ctx->work, t);
+}
+
+// The bank-class order of the tiles' rows in `local`, for the kernels that
+// read it instead of the slices (once per tiling).
+int ensure_bank_order(ljgpu_ctx* ctx) {
+  DevTiles& t = ctx->tiles;
+  if (t.blocks <= 0 || t.bank_done || !ctx->bank_order) return LJGPU_OK;
+  TRY(dev_bank_order(ctx->stream, tile_row_starts(ctx), t, t.local.as<uint16_t>()));
+  t.bank_done = true;
+  return LJGPU_OK;
 }
 
 int prepare_layouts(ljgpu_ctx* ctx, const PosIn* q, double box, double cl2) {
   if (ctx->lanes == 1) return ensure_ell(ctx);
-  TRY(ensure_tiles(ctx, q, box, cl2));
-  return ensure_sliced(ctx);
+  TRY(ensure_tiles(ctx, q, box));
+  TRY(ensure_sliced(ctx, q, box, cl2));
+  return ctx->tile_offsets_lds || ctx->tiles.sliced_lanes == 0 ? ensure_bank_order(ctx) : LJGPU_OK;
 }
 
 PosIn positions_of(const ForceArgs& fa) {
@@ -1041,9 +1055,21 @@ int ljgpu_get_tiles(ljgpu_ctx* ctx, int32_t* desc, int64_t desc_capacity, int32_
     return set_error(LJGPU_ERR_CAPACITY, "get_tiles: output too small");
   HIP_TRY(hipMemcpyAsync(desc, t.desc.p, sizeof(int32_t) * 8 * t.blocks, hipMemcpyDeviceToHost,
                          ctx->stream), "hipMemcpyAsync");
-  if (ctx->eval.e > 0)
-    HIP_TRY(hipMemcpyAsync(local, t.local.p, sizeof(uint16_t) * ctx->eval.e, hipMemcpyDeviceToHost,
-                           ctx->stream), "hipMemcpyAsync");
+  if (ctx->eval.e > 0) {
+    // The rows in the bank-class order, made in a copy: the evaluated
+    // offsets stay as they are.
+    const size_t bytes = sizeof(uint16_t) * ctx->eval.e;
+    const void* src = t.local.p;
+    if (ctx->bank_order && !t.bank_done) {
+      TRY(dev_reserve(ctx->work.tmp, bytes, ctx->stream));
+      HIP_TRY(hipMemcpyAsync(ctx->work.tmp.p, src, bytes, hipMemcpyDeviceToDevice, ctx->stream),
+              "hipMemcpyAsync");
+      TRY(dev_bank_order(ctx->stream, tile_row_starts(ctx), t, ctx->work.tmp.as<uint16_t>()));
+      src = ctx->work.tmp.p;
+    }
+    HIP_TRY(hipMemcpyAsync(local, src, bytes, hipMemcpyDeviceToHost, ctx->stream),
+            "hipMemcpyAsync");
+  }
   if (t.stage_stride == 0) {
     if (t.staged > 0)
       HIP_TRY(hipMemcpyAsync(stage, t.stage.p, sizeof(int32_t) * t.staged, hipMemcpyDeviceToHost,

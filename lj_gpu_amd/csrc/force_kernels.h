@@ -652,13 +652,15 @@ k_tile(P pos, M mom, const int32_t* __restrict__ nop, const int32_t* __restrict_
 // pair arithmetic, with the energy policy): each workgroup walks its tiles
 // as k_tile does and writes weight * 4 * sum s^3 (s^3 - 1) and weight * the
 // pair count into part_u / part_c[blockIdx.x] (fixed-order sums, so the
-// result does not depend on scheduling). Row offsets from `local`.
-template <int TPI, int U, bool PBC>
+// result does not depend on scheduling). Row offsets from the slices where
+// they are cut for TPI lanes and U entries (SL), else from `local`.
+template <int TPI, int U, bool PBC, bool SL>
 __global__ void __launch_bounds__(1024)
 k_tile_energy(PosAos pos, const int32_t* __restrict__ member,
               const int32_t* __restrict__ slot_ptr, const int4* __restrict__ desc,
               const int32_t* __restrict__ stage, const uint16_t* __restrict__ local,
-              int32_t nblocks, PairParams pp, double reach, double weight,
+              const uint16_t* __restrict__ sliced, const int32_t* __restrict__ wave_off,
+              int32_t wpb, int32_t nblocks, PairParams pp, double reach, double weight,
               double* __restrict__ part_u, double* __restrict__ part_c) {
   extern __shared__ double lds[];
   int* flag = reinterpret_cast<int*>(lds);
@@ -671,8 +673,8 @@ k_tile_energy(PosAos pos, const int32_t* __restrict__ member,
   const int stride = static_cast<int>(gridDim.x) / kXcds;
   const int t_end = min(nblocks, (xcd + 1) * per);
   for (int b = xcd * per + static_cast<int>(blockIdx.x) / kXcds; b < t_end; b += stride) {
-    tile_body<TPI, U, kEnergy, PosAos, MomAos, PBC, false, false>(
-        pos, MomAos{nullptr}, nullptr, member, slot_ptr, desc, stage, local, nullptr, nullptr, 0,
+    tile_body<TPI, U, kEnergy, PosAos, MomAos, PBC, false, SL>(
+        pos, MomAos{nullptr}, nullptr, member, slot_ptr, desc, stage, local, sliced, wave_off, wpb,
         b, pp, reach, nullptr, lb, flag, eacc);
     __syncthreads();
   }
@@ -731,16 +733,18 @@ inline int run_energy_tiles(hipStream_t s, const double* q, const ListView& lv, 
   const size_t lds_bytes =
       kTileLdsHeader + std::max<size_t>(static_cast<size_t>(lv.tile_max_stage) * 24, 16 * 16);
   PosAos pos{q};
-  if (box > 0.0)
-    hipLaunchKernelGGL((k_tile_energy<kLanes, 4, true>), dim3(grid), dim3(threads), lds_bytes, s,
-                       pos, lv.tile_member, lv.tile_slot_ptr,
-                       reinterpret_cast<const int4*>(lv.tile_desc), lv.tile_stage, lv.tile_local,
-                       lv.tile_blocks, pp, reach, weight, part_u, part_c);
-  else
-    hipLaunchKernelGGL((k_tile_energy<kLanes, 4, false>), dim3(grid), dim3(threads), lds_bytes, s,
-                       pos, lv.tile_member, lv.tile_slot_ptr,
-                       reinterpret_cast<const int4*>(lv.tile_desc), lv.tile_stage, lv.tile_local,
-                       lv.tile_blocks, pp, reach, weight, part_u, part_c);
+  constexpr int kUnroll = 4;
+  const bool sl = lv.tile_sliced && lv.tile_sliced_lanes == kLanes && lv.tile_sliced_unroll == kUnroll;
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), lds_bytes, s, pos, lv.tile_member,
+                       lv.tile_slot_ptr, reinterpret_cast<const int4*>(lv.tile_desc),
+                       lv.tile_stage, lv.tile_local, lv.tile_sliced, lv.tile_wave_off,
+                       lv.tile_waves_per_block, lv.tile_blocks, pp, reach, weight, part_u, part_c);
+  };
+  if (box > 0.0) sl ? launch(k_tile_energy<kLanes, kUnroll, true, true>)
+                    : launch(k_tile_energy<kLanes, kUnroll, true, false>);
+  else sl ? launch(k_tile_energy<kLanes, kUnroll, false, true>)
+          : launch(k_tile_energy<kLanes, kUnroll, false, false>);
   return launch_status("tiled energy kernel launch");
 }
 

@@ -65,6 +65,13 @@ struct DevTiles {
   DevMem sliced;      // uint16
   DevMem wave_off;    // int32 per (block, wavefront slot): start of its slice
   int32_t sliced_lanes = 0, sliced_unroll = 0, waves_per_block = 0;
+
+  // Cutoff classes (cut): the rows of local hold their inner entries first,
+  // inner[s] of them in slot s's row. bank_done: local's rows are in the
+  // bank-class order as well (dev_bank_order).
+  bool cut = false, bank_done = false;
+  DevMem inner;          // int32 per slot
+  int32_t longest = 0;   // longest row
 };
 void dev_release(DevTiles& t);
 
@@ -82,6 +89,7 @@ struct ListWork {
   DevMem tmp;         // int32 per list entry
   DevMem tile_ns;     // int32 per tile (+1)
   DevMem tile_soff;   // int32 per tile (+1)
+  DevMem tile_stats;  // int4 per tile
   DevMem tile_geo;    // int32 x 4 per tile: first particle, count, replica
   DevMem rep_of;      // int32 per particle: replica index
   DevMem order;       // int32 per particle: spatial tile order
@@ -148,20 +156,10 @@ int dev_make_ell(hipStream_t s, const DevCSR& c, int32_t width, DevMem& ell);
 // evaluates untiled).
 // `member` (device, one particle per slot, a permutation that keeps every
 // replica's particles within its own slot range) orders the particles the
-// blocks cover; null takes them in index order. bank_order puts each row's
-// entries in the LDS bank-class order (bank_class_order), as the host model
-// does; without it rows keep the list order.
-// With bank_order and positions in `cut` (cut->q.x non-null), the rows
-// first take the cutoff classes (cut_partition) of those positions.
-struct CutHint {
-  PosIn q;                        // positions in the caller's particle order
-  double box = 0.0;               // single system: periodic box (<= 0 open)
-  const double* rep_box = nullptr;  // replicas: (box, 1/box) per replica on the device
-  double cl2 = 9.0;
-};
+// blocks cover; null takes them in index order.
 int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t tile_particles,
-                   const std::vector<int32_t>& replicas, const int32_t* member, bool bank_order,
-                   const CutHint* cut, ListWork& w, DevTiles& out);
+                   const std::vector<int32_t>& replicas, const int32_t* member, ListWork& w,
+                   DevTiles& out);
 
 // The tiles' entry offsets sliced per wavefront, for a tile kernel in
 // which `lanes` consecutive lanes own one row and take entries in batches
@@ -172,10 +170,25 @@ int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t tile_particles,
 // (as many as its longest row needs) 64 * unroll offsets, slot by slot,
 // each slot the 64 lanes' entries in lane order, so one offset load of the
 // kernel reads 64 consecutive values. Slots past a row's end hold 0.
-// Needs local, desc and the slot row starts of a built tiling; a slicing
-// whose total does not fit int32 is not built (sliced_lanes stays 0).
+// Needs local, desc and the slot row starts of a built tiling of n particles; a slicing
+// whose total does not fit int32 is not built (sliced_lanes stays 0). With
+// bank_order, the rows of local first take the cutoff classes
+// (cut_partition) of the positions in `cut`, if it has any and they have
+// none yet, and the places of a row (its inner ones, then the others) are given out so
+// that the lanes that read LDS together mostly read different banks
+// (slice_part). Without it places follow local.
+struct CutHint {
+  PosIn q;                        // positions in the caller's particle order
+  double box = 0.0;               // single system: periodic box (<= 0 open)
+  const double* rep_box = nullptr;  // replicas: (box, 1/box) per replica on the device
+  double cl2 = 9.0;
+};
 int dev_slice_tiles(hipStream_t s, const int32_t* slot_ptr, int32_t lanes, int32_t unroll,
-                    ListWork& w, DevTiles& t);
+                    bool bank_order, int32_t n, const CutHint* cut, ListWork& w, DevTiles& t);
+
+// The bank-class order (bank_class_order) of a tiling's rows, in place in
+// `local` (t.local or a copy of it); nothing when t.bank_done.
+int dev_bank_order(hipStream_t s, const int32_t* slot_ptr, const DevTiles& t, uint16_t* local);
 
 // Spatial particle order for LDS tiles, into w.order: each periodic system
 // (the whole set, or every replica of `replicas` with its box) is cut into

@@ -20,6 +20,7 @@
 #include <algorithm>
 #include <climits>
 #include <cmath>
+#include <cstring>
 #include <string>
 #include <type_traits>
 #include <vector>
@@ -803,32 +804,40 @@ __global__ __launch_bounds__(kBlock) void k_pairs_wave(int32_t ncell,
 // ---------------------------------------------------------------------------
 // LDS tiles
 // ---------------------------------------------------------------------------
-constexpr int kTileHashBits = 12;
-constexpr int kTileHash = 1 << kTileHashBits;          // open-addressing table slots
-constexpr int kTileHashLimit = 3072;                   // distinct keys before giving up
 constexpr int kTileMaxStage = kTileLdsBudget / 24 + 1; // staged positions that can fit
-constexpr int kTileUniq = 4096;                        // sort buffer (power of two)
-constexpr int kTileBatch = 8;                          // list entries loaded ahead per thread
 constexpr int64_t kTileOnePassBytes = int64_t{4} << 30;  // staging slots of the one-pass build
-static_assert(kTileMaxStage <= kTileHashLimit, "the hash limit must cover every tile that fits");
-static_assert(kTileHashLimit + kBlock < kTileHash, "probing must always find a free slot");
-static_assert(kTileHashLimit <= kTileUniq, "the sort buffer must hold every distinct key");
-
-__device__ __forceinline__ uint32_t tile_hash(int32_t key) {
-  return (static_cast<uint32_t>(key) * 2654435761u) >> (32 - kTileHashBits);
-}
-
 // Wavefronts per tile of the sliced offsets: at most 1024 threads.
 constexpr int kSliceWavesMax = 16;
-// A block's rows, staged in LDS: slot i0 + s holds particle mem[s], whose
-// row is list[src[s] ..) and covers entries [beg[s], beg[s + 1]) of the
-// block (beg[ni] = ne).
-constexpr int kTileRowsMax = 1024;
-struct TileRows {
-  int32_t mem[kTileRowsMax];
-  int32_t src[kTileRowsMax];
-  int32_t beg[kTileRowsMax + 1];
-};
+constexpr int kTileRowsMax = 1024;  // rows of a tile
+constexpr int kSliceRows = 64;      // rows whose slices are made together
+constexpr size_t kTileLdsMax = 64000;  // dynamic LDS of the row-order kernels
+
+// The set of a tile's partners, kept in LDS as a hash table of words: word
+// w stands for the 16 slots [16 w, 16 w + 16), its entry holds the key w and
+// a 16-bit mask of the slots present (later also the rank of its first
+// slot). Partners of a compact tile are runs of consecutive slots, so a tile
+// of about 750 partners and 9,000 entries has some 100 to 200 words: nearly
+// every entry finds its bit set already, and the words are few enough to be
+// ranked by comparing all pairs. A tile that fits the LDS budget has at most
+// kTileMaxStage words, below kWordLimit.
+constexpr int kWordBits = 12;
+constexpr int kWords = 1 << kWordBits;
+constexpr int kWordLimit = 3000;
+constexpr int kWordLanes = 16;  // lanes that walk one row together
+constexpr int kWordBatch = 4;   // entries per lane in flight
+constexpr int kSeedRows = 8;    // one row in so many fills the set first
+constexpr int32_t kTileCodeMax = 12288;  // entry codes kept in LDS
+static_assert(kTileMaxStage <= kWordLimit, "the word limit must cover every tile that fits");
+static_assert(kWordLimit + 1024 < kWords, "probing must always find a free entry");
+
+__device__ __forceinline__ uint32_t word_hash(int32_t w) {
+  return (static_cast<uint32_t>(w) * 2654435761u) >> (32 - kWordBits);
+}
+
+template <class T>
+__device__ __forceinline__ T lds_load(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
 
 struct TileGeom {
   int32_t i0, ni, ne, rid;
@@ -848,249 +857,170 @@ __device__ __forceinline__ TileGeom tile_geom(int32_t b, const int32_t* __restri
   return g;
 }
 
-// Fill the row table of block g. Returns the list position of the block's
-// first entry when its rows lie back to back in the list (index order), so
-// entry u is list[base + u]; -1 when they are scattered (entry u is then
-// found by a binary search over beg).
-__device__ int32_t tile_rows(const TileGeom& g, const int32_t* __restrict__ member,
-                             const int32_t* __restrict__ ptr, const int32_t* __restrict__ slot_ptr,
-                             TileRows& r) {
-  for (int32_t t = threadIdx.x; t < g.ni; t += kBlock) {
-    const int32_t i = member ? member[g.i0 + t] : g.i0 + t;
-    r.mem[t] = i;
-    r.src[t] = ptr[i];
-    r.beg[t] = slot_ptr[g.i0 + t] - static_cast<int32_t>(g.e0);
-  }
-  if (threadIdx.x == 0) r.beg[g.ni] = g.ne;
-  __syncthreads();
-  const int32_t base = r.src[0];
-  int ok = 1;
-  for (int32_t t = threadIdx.x; t < g.ni; t += kBlock) ok &= (r.src[t] - r.beg[t] == base);
-  return __syncthreads_and(ok) ? base : -1;
-}
-
-// Partner of the block's entry u (0 <= u < ne).
-__device__ __forceinline__ int32_t tile_entry(const TileRows& r, int32_t ni, int32_t base,
-                                              const int32_t* __restrict__ list, int32_t u) {
-  if (base >= 0) return list[base + u];
-  int32_t lo = 0, hi = ni;  // beg[lo] <= u < beg[hi]
-  while (hi - lo > 1) {
-    const int32_t mid = (lo + hi) >> 1;
-    if (r.beg[mid] <= u) lo = mid;
-    else hi = mid;
-  }
-  return list[r.src[lo] + (u - r.beg[lo])];
-}
-
-// Insert the block's keys (the slots of its own particles and of every
-// entry's partner; slot_of null: index order, slot = particle) into an LDS
-// hash set. Returns the number of distinct keys, or -1 when there are more
-// than kTileHashLimit (such a block cannot fit the LDS budget).
-__device__ int32_t tile_insert(const TileGeom& g, const TileRows& rows, int32_t base,
-                               const int32_t* __restrict__ list,
-                               const int32_t* __restrict__ slot_of, int32_t* table,
-                               int32_t* counter) {
-  for (int32_t t = threadIdx.x; t < kTileHash; t += kBlock) table[t] = -1;
-  if (threadIdx.x == 0) *counter = 0;
-  __syncthreads();
-  const int64_t m = g.ni + static_cast<int64_t>(g.ne);
-  // Keys are loaded kTileBatch at a time before any is inserted, so each
-  // thread waits for memory once per batch rather than once per key.
-  for (int64_t t0 = 0; t0 < m; t0 += kTileBatch * kBlock) {
-    int32_t keys[kTileBatch];
-#pragma unroll
-    for (int r = 0; r < kTileBatch; r++) {
-      const int64_t t = t0 + r * kBlock + threadIdx.x;
-      keys[r] = t >= m     ? -1
-                : t < g.ni ? -2 - static_cast<int32_t>(t)  // own slot g.i0 + t, below
-                           : tile_entry(rows, g.ni, base, list, static_cast<int32_t>(t - g.ni));
+// Add one slot (its word w, hashed to h, and bit) to the set. Returns the
+// word's table entry; once more than kWordLimit words are present the tile
+// cannot fit, and the search ends at any entry.
+__device__ __forceinline__ uint32_t word_add(int32_t w, uint32_t h, uint32_t bit, int32_t* keys,
+                                             uint32_t* masks, int32_t* counter) {
+  while (lds_load(counter) <= kWordLimit) {
+    const int32_t prev = atomicCAS(&keys[h], -1, w);
+    if (prev == -1) atomicAdd(counter, 1);
+    if (prev == -1 || prev == w) {
+      atomicOr(&masks[h], 1u << bit);
+      break;
     }
-#pragma unroll
-    for (int r = 0; r < kTileBatch; r++) {
-      if (keys[r] <= -2) keys[r] = g.i0 - 2 - keys[r];
-      else if (keys[r] >= 0 && slot_of) keys[r] = slot_of[keys[r]];
-    }
-#pragma unroll
-    for (int r = 0; r < kTileBatch; r++) {
-      const int32_t key = keys[r];
-      if (key < 0) continue;
-      uint32_t h = tile_hash(key);
-      while (__hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) <=
-             kTileHashLimit) {
-        const int32_t prev = atomicCAS(&table[h], -1, key);
-        if (prev == -1) {
-          atomicAdd(counter, 1);
-          break;
-        }
-        if (prev == key) break;
-        h = (h + 1) & (kTileHash - 1);
-      }
-    }
+    h = (h + 1) & (kWords - 1);
   }
-  __syncthreads();
-  const int32_t ns = *counter;
-  __syncthreads();
-  return ns > kTileHashLimit ? -1 : ns;
+  return h;
 }
 
-// Slot of a key known to be in the table.
-__device__ __forceinline__ int32_t tile_find(const int32_t* table, int32_t key) {
-  uint32_t h = tile_hash(key);
-  while (table[h] != key) h = (h + 1) & (kTileHash - 1);
-  return static_cast<int32_t>(h);
-}
-
-// Ascending sort of uniq[0 .. kBlock * R) by the workgroup's wavefronts:
-// element e = w*64R + r*64 + lane sits in register r of lane `lane` of
-// wavefront w. Bitonic network: exchanges closer than 64 go through lane
-// shuffles, closer than 64R between a lane's own registers, and only the
-// farther ones (log2(waves) stages per merge size beyond 64R) through LDS.
-template <int R>
-__device__ void block_bitonic(int32_t* uniq) {
-  constexpr int kSpan = 64 * R;
-  constexpr int P = kBlock * R;
-  const int lane = threadIdx.x & 63;
-  const int wbase = static_cast<int>(threadIdx.x >> 6) * kSpan;
-  int32_t v[R];
-#pragma unroll
-  for (int r = 0; r < R; r++) v[r] = uniq[wbase + r * 64 + lane];
-  for (int k = 2; k <= P; k <<= 1) {
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      if (j >= kSpan) {
-#pragma unroll
-        for (int r = 0; r < R; r++) uniq[wbase + r * 64 + lane] = v[r];
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-          const int e = wbase + r * 64 + lane;
-          const int32_t other = uniq[e ^ j];
-          const bool keep_min = ((e & j) == 0) == ((e & k) == 0);
-          v[r] = keep_min ? min(v[r], other) : max(v[r], other);
-        }
-        __syncthreads();
-      } else if (j >= 64) {
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-          const int pr = r ^ (j / 64);
-          if (pr > r) {
-            const bool up = ((wbase + r * 64 + lane) & k) == 0;
-            const int32_t a = v[r], c = v[pr];
-            v[r] = up ? min(a, c) : max(a, c);
-            v[pr] = up ? max(a, c) : min(a, c);
-          }
-        }
-      } else {
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-          const int32_t other = __shfl_xor(v[r], j, 64);
-          const bool up = ((wbase + r * 64 + lane) & k) == 0;
-          const bool keep_min = ((lane & j) == 0) == up;
-          v[r] = keep_min ? min(v[r], other) : max(v[r], other);
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < R; r++) uniq[wbase + r * 64 + lane] = v[r];
-}
-
-// Pass 1: distinct staged particles per block; flags blocks that exceed the
-// LDS budget. stats: [0] overflow, [1] max staged, [2] max LDS bytes.
-__global__ __launch_bounds__(kBlock) void k_tile_count(const int32_t* __restrict__ geo, int32_t nblocks,
-                                                       const int32_t* __restrict__ member,
-                                                       const int32_t* __restrict__ slot_of,
-                                                       const int32_t* __restrict__ slot_ptr,
-                                                       const int32_t* __restrict__ ptr,
-                                                       const int32_t* __restrict__ list,
-                                                       int32_t* __restrict__ ns_out,
-                                                       int32_t* __restrict__ stats) {
-  __shared__ int32_t table[kTileHash];
-  __shared__ TileRows rows;
-  __shared__ int32_t counter;
+// One workgroup per tile. Every partner's slot (and the tile's own slots)
+// enters the word set; the words are ranked, each slot's rank being its
+// word's base plus the set bits below it, which is the ascending order of
+// slots; the staged particles are written in that order and each entry's LDS
+// offset 24 * rank in row order. What an entry needs to find its rank (table
+// entry and bit, 16 bits) stays in LDS between the two, so the list and
+// slot_of are read once; entries beyond `ecap` are looked up again.
+//   Sixteen lanes share a row (no search for the row of an entry), four
+// entries per lane in flight, with every first probe of a batch issued
+// before any is used. soff null: tile b stages at b * kTileMaxStage, and
+// nothing more is done for a tile over the LDS budget; else at soff[b].
+// COUNT stops after the set: ns_out[b] distinct slots. stats[b]: distinct
+// slots (-1: too many words), LDS bytes, longest row (k_tile_stats reduces
+// them: an atomic per tile on one address costs more than the tile).
+template <bool COUNT>
+__global__ __launch_bounds__(1024) void k_tile_fill(
+    const int32_t* __restrict__ geo, int32_t nblocks, const int32_t* __restrict__ member,
+    const int32_t* __restrict__ slot_of, const int32_t* __restrict__ slot_ptr,
+    const int32_t* __restrict__ ptr, const int32_t* __restrict__ list,
+    const int32_t* __restrict__ soff, int32_t ecap, int32_t* __restrict__ ns_out,
+    int32_t* __restrict__ desc, int32_t* __restrict__ stage, int32_t* __restrict__ stage_slot,
+    uint16_t* __restrict__ local, int4* __restrict__ stats) {
+  __shared__ int32_t keys[kWords];
+  __shared__ uint32_t masks[kWords];  // slots present, then also the base rank << 16
+  __shared__ uint16_t words[kWordLimit];  // table entries in use
+  __shared__ int32_t counter, nwords, total, longest;
+  extern __shared__ uint16_t code[];  // ecap: table entry << 4 | bit of each entry
+  const int nt = static_cast<int>(blockDim.x), tid = static_cast<int>(threadIdx.x);
+  const int lane = tid & (kWordLanes - 1), group = tid / kWordLanes, groups = nt / kWordLanes;
   for (int32_t b = blockIdx.x; b < nblocks; b += gridDim.x) {
     const TileGeom g = tile_geom(b, geo, slot_ptr);
-    const int32_t base = tile_rows(g, member, ptr, slot_ptr, rows);
-    const int32_t ns = tile_insert(g, rows, base, list, slot_of, table, &counter);
-    if (threadIdx.x == 0) {
-      ns_out[b] = ns < 0 ? 0 : ns;
-      const int64_t bytes = ns < 0 ? INT32_MAX : tile_lds_bytes(ns, g.ne);
-      if (bytes > kTileLdsBudget) atomicOr(&stats[0], 1);
-      atomicMax(&stats[1], ns);
-      atomicMax(&stats[2], static_cast<int32_t>(std::min<int64_t>(bytes, INT32_MAX)));
+    for (int t = tid; t < kWords; t += nt) {
+      keys[t] = -1;
+      masks[t] = 0;
     }
-  }
-}
-
-// Pass 2 (every block fits): the distinct keys sorted ascending become the
-// block's staged particles; each entry's LDS offset is 24 * the rank of its
-// partner, looked up through the hash table.
-__global__ __launch_bounds__(kBlock) void k_tile_fill(const int32_t* __restrict__ geo, int32_t nblocks,
-                                                      const int32_t* __restrict__ member,
-                                                      const int32_t* __restrict__ slot_of,
-                                                      const int32_t* __restrict__ slot_ptr,
-                                                      const int32_t* __restrict__ ptr,
-                                                      const int32_t* __restrict__ list,
-                                                      const int32_t* __restrict__ soff,
-                                                      int32_t* __restrict__ desc,
-                                                      int32_t* __restrict__ stage,
-                                                      int32_t* __restrict__ stage_slot,
-                                                      uint16_t* __restrict__ local,
-                                                      int32_t* __restrict__ stats,
-                                                      unsigned long long* __restrict__ staged) {
-  __shared__ int32_t table[kTileHash];
-  __shared__ uint16_t rank_of[kTileHash];
-  __shared__ int32_t uniq[kTileUniq];
-  __shared__ TileRows rows;
-  __shared__ int32_t counter;
-  __shared__ int64_t sh[kBlock / 64];
-  constexpr int32_t C = kTileHash / kBlock;
-  for (int32_t b = blockIdx.x; b < nblocks; b += gridDim.x) {
-    const TileGeom g = tile_geom(b, geo, slot_ptr);
-    const int32_t base = tile_rows(g, member, ptr, slot_ptr, rows);
-    const int32_t ns = tile_insert(g, rows, base, list, slot_of, table, &counter);
-    if (!soff) {
-      // One pass: block b stages at b * kTileMaxStage, and the budget check
-      // of k_tile_count happens here (stats as there, plus the total staged).
-      const int64_t bytes = ns < 0 ? INT32_MAX : tile_lds_bytes(ns, g.ne);
-      const bool over = bytes > kTileLdsBudget;
-      if (threadIdx.x == 0) {
-        if (over) atomicOr(&stats[0], 1);
-        atomicMax(&stats[1], ns);
-        atomicMax(&stats[2], static_cast<int32_t>(std::min<int64_t>(bytes, INT32_MAX)));
-        if (!over) atomicAdd(staged, static_cast<unsigned long long>(ns));
-      }
-      if (over) continue;  // the whole block (ns is uniform); the caller retries smaller
-    }
-    // Compact the occupied slots (C per thread) into uniq[0..ns), pad, sort.
-    int32_t cnt = 0;
-    for (int32_t t = threadIdx.x * C; t < (threadIdx.x + 1) * C; t++) cnt += table[t] != -1;
-    int64_t total;
-    int64_t off = block_exclusive(cnt, &total, sh);
-    for (int32_t t = threadIdx.x * C; t < (threadIdx.x + 1) * C; t++)
-      if (table[t] != -1) uniq[off++] = table[t];
-    int32_t P = kBlock;
-    while (P < ns) P <<= 1;
-    for (int32_t t = ns + threadIdx.x; t < P; t += kBlock) uniq[t] = INT32_MAX;
+    if (tid == 0) counter = nwords = total = longest = 0;
     __syncthreads();
-    switch (P / kBlock) {
-      case 1: block_bitonic<1>(uniq); break;
-      case 2: block_bitonic<2>(uniq); break;
-      case 4: block_bitonic<4>(uniq); break;
-      case 8: block_bitonic<8>(uniq); break;
-      default: block_bitonic<16>(uniq); break;
+    for (int t = tid; t < g.ni; t += nt) {
+      const int32_t key = g.i0 + t;
+      (void)word_add(key >> 4, word_hash(key >> 4), key & 15, keys, masks, &counter);
+    }
+    // One row in kSeedRows first, spread over all the groups: it brings in most
+    // of the words and bits, so that the other rows nearly always find theirs
+    // (all rows at once would all meet the empty table).
+    auto walk = [&](int r, int32_t k0, int32_t step) {
+      const int32_t a = slot_ptr[g.i0 + r];
+      const int32_t m = slot_ptr[g.i0 + r + 1] - a;
+      const int32_t src = ptr[member ? member[g.i0 + r] : g.i0 + r];
+      const int32_t eoff = a - static_cast<int32_t>(g.e0);
+      if (k0 == 0) atomicMax(&longest, m);
+      for (; k0 < m; k0 += step * kWordBatch) {
+        int32_t key[kWordBatch], w0[kWordBatch];
+        uint32_t h[kWordBatch], m0[kWordBatch];
+#pragma unroll
+        for (int u = 0; u < kWordBatch; u++) {
+          const int32_t k = k0 + u * step;
+          key[u] = k < m ? list[src + k] : -1;
+        }
+        if (slot_of) {
+#pragma unroll
+          for (int u = 0; u < kWordBatch; u++)
+            if (key[u] >= 0) key[u] = slot_of[key[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < kWordBatch; u++) {
+          h[u] = word_hash(key[u] >> 4);
+          w0[u] = lds_load(&keys[h[u]]);
+          m0[u] = lds_load(&masks[h[u]]);
+        }
+#pragma unroll
+        for (int u = 0; u < kWordBatch; u++) {
+          if (key[u] < 0) continue;
+          const uint32_t bit = key[u] & 15;
+          if (w0[u] != key[u] >> 4)
+            h[u] = word_add(key[u] >> 4, h[u], bit, keys, masks, &counter);
+          else if (!((m0[u] >> bit) & 1))
+            atomicOr(&masks[h[u]], 1u << bit);
+          const int32_t e = eoff + k0 + u * step;
+          if (!COUNT && e < ecap) code[e] = static_cast<uint16_t>(h[u] << 4 | bit);
+        }
+      }
+    };
+    const int seeds = (g.ni + kSeedRows - 1) / kSeedRows;
+    const int share = max(1, groups / seeds);  // groups to a seed row
+    for (int q = group; q < seeds * share; q += groups)
+      walk(q / share * kSeedRows, (q % share) * kWordLanes + lane, share * kWordLanes);
+    __syncthreads();
+    for (int q = group; q < g.ni - seeds; q += groups)
+      walk(q / (kSeedRows - 1) * kSeedRows + q % (kSeedRows - 1) + 1, lane, kWordLanes);
+    __syncthreads();
+    const bool full = counter > kWordLimit;
+    // The table entries in use, in any order, and the distinct slots.
+    if (!full) {
+      int32_t cnt = 0;
+      for (int t = tid; t < kWords; t += nt) {
+        if (keys[t] == -1) continue;
+        words[atomicAdd(&nwords, 1)] = static_cast<uint16_t>(t);
+        cnt += __popc(masks[t]);
+      }
+      if (cnt) atomicAdd(&total, cnt);
+    }
+    __syncthreads();
+    const int32_t nw = nwords;
+    const int32_t ns = full ? -1 : total;
+    const int64_t bytes = full ? INT32_MAX : tile_lds_bytes(ns, g.ne);
+    const bool over = bytes > kTileLdsBudget;
+    if (tid == 0) {
+      if (COUNT) ns_out[b] = full ? 0 : ns;
+      stats[b] = make_int4(ns, static_cast<int32_t>(std::min<int64_t>(bytes, INT32_MAX)), longest, 0);
+    }
+    if (COUNT || (over && !soff)) {  // uniform over the workgroup
+      __syncthreads();
+      continue;
+    }
+    // Base rank of each word: the slots of all smaller words, eight lanes to
+    // a word.
+    for (int t0 = 0; t0 < nw; t0 += nt / 8) {
+      const int t = t0 + tid / 8;
+      int32_t base = 0;
+      if (t < nw) {
+        const int32_t w = keys[words[t]];
+        for (int v = tid & 7; v < nw; v += 8) {
+          const int x = words[v];
+          base += keys[x] < w ? __popc(masks[x] & 0xffffu) : 0;
+        }
+      }
+#pragma unroll
+      for (int d = 4; d > 0; d >>= 1) base += __shfl_xor(base, d, 8);
+      // Only the low halves are read above, so the base can go in at once.
+      if (t < nw && (tid & 7) == 0) atomicOr(&masks[words[t]], static_cast<uint32_t>(base) << 16);
     }
     __syncthreads();
     const int64_t s0 = soff ? soff[b] : static_cast<int64_t>(b) * kTileMaxStage;
     // Staged particles in slot order: stage holds the particles, stage_slot
     // (spatial order only) their slots.
-    for (int32_t t = threadIdx.x; t < ns; t += kBlock) {
-      const int32_t key = uniq[t];
-      stage[s0 + t] = member ? member[key] : key;
-      if (stage_slot) stage_slot[s0 + t] = key;
-      rank_of[tile_find(table, key)] = static_cast<uint16_t>(t);
+    for (int t = tid; t < nw * 16; t += nt) {
+      const int x = words[t >> 4];
+      const uint32_t v = masks[x], bit = t & 15;
+      if (!((v >> bit) & 1)) continue;
+      const int32_t key = keys[x] << 4 | bit;
+      const int64_t d = s0 + (v >> 16) + __popc(v & ((1u << bit) - 1));
+      stage[d] = member ? member[key] : key;
+      if (stage_slot) stage_slot[d] = key;
     }
-    if (threadIdx.x == 0) {
+    if (tid == 0) {
       int32_t* d = desc + static_cast<int64_t>(b) * 8;
+      const int32_t mid = g.i0 + g.ni / 2;
       d[0] = g.i0;
       d[1] = g.ni;
       d[2] = static_cast<int32_t>(s0);
@@ -1098,80 +1028,290 @@ __global__ __launch_bounds__(kBlock) void k_tile_fill(const int32_t* __restrict_
       d[4] = static_cast<int32_t>(g.e0);
       d[5] = g.ne;
       d[6] = g.rid;
-      d[7] = rows.mem[g.ni / 2];  // middle particle: the periodic unwrap's reference
+      d[7] = member ? member[mid] : mid;  // middle particle: the periodic unwrap's reference
     }
-    __syncthreads();
-    for (int32_t e0 = 0; e0 < g.ne; e0 += kTileBatch * kBlock) {
-      int32_t js[kTileBatch];
-#pragma unroll
-      for (int r = 0; r < kTileBatch; r++) {
-        const int32_t e = e0 + r * kBlock + threadIdx.x;
-        js[r] = e < g.ne ? tile_entry(rows, g.ni, base, list, e) : -1;
-      }
-      if (slot_of) {
-#pragma unroll
-        for (int r = 0; r < kTileBatch; r++)
-          if (js[r] >= 0) js[r] = slot_of[js[r]];
-      }
-#pragma unroll
-      for (int r = 0; r < kTileBatch; r++) {
-        const int32_t e = e0 + r * kBlock + threadIdx.x;
-        if (js[r] >= 0) local[g.e0 + e] = static_cast<uint16_t>(rank_of[tile_find(table, js[r])] * 24);
+    const int32_t ncode = min(g.ne, ecap);
+    for (int32_t e = tid; e < ncode; e += nt) {
+      const uint32_t v = masks[code[e] >> 4], bit = code[e] & 15;
+      local[g.e0 + e] = static_cast<uint16_t>(((v >> 16) + __popc(v & ((1u << bit) - 1))) * 24);
+    }
+    if (g.ne > ecap) {
+      for (int r = group; r < g.ni; r += groups) {
+        const int32_t a = slot_ptr[g.i0 + r];
+        const int32_t m = slot_ptr[g.i0 + r + 1] - a;
+        const int32_t src = ptr[member ? member[g.i0 + r] : g.i0 + r];
+        const int32_t eoff = a - static_cast<int32_t>(g.e0);
+        for (int32_t k = lane; k < m; k += kWordLanes) {
+          if (eoff + k < ecap) continue;
+          int32_t key = list[src + k];
+          if (slot_of) key = slot_of[key];
+          uint32_t h = word_hash(key >> 4);
+          while (keys[h] != key >> 4) h = (h + 1) & (kWords - 1);
+          const uint32_t v = masks[h], bit = key & 15;
+          local[a + k] = static_cast<uint16_t>(((v >> 16) + __popc(v & ((1u << bit) - 1))) * 24);
+        }
       }
     }
     __syncthreads();
   }
 }
 
-// The row order of every tile row: with positions (cut.q.x non-null) the
-// cutoff classes (cut_partition over cut_inner, partners found through the
-// block's staged particles), then the bank-class order of each class
-// (bank_class_order). One wavefront per tile, one row per lane, each lane's
-// buffers in LDS.
-struct CutDev {
-  PosIn q;
-  const int32_t* desc;
-  const int32_t* stage;
-  const int32_t* member;
-  double box;
-  const double* rep_box;
-  double cl2;
-};
+// The tiles' stats in one: out[0] a tile over the LDS budget, [1] most staged,
+// [2] most LDS bytes, [3] longest row, [4] a tile with too many pages, [6..7]
+// the total staged (64 bits). One workgroup.
+__global__ __launch_bounds__(1024) void k_tile_stats(int32_t nblocks, const int4* __restrict__ stats,
+                                                     int32_t* __restrict__ out) {
+  __shared__ int32_t mx[5];
+  __shared__ unsigned long long sum;
+  if (threadIdx.x < 5) mx[threadIdx.x] = threadIdx.x == 1 ? -1 : 0;
+  if (threadIdx.x == 5) sum = 0;
+  __syncthreads();
+  int32_t v[5] = {0, -1, 0, 0, 0};
+  unsigned long long n = 0;
+  for (int32_t b = threadIdx.x; b < nblocks; b += blockDim.x) {
+    const int4 t = stats[b];
+    const bool over = t.y > kTileLdsBudget;
+    v[0] |= over;
+    v[1] = max(v[1], t.x);
+    v[2] = max(v[2], t.y);
+    v[3] = max(v[3], t.z);
+    v[4] |= t.w;
+    n += over ? 0 : max(t.x, 0);
+  }
+  for (int d = 32; d > 0; d >>= 1) {
+#pragma unroll
+    for (int k = 0; k < 5; k++) v[k] = max(v[k], __shfl_xor(v[k], d, 64));
+    n += __shfl_xor(n, d, 64);
+  }
+  if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+    for (int k = 0; k < 5; k++) atomicMax(&mx[k], v[k]);
+    atomicAdd(&sum, n);
+  }
+  __syncthreads();
+  if (threadIdx.x < 5) out[threadIdx.x] = mx[threadIdx.x];
+  if (threadIdx.x == 5) *reinterpret_cast<unsigned long long*>(out + 6) = sum;
+}
+
+// The same tiles as k_tile_fill<false>, for tiles whose partners lie in few
+// pages of 2^pshift consecutive slots (any spatially ordered list: a column's
+// slots are consecutive, and a tile meets about 25 columns). The set is
+// then a byte per slot of the pages in use, filled by plain stores, with no atomics
+// and no search:
+//   1. every entry marks its page in a directory of all pages;
+//   2. a scan numbers the marked pages in ascending order;
+//   3. every entry marks its slot in its page's bytes;
+//   4. a scan over the bytes, 16 at a time, leaves a 16-bit mask and a base rank
+//      for each sixteen slots, from which every entry takes its rank.
+// A row's entries stay in registers (kPageLanes lanes to a row, up to
+// kPageKeys of them each; more are loaded again). What a tile takes is mostly
+// the latency of its dependent loads and barriers, so the workgroup is sized
+// for three of them to a CU (80 VGPRs; at four the 24 spilled registers cost
+// more: 87 against 64 us at 119,000 particles, 521 against 364 us at a
+// million). The hashed set of k_tile_fill takes 119 and 742 us there. A tile with more pages
+// than fit kPageBytes says so in stats[b].w, and the caller uses k_tile_fill.
+constexpr int kPageLanes = 8;
+constexpr int kPageKeys = 20;
+constexpr int kPageBytes = 24576;
+constexpr int kPageDir = 32768;  // most pages of a list
+static_assert(kPageBytes / 128 < 255, "a page number fits a byte");
+
+// Exclusive scan over the workgroup; *total receives the sum. sh: one value
+// per wavefront.
+__device__ __forceinline__ int32_t group_exclusive(int32_t v, int32_t* total, int32_t* sh) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  int32_t inc = v;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int32_t t = __shfl_up(inc, d, 64);
+    if (lane >= d) inc += t;
+  }
+  if (lane == 63) sh[wid] = inc;
+  __syncthreads();
+  int32_t off = 0, tot = 0;
+  for (int w = 0; w < static_cast<int>(blockDim.x) / 64; w++) {
+    const int32_t x = sh[w];
+    off += w < wid ? x : 0;
+    tot += x;
+  }
+  __syncthreads();
+  *total = tot;
+  return off + inc - v;
+}
+
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6))) void k_tile_pages(
+    const int32_t* __restrict__ geo, int32_t nblocks, const int32_t* __restrict__ member,
+    const int32_t* __restrict__ slot_of, const int32_t* __restrict__ slot_ptr,
+    const int32_t* __restrict__ ptr, const int32_t* __restrict__ list, int32_t pshift,
+    int32_t npages, int32_t* __restrict__ desc, int32_t* __restrict__ stage,
+    int32_t* __restrict__ stage_slot, uint16_t* __restrict__ local, int4* __restrict__ stats) {
+  extern __shared__ uint32_t page_lds[];
+  __shared__ uint32_t table[kPageBytes / 16];  // slots present, base rank << 16
+  __shared__ uint32_t used[kPageBytes / 4];    // a byte per slot of the pages in use
+  __shared__ int32_t page_of[256];
+  __shared__ int32_t sh[16];
+  __shared__ int32_t longest;
+  uint8_t* dir = reinterpret_cast<uint8_t*>(page_lds);  // npages, a multiple of 4 bytes
+  uint8_t* mark = reinterpret_cast<uint8_t*>(used);
+  const int nt = static_cast<int>(blockDim.x), tid = static_cast<int>(threadIdx.x);
+  const int lane = tid & (kPageLanes - 1), group = tid / kPageLanes, groups = nt / kPageLanes;
+  const int32_t low = (1 << pshift) - 1;
+  const int32_t chunk = ((npages + nt - 1) / nt + 3) / 4;  // directory words per thread
+  for (int32_t b = blockIdx.x; b < nblocks; b += gridDim.x) {
+    const TileGeom g = tile_geom(b, geo, slot_ptr);
+    for (int t = tid; t < (npages + 3) / 4; t += nt) page_lds[t] = 0;
+    if (tid == 0) longest = 0;
+    // The group's first row, in registers; places past its end hold the tile's
+    // first slot, which belongs to the set anyway.
+    int32_t key[kPageKeys];
+    int32_t mine = 0;  // the row's entries from this lane's first on
+    const int32_t* row = list + lane;
+    uint16_t* out = local + lane;
+    if (group < g.ni) {
+      const int32_t a = slot_ptr[g.i0 + group];
+      mine = slot_ptr[g.i0 + group + 1] - a - lane;
+      row += ptr[member ? member[g.i0 + group] : g.i0 + group];
+      out += a;
+    }
+#pragma unroll
+    for (int u = 0; u < kPageKeys; u++) {
+      key[u] = slot_of ? -1 : g.i0;
+      if (u * kPageLanes < mine) key[u] = row[u * kPageLanes];
+    }
+    if (slot_of) {
+#pragma unroll
+      for (int u = 0; u < kPageKeys; u++)
+        key[u] = key[u] >= 0 ? slot_of[static_cast<uint32_t>(key[u])] : g.i0;
+    }
+    // f(slot, entry) of every other entry of the block.
+    auto others = [&](auto&& f) {
+      for (int r = group; r < g.ni; r += groups) {
+        const int32_t a = slot_ptr[g.i0 + r];
+        const int32_t m = slot_ptr[g.i0 + r + 1] - a;
+        const int32_t src = ptr[member ? member[g.i0 + r] : g.i0 + r];
+        for (int32_t k = lane + (r == group ? kPageKeys * kPageLanes : 0); k < m; k += kPageLanes) {
+          const int32_t j = list[src + k];
+          f(slot_of ? slot_of[j] : j, a + k);
+        }
+        if (lane == 0) atomicMax(&longest, m);
+      }
+    };
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kPageKeys; u++) dir[key[u] >> pshift] = 1;
+    others([&](int32_t s, int32_t) { dir[s >> pshift] = 1; });
+    for (int t = tid; t < g.ni; t += nt) dir[(g.i0 + t) >> pshift] = 1;
+    __syncthreads();
+    int32_t pages = 0;
+    {
+      int32_t c = 0;
+      for (int w = tid * chunk; w < min((tid + 1) * chunk, (npages + 3) / 4); w++)
+        c += __popc(page_lds[w]);
+      int32_t p = group_exclusive(c, &pages, sh);
+      if ((pages << pshift) <= kPageBytes && c > 0)
+        for (int t = tid * chunk * 4; t < min((tid + 1) * chunk * 4, npages); t++)
+          if (dir[t]) {
+            page_of[p] = t;
+            dir[t] = static_cast<uint8_t>(p++);
+          }
+    }
+    if ((pages << pshift) > kPageBytes) {  // uniform over the workgroup
+      if (tid == 0) stats[b] = make_int4(0, 0, 0, 1);
+      __syncthreads();
+      continue;
+    }
+    const int nwords = (pages << pshift) / 16;
+    for (int t = tid; t < nwords * 4; t += nt) used[t] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kPageKeys; u++) {
+      key[u] = dir[key[u] >> pshift] << pshift | (key[u] & low);  // its byte from here on
+      mark[key[u]] = 1;
+    }
+    others([&](int32_t s, int32_t) { mark[dir[s >> pshift] << pshift | (s & low)] = 1; });
+    for (int t = tid; t < g.ni; t += nt) {
+      const int32_t s = g.i0 + t;
+      mark[dir[s >> pshift] << pshift | (s & low)] = 1;
+    }
+    __syncthreads();
+    int32_t ns = 0;
+    for (int w0 = 0; w0 < nwords; w0 += nt) {
+      const int w = w0 + tid;
+      uint32_t mask = 0;
+      if (w < nwords) {
+#pragma unroll
+        for (int q = 0; q < 4; q++)  // four bytes of 0 or 1 to four bits
+          mask |= ((used[4 * w + q] * 0x01020408u) >> 24 & 15u) << (4 * q);
+      }
+      int32_t n = 0;
+      const int32_t base = ns + group_exclusive(__popc(mask), &n, sh);
+      if (w < nwords) table[w] = mask | static_cast<uint32_t>(base) << 16;
+      ns += n;
+    }
+    __syncthreads();
+    const int64_t bytes = tile_lds_bytes(ns, g.ne);
+    const bool over = bytes > kTileLdsBudget;
+    if (tid == 0)
+      stats[b] = make_int4(ns, static_cast<int32_t>(std::min<int64_t>(bytes, INT32_MAX)), longest, 0);
+    if (over) {  // uniform; the caller retries smaller
+      __syncthreads();
+      continue;
+    }
+    const int64_t s0 = static_cast<int64_t>(b) * kTileMaxStage;
+    for (int t = tid; t < nwords * 16; t += nt) {
+      const uint32_t v = table[t >> 4], bit = t & 15;
+      if (!((v >> bit) & 1)) continue;
+      const int32_t slot = page_of[t >> pshift] << pshift | (t & low);
+      const int64_t d = s0 + (v >> 16) + __popc(v & ((1u << bit) - 1));
+      stage[d] = member ? member[slot] : slot;
+      if (stage_slot) stage_slot[d] = slot;
+    }
+    if (tid == 0) {
+      int32_t* d = desc + static_cast<int64_t>(b) * 8;
+      const int32_t mid = g.i0 + g.ni / 2;
+      d[0] = g.i0;
+      d[1] = g.ni;
+      d[2] = static_cast<int32_t>(s0);
+      d[3] = ns;
+      d[4] = static_cast<int32_t>(g.e0);
+      d[5] = g.ne;
+      d[6] = g.rid;
+      d[7] = member ? member[mid] : mid;  // middle particle: the periodic unwrap's reference
+    }
+    auto offset = [&](int32_t at) {
+      const uint32_t v = table[at >> 4];
+      return static_cast<uint16_t>(((v >> 16) + __popc(v & ((1u << (at & 15)) - 1))) * 24);
+    };
+#pragma unroll
+    for (int u = 0; u < kPageKeys; u++) {
+      const uint16_t v = offset(key[u]);
+      if (u * kPageLanes < mine) out[u * kPageLanes] = v;
+    }
+    others([&](int32_t s, int32_t e) { local[e] = offset(dir[s >> pshift] << pshift | (s & low)); });
+    __syncthreads();
+  }
+}
+
+// The bank-class order (bank_class_order) of rows in cutoff classes, for the
+// layouts that read `local` itself. One wavefront per tile, one row per
+// lane, each lane's buffers in LDS.
 constexpr int kBankBlock = 64;
-__global__ __launch_bounds__(kBankBlock) void k_bank_order(const int32_t* __restrict__ geo,
+__global__ __launch_bounds__(kBankBlock) void k_bank_order(const int32_t* __restrict__ desc,
                                                            int32_t nblocks,
                                                            const int32_t* __restrict__ slot_ptr,
-                                                           uint16_t* __restrict__ local,
-                                                           CutDev cut) {
+                                                           const int32_t* __restrict__ inner,
+                                                           uint16_t* __restrict__ local) {
   __shared__ uint16_t buf[kBankBlock][kBankRowMax];
   __shared__ uint16_t cnt[kBankBlock][kBankClasses];
   __shared__ uint16_t nxt[kBankBlock][kBankClasses];
   const int t = static_cast<int>(threadIdx.x);
-  const int64_t st = cut.q.stride;
   for (int32_t b = blockIdx.x; b < nblocks; b += gridDim.x) {
-    const int32_t i0 = geo[4 * b], ni = geo[4 * b + 1];
+    const int32_t i0 = desc[8 * static_cast<int64_t>(b)], ni = desc[8 * static_cast<int64_t>(b) + 1];
     for (int32_t r = t; r < ni; r += kBankBlock) {
       const int32_t a = slot_ptr[i0 + r];
       const int m = slot_ptr[i0 + r + 1] - a;
+      const int nin = inner ? inner[i0 + r] : m;
       uint16_t* row = local + a;
-      int nin = 0;
-      if (cut.q.x && m <= kBankRowMax) {
-        const int64_t i = cut.member ? cut.member[i0 + r] : i0 + r;
-        const double xi = cut.q.x[i * st], yi = cut.q.y[i * st], zi = cut.q.z[i * st];
-        const int32_t soff = cut.desc[8 * static_cast<int64_t>(b) + 2];
-        const double box = cut.rep_box ? cut.rep_box[2 * geo[4 * b + 2]] : cut.box;
-        int nout = 0;
-        for (int k = 0; k < m; k++) {
-          const uint16_t o = row[k];
-          const int64_t j = cut.stage[soff + o / 24];
-          if (cut_inner(xi, yi, zi, cut.q.x[j * st], cut.q.y[j * st], cut.q.z[j * st], box,
-                        cut.cl2))
-            row[nin++] = o;
-          else
-            buf[t][nout++] = o;
-        }
-        for (int k = 0; k < nout; k++) row[nin + k] = buf[t][k];
-      }
       bank_class_order(row, nin, r, 0, buf[t], cnt[t], nxt[t]);
       bank_class_order(row + nin, m - nin, r, nin, buf[t], cnt[t], nxt[t]);
     }
@@ -1196,41 +1336,232 @@ __global__ void k_wave_slices(const int32_t* __restrict__ desc, int32_t nblocks,
   len[id] = batches * 64 * unroll;
 }
 
-// The slices of one block per workgroup, written in order: slice position
-// p of wavefront w (batch j = p / (64 unroll), slot u, lane l) holds entry
-// k = j * lanes * unroll + u * lanes + l % lanes of the block's row
-// w * (64 / lanes) + l / lanes, or 0 past the row's end (padding). The
-// writes are contiguous; the reads gather short runs of `local` (the
-// block's rows, a few KB, served by the cache). Row starts and the block's
-// slice offsets come from LDS; lanes and unroll are powers of two, so the
-// position arithmetic is shifts and masks.
-__global__ __launch_bounds__(kBlock) void k_slice_gather(
-    const int32_t* __restrict__ desc, int32_t nblocks, int32_t wpb,
-    const int32_t* __restrict__ slot_ptr, const uint16_t* __restrict__ local, int32_t lanes,
-    int32_t unroll, const int32_t* __restrict__ wave_off, uint16_t* __restrict__ sliced) {
-  __shared__ int32_t rs[kTileRowsMax + 1];
-  __shared__ int32_t wo[kSliceWavesMax + 1];
-  const int32_t lsh = 31 - __clz(lanes), ush = 31 - __clz(unroll);
-  const int32_t bsh = 6 + ush;  // log2 of a batch's 64 * unroll positions
-  for (int32_t b = blockIdx.x; b < nblocks; b += gridDim.x) {
-    const int32_t i0 = desc[8 * static_cast<int64_t>(b)], ni = desc[8 * static_cast<int64_t>(b) + 1];
-    for (int32_t r = threadIdx.x; r <= ni; r += kBlock) rs[r] = slot_ptr[i0 + r];
-    for (int32_t w = threadIdx.x; w <= wpb; w += kBlock)
-      wo[w] = wave_off[static_cast<int64_t>(b) * wpb + w];
-    __syncthreads();
-    for (int32_t w = 0; w < wpb; w++) {
-      const int32_t p0 = wo[w], len = wo[w + 1] - p0;
-      const int32_t row0 = w << (6 - lsh);
-      for (int32_t off = threadIdx.x; off < len; off += kBlock) {
-        const int32_t j = off >> bsh, u = (off >> 6) & (unroll - 1), l = off & 63;
-        const int32_t row = row0 + (l >> lsh);
-        const int32_t k = (j << (lsh + ush)) + (u << lsh) + (l & (lanes - 1));
-        uint16_t v = 0;
-        if (row < ni && k < rs[row + 1] - rs[row]) v = local[rs[row] + k];
-        sliced[p0 + off] = v;
-      }
+// The places of one part of a row (its inner entries, or the others), by one
+// lane: n ranks in[0], in[step], ... take the places out[0 .. n), whose first
+// one has target class `phase`. cnt is this lane's column of the class counts
+// (kBankClasses words, kSliceRows apart). The q-th entry of a class takes the
+// q-th place that has the class as its target; the entries beyond those fill,
+// in order, the places whose class ran out. No entry waits for the one
+// before it, unlike bank_class_order's walk over the classes left, and a row
+// that runs out of a class leaves only that place to chance.
+__device__ __forceinline__ void slice_part(uint16_t* in, int step, uint16_t* out, uint32_t* cnt,
+                                           int phase, int n) {
+  constexpr int kB = 8;  // entries in flight
+#pragma unroll
+  for (int c = 0; c < kBankClasses; c++) cnt[c * kSliceRows] = 0;
+  int left = 0;
+  for (int k0 = 0; k0 < n; k0 += kB) {
+    int x[kB];
+    uint32_t q[kB];
+#pragma unroll
+    for (int u = 0; u < kB; u++) x[u] = in[min(k0 + u, n - 1) * step];
+#pragma unroll
+    for (int u = 0; u < kB; u++)
+      q[u] = atomicAdd(&cnt[(x[u] & (kBankClasses - 1)) * kSliceRows], k0 + u < n ? 1u : 0u);
+#pragma unroll
+    for (int u = 0; u < kB; u++) {
+      if (k0 + u >= n) continue;
+      const int d = ((x[u] - phase) & (kBankClasses - 1)) + kBankClasses * static_cast<int>(q[u]);
+      if (d < n) out[d] = static_cast<uint16_t>(x[u]);
+      else in[left++ * step] = static_cast<uint16_t>(x[u]);  // where it was read already
     }
-    __syncthreads();
+  }
+  int at = 0;
+  for (int k0 = 0; k0 < n; k0 += kB) {
+    uint32_t q[kB];
+    uint16_t x[kB];
+    bool hole[kB];
+#pragma unroll
+    for (int u = 0; u < kB; u++) q[u] = cnt[((phase + k0 + u) & (kBankClasses - 1)) * kSliceRows];
+#pragma unroll
+    for (int u = 0; u < kB; u++) {
+      hole[u] = k0 + u < n && static_cast<uint32_t>(k0 + u) / kBankClasses >= q[u];
+      x[u] = in[min(at, n - 1) * step];
+      at += hole[u] ? 1 : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < kB; u++)
+      if (hole[u]) out[k0 + u] = x[u];
+  }
+}
+
+struct CutDev {
+  PosIn q;
+  const int32_t* stage;
+  const int32_t* member;
+  double box;
+  const double* rep_box;
+  double cl2;
+};
+constexpr int kRowLanes = 8;  // lanes that read one row together
+constexpr int kRowBatch = 5;  // entries per lane in flight
+
+// The slices of one block per workgroup, rows in groups of `grows` (at most
+// kSliceRows, a multiple of a wavefront's rows): slice position p of
+// wavefront w (batch j = p / (64 unroll), slot u, lane l) holds place k = j
+// * lanes * unroll + u * lanes + l % lanes of the block's row w * (64 /
+// lanes) + l / lanes, or 0 past the row's end (padding).
+//   CUT first puts the rows in cutoff classes (cut_partition over cut_inner):
+// inner entries first, the others behind them, both in list order, in
+// `local` as well; inner[s] receives the inner count of slot s's row. The
+// partners' positions are staged in LDS (POS_LDS) or, where they do not fit,
+// read from memory.
+//   ORDER gives the places of each class out by slice_part, so that the 32
+// lanes that read LDS together mostly read different banks (the row's phase
+// is its first lane's place among them): one lane per row, all of a group in
+// one wavefront, on ranks in LDS, rows `stride` (an odd number of dwords)
+// apart, inner entries forward from the row's start, the others backward from
+// its end. At density 1 a half-wavefront's read then takes 2.3 passes over the
+// banks (modelled on the tiles of 119,164 particles) against 2.6 in the
+// bank-class order: FP64 forces 2.4 %, mixed 4 % faster.
+//   Rows of more than kBankRowMax entries, and all rows without ORDER, keep
+// the order of `local`.
+template <bool CUT, bool POS_LDS, bool ORDER>
+__global__ __launch_bounds__(512) void k_tile_slices(
+    const int32_t* __restrict__ desc, int32_t nblocks, const int32_t* __restrict__ slot_ptr,
+    int32_t* __restrict__ inner, uint16_t* __restrict__ local, CutDev cut, int32_t grows,
+    int32_t stride, int32_t lanes, int32_t wpb, const int32_t* __restrict__ wave_off,
+    uint16_t* __restrict__ sliced) {
+  extern __shared__ double slice_lds[];
+  __shared__ int32_t start[kSliceRows], len[kSliceRows], in_len[kSliceRows];
+  // The rows; then the staged positions, whose place the class counts and the
+  // ordered rows take afterwards.
+  uint16_t* in = reinterpret_cast<uint16_t*>(slice_lds);
+  double* pos = slice_lds + (grows * stride + 3) / 4;
+  uint32_t* cnt = reinterpret_cast<uint32_t*>(pos);
+  uint16_t* out = ORDER ? reinterpret_cast<uint16_t*>(cnt + kBankClasses * kSliceRows) : in;
+  const int tid = static_cast<int>(threadIdx.x), nt = static_cast<int>(blockDim.x);
+  const int lane = tid & (kRowLanes - 1), seg = (tid & 63) & ~(kRowLanes - 1);
+  const int lsh = 31 - __clz(lanes);
+  const int rpw = 64 >> lsh;  // rows per wavefront
+  const int64_t st = cut.q.stride;
+  for (int32_t b = blockIdx.x; b < nblocks; b += gridDim.x) {
+    const int32_t* d = desc + 8 * static_cast<int64_t>(b);
+    const int32_t i0 = d[0], ni = d[1], soff = d[2], ns = d[3];
+    double box = cut.box;
+    if (CUT && cut.rep_box) box = cut.rep_box[2 * d[6]];
+    for (int32_t g0 = 0; g0 < ni; g0 += grows) {
+      const int nr = min(grows, ni - g0);
+      if (tid < nr) {
+        const int32_t a = slot_ptr[i0 + g0 + tid];
+        const int32_t m = slot_ptr[i0 + g0 + tid + 1] - a;
+        start[tid] = a;
+        len[tid] = m;
+        in_len[tid] = !CUT && inner ? inner[i0 + g0 + tid] : m;
+      }
+      if (CUT && POS_LDS) {
+        for (int t = tid; t < ns; t += nt) {
+          const int64_t j = static_cast<int64_t>(cut.stage[soff + t]) * st;
+          pos[3 * t] = cut.q.x[j];
+          pos[3 * t + 1] = cut.q.y[j];
+          pos[3 * t + 2] = cut.q.z[j];
+        }
+      }
+      __syncthreads();
+      for (int r = tid / kRowLanes; r < nr; r += nt / kRowLanes) {
+        const int32_t a = start[r];
+        const int m = len[r];
+        if (m > kBankRowMax) {
+          if (CUT && lane == 0) inner[i0 + g0 + r] = m;
+          continue;
+        }
+        uint16_t* row = in + r * stride;
+        int nin = CUT ? 0 : in_len[r], nout = 0;
+        double xi = 0.0, yi = 0.0, zi = 0.0;
+        if (CUT) {
+          const int32_t slot = i0 + g0 + r;
+          const int64_t i = static_cast<int64_t>(cut.member ? cut.member[slot] : slot) * st;
+          xi = cut.q.x[i];
+          yi = cut.q.y[i];
+          zi = cut.q.z[i];
+        }
+        for (int k0 = 0; k0 < m; k0 += kRowBatch * kRowLanes) {
+          int rank[kRowBatch];
+#pragma unroll
+          for (int u = 0; u < kRowBatch; u++) {
+            const int k = k0 + u * kRowLanes + lane;
+            rank[u] = k < m ? local[a + k] / 24 : -1;
+          }
+          if (!CUT) {
+#pragma unroll
+            for (int u = 0; u < kRowBatch; u++) {
+              const int k = k0 + u * kRowLanes + lane;
+              if (rank[u] >= 0)
+                row[ORDER && k >= nin ? m - 1 - (k - nin) : k] = static_cast<uint16_t>(rank[u]);
+            }
+            continue;
+          }
+          bool in_u[kRowBatch];
+#pragma unroll
+          for (int u = 0; u < kRowBatch; u++) {
+            const int t = max(rank[u], 0);
+            double xj, yj, zj;
+            if (POS_LDS) {
+              xj = pos[3 * t];
+              yj = pos[3 * t + 1];
+              zj = pos[3 * t + 2];
+            } else {
+              const int64_t j = static_cast<int64_t>(cut.stage[soff + t]) * st;
+              xj = cut.q.x[j];
+              yj = cut.q.y[j];
+              zj = cut.q.z[j];
+            }
+            in_u[u] = cut_inner(xi, yi, zi, xj, yj, zj, box, cut.cl2);
+          }
+#pragma unroll
+          for (int u = 0; u < kRowBatch; u++) {
+            const bool valid = rank[u] >= 0;
+            constexpr uint32_t kSeg = (1u << kRowLanes) - 1;
+            const uint32_t vm = kSeg & static_cast<uint32_t>(__ballot(valid) >> seg);
+            const uint32_t im = kSeg & static_cast<uint32_t>(__ballot(valid && in_u[u]) >> seg);
+            const uint32_t below = (1u << lane) - 1;
+            if (valid)
+              row[in_u[u] ? nin + __popc(im & below) : m - 1 - nout - __popc(vm & ~im & below)] =
+                  static_cast<uint16_t>(rank[u]);
+            nin += __popc(im);
+            nout += __popc(vm & ~im);
+          }
+        }
+        if (CUT) {
+          if (lane == 0) {
+            inner[i0 + g0 + r] = nin;
+            in_len[r] = nin;
+          }
+          // The row goes back in its new order (its lanes belong to one
+          // wavefront, so their LDS writes come before these reads).
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          if (nout > 0)
+            for (int k = lane; k < m; k += kRowLanes)
+              local[a + k] = static_cast<uint16_t>(row[k < nin ? k : m - 1 - (k - nin)] * 24);
+        }
+      }
+      __syncthreads();
+      if (ORDER) {
+        if (tid < nr && len[tid] <= kBankRowMax) {
+          const int m = len[tid], nin = in_len[tid];
+          const int phase = (g0 + tid) << lsh;
+          uint16_t* row = in + tid * stride;
+          if (nin > 0) slice_part(row, 1, out + tid * stride, cnt + tid, phase, nin);
+          if (m > nin)
+            slice_part(row + m - 1, -1, out + tid * stride + nin, cnt + tid, phase + nin, m - nin);
+        }
+        __syncthreads();
+      }
+      for (int w = g0 / rpw + tid / 64; w < min(wpb, (g0 + grows) / rpw); w += nt / 64) {
+        const int32_t p0 = wave_off[static_cast<int64_t>(b) * wpb + w];
+        const int32_t n = wave_off[static_cast<int64_t>(b) * wpb + w + 1] - p0;
+        const int r = w * rpw + ((tid & 63) >> lsh) - g0;
+        const int m = r < nr ? len[r] : 0;
+        const bool direct = m > kBankRowMax;
+        const uint16_t* src = direct ? local + start[r] : out + min(r, grows - 1) * stride;
+        const int scale = direct ? 1 : 24;
+        int k = tid & (lanes - 1);
+#pragma unroll 4
+        for (int32_t p = tid & 63; p < n; p += 64, k += lanes)
+          sliced[p0 + p] = k < m ? static_cast<uint16_t>(src[k] * scale) : uint16_t{0};
+      }
+      __syncthreads();
+    }
   }
 }
 
@@ -1410,6 +1741,8 @@ void dev_release(DevTiles& t) {
   dev_release(t.member);
   dev_release(t.slot_ptr);
   dev_release(t.stage_slot);
+  dev_release(t.inner);
+  t.cut = t.bank_done = false;
   t.tile_particles = 0;
   t.blocks = 0;
   t.staged = 0;
@@ -1419,7 +1752,7 @@ void dev_release(DevTiles& t) {
 
 void dev_release(ListWork& w) {
   for (DevMem* m : {&w.scan_sums, &w.small, &w.cell_count, &w.cell_start, &w.cell_slot, &w.cell_of,
-                    &w.cell_sorted, &w.cpos, &w.counts, &w.tmp, &w.tile_ns, &w.tile_soff,
+                    &w.cell_sorted, &w.cpos, &w.counts, &w.tmp, &w.tile_ns, &w.tile_soff, &w.tile_stats,
                     &w.tile_geo, &w.rep_of, &w.order, &w.order_grid, &w.slot_of})
     dev_release(*m);
   dev_release(w.part);
@@ -1835,8 +2168,7 @@ int dev_length_sort(hipStream_t s, const DevCSR& c, int32_t T, const std::vector
 }
 
 int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<int32_t>& reps,
-                   const int32_t* member, bool bank_order, const CutHint* cut, ListWork& w,
-                   DevTiles& out) {
+                   const int32_t* member, ListWork& w, DevTiles& out) {
   out.tile_particles = 0;
   out.blocks = 0;
   if (T <= 0 || T > kTileRowsMax || c.n <= 0) return LJGPU_OK;
@@ -1881,10 +2213,8 @@ int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<
                       hipMemcpyHostToDevice, s), "hipMemcpyAsync");
   const int32_t* dgeo = w.tile_geo.as<int32_t>();
   LCHECK(dev_reserve(w.small, sizeof(int64_t) * 8, s));
-  int32_t* stats = w.small.as<int32_t>() + 4;
-  unsigned long long* staged_dev = w.small.as<unsigned long long>() + 4;
-  LCHECK(fill<int32_t>(s, stats, 3, 0));
-  LCHECK(fill<unsigned long long>(s, staged_dev, 1, 0ull));
+  LCHECK(dev_reserve(w.tile_stats, sizeof(int4) * static_cast<size_t>(nb), s));
+  int4* stats = w.tile_stats.as<int4>();
   const int grid = std::min(nb, 65535);
   // The force kernel copies entry offsets in whole 16-byte chunks: pad.
   const int64_t nlocal = c.e + kTileLocalPad;
@@ -1898,31 +2228,60 @@ int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<
       slots * static_cast<int64_t>(sizeof(int32_t)) * (member ? 2 : 1) <= kTileOnePassBytes &&
       slots <= INT32_MAX;
   int64_t staged = 0;
-  int32_t h[3];
+  int32_t h[4];
+  // Sixteen lanes to a row, all rows of a tile of 64 at once; entry codes in
+  // LDS for tiles up to a quarter longer than the average row makes them.
+  const int threads = std::min(1024, std::max(256, T * kWordLanes));
+  const int32_t ecap = static_cast<int32_t>(std::min<int64_t>(
+      kTileCodeMax, (c.e / c.n + 1) * T * 5 / 4 + 64));
+  const size_t code_bytes = sizeof(uint16_t) * ecap;
+  auto read_stats = [&](int32_t (&back)[8]) -> int {
+    k_tile_stats<<<1, 1024, 0, s>>>(nb, stats, w.small.as<int32_t>());
+    LTRY(hipGetLastError(), "tile stats kernel");
+    LTRY(hipMemcpyAsync(back, w.small.p, sizeof(back), hipMemcpyDeviceToHost, s), "hipMemcpyAsync");
+    LTRY(hipStreamSynchronize(s), "hipStreamSynchronize");
+    return LJGPU_OK;
+  };
   if (one_pass) {
     LCHECK(dev_reserve(out.stage, sizeof(int32_t) * slots, s));
     if (member) LCHECK(dev_reserve(out.stage_slot, sizeof(int32_t) * slots, s));
-    k_tile_fill<<<grid, kBlock, 0, s>>>(dgeo, nb, mem, slot_of, sptr, c.ptr.as<int32_t>(),
-                                        c.list.as<int32_t>(), nullptr, out.desc.as<int32_t>(),
-                                        out.stage.as<int32_t>(),
-                                        member ? out.stage_slot.as<int32_t>() : nullptr,
-                                        out.local.as<uint16_t>(), stats, staged_dev);
-    LTRY(hipGetLastError(), "tile fill kernel");
+    // Pages of 128 slots or more, so that the directory of a large system
+    // fits LDS too.
+    int32_t pshift = 7;
+    while ((c.n >> pshift) >= kPageDir) pshift++;
+    const int32_t npages = (c.n >> pshift) + 1;
     unsigned long long st = 0;
-    LTRY(hipMemcpyAsync(h, stats, sizeof(h), hipMemcpyDeviceToHost, s), "hipMemcpyAsync");
-    LTRY(hipMemcpyAsync(&st, staged_dev, sizeof(st), hipMemcpyDeviceToHost, s), "hipMemcpyAsync");
-    LTRY(hipStreamSynchronize(s), "hipStreamSynchronize");
+    for (int pass = 0; pass < 2; pass++) {
+      if (pass == 0)
+        k_tile_pages<<<grid, std::min(512, std::max(256, T * kPageLanes)), (npages + 15) / 16 * 16, s>>>(
+            dgeo, nb, mem, slot_of, sptr, c.ptr.as<int32_t>(), c.list.as<int32_t>(), pshift,
+            npages, out.desc.as<int32_t>(), out.stage.as<int32_t>(),
+            member ? out.stage_slot.as<int32_t>() : nullptr, out.local.as<uint16_t>(), stats);
+      else
+        k_tile_fill<false><<<grid, threads, code_bytes, s>>>(
+            dgeo, nb, mem, slot_of, sptr, c.ptr.as<int32_t>(), c.list.as<int32_t>(), nullptr, ecap,
+            nullptr, out.desc.as<int32_t>(), out.stage.as<int32_t>(),
+            member ? out.stage_slot.as<int32_t>() : nullptr, out.local.as<uint16_t>(), stats);
+      LTRY(hipGetLastError(), "tile fill kernel");
+      int32_t back[8];
+      LCHECK(read_stats(back));
+      std::copy(back, back + 4, h);
+      std::memcpy(&st, back + 6, sizeof(st));
+      if (back[4] == 0) break;  // else partners over too many pages: the hashed set
+    }
     if (h[0] != 0) return LJGPU_OK;  // does not fit: caller retries smaller or runs untiled
     staged = static_cast<int64_t>(st);
     out.stage_stride = kTileMaxStage;
   } else {
     LCHECK(dev_reserve(w.tile_ns, sizeof(int32_t) * (static_cast<size_t>(nb) + 1), s));
     LCHECK(dev_reserve(w.tile_soff, sizeof(int32_t) * (static_cast<size_t>(nb) + 1), s));
-    k_tile_count<<<grid, kBlock, 0, s>>>(dgeo, nb, mem, slot_of, sptr, c.ptr.as<int32_t>(),
-                                         c.list.as<int32_t>(), w.tile_ns.as<int32_t>(), stats);
+    k_tile_fill<true><<<grid, threads, 0, s>>>(
+        dgeo, nb, mem, slot_of, sptr, c.ptr.as<int32_t>(), c.list.as<int32_t>(), nullptr, 0,
+        w.tile_ns.as<int32_t>(), nullptr, nullptr, nullptr, nullptr, stats);
     LTRY(hipGetLastError(), "tile count kernel");
-    LTRY(hipMemcpyAsync(h, stats, sizeof(h), hipMemcpyDeviceToHost, s), "hipMemcpyAsync");
-    LTRY(hipStreamSynchronize(s), "hipStreamSynchronize");
+    int32_t back[8];
+    LCHECK(read_stats(back));
+    std::copy(back, back + 4, h);
     if (h[0] != 0) return LJGPU_OK;  // does not fit: caller retries smaller or runs untiled
     LCHECK(dev_scan(s, w.tile_ns.as<int32_t>(), w.tile_soff.as<int32_t>(), nb, w, &staged));
     if (staged > INT32_MAX) return LJGPU_OK;
@@ -1931,28 +2290,17 @@ int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<
     // positions and momenta in slot order.
     if (member)
       LCHECK(dev_reserve(out.stage_slot, sizeof(int32_t) * std::max<int64_t>(staged, 1), s));
-    k_tile_fill<<<grid, kBlock, 0, s>>>(dgeo, nb, mem, slot_of, sptr, c.ptr.as<int32_t>(),
-                                        c.list.as<int32_t>(), w.tile_soff.as<int32_t>(),
-                                        out.desc.as<int32_t>(), out.stage.as<int32_t>(),
-                                        member ? out.stage_slot.as<int32_t>() : nullptr,
-                                        out.local.as<uint16_t>(), stats, staged_dev);
+    k_tile_fill<false><<<grid, threads, code_bytes, s>>>(
+        dgeo, nb, mem, slot_of, sptr, c.ptr.as<int32_t>(), c.list.as<int32_t>(),
+        w.tile_soff.as<int32_t>(), ecap, nullptr, out.desc.as<int32_t>(),
+        out.stage.as<int32_t>(), member ? out.stage_slot.as<int32_t>() : nullptr,
+        out.local.as<uint16_t>(), stats);
     LTRY(hipGetLastError(), "tile fill kernel");
     out.stage_stride = 0;
   }
-  if (bank_order) {
-    CutDev cd{};
-    if (cut && cut->q.x) {
-      cd.q = cut->q;
-      cd.desc = out.desc.as<int32_t>();
-      cd.stage = out.stage.as<int32_t>();
-      cd.member = mem;
-      cd.box = cut->box;
-      cd.rep_box = reps.empty() ? nullptr : cut->rep_box;
-      cd.cl2 = cut->cl2;
-    }
-    k_bank_order<<<grid, kBankBlock, 0, s>>>(dgeo, nb, sptr, out.local.as<uint16_t>(), cd);
-    LTRY(hipGetLastError(), "tile bank order kernel");
-  }
+  out.cut = false;
+  out.bank_done = false;
+  out.longest = h[3];
   out.tile_particles = T;
   out.blocks = nb;
   out.staged = staged;
@@ -1962,7 +2310,7 @@ int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<
 }
 
 int dev_slice_tiles(hipStream_t s, const int32_t* slot_ptr, int32_t lanes, int32_t unroll,
-                    ListWork& w, DevTiles& t) {
+                    bool bank_order, int32_t n, const CutHint* hint, ListWork& w, DevTiles& t) {
   t.sliced_lanes = t.sliced_unroll = t.waves_per_block = 0;
   if (t.blocks <= 0 || lanes < 1 || lanes > 64 || (64 % lanes) != 0 || unroll < 1 ||
       (unroll & (unroll - 1)) != 0)
@@ -1983,13 +2331,51 @@ int dev_slice_tiles(hipStream_t s, const int32_t* slot_ptr, int32_t lanes, int32
   if (total + pad > INT32_MAX) return LJGPU_OK;
   LCHECK(dev_reserve(t.sliced, sizeof(uint16_t) * (total + pad), s));
   LCHECK(fill<uint16_t>(s, t.sliced.as<uint16_t>() + total, pad, 0));
-  k_slice_gather<<<std::min(t.blocks, 65535), kBlock, 0, s>>>(
-      t.desc.as<int32_t>(), t.blocks, wpb, slot_ptr, t.local.as<uint16_t>(), lanes, unroll,
-      t.wave_off.as<int32_t>(), t.sliced.as<uint16_t>());
-  LTRY(hipGetLastError(), "slice gather kernel");
+  CutDev cd{};
+  const bool cut = bank_order && hint && hint->q.x && !t.cut;
+  if (cut) {
+    cd.q = hint->q;
+    cd.stage = t.stage.as<int32_t>();
+    cd.member = t.order == LJGPU_TILE_ORDER_SPATIAL ? t.member.as<int32_t>() : nullptr;
+    cd.box = hint->box;
+    cd.rep_box = hint->rep_box;
+    cd.cl2 = hint->cl2;
+    LCHECK(dev_reserve(t.inner, sizeof(int32_t) * n, s));
+  }
+  // Rows an odd number of dwords apart, so that lanes walking one row each
+  // read different banks; fewer rows at a time where long ones would not fit.
+  const int32_t longest = std::min(std::max(t.longest, 2), kBankRowMax);
+  const int32_t stride = 2 * ((longest + 1) / 2 | 1);
+  int32_t grows = kSliceRows;
+  size_t rows = 0, order = 0;
+  for (;; grows /= 2) {
+    rows = (sizeof(uint16_t) * stride * grows + 7) / 8 * 8;
+    order = bank_order ? rows + sizeof(uint32_t) * kBankClasses * kSliceRows : 0;
+    if (grows == kSliceRows / 2 || rows + order <= kTileLdsMax) break;
+  }
+  const size_t pos = cut ? sizeof(double) * 3 * static_cast<size_t>(t.max_stage) : 0;
+  const bool pos_lds = rows + pos <= kTileLdsMax;
+  auto kernel = !bank_order ? k_tile_slices<false, false, false>
+                : !cut      ? k_tile_slices<false, false, true>
+                : pos_lds   ? k_tile_slices<true, true, true>
+                            : k_tile_slices<true, false, true>;
+  kernel<<<std::min(t.blocks, 65535), 512, rows + std::max(order, pos_lds ? pos : 0), s>>>(
+      t.desc.as<int32_t>(), t.blocks, slot_ptr,
+      t.cut || cut ? t.inner.as<int32_t>() : nullptr, t.local.as<uint16_t>(), cd, grows, stride,
+      lanes, wpb, t.wave_off.as<int32_t>(), t.sliced.as<uint16_t>());
+  LTRY(hipGetLastError(), "tile slice kernel");
+  if (cut) t.cut = true;
   t.sliced_lanes = lanes;
   t.sliced_unroll = unroll;
   t.waves_per_block = wpb;
+  return LJGPU_OK;
+}
+
+int dev_bank_order(hipStream_t s, const int32_t* slot_ptr, const DevTiles& t, uint16_t* local) {
+  if (t.blocks <= 0 || t.bank_done) return LJGPU_OK;
+  k_bank_order<<<std::min(t.blocks, 65535), kBankBlock, 0, s>>>(
+      t.desc.as<int32_t>(), t.blocks, slot_ptr, t.cut ? t.inner.as<int32_t>() : nullptr, local);
+  LTRY(hipGetLastError(), "tile bank order kernel");
   return LJGPU_OK;
 }
 

@@ -1,0 +1,85 @@
+"""The device tile builder at the sizes where it branches: tiles of one to
+128 particles with a ragged last one, rows longer than the 256 entries that
+are put in order, partners spread over the whole system (the hashed set) or
+in a few runs of slots (the paged one), rows of very different lengths, open
+and periodic boxes. The tiles must equal the host model's (ljgpu_make_tiles_*)
+and the forces over them, whose entry order is the slices' own, the oracle's.
+"""
+import functools
+
+import numpy as np
+import pytest
+
+import lj_gpu_amd as G
+import oracle as O
+from helpers import FP64_TOL, normwise
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    if G.device_count() < 1:
+        pytest.skip("no HIP device")
+    c = G.Context(0)
+    yield c
+    c.close()
+
+
+@functools.lru_cache(maxsize=None)
+def system(name):
+    """(q, box, full list, oracle force)."""
+    rng = np.random.default_rng(5)
+    if name == "ragged":        # vacancies, shuffled: N = 859
+        q, box = G.lattice_periodic(6, 1.0, 3)
+        q = q[rng.permutation(q.shape[0])[:-5]]
+    elif name == "long_rows":   # about 300 partners: rows past the order's limit
+        q, box = G.lattice_periodic(6, 2.0, 3)
+    elif name == "mixed_rows":  # rows of about 140 to 310 entries in one box
+        q, box = G.lattice_periodic(8, 2.0, 3)
+        keep = (q[:, 0] < 0.5 * box) | (rng.random(q.shape[0]) < 0.4)
+        q = q[keep]
+    elif name == "scattered":   # open box in a shuffled index order
+        q, box = G.lattice_reference(1.0, 22.0), 0.0
+        q = q[rng.permutation(q.shape[0])]
+    else:                       # open box in lattice order
+        assert name == "open"
+        q, box = G.lattice_reference(0.5, 22.0), 0.0
+    q = np.ascontiguousarray(q)
+    full = G.makepair(q, box, G.LIST_FULL)
+    f = np.zeros_like(q)
+    O.force_aos(O.CSR(full.number_of_partners, full.pointer, full.sorted_list, "full"), q, f, 1.0,
+                O.CL2, box, steps=1, method="full")
+    return q, box, full, f
+
+
+@pytest.mark.parametrize("name", ["ragged", "long_rows", "mixed_rows", "scattered", "open"])
+@pytest.mark.parametrize("lanes,unroll,tile", [(4, 4, 64), (4, 2, 48), (4, 4, 1), (2, 1, 128),
+                                               (8, 2, 32), (64, 1, 16)])
+def test_built_tiles_and_their_forces(ctx, name, lanes, unroll, tile):
+    q, box, full, f = system(name)
+    print(f"{name} lanes={lanes} unroll={unroll} tile={tile}", flush=True)
+    ctx.set_kernel_config(lanes, 256, unroll)
+    ctx.set_tiling(tile)
+    ctx.set_half_mode(G.HALF_AUTO)
+    dq, dp = ctx.array(q), ctx.zeros(q.shape)
+    ctx.build_list(dq, q.shape[0], box, G.LIST_FULL)
+    for steps in (1, 20):
+        dp.zero()
+        ctx.force_aos_f64(dq, dp, 1.0 / steps, G.CL2, box, steps)
+        ctx.sync()
+        assert normwise(dp.download(), f) < FP64_TOL
+    t = ctx.get_tiles()
+    used = ctx.list_info().tile_particles
+    order, member = ctx.get_tile_order()
+    assert order == (G.TILE_ORDER_SPATIAL if box > 0 else G.TILE_ORDER_INDEX)
+    h = G.make_tiles(full, used, member=member, q=q, box=box, cl2=G.CL2)
+    if np.all(h.desc[:-1, 1] == used):
+        np.testing.assert_array_equal(t.desc, h.desc)
+        np.testing.assert_array_equal(t.stage, h.stage)
+        np.testing.assert_array_equal(t.local, h.local)
+    # Inspection left the evaluated layout as it was.
+    dp.zero()
+    ctx.force_aos_f64(dq, dp, 1.0, G.CL2, box, 1)
+    ctx.sync()
+    assert normwise(dp.download(), f) < FP64_TOL
