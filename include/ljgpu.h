@@ -67,8 +67,10 @@ extern "C" {
 #define LJGPU_HALF_AUTO 0       /* library choice (autotuned)               */
 #define LJGPU_HALF_ATOMIC 1     /* scatter to j with FP64 atomics, like the
                                    reference's *_with_aar kernels
-                                   (cuda/kernel.cuh:238-469); summation
-                                   order is not deterministic               */
+                                   (cuda/kernel.cuh:238-469), in LDS over
+                                   tiles that share partners, in memory
+                                   otherwise; summation order is not
+                                   deterministic                            */
 #define LJGPU_HALF_EXPAND 2     /* expand to the full list once at
                                    set-list time; deterministic             */
 
@@ -199,8 +201,9 @@ int ljgpu_set_kernel_config(ljgpu_ctx* ctx, int lanes_per_particle, int block_si
  * LDS offset. The particles of a block are consecutive in the order chosen
  * by ljgpu_set_tile_order. 0 turns tiling off (global-gather
  * kernels). The tile actually used is capped at 1024 / lanes_per_particle
- * particles (one workgroup per tile); ELL lists and half lists evaluated
- * with atomics are never tiled. stage_offsets = 1 also stages each tile's
+ * particles (one workgroup per tile); ELL lists are never tiled, and the
+ * tiles of half lists evaluated with atomics are internal (reported as
+ * untiled). stage_offsets = 1 also stages each tile's
  * entry offsets in LDS (more LDS per workgroup); 0 streams them from HBM.
  * resident_per_cu > 0 launches a persistent grid of that many workgroups per
  * compute unit, each looping over tiles; 0 launches one workgroup per tile.

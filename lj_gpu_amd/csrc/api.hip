@@ -112,7 +112,7 @@ int ensure_ell(ljgpu_ctx* ctx) {
 // order. A tiling derived without positions is derived again, once, when
 // positions first come.
 int ensure_tiles(ljgpu_ctx* ctx, const PosIn* q, double box) {
-  const int32_t want = ctx->eval_half ? 0 : effective_tile(ctx);
+  const int32_t want = ctx->eval_half && !ctx->rep_off.empty() ? 0 : effective_tile(ctx);
   const bool spatial = ctx->tile_order == LJGPU_TILE_ORDER_SPATIAL && want > 0;
   if (want == ctx->tiles_for && (ctx->tiles_ordered || !q || want == 0)) return LJGPU_OK;
   ctx->tiles.tile_particles = 0;
@@ -126,8 +126,15 @@ int ensure_tiles(ljgpu_ctx* ctx, const PosIn* q, double box) {
   const int32_t* member = ordered ? ctx->work.order.as<int32_t>() : nullptr;
   for (int32_t tp = want; tp >= 1 && ctx->eval.n > 0; tp /= 2) {
     TRY(dev_make_tiles(ctx->stream, ctx->eval, tp, ctx->rep_off, member, ctx->work, ctx->tiles));
-    if (ctx->tiles.tile_particles > 0) break;
+    if (ctx->tiles.tile_particles == 0) continue;
+    if (!ctx->eval_half || ctx->tiles.max_stage <= kHalfMaxStage) break;
+    ctx->tiles.tile_particles = ctx->tiles.blocks = 0;
   }
+  // A half list's tile writes a force sum per staged partner. Where partners
+  // are hardly shared (scattered particles of an open box) there are nearly
+  // as many as pairs, and the untiled kernel stays.
+  if (ctx->eval_half && 2 * ctx->tiles.staged > ctx->eval.e)
+    ctx->tiles.tile_particles = ctx->tiles.blocks = 0;
   // The slot-order copies that calls of kSlotMinSteps or more steps run over
   // are reserved with the tiles, so a force call never allocates.
   if (ctx->tiles.blocks > 0 && ctx->tiles.order == LJGPU_TILE_ORDER_SPATIAL &&
@@ -151,8 +158,9 @@ const int32_t* tile_row_starts(const ljgpu_ctx* ctx) {
 // a new tiling comes with.
 int ensure_sliced(ljgpu_ctx* ctx, const PosIn* q, double box, double cl2) {
   DevTiles& t = ctx->tiles;
-  if (t.blocks <= 0 || (t.sliced_lanes == ctx->lanes && t.sliced_unroll == ctx->unroll))
-    return LJGPU_OK;
+  const int lanes = ctx->eval_half ? kHalfLanes : ctx->lanes;
+  const int unroll = ctx->eval_half ? 4 : ctx->unroll;
+  if (t.blocks <= 0 || (t.sliced_lanes == lanes && t.sliced_unroll == unroll)) return LJGPU_OK;
   CutHint cut;
   if (q) {
     cut.q = *q;
@@ -160,8 +168,13 @@ int ensure_sliced(ljgpu_ctx* ctx, const PosIn* q, double box, double cl2) {
     cut.rep_box = ctx->rep_off.empty() ? nullptr : ctx->rep_box_dev.as<double>();
     cut.cl2 = cl2;
   }
-  return dev_slice_tiles(ctx->stream, tile_row_starts(ctx), ctx->lanes, ctx->unroll,
-                         ctx->bank_order && !t.bank_done, ctx->eval.n, &cut, ctx->work, t);
+  TRY(dev_slice_tiles(ctx->stream, tile_row_starts(ctx), lanes, unroll,
+                      ctx->eval_half ? kHalfStride : 24, ctx->bank_order && !t.bank_done,
+                      ctx->eval.n, &cut, ctx->work, t));
+  if (!ctx->eval_half) return LJGPU_OK;
+  // The half-list kernel reads the slices only.
+  if (t.sliced_lanes == 0) t.tile_particles = t.blocks = 0;
+  return dev_half_tiles(ctx->stream, ctx->eval.n, ctx->work, t);
 }
 
 // The bank-class order of the tiles' rows in `local`, for the kernels that
@@ -178,6 +191,7 @@ int prepare_layouts(ljgpu_ctx* ctx, const PosIn* q, double box, double cl2) {
   if (ctx->lanes == 1) return ensure_ell(ctx);
   TRY(ensure_tiles(ctx, q, box));
   TRY(ensure_sliced(ctx, q, box, cl2));
+  if (ctx->eval_half) return LJGPU_OK;
   return ctx->tile_offsets_lds || ctx->tiles.sliced_lanes == 0 ? ensure_bank_order(ctx) : LJGPU_OK;
 }
 
@@ -358,7 +372,7 @@ int force_view(ljgpu_ctx* ctx, const ForceArgs& fa, ListView* lv, LaunchConfig* 
     lv->ell_width = ctx->ell_width;
   } else {
     lv->list = ctx->eval.list.as<int32_t>();
-    if (ctx->tiles.blocks > 0 && !ctx->eval_half) tile_fields(ctx, lv);
+    if (ctx->tiles.blocks > 0) tile_fields(ctx, lv);
   }
   return LJGPU_OK;
 }
@@ -379,6 +393,12 @@ void tile_fields(const ljgpu_ctx* ctx, ListView* lv) {
     lv->tile_waves_per_block = ctx->tiles.waves_per_block;
     lv->tile_sliced_lanes = ctx->tiles.sliced_lanes;
     lv->tile_sliced_unroll = ctx->tiles.sliced_unroll;
+  }
+  if (ctx->eval_half) {
+    lv->half_tile = ctx->tiles.half_tile.as<int32_t>();
+    lv->half_first = ctx->tiles.half_first.as<int32_t>();
+    lv->half_at = ctx->tiles.half_at.as<int32_t>();
+    lv->half_part = ctx->tiles.half_part.as<double>();
   }
   if (ctx->tiles.order == LJGPU_TILE_ORDER_SPATIAL) {
     lv->tile_member = ctx->tiles.member.as<int32_t>();
@@ -473,6 +493,10 @@ StepKey step_key(const ForceArgs& fa, const ListView& lv, const LaunchConfig& lc
   k.add(lv.tile_waves_per_block);
   k.add(lv.tile_sliced_lanes);
   k.add(lv.tile_sliced_unroll);
+  k.add(lv.half_tile);
+  k.add(lv.half_first);
+  k.add(lv.half_at);
+  k.add(lv.half_part);
   k.add(lv.replica_box);
   k.add(lc.lanes);
   k.add(lc.unroll);
@@ -662,8 +686,11 @@ int run_steps(ljgpu_ctx* ctx, const ForceArgs& caller, int32_t steps, bool mixed
   // Over enough tiles, the tiles in `chains` contiguous parts, each a chain
   // of launches on its own stream, forked from and joined back into the
   // context stream (see kMaxChains).
-  const int chains =
-      (lv.tile_blocks >= kMinChainTiles * ctx->chains && steps >= kGraphMinSteps) ? ctx->chains : 1;
+  // Tiles of a half list share particles, so they form one chain.
+  const int chains = (lv.tile_blocks >= kMinChainTiles * ctx->chains && steps >= kGraphMinSteps &&
+                      !lc.half_atomic)
+                         ? ctx->chains
+                         : 1;
   if (chains > 1) {
     HIP_TRY(hipEventRecord(ctx->ev_fork, ctx->stream), "hipEventRecord");
     ListView part[kMaxChains];

@@ -648,6 +648,159 @@ k_tile(P pos, M mom, const int32_t* __restrict__ nop, const int32_t* __restrict_
   }
 }
 
+// Half lists over tiles: every pair once, -f to its partner j. As in k_tile a
+// workgroup stages its tile's partners in LDS, here kHalfStride bytes each:
+// the position, then the sum of the tile's forces on that particle, to which
+// rows add with LDS atomics (the rows' own sums included: a tile's own
+// particles are staged, in slot order, from half_tile[b].y on). The sums leave
+// as half_tile[b].x ... of `part`, three doubles each, and k_half_gather adds
+// each particle's sums (about seven at density 0.8) to its momentum. Memory
+// atomics run at about 30 to 50 G/s here: at 62,463 particles (density 0.8)
+// one per pair and component took 267 us a launch, one per staged partner and
+// component 35 us, the sums and their gather 29 us (21 of them bound by the LDS
+// atomics). The stride of 14 dwords keeps the 32 bank classes of the 24-byte
+// one. Four lanes per row, offsets from the slices (kHalfStride * rank, in
+// batches of 4 * kHalfUnroll entries). LDS sums come in no fixed order.
+constexpr int kHalfUnroll = 4;
+
+template <int PREC, class P, bool PBC>
+__global__ void __launch_bounds__(1024)
+k_tile_half(P pos, const int32_t* __restrict__ member,
+            const int32_t* __restrict__ slot_ptr, const int4* __restrict__ desc,
+            const int32_t* __restrict__ stage, const uint16_t* __restrict__ sliced,
+            const int32_t* __restrict__ wave_off, int32_t wpb, const int2* __restrict__ half_tile,
+            double* __restrict__ part, int32_t nblocks, PairParams pp, double reach) {
+  constexpr int TPI = kHalfLanes, U = kHalfUnroll;
+  extern __shared__ double lds[];
+  int* flag = reinterpret_cast<int*>(lds);
+  double* cell = lds + kTileLdsHeader / 8;
+  const int tid = static_cast<int>(threadIdx.x), nt = static_cast<int>(blockDim.x);
+  if (tid == 0) *flag = 0;
+  __syncthreads();
+  const int per = (nblocks + kXcds - 1) / kXcds;
+  const int b = static_cast<int>(blockIdx.x) % kXcds * per + static_cast<int>(blockIdx.x) / kXcds;
+  if (static_cast<int>(blockIdx.x) / kXcds >= per || b >= nblocks) return;
+  const int4 d0 = desc[2 * b];
+  const int4 d1 = desc[2 * b + 1];
+  const int i0 = d0.x, ni = d0.y, soff = d0.z, ns = d0.w;
+  double cx = 0.0, cy = 0.0, cz = 0.0;
+  if constexpr (PBC) pos.ld(member ? d1.w : i0 + ni / 2, cx, cy, cz);
+  const int seg = tid / TPI, sub = tid & (TPI - 1);
+  const bool active = seg < ni;
+  const int slot = i0 + (active ? seg : 0);
+  const int i = member ? member[slot] : slot;
+  const int np = active ? slot_ptr[slot + 1] - slot_ptr[slot] : 0;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const uint16_t* row = sliced + wave_off[static_cast<int64_t>(b) * wpb + wave] + (tid & 63);
+  double xi, yi, zi;
+  pos.ld(i, xi, yi, zi);
+  uint32_t o[U];
+#pragma unroll
+  for (int u = 0; u < U; u++) o[u] = row[64 * u];
+  for (int t = tid; t < ns; t += nt) {
+    double x, y, z;
+    pos.ld(stage[soff + t], x, y, z);
+    unwrap_near<PBC>(x, y, z, cx, cy, cz, pp);
+    double* c = cell + kHalfStride / 8 * t;
+    c[0] = x;
+    c[1] = y;
+    c[2] = z;
+    c[3] = c[4] = c[5] = 0.0;
+  }
+  if constexpr (PBC) {
+    unwrap_near<PBC>(xi, yi, zi, cx, cy, cz, pp);
+    if (active && (fabs(xi - cx) >= reach || fabs(yi - cy) >= reach || fabs(zi - cz) >= reach))
+      *flag = 1;
+  }
+  __syncthreads();
+  const bool any_far = PBC && *flag != 0;
+  Accum<PREC> acc;
+  char* base = reinterpret_cast<char*>(cell);
+  for (int k0 = 0; k0 < np; k0 += TPI * U) {
+    double dx[U], dy[U], dz[U];
+    uint32_t at[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      at[u] = o[u];
+      const double* c = reinterpret_cast<const double*>(base + at[u]);
+      dx[u] = c[0] - xi;
+      dy[u] = c[1] - yi;
+      dz[u] = c[2] - zi;
+    }
+    row += 64 * U;
+    // The next batch (the slices are padded past their ends).
+#pragma unroll
+    for (int u = 0; u < U; u++) o[u] = row[64 * u];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (PBC && any_far) min_image<PBC>(dx[u], dy[u], dz[u], pp);
+      const double r2 = fma(dz[u], dz[u], fma(dy[u], dy[u], dx[u] * dx[u]));
+      // Places past the row's end read its tile's first partner.
+      if (k0 + u * TPI + sub >= np || r2 > pp.cl2) continue;
+      double df;
+      float dff = 0.0f;
+      if constexpr (PREC == kF64) {
+        df = lj_df_f64(r2, pp);
+      } else {
+        dff = lj_df_mixed(r2, pp);
+        df = static_cast<double>(dff);
+      }
+      acc.add(df, dff, dx[u], dy[u], dz[u]);
+      double* f = reinterpret_cast<double*>(base + at[u]) + 3;
+      unsafeAtomicAdd(f, -df * dx[u]);
+      unsafeAtomicAdd(f + 1, -df * dy[u]);
+      unsafeAtomicAdd(f + 2, -df * dz[u]);
+    }
+  }
+  const double fx = segment_sum<TPI>(acc.vx());
+  const double fy = segment_sum<TPI>(acc.vy());
+  const double fz = segment_sum<TPI>(acc.vz());
+  const int2 ht = half_tile[b];
+  if (active && sub == 0) {
+    double* f = cell + kHalfStride / 8 * (ht.y + seg) + 3;
+    unsafeAtomicAdd(f, fx);
+    unsafeAtomicAdd(f + 1, fy);
+    unsafeAtomicAdd(f + 2, fz);
+  }
+  __syncthreads();
+  double* out = part + 3 * static_cast<int64_t>(ht.x);
+  for (int t = tid; t < 3 * ns; t += nt) {
+    const int j = t / 3;
+    out[t] = cell[kHalfStride / 8 * j + 3 + t - 3 * j];
+  }
+}
+
+// Each particle's force sums (rows at[first[s]], ... of part, slot s) onto its
+// momentum.
+template <class M>
+__global__ void __launch_bounds__(256)
+k_half_gather(M mom, int32_t n, const int32_t* __restrict__ member,
+              const int32_t* __restrict__ first, const int32_t* __restrict__ at,
+              const double* __restrict__ part) {
+  const int s = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
+  if (s >= n) return;
+  constexpr int kB = 4;
+  double x = 0.0, y = 0.0, z = 0.0;
+  const int e = first[s + 1];
+  for (int k = first[s]; k < e; k += kB) {
+    double v[kB][3];
+#pragma unroll
+    for (int u = 0; u < kB; u++) {
+      const double* r = part + 3 * static_cast<int64_t>(at[min(k + u, e - 1)]);
+      v[u][0] = r[0];
+      v[u][1] = r[1];
+      v[u][2] = r[2];
+    }
+#pragma unroll
+    for (int u = 0; u < kB; u++) {
+      x += k + u < e ? v[u][0] : 0.0;
+      y += k + u < e ? v[u][1] : 0.0;
+      z += k + u < e ? v[u][2] : 0.0;
+    }
+  }
+  mom.add(member ? member[s] : s, x, y, z);
+}
+
 // Potential energy over the tiles (the force kernel's staging, offsets and
 // pair arithmetic, with the energy policy): each workgroup walks its tiles
 // as k_tile does and writes weight * 4 * sum s^3 (s^3 - 1) and weight * the
@@ -790,6 +943,25 @@ int run_tile(hipStream_t s, P pos, M mom, const ListView& lv, const PairParams& 
   return launch_status("tiled force kernel launch");
 }
 
+template <int PREC, class P, class M, bool PBC>
+int run_tile_half(hipStream_t s, P pos, M mom, const ListView& lv, const PairParams& pp) {
+  const int threads = (lv.tile_particles * kHalfLanes + 63) / 64 * 64;
+  if (threads > 1024 || lv.tile_sliced_lanes != kHalfLanes ||
+      lv.tile_sliced_unroll != kHalfUnroll || !lv.half_tile || lv.tile_first != 0)
+    return set_error(LJGPU_ERR_INVALID_ARGUMENT, "tiled half list: launch shape");
+  const int grid = (lv.tile_blocks + kXcds - 1) / kXcds * kXcds;
+  const size_t lds_bytes = kTileLdsHeader + static_cast<size_t>(lv.tile_max_stage) * kHalfStride;
+  const double reach = 0.5 * pp.box - sqrt(pp.cl2);
+  double* part = const_cast<double*>(lv.half_part);
+  hipLaunchKernelGGL((k_tile_half<PREC, P, PBC>), dim3(grid), dim3(threads), lds_bytes, s, pos,
+                     lv.tile_member, lv.tile_slot_ptr, reinterpret_cast<const int4*>(lv.tile_desc),
+                     lv.tile_stage, lv.tile_sliced, lv.tile_wave_off, lv.tile_waves_per_block,
+                     reinterpret_cast<const int2*>(lv.half_tile), part, lv.tile_blocks, pp, reach);
+  hipLaunchKernelGGL((k_half_gather<M>), dim3((lv.n + 255) / 256), dim3(256), 0, s, mom, lv.n,
+                     lv.tile_member, lv.half_first, lv.half_at, part);
+  return launch_status("tiled half-list kernel launch");
+}
+
 template <int TPI, int U, int PREC, class P, class M, bool PBC>
 int run_tile_layout(hipStream_t s, P pos, M mom, const ListView& lv, const PairParams& pp,
                     const LaunchConfig& lc) {
@@ -888,7 +1060,10 @@ int run_layout(hipStream_t s, P pos, M mom, const ListView& lv, const PairParams
                        "tiling on, no atomic half list)");
     return run_tile_lanes<PREC, P, M, true>(s, pos, mom, lv, pp, lc);
   }
-  if (lv.tile_blocks > 0 && !lc.half_atomic) {
+  if (lv.tile_blocks > 0 && lc.half_atomic)
+    return pbc ? run_tile_half<PREC, P, M, true>(s, pos, mom, lv, pp)
+               : run_tile_half<PREC, P, M, false>(s, pos, mom, lv, pp);
+  if (lv.tile_blocks > 0) {
     return pbc ? run_tile_lanes<PREC, P, M, true>(s, pos, mom, lv, pp, lc)
                : run_tile_lanes<PREC, P, M, false>(s, pos, mom, lv, pp, lc);
   }

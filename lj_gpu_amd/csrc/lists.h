@@ -72,6 +72,9 @@ struct DevTiles {
   bool cut = false, bank_done = false;
   DevMem inner;          // int32 per slot
   int32_t longest = 0;   // longest row
+
+  // Half lists (dev_half_tiles): see ListView.
+  DevMem half_tile, half_first, half_at, half_part;
 };
 void dev_release(DevTiles& t);
 
@@ -167,7 +170,8 @@ int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t tile_particles,
 // (k / lanes) % unroll, lane k % lanes). Wavefront w of block b holds the
 // block's rows [w * 64/lanes, (w+1) * 64/lanes) and owns the slice that
 // starts at wave_off[b * waves_per_block + w]: for each of its batches
-// (as many as its longest row needs) 64 * unroll offsets, slot by slot,
+// (as many as its longest row needs) 64 * unroll offsets (scale * rank, scale
+// the bytes per staged partner), slot by slot,
 // each slot the 64 lanes' entries in lane order, so one offset load of the
 // kernel reads 64 consecutive values. Slots past a row's end hold 0.
 // Needs local, desc and the slot row starts of a built tiling of n particles; a slicing
@@ -184,7 +188,13 @@ struct CutHint {
   double cl2 = 9.0;
 };
 int dev_slice_tiles(hipStream_t s, const int32_t* slot_ptr, int32_t lanes, int32_t unroll,
-                    bool bank_order, int32_t n, const CutHint* cut, ListWork& w, DevTiles& t);
+                    int32_t scale, bool bank_order, int32_t n, const CutHint* cut, ListWork& w,
+                    DevTiles& t);
+
+// What the tiled half-list kernel needs beyond a tiling of n particles: where
+// each tile writes its staged partners' force sums, and which of them belong
+// to each slot (in ascending order).
+int dev_half_tiles(hipStream_t s, int32_t n, ListWork& w, DevTiles& t);
 
 // The bank-class order (bank_class_order) of a tiling's rows, in place in
 // `local` (t.local or a copy of it); nothing when t.bank_done.

@@ -1400,7 +1400,8 @@ constexpr int kRowBatch = 5;  // entries per lane in flight
 // kSliceRows, a multiple of a wavefront's rows): slice position p of
 // wavefront w (batch j = p / (64 unroll), slot u, lane l) holds place k = j
 // * lanes * unroll + u * lanes + l % lanes of the block's row w * (64 /
-// lanes) + l / lanes, or 0 past the row's end (padding).
+// lanes) + l / lanes as `scale` times its rank, or 0 past the row's end
+// (padding).
 //   CUT first puts the rows in cutoff classes (cut_partition over cut_inner):
 // inner entries first, the others behind them, both in list order, in
 // `local` as well; inner[s] receives the inner count of slot s's row. The
@@ -1420,8 +1421,8 @@ template <bool CUT, bool POS_LDS, bool ORDER>
 __global__ __launch_bounds__(512) void k_tile_slices(
     const int32_t* __restrict__ desc, int32_t nblocks, const int32_t* __restrict__ slot_ptr,
     int32_t* __restrict__ inner, uint16_t* __restrict__ local, CutDev cut, int32_t grows,
-    int32_t stride, int32_t lanes, int32_t wpb, const int32_t* __restrict__ wave_off,
-    uint16_t* __restrict__ sliced) {
+    int32_t stride, int32_t lanes, int32_t wpb, int32_t scale,
+    const int32_t* __restrict__ wave_off, uint16_t* __restrict__ sliced) {
   extern __shared__ double slice_lds[];
   __shared__ int32_t start[kSliceRows], len[kSliceRows], in_len[kSliceRows];
   // The rows; then the staged positions, whose place the class counts and the
@@ -1554,13 +1555,51 @@ __global__ __launch_bounds__(512) void k_tile_slices(
         const int m = r < nr ? len[r] : 0;
         const bool direct = m > kBankRowMax;
         const uint16_t* src = direct ? local + start[r] : out + min(r, grows - 1) * stride;
-        const int scale = direct ? 1 : 24;
         int k = tid & (lanes - 1);
 #pragma unroll 4
         for (int32_t p = tid & 63; p < n; p += 64, k += lanes)
-          sliced[p0 + p] = k < m ? static_cast<uint16_t>(src[k] * scale) : uint16_t{0};
+          sliced[p0 + p] =
+              k < m ? static_cast<uint16_t>((direct ? src[k] / 24 : src[k]) * scale) : uint16_t{0};
       }
       __syncthreads();
+    }
+  }
+}
+
+// Half lists over tiles. Staged counts of the tiles; then per tile its first
+// row of force sums and the rank of its own first slot (keys: the staged
+// slots, ascending), and the number of staged places of each slot.
+__global__ void k_half_counts(int32_t nblocks, const int32_t* __restrict__ desc,
+                              int32_t* __restrict__ ns) {
+  const int64_t b = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+  if (b < nblocks) ns[b] = desc[8 * b + 3];
+}
+
+__global__ __launch_bounds__(kBlock) void k_half_places(
+    int32_t nblocks, const int32_t* __restrict__ desc, const int32_t* __restrict__ keys,
+    const int32_t* __restrict__ first_row, int2* __restrict__ tile, int32_t* __restrict__ count) {
+  for (int32_t b = blockIdx.x; b < nblocks; b += gridDim.x) {
+    const int32_t* d = desc + 8 * static_cast<int64_t>(b);
+    const int32_t i0 = d[0], soff = d[2], ns = d[3];
+    for (int t = threadIdx.x; t < ns; t += kBlock) {
+      const int32_t s = keys[soff + t];
+      atomicAdd(&count[s], 1);
+      if (s == i0) tile[b] = make_int2(first_row[b], t);
+    }
+  }
+}
+
+// The rows of each slot, in any order, then ascending.
+__global__ __launch_bounds__(kBlock) void k_half_fill(
+    int32_t nblocks, const int32_t* __restrict__ desc, const int32_t* __restrict__ keys,
+    const int32_t* __restrict__ first_row, const int32_t* __restrict__ first,
+    int32_t* __restrict__ used, int32_t* __restrict__ at) {
+  for (int32_t b = blockIdx.x; b < nblocks; b += gridDim.x) {
+    const int32_t* d = desc + 8 * static_cast<int64_t>(b);
+    const int32_t soff = d[2], ns = d[3];
+    for (int t = threadIdx.x; t < ns; t += kBlock) {
+      const int32_t s = keys[soff + t];
+      at[first[s] + atomicAdd(&used[s], 1)] = first_row[b] + t;
     }
   }
 }
@@ -1742,6 +1781,7 @@ void dev_release(DevTiles& t) {
   dev_release(t.slot_ptr);
   dev_release(t.stage_slot);
   dev_release(t.inner);
+  for (DevMem* m : {&t.half_tile, &t.half_first, &t.half_at, &t.half_part}) dev_release(*m);
   t.cut = t.bank_done = false;
   t.tile_particles = 0;
   t.blocks = 0;
@@ -2310,7 +2350,8 @@ int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<
 }
 
 int dev_slice_tiles(hipStream_t s, const int32_t* slot_ptr, int32_t lanes, int32_t unroll,
-                    bool bank_order, int32_t n, const CutHint* hint, ListWork& w, DevTiles& t) {
+                    int32_t scale, bool bank_order, int32_t n, const CutHint* hint, ListWork& w,
+                    DevTiles& t) {
   t.sliced_lanes = t.sliced_unroll = t.waves_per_block = 0;
   if (t.blocks <= 0 || lanes < 1 || lanes > 64 || (64 % lanes) != 0 || unroll < 1 ||
       (unroll & (unroll - 1)) != 0)
@@ -2362,12 +2403,46 @@ int dev_slice_tiles(hipStream_t s, const int32_t* slot_ptr, int32_t lanes, int32
   kernel<<<std::min(t.blocks, 65535), 512, rows + std::max(order, pos_lds ? pos : 0), s>>>(
       t.desc.as<int32_t>(), t.blocks, slot_ptr,
       t.cut || cut ? t.inner.as<int32_t>() : nullptr, t.local.as<uint16_t>(), cd, grows, stride,
-      lanes, wpb, t.wave_off.as<int32_t>(), t.sliced.as<uint16_t>());
+      lanes, wpb, scale, t.wave_off.as<int32_t>(), t.sliced.as<uint16_t>());
   LTRY(hipGetLastError(), "tile slice kernel");
   if (cut) t.cut = true;
   t.sliced_lanes = lanes;
   t.sliced_unroll = unroll;
   t.waves_per_block = wpb;
+  return LJGPU_OK;
+}
+
+int dev_half_tiles(hipStream_t s, int32_t n, ListWork& w, DevTiles& t) {
+  if (t.blocks <= 0) return LJGPU_OK;
+  const int32_t nb = t.blocks;
+  LCHECK(dev_reserve(w.tile_ns, sizeof(int32_t) * (static_cast<size_t>(nb) + 1), s));
+  LCHECK(dev_reserve(w.tile_soff, sizeof(int32_t) * (static_cast<size_t>(nb) + 1), s));
+  LCHECK(dev_reserve(w.counts, sizeof(int32_t) * (static_cast<size_t>(n) + 1), s));
+  LCHECK(dev_reserve(t.half_tile, sizeof(int2) * static_cast<size_t>(nb), s));
+  LCHECK(dev_reserve(t.half_first, sizeof(int32_t) * (static_cast<size_t>(n) + 1), s));
+  const int32_t* desc = t.desc.as<int32_t>();
+  const int32_t* keys = t.order == LJGPU_TILE_ORDER_SPATIAL ? t.stage_slot.as<int32_t>()
+                                                            : t.stage.as<int32_t>();
+  int32_t* count = w.counts.as<int32_t>();
+  int32_t* first = t.half_first.as<int32_t>();
+  k_half_counts<<<grid_for(nb, kBlock), kBlock, 0, s>>>(nb, desc, w.tile_ns.as<int32_t>());
+  LTRY(hipGetLastError(), "half tile count kernel");
+  int64_t total = 0;
+  LCHECK(dev_scan(s, w.tile_ns.as<int32_t>(), w.tile_soff.as<int32_t>(), nb, w, &total));
+  if (total > INT32_MAX) return set_error(LJGPU_ERR_CAPACITY, "half list: too many staged partners");
+  LCHECK(dev_reserve(t.half_at, sizeof(int32_t) * std::max<int64_t>(total, 1), s));
+  LCHECK(dev_reserve(t.half_part, sizeof(double) * 3 * std::max<int64_t>(total, 1), s));
+  const int grid = std::min(nb, 65535);
+  LCHECK(fill<int32_t>(s, count, n, 0));
+  k_half_places<<<grid, kBlock, 0, s>>>(nb, desc, keys, w.tile_soff.as<int32_t>(),
+                                        t.half_tile.as<int2>(), count);
+  LTRY(hipGetLastError(), "half tile place kernel");
+  LCHECK(dev_scan(s, count, first, n, w, &total));
+  LCHECK(fill<int32_t>(s, count, n, 0));
+  k_half_fill<<<grid, kBlock, 0, s>>>(nb, desc, keys, w.tile_soff.as<int32_t>(), first, count,
+                                      t.half_at.as<int32_t>());
+  k_order_sort<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, first, t.half_at.as<int32_t>());
+  LTRY(hipGetLastError(), "half tile fill kernels");
   return LJGPU_OK;
 }
 

@@ -72,6 +72,14 @@ struct ListView {
   const int32_t* tile_wave_off = nullptr;
   int32_t tile_waves_per_block = 0, tile_sliced_lanes = 0, tile_sliced_unroll = 0;
 
+  // Half lists over tiles: per tile its first row of half_part (a row of
+  // three doubles per staged partner) and the rank of its own first particle;
+  // per slot (+1) the start in half_at of the rows that hold its force sums.
+  const int32_t* half_tile = nullptr;  // 2 ints per tile
+  const int32_t* half_first = nullptr;
+  const int32_t* half_at = nullptr;
+  const double* half_part = nullptr;
+
   // Batched replicas (tiled kernel only): per replica (box, 1/box), indexed
   // by descriptor slot 6; null for a single system.
   const double* replica_box = nullptr;
@@ -100,6 +108,13 @@ constexpr int32_t kTileLocalPad = 512;
 LJ_HD inline int64_t tile_lds_bytes(int64_t ns, int64_t ne) {
   return ((ns * 24 + 15) / 16) * 16 + ((ne + 14 + 7) / 8) * 16;
 }
+
+// Half lists over tiles (atomic mode): four lanes per row, and per staged
+// partner its position and force sum in kHalfStride bytes of LDS, so its
+// 16-bit offsets reach kHalfMaxStage partners.
+constexpr int kHalfLanes = 4;
+constexpr int32_t kHalfStride = 56;
+constexpr int32_t kHalfMaxStage = (65536 - kTileLdsHeader) / kHalfStride;
 
 // Entry order within a tile row, chosen so that the partner reads of one
 // LDS instruction spread over the banks. The staged position of rank t

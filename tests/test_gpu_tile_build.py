@@ -83,3 +83,37 @@ def test_built_tiles_and_their_forces(ctx, name, lanes, unroll, tile):
     ctx.force_aos_f64(dq, dp, 1.0, G.CL2, box, 1)
     ctx.sync()
     assert normwise(dp.download(), f) < FP64_TOL
+
+
+@pytest.mark.parametrize("name", ["ragged", "long_rows", "mixed_rows", "scattered", "open"])
+@pytest.mark.parametrize("layout", ["aos", "soa", "aos3"])
+@pytest.mark.parametrize("tile", [64, 16, 1])
+def test_atomic_half_lists_over_tiles(ctx, name, layout, tile):
+    """Half lists scattered to both particles: over tiles where partners are
+    shared (LDS sums, one addition to memory per staged partner), else the
+    untiled kernel; reported as untiled either way."""
+    q, box, full, f = system(name)
+    n = q.shape[0]
+    print(f"{name} {layout} tile={tile}", flush=True)
+    ctx.set_kernel_config(4, 256, 4)
+    ctx.set_tiling(tile)
+    ctx.set_half_mode(G.HALF_ATOMIC)
+    if layout == "soa":
+        dq = [ctx.array(np.ascontiguousarray(q[:, c])) for c in range(3)]
+        dp = [ctx.zeros(n) for _ in range(3)]
+        build, force = ctx.build_list_soa, ctx.force_soa_f64
+    else:
+        w = 4 if layout == "aos" else 3
+        dq, dp = ctx.array(np.ascontiguousarray(q[:, :w])), ctx.zeros((n, w))
+        build = ctx.build_list if w == 4 else ctx.build_list_aos3
+        force = ctx.force_aos_f64 if w == 4 else ctx.force_aos3_f64
+    build(dq, n, box, G.LIST_HALF)
+    for steps in (1, 5, 20):
+        for a in dp if layout == "soa" else [dp]:
+            a.zero()
+        force(dq, dp, 1.0 / steps, G.CL2, box, steps)
+        ctx.sync()
+        p = np.stack([a.download() for a in dp], 1) if layout == "soa" else dp.download()
+        assert normwise(p, f) < FP64_TOL
+    assert ctx.list_info().tile_particles == 0 and ctx.get_tiles() is None
+    ctx.set_half_mode(G.HALF_AUTO)
