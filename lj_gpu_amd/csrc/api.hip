@@ -119,13 +119,15 @@ int ensure_tiles(ljgpu_ctx* ctx, const PosIn* q, double box) {
   ctx->tiles.blocks = 0;
   ctx->tiles.sliced_lanes = ctx->tiles.sliced_unroll = 0;
   bool ordered = false;
-  if (spatial && q && ctx->eval.n > 0)
+  if (ctx->order_begun)
+    ordered = dev_tile_order_end(ctx->work);  // the list build has synchronised since
+  else if (spatial && q && ctx->eval.n > 0)
     TRY(dev_tile_order(ctx->stream, *q, ctx->eval.n, box, ctx->rep_off, ctx->rep_boxes, want,
                        ctx->work, &ordered));
-  if (ordered) TRY(dev_length_sort(ctx->stream, ctx->eval, want, ctx->rep_off, ctx->work));
-  const int32_t* member = ordered ? ctx->work.order.as<int32_t>() : nullptr;
+  if (ordered)
+    TRY(dev_tile_slots(ctx->stream, ctx->eval, want, ctx->rep_off, ctx->work, ctx->tiles));
   for (int32_t tp = want; tp >= 1 && ctx->eval.n > 0; tp /= 2) {
-    TRY(dev_make_tiles(ctx->stream, ctx->eval, tp, ctx->rep_off, member, ctx->work, ctx->tiles));
+    TRY(dev_make_tiles(ctx->stream, ctx->eval, tp, ctx->rep_off, ordered, ctx->work, ctx->tiles));
     if (ctx->tiles.tile_particles == 0) continue;
     if (!ctx->eval_half || ctx->tiles.max_stage <= kHalfMaxStage) break;
     ctx->tiles.tile_particles = ctx->tiles.blocks = 0;
@@ -305,6 +307,17 @@ int build_list(ljgpu_ctx* ctx, const PosIn& q, int32_t n, double box, double sea
   TRY(use_device(ctx));
   reset_list(ctx);
   const bool expand = kind == LJGPU_LIST_FULL || ctx->half_mode_req != LJGPU_HALF_ATOMIC;
+  // The spatial tile order needs the positions only: enqueued first, it is
+  // decided by the pair search's synchronisation.
+  struct OrderBegun {
+    ljgpu_ctx* c;
+    ~OrderBegun() { c->order_begun = false; }
+  } order_begun_guard{ctx};
+  const int32_t tile = effective_tile(ctx);
+  if (tile > 0 && n > 0 && ctx->tile_order == LJGPU_TILE_ORDER_SPATIAL &&
+      (expand || ctx->rep_off.empty()))
+    TRY(dev_tile_order_begin(ctx->stream, q, n, box, ctx->rep_off, ctx->rep_boxes, tile, ctx->work,
+                             &ctx->order_begun));
   // A full list is the symmetric closure of the half list (the pair
   // predicate is exactly symmetric), so an expanded half list is built
   // directly as the full list.
@@ -322,7 +335,10 @@ int build_list(ljgpu_ctx* ctx, const PosIn& q, int32_t n, double box, double sea
   ctx->n_entries = (kind == LJGPU_LIST_HALF && expand) ? ctx->eval.e / 2 : ctx->eval.e;
   if (kind == LJGPU_LIST_HALF && expand)
     TRY(dev_half_row_stats(ctx->stream, ctx->eval, ctx->work, &ctx->min_np, &ctx->max_np));
-  else
+  else if (ctx->rep_off.empty()) {
+    ctx->min_np = ctx->work.row_min;
+    ctx->max_np = ctx->work.row_max;
+  } else
     TRY(dev_minmax(ctx->stream, ctx->eval.nop.as<int32_t>(), n, ctx->work, &ctx->min_np,
                    &ctx->max_np));
   ctx->ell_ready = false;

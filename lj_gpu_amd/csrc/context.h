@@ -114,6 +114,7 @@ struct ljgpu_ctx {
   int cus = 0;                    // compute units of the device
   int32_t tiles_for = 0;          // effective tile size the tiling was derived for (0: none)
   int tile_order = LJGPU_TILE_ORDER_SPATIAL;  // requested order of the particles in tiles
+  bool order_begun = false;       // within build_list: dev_tile_order_begin is enqueued
   bool tiles_ordered = false;     // the tiling was derived with positions (order, cutoff classes)
   bool bank_order = true;         // tile rows in the LDS bank-class order (bank_class_order)
   ljgpu::DevTiles tiles;

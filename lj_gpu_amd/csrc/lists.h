@@ -78,6 +78,19 @@ struct DevTiles {
 };
 void dev_release(DevTiles& t);
 
+// Results of enqueued kernels, in pinned memory that they write: valid once
+// the stream has been synchronised after the kernel.
+struct ScanStats {
+  int64_t total;
+  int32_t lo, hi;  // smallest and largest value scanned
+};
+struct ListResults {
+  ScanStats scan;    // of dev_scan
+  ScanStats cells;   // particles per cell
+  ScanStats order;   // particles per bin of the spatial tile order
+  int32_t tiles[8];  // k_tile_stats
+};
+
 // Scratch buffers reused across builds.
 struct ListWork {
   DevMem scan_sums;   // int64 per scan tile
@@ -100,6 +113,10 @@ struct ListWork {
   DevMem slot_of;     // int32 per particle: its slot in the tile order
   DevCSR part;        // one replica's list during a batched build
   int32_t last_max_row = 0;  // longest row of the last device build (slab size hint)
+  int32_t row_min = 0, row_max = 0;  // row lengths of the last device build
+  ListResults* results = nullptr;    // pinned
+  std::vector<int32_t> geo_host;     // blocks of a replicas' tiling, as uploaded
+  std::vector<char> order_host;      // bins and offsets of a replicas' tile order, as uploaded
 };
 void dev_release(ListWork& w);
 
@@ -112,8 +129,8 @@ struct PosIn {
   int stride = 4;
 };
 
-// Exclusive scan of in[0..n) into out[0..n], out[n] = total; *total receives
-// the sum (synchronises the stream).
+// Exclusive scan of in[0..n) into out[0..n], out[n] = total, both 16-byte
+// aligned; *total receives the sum (synchronises the stream).
 int dev_scan(hipStream_t s, const int32_t* in, int32_t* out, int64_t n, ListWork& w,
              int64_t* total);
 
@@ -151,18 +168,22 @@ int dev_half_row_stats(hipStream_t s, const DevCSR& full, ListWork& w, int32_t* 
 // row (at least 1), zero padded.
 int dev_make_ell(hipStream_t s, const DevCSR& c, int32_t width, DevMem& ell);
 
+// The slots of the spatial order in w.order (dev_tile_order): within each
+// block of tile_particles consecutive slots (restarted at every replica
+// boundary) the particles by row length, longest first, ties in the order
+// given. Sets out.member, out.slot_ptr and w.slot_of.
+int dev_tile_slots(hipStream_t s, const DevCSR& c, int32_t tile_particles,
+                   const std::vector<int32_t>& replicas, ListWork& w, DevTiles& out);
+
 // LDS tiling of a row-ordered full list with blocks of `tile_particles`
 // consecutive particles, restarted at each replica boundary of `replicas`
 // (host offsets; empty for a single system), descriptor slot 6 holding the
 // block's replica. Returns LJGPU_OK with out.tile_particles = 0 when a block
 // does not fit the LDS budget (the caller then halves the tile size or
-// evaluates untiled).
-// `member` (device, one particle per slot, a permutation that keeps every
-// replica's particles within its own slot range) orders the particles the
-// blocks cover; null takes them in index order.
+// evaluates untiled). With `spatial` the blocks cover the slots of
+// dev_tile_slots, else particles in index order.
 int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t tile_particles,
-                   const std::vector<int32_t>& replicas, const int32_t* member, ListWork& w,
-                   DevTiles& out);
+                   const std::vector<int32_t>& replicas, bool spatial, ListWork& w, DevTiles& out);
 
 // The tiles' entry offsets sliced per wavefront, for a tile kernel in
 // which `lanes` consecutive lanes own one row and take entries in batches
@@ -211,13 +232,13 @@ int dev_bank_order(hipStream_t s, const int32_t* slot_ptr, const DevTiles& t, ui
 int dev_tile_order(hipStream_t s, const PosIn& q, int32_t n, double box,
                    const std::vector<int32_t>& replicas, const std::vector<double>& boxes,
                    int32_t tile_particles, ListWork& w, bool* ok);
-
-// Within each block of tile_particles consecutive slots of w.order (restarted
-// at every replica boundary, as dev_make_tiles forms its blocks), the slots
-// reordered by the row length of their particles in c, longest first, ties
-// in the previous order.
-int dev_length_sort(hipStream_t s, const DevCSR& c, int32_t tile_particles,
-                    const std::vector<int32_t>& replicas, ListWork& w);
+// The same in two steps, so that a caller's next synchronisation serves it
+// too: begin enqueues it (*begun = false: no order for this box), end tells
+// after that synchronisation whether the order holds.
+int dev_tile_order_begin(hipStream_t s, const PosIn& q, int32_t n, double box,
+                         const std::vector<int32_t>& replicas, const std::vector<double>& boxes,
+                         int32_t tile_particles, ListWork& w, bool* begun);
+bool dev_tile_order_end(const ListWork& w);
 
 // Batched replicas: lists of every replica (particles [off[r], off[r+1]),
 // box boxes[r]) built on the device into one CSR with global indices.

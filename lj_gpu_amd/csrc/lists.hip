@@ -49,6 +49,8 @@ int hip_err(hipError_t e, const char* what) {
 constexpr int kBlock = 256;
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kBlock * kScanItems;
+constexpr int64_t kScanSmall = 16384;  // values scanned by one workgroup
+constexpr int64_t kScanTiles = 1024;   // tiles whose sums every workgroup adds up itself
 
 int grid_for(int64_t items, int block, int cap = 65535 * 8) {
   const int64_t g = (items + block - 1) / block;
@@ -73,29 +75,23 @@ int fill(hipStream_t s, T* a, int64_t n, T v) {
   return LJGPU_OK;
 }
 
-// Inclusive scan of one value per lane over a wavefront.
-__device__ __forceinline__ int64_t wave_inclusive(int64_t v) {
-  const int lane = threadIdx.x & 63;
+// Exclusive scan of one value per thread over the workgroup; *total receives
+// the sum. `sh` holds one value per wavefront.
+template <class T>
+__device__ __forceinline__ T block_exclusive(T v, T* total, T* sh) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  T inc = v;
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
-    const int64_t t = __shfl_up(v, d, 64);
-    if (lane >= d) v += t;
+    const T t = __shfl_up(inc, d, 64);
+    if (lane >= d) inc += t;
   }
-  return v;
-}
-
-// Exclusive scan of one value per thread over a kBlock-thread workgroup;
-// *total receives the workgroup sum. `sh` holds kBlock/64 values.
-__device__ __forceinline__ int64_t block_exclusive(int64_t v, int64_t* total, int64_t* sh) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int64_t inc = wave_inclusive(v);
   if (lane == 63) sh[wid] = inc;
   __syncthreads();
-  int64_t off = 0, tot = 0;
-#pragma unroll
-  for (int w = 0; w < kBlock / 64; w++) {
-    const int64_t x = sh[w];
-    off += (w < wid) ? x : 0;
+  T off = 0, tot = 0;
+  for (int w = 0; w < static_cast<int>(blockDim.x) / 64; w++) {
+    const T x = sh[w];
+    off += w < wid ? x : 0;
     tot += x;
   }
   __syncthreads();
@@ -103,57 +99,174 @@ __device__ __forceinline__ int64_t block_exclusive(int64_t v, int64_t* total, in
   return off + inc - v;
 }
 
-// Scan pass 1: per-tile sums.
-__global__ __launch_bounds__(kBlock) void k_scan_reduce(const int32_t* __restrict__ in, int64_t n,
-                                                        int64_t* __restrict__ sums) {
-  __shared__ int64_t sh[kBlock / 64];
-  const int64_t base = static_cast<int64_t>(blockIdx.x) * kScanTile;
-  int64_t v = 0;
-  for (int r = 0; r < kScanItems; r++) {
-    const int64_t t = base + r * kBlock + threadIdx.x;
-    if (t < n) v += in[t];
+// Smallest and largest of one pair per thread over the workgroup, for thread 0.
+__device__ __forceinline__ void block_extrema(int32_t& lo, int32_t& hi, int32_t* slo,
+                                              int32_t* shi) {
+  for (int d = 32; d > 0; d >>= 1) {
+    lo = min(lo, __shfl_xor(lo, d, 64));
+    hi = max(hi, __shfl_xor(hi, d, 64));
   }
-  int64_t total;
-  (void)block_exclusive(v, &total, sh);
-  if (threadIdx.x == 0) sums[blockIdx.x] = total;
+  if ((threadIdx.x & 63) == 0) {
+    slo[threadIdx.x >> 6] = lo;
+    shi[threadIdx.x >> 6] = hi;
+  }
+  __syncthreads();
+  for (int w = 0; w < static_cast<int>(blockDim.x) / 64; w++) {
+    lo = min(lo, slo[w]);
+    hi = max(hi, shi[w]);
+  }
+  __syncthreads();
 }
 
-// Scan pass 2: exclusive scan of the tile sums in place (one workgroup).
-__global__ __launch_bounds__(kBlock) void k_scan_sums(int64_t* __restrict__ sums, int64_t nb,
-                                                      int64_t* __restrict__ total_out) {
+__device__ __forceinline__ int32_t clamp_i32(int64_t v) {
+  return static_cast<int32_t>(std::min<int64_t>(v, INT32_MAX));
+}
+
+// Exclusive scan (values clamped to int32; the host rejects totals above
+// INT32_MAX), out[n] = total, with the sum and extrema of the input in *res
+// (null: not wanted). Up to kScanSmall values: one workgroup, a contiguous
+// piece per thread. More: a pass that sums tiles of kScanTile values, and one that scans
+// each tile from the sum of the tiles before it, which every workgroup adds
+// up itself (SUMS: taken from sums scanned by k_scan_sums, for lists of many
+// tiles).
+__global__ __launch_bounds__(1024) void k_scan_small(const int32_t* __restrict__ in, int32_t n,
+                                                     int32_t* __restrict__ out,
+                                                     ScanStats* __restrict__ res) {
+  __shared__ int64_t sh[16];
+  __shared__ int32_t slo[16], shi[16];
+  const int32_t piece = ((n + 1023) / 1024 + 3) / 4 * 4;
+  const int32_t t0 = threadIdx.x * piece, t1 = min(t0 + piece, n);
+  int64_t v = 0;
+  int32_t lo = INT32_MAX, hi = INT32_MIN;
+#pragma unroll 4
+  for (int32_t t = t0; t < t1; t++) {
+    const int32_t x = in[t];
+    v += x;
+    lo = min(lo, x);
+    hi = max(hi, x);
+  }
+  int64_t total;
+  int64_t run = block_exclusive<int64_t>(v, &total, sh);
+#pragma unroll 4
+  for (int32_t t = t0; t < t1; t++) {
+    out[t] = clamp_i32(run);
+    run += in[t];
+  }
+  if (threadIdx.x == 0) out[n] = clamp_i32(total);
+  if (!res) return;
+  block_extrema(lo, hi, slo, shi);
+  if (threadIdx.x == 0) *res = ScanStats{total, lo, hi};
+}
+
+struct ScanTile {
+  int64_t sum;
+  int32_t lo, hi;
+};
+
+// The kScanItems values of this thread in its tile (0 past the end).
+__device__ __forceinline__ void scan_load(const int32_t* __restrict__ in, int64_t n, int64_t base,
+                                          int32_t (&v)[kScanItems]) {
+  if (base + kScanItems <= n) {
+#pragma unroll
+    for (int q = 0; q < kScanItems / 4; q++) {
+      const int4 x = reinterpret_cast<const int4*>(in + base)[q];
+      v[4 * q] = x.x;
+      v[4 * q + 1] = x.y;
+      v[4 * q + 2] = x.z;
+      v[4 * q + 3] = x.w;
+    }
+  } else {
+#pragma unroll
+    for (int r = 0; r < kScanItems; r++) v[r] = base + r < n ? in[base + r] : 0;
+  }
+}
+
+__global__ __launch_bounds__(kBlock) void k_scan_reduce(const int32_t* __restrict__ in, int64_t n,
+                                                        ScanTile* __restrict__ tiles) {
+  __shared__ int64_t sh[kBlock / 64];
+  __shared__ int32_t slo[kBlock / 64], shi[kBlock / 64];
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * kScanTile + threadIdx.x * kScanItems;
+  int32_t v[kScanItems];
+  scan_load(in, n, base, v);
+  int64_t sum = 0;
+  int32_t lo = INT32_MAX, hi = INT32_MIN;
+#pragma unroll
+  for (int r = 0; r < kScanItems; r++) {
+    sum += v[r];
+    if (base + r < n) {
+      lo = min(lo, v[r]);
+      hi = max(hi, v[r]);
+    }
+  }
+  int64_t total;
+  (void)block_exclusive<int64_t>(sum, &total, sh);
+  block_extrema(lo, hi, slo, shi);
+  if (threadIdx.x == 0) tiles[blockIdx.x] = ScanTile{total, lo, hi};
+}
+
+// Exclusive scan of the tile sums in place (one workgroup).
+__global__ __launch_bounds__(kBlock) void k_scan_sums(ScanTile* __restrict__ tiles, int64_t nb) {
   __shared__ int64_t sh[kBlock / 64];
   int64_t carry = 0;
   for (int64_t b0 = 0; b0 < nb; b0 += kBlock) {
     const int64_t t = b0 + threadIdx.x;
-    const int64_t v = t < nb ? sums[t] : 0;
+    const int64_t v = t < nb ? tiles[t].sum : 0;
     int64_t tot;
-    const int64_t ex = block_exclusive(v, &tot, sh);
-    if (t < nb) sums[t] = carry + ex;
+    const int64_t ex = block_exclusive<int64_t>(v, &tot, sh);
+    if (t < nb) tiles[t].sum = carry + ex;
     carry += tot;
   }
-  if (threadIdx.x == 0) *total_out = carry;
 }
 
-// Scan pass 3: exclusive scan within each tile plus the tile offset; the
-// last tile also writes out[n] = total (clamped to int32; the host rejects
-// totals above INT32_MAX).
+template <bool SUMS>
 __global__ __launch_bounds__(kBlock) void k_scan_apply(const int32_t* __restrict__ in, int64_t n,
-                                                       const int64_t* __restrict__ sums,
-                                                       const int64_t* __restrict__ total,
-                                                       int32_t* __restrict__ out) {
+                                                       const ScanTile* __restrict__ tiles,
+                                                       int32_t* __restrict__ out,
+                                                       ScanStats* __restrict__ res) {
   __shared__ int64_t sh[kBlock / 64];
-  const int64_t base = static_cast<int64_t>(blockIdx.x) * kScanTile;
-  int64_t carry = sums[blockIdx.x];
-  for (int r = 0; r < kScanItems; r++) {
-    const int64_t t = base + r * kBlock + threadIdx.x;
-    const int64_t v = t < n ? in[t] : 0;
-    int64_t tot;
-    const int64_t ex = block_exclusive(v, &tot, sh);
-    if (t < n) out[t] = static_cast<int32_t>(std::min<int64_t>(carry + ex, INT32_MAX));
-    carry += tot;
+  __shared__ int32_t slo[kBlock / 64], shi[kBlock / 64];
+  int64_t carry = 0;
+  if (SUMS) {
+    carry = tiles[blockIdx.x].sum;
+  } else {
+    int64_t before = 0;
+    for (int t = threadIdx.x; t < static_cast<int>(blockIdx.x); t += kBlock) before += tiles[t].sum;
+    (void)block_exclusive<int64_t>(before, &carry, sh);
   }
-  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0)
-    out[n] = static_cast<int32_t>(std::min<int64_t>(*total, INT32_MAX));
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * kScanTile + threadIdx.x * kScanItems;
+  int32_t v[kScanItems];
+  scan_load(in, n, base, v);
+  int64_t sum = 0;
+#pragma unroll
+  for (int r = 0; r < kScanItems; r++) sum += v[r];
+  int64_t tot;
+  int64_t run = carry + block_exclusive<int64_t>(sum, &tot, sh);
+  int32_t o[kScanItems];
+#pragma unroll
+  for (int r = 0; r < kScanItems; r++) {
+    o[r] = clamp_i32(run);
+    run += v[r];
+  }
+  if (base + kScanItems <= n) {
+#pragma unroll
+    for (int q = 0; q < kScanItems / 4; q++)
+      reinterpret_cast<int4*>(out + base)[q] =
+          make_int4(o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]);
+  } else {
+#pragma unroll
+    for (int r = 0; r < kScanItems; r++)
+      if (base + r < n) out[base + r] = o[r];
+  }
+  if (blockIdx.x != gridDim.x - 1) return;
+  if (threadIdx.x == 0) out[n] = clamp_i32(carry + tot);
+  if (!res) return;
+  int32_t lo = INT32_MAX, hi = INT32_MIN;
+  for (int t = threadIdx.x; t < static_cast<int>(gridDim.x); t += kBlock) {
+    lo = min(lo, tiles[t].lo);
+    hi = max(hi, tiles[t].hi);
+  }
+  block_extrema(lo, hi, slo, shi);
+  if (threadIdx.x == 0) *res = ScanStats{carry + tot, lo, hi};
 }
 
 // ---------------------------------------------------------------------------
@@ -478,24 +591,52 @@ __global__ void k_cell_scatter(int32_t n, PosIn q, const int32_t* __restrict__ c
   }
 }
 
-// Each cell's particles by ascending index (insertion sort, one thread per
-// cell): the scatter's atomic slots leave them in arrival order. Used only
-// when no cell holds more than kCellOrderMax particles.
+// Cells (or bins) in a fixed order: the particles of each by ascending index.
+// Their atomic slots leave them in arrival order (k_bin_index); each then takes the rank of
+// its index among its bin's, which cost a few loads that do not wait for
+// each other where a sort by one thread per bin waits for each exchange. Bins of
+// more than kCellOrderMax particles keep the arrival order; the callers look
+// at the largest bin.
 constexpr int32_t kCellOrderMax = 256;
-__global__ void k_cell_order(int64_t ncell, const int32_t* __restrict__ cell_start,
-                             double4* __restrict__ cpos) {
-  for (int64_t c = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; c < ncell;
-       c += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    const int32_t a = cell_start[c], b = cell_start[c + 1];
-    for (int32_t k = a + 1; k < b; k++) {
-      const double4 v = cpos[k];
-      int32_t m = k;
-      while (m > a && cpos[m - 1].w > v.w) {
-        cpos[m] = cpos[m - 1];
-        m--;
-      }
-      cpos[m] = v;
-    }
+__global__ void k_bin_index(int32_t n, const int32_t* __restrict__ bin_of,
+                            const int32_t* __restrict__ slot, const int32_t* __restrict__ start,
+                            int32_t* __restrict__ arrival) {
+  for (int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; t < n;
+       t += static_cast<int64_t>(gridDim.x) * blockDim.x)
+    arrival[start[bin_of[t]] + slot[t]] = static_cast<int32_t>(t);
+}
+
+// The place of arrival t, whose particle is i.
+__device__ __forceinline__ int32_t bin_place(int64_t t, int32_t i, const int32_t* __restrict__ bin_of,
+                                             const int32_t* __restrict__ start,
+                                             const int32_t* __restrict__ arrival) {
+  const int32_t c = bin_of[i];
+  const int32_t a = start[c], b = start[c + 1];
+  if (b - a > kCellOrderMax) return static_cast<int32_t>(t);
+  int32_t r = a;
+  for (int32_t u = a; u < b; u++) r += arrival[u] < i ? 1 : 0;
+  return r;
+}
+
+__global__ void k_order_place(int32_t n, const int32_t* __restrict__ bin_of,
+                              const int32_t* __restrict__ start,
+                              const int32_t* __restrict__ arrival, int32_t* __restrict__ order) {
+  for (int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; t < n;
+       t += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    const int32_t i = arrival[t];
+    order[bin_place(t, i, bin_of, start, arrival)] = i;
+  }
+}
+
+__global__ void k_cell_place(int32_t n, PosIn q, const int32_t* __restrict__ cell_of,
+                             const int32_t* __restrict__ start,
+                             const int32_t* __restrict__ arrival, double4* __restrict__ cpos) {
+  for (int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; t < n;
+       t += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    const int32_t i = arrival[t];
+    const int64_t o = static_cast<int64_t>(i) * q.stride;
+    cpos[bin_place(t, i, cell_of, start, arrival)] =
+        make_double4(q.x[o], q.y[o], q.z[o], static_cast<double>(i));
   }
 }
 
@@ -839,19 +980,34 @@ __device__ __forceinline__ T lds_load(const T* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
+// The blocks of a tiling: geo (4 ints per block: first slot, count, replica)
+// for replicas, else (null) blocks of T consecutive slots of n.
+struct TileSpans {
+  const int32_t* geo;
+  int32_t T, n;
+};
+struct TileSpan {
+  int32_t i0, ni, rid;
+};
+__device__ __forceinline__ TileSpan tile_span(const TileSpans& g, int32_t b) {
+  if (g.geo) return TileSpan{g.geo[4 * b], g.geo[4 * b + 1], g.geo[4 * b + 2]};
+  return TileSpan{b * g.T, min(g.T, g.n - b * g.T), 0};
+}
+
 struct TileGeom {
   int32_t i0, ni, ne, rid;
   int64_t e0;
 };
 
-// Block b covers slots [geo[4b], geo[4b] + geo[4b+1]) of replica geo[4b+2];
-// its entries are [slot_ptr[i0], slot_ptr[i0 + ni]) of the slot-ordered rows.
-__device__ __forceinline__ TileGeom tile_geom(int32_t b, const int32_t* __restrict__ geo,
+// Block b's entries are [slot_ptr[i0], slot_ptr[i0 + ni]) of the slot-ordered
+// rows.
+__device__ __forceinline__ TileGeom tile_geom(const TileSpans& spans, int32_t b,
                                               const int32_t* __restrict__ slot_ptr) {
+  const TileSpan t = tile_span(spans, b);
   TileGeom g;
-  g.i0 = geo[4 * b];
-  g.ni = geo[4 * b + 1];
-  g.rid = geo[4 * b + 2];
+  g.i0 = t.i0;
+  g.ni = t.ni;
+  g.rid = t.rid;
   g.e0 = slot_ptr[g.i0];
   g.ne = slot_ptr[g.i0 + g.ni] - static_cast<int32_t>(g.e0);
   return g;
@@ -890,7 +1046,7 @@ __device__ __forceinline__ uint32_t word_add(int32_t w, uint32_t h, uint32_t bit
 // them: an atomic per tile on one address costs more than the tile).
 template <bool COUNT>
 __global__ __launch_bounds__(1024) void k_tile_fill(
-    const int32_t* __restrict__ geo, int32_t nblocks, const int32_t* __restrict__ member,
+    TileSpans spans, int32_t nblocks, const int32_t* __restrict__ member,
     const int32_t* __restrict__ slot_of, const int32_t* __restrict__ slot_ptr,
     const int32_t* __restrict__ ptr, const int32_t* __restrict__ list,
     const int32_t* __restrict__ soff, int32_t ecap, int32_t* __restrict__ ns_out,
@@ -904,7 +1060,7 @@ __global__ __launch_bounds__(1024) void k_tile_fill(
   const int nt = static_cast<int>(blockDim.x), tid = static_cast<int>(threadIdx.x);
   const int lane = tid & (kWordLanes - 1), group = tid / kWordLanes, groups = nt / kWordLanes;
   for (int32_t b = blockIdx.x; b < nblocks; b += gridDim.x) {
-    const TileGeom g = tile_geom(b, geo, slot_ptr);
+    const TileGeom g = tile_geom(spans, b, slot_ptr);
     for (int t = tid; t < kWords; t += nt) {
       keys[t] = -1;
       masks[t] = 0;
@@ -1060,7 +1216,10 @@ __global__ __launch_bounds__(1024) void k_tile_fill(
 // [2] most LDS bytes, [3] longest row, [4] a tile with too many pages, [6..7]
 // the total staged (64 bits). One workgroup.
 __global__ __launch_bounds__(1024) void k_tile_stats(int32_t nblocks, const int4* __restrict__ stats,
+                                                     uint16_t* __restrict__ pad,
                                                      int32_t* __restrict__ out) {
+  // The offsets' padding, too (the force kernels read past the last row).
+  for (int t = threadIdx.x; pad && t < kTileLocalPad; t += blockDim.x) pad[t] = 0;
   __shared__ int32_t mx[5];
   __shared__ unsigned long long sum;
   if (threadIdx.x < 5) mx[threadIdx.x] = threadIdx.x == 1 ? -1 : 0;
@@ -1116,31 +1275,8 @@ constexpr int kPageBytes = 24576;
 constexpr int kPageDir = 32768;  // most pages of a list
 static_assert(kPageBytes / 128 < 255, "a page number fits a byte");
 
-// Exclusive scan over the workgroup; *total receives the sum. sh: one value
-// per wavefront.
-__device__ __forceinline__ int32_t group_exclusive(int32_t v, int32_t* total, int32_t* sh) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  int32_t inc = v;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int32_t t = __shfl_up(inc, d, 64);
-    if (lane >= d) inc += t;
-  }
-  if (lane == 63) sh[wid] = inc;
-  __syncthreads();
-  int32_t off = 0, tot = 0;
-  for (int w = 0; w < static_cast<int>(blockDim.x) / 64; w++) {
-    const int32_t x = sh[w];
-    off += w < wid ? x : 0;
-    tot += x;
-  }
-  __syncthreads();
-  *total = tot;
-  return off + inc - v;
-}
-
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6))) void k_tile_pages(
-    const int32_t* __restrict__ geo, int32_t nblocks, const int32_t* __restrict__ member,
+    TileSpans spans, int32_t nblocks, const int32_t* __restrict__ member,
     const int32_t* __restrict__ slot_of, const int32_t* __restrict__ slot_ptr,
     const int32_t* __restrict__ ptr, const int32_t* __restrict__ list, int32_t pshift,
     int32_t npages, int32_t* __restrict__ desc, int32_t* __restrict__ stage,
@@ -1158,7 +1294,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6))) void k
   const int32_t low = (1 << pshift) - 1;
   const int32_t chunk = ((npages + nt - 1) / nt + 3) / 4;  // directory words per thread
   for (int32_t b = blockIdx.x; b < nblocks; b += gridDim.x) {
-    const TileGeom g = tile_geom(b, geo, slot_ptr);
+    const TileGeom g = tile_geom(spans, b, slot_ptr);
     for (int t = tid; t < (npages + 3) / 4; t += nt) page_lds[t] = 0;
     if (tid == 0) longest = 0;
     // The group's first row, in registers; places past its end hold the tile's
@@ -1207,7 +1343,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6))) void k
       int32_t c = 0;
       for (int w = tid * chunk; w < min((tid + 1) * chunk, (npages + 3) / 4); w++)
         c += __popc(page_lds[w]);
-      int32_t p = group_exclusive(c, &pages, sh);
+      int32_t p = block_exclusive<int32_t>(c, &pages, sh);
       if ((pages << pshift) <= kPageBytes && c > 0)
         for (int t = tid * chunk * 4; t < min((tid + 1) * chunk * 4, npages); t++)
           if (dir[t]) {
@@ -1244,7 +1380,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6))) void k
           mask |= ((used[4 * w + q] * 0x01020408u) >> 24 & 15u) << (4 * q);
       }
       int32_t n = 0;
-      const int32_t base = ns + group_exclusive(__popc(mask), &n, sh);
+      const int32_t base = ns + block_exclusive<int32_t>(__popc(mask), &n, sh);
       if (w < nwords) table[w] = mask | static_cast<uint32_t>(base) << 16;
       ns += n;
     }
@@ -1421,7 +1557,7 @@ template <bool CUT, bool POS_LDS, bool ORDER>
 __global__ __launch_bounds__(512) void k_tile_slices(
     const int32_t* __restrict__ desc, int32_t nblocks, const int32_t* __restrict__ slot_ptr,
     int32_t* __restrict__ inner, uint16_t* __restrict__ local, CutDev cut, int32_t grows,
-    int32_t stride, int32_t lanes, int32_t wpb, int32_t scale,
+    int32_t stride, int32_t lanes, int32_t wpb, int32_t scale, int32_t pad,
     const int32_t* __restrict__ wave_off, uint16_t* __restrict__ sliced) {
   extern __shared__ double slice_lds[];
   __shared__ int32_t start[kSliceRows], len[kSliceRows], in_len[kSliceRows];
@@ -1436,6 +1572,10 @@ __global__ __launch_bounds__(512) void k_tile_slices(
   const int lsh = 31 - __clz(lanes);
   const int rpw = 64 >> lsh;  // rows per wavefront
   const int64_t st = cut.q.stride;
+  // The kernels' offset prefetch reads past the last slice.
+  if (blockIdx.x == 0)
+    for (int t = tid; t < pad; t += nt)
+      sliced[wave_off[static_cast<int64_t>(nblocks) * wpb] + t] = 0;
   for (int32_t b = blockIdx.x; b < nblocks; b += gridDim.x) {
     const int32_t* d = desc + 8 * static_cast<int64_t>(b);
     const int32_t i0 = d[0], ni = d[1], soff = d[2], ns = d[3];
@@ -1589,7 +1729,7 @@ __global__ __launch_bounds__(kBlock) void k_half_places(
   }
 }
 
-// The rows of each slot, in any order, then ascending.
+// The rows of each slot, in arrival order, then ascending (k_half_sort, a few rows each).
 __global__ __launch_bounds__(kBlock) void k_half_fill(
     int32_t nblocks, const int32_t* __restrict__ desc, const int32_t* __restrict__ keys,
     const int32_t* __restrict__ first_row, const int32_t* __restrict__ first,
@@ -1641,6 +1781,19 @@ __global__ void k_check_replicas(int32_t n, const int32_t* __restrict__ nop,
   }
 }
 
+__global__ void k_half_sort(int32_t n, const int32_t* __restrict__ first,
+                            int32_t* __restrict__ at) {
+  const int64_t c = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+  if (c >= n) return;
+  const int32_t a = first[c], b = first[c + 1];
+  for (int32_t k = a + 1; k < b; k++) {
+    const int32_t v = at[k];
+    int32_t m = k;
+    for (; m > a && at[m - 1] > v; m--) at[m] = at[m - 1];
+    at[m] = v;
+  }
+}
+
 // Spatial tile order: bins of one system (dev_tile_order).
 struct OrderGrid {
   double w[3];     // bin widths: x bins, y and z columns
@@ -1649,12 +1802,12 @@ struct OrderGrid {
   int32_t key0;    // first key of the system
 };
 
-__global__ void k_order_key(int32_t n, PosIn q, const OrderGrid* __restrict__ grids,
+__global__ void k_order_key(int32_t n, PosIn q, OrderGrid one, const OrderGrid* __restrict__ grids,
                             const int32_t* __restrict__ rep_of, int32_t* __restrict__ count,
                             int32_t* __restrict__ slot, int32_t* __restrict__ key_of) {
   for (int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; t < n;
        t += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    const OrderGrid g = grids[rep_of ? rep_of[t] : 0];
+    const OrderGrid g = rep_of ? grids[rep_of[t]] : one;
     const int64_t o = t * q.stride;
     const int cx = cell_coord(q.x[o], 0.0, g.w[0], g.nc[0], g.box);
     const int cy = cell_coord(q.y[o], 0.0, g.w[1], g.nc[1], g.box);
@@ -1665,75 +1818,37 @@ __global__ void k_order_key(int32_t n, PosIn q, const OrderGrid* __restrict__ gr
   }
 }
 
-__global__ void k_order_scatter(int32_t n, const int32_t* __restrict__ key_of,
-                                const int32_t* __restrict__ slot,
-                                const int32_t* __restrict__ start, int32_t* __restrict__ order) {
-  for (int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; t < n;
-       t += static_cast<int64_t>(gridDim.x) * blockDim.x)
-    order[start[key_of[t]] + slot[t]] = static_cast<int32_t>(t);
-}
-
-// Each bin's particles by ascending index (insertion sort, one thread per
-// bin; bins hold at most kCellOrderMax particles).
-__global__ void k_order_sort(int64_t nkey, const int32_t* __restrict__ start,
-                             int32_t* __restrict__ order) {
-  for (int64_t c = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; c < nkey;
-       c += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    const int32_t a = start[c], b = start[c + 1];
-    for (int32_t k = a + 1; k < b; k++) {
-      const int32_t v = order[k];
-      int32_t m = k;
-      while (m > a && order[m - 1] > v) {
-        order[m] = order[m - 1];
-        m--;
-      }
-      order[m] = v;
-    }
-  }
-}
-
-// slot_of[member[s]] = s.
-__global__ void k_inverse(int32_t n, const int32_t* __restrict__ member,
-                          int32_t* __restrict__ slot_of) {
-  for (int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; t < n;
-       t += static_cast<int64_t>(gridDim.x) * blockDim.x)
-    slot_of[member[t]] = static_cast<int32_t>(t);
-}
-
-// Each group of slots (geo: first slot, count) reordered by the row length
-// of its particles, longest first, ties in the previous slot order: the
-// wavefronts of a tile then hold rows of similar length, which need similar
-// numbers of batches.
-__global__ __launch_bounds__(kBlock) void k_group_length_sort(const int32_t* __restrict__ geo,
-                                                              int32_t ngroups,
-                                                              const int32_t* __restrict__ nop,
-                                                              int32_t* __restrict__ order) {
+// The slots of a spatial order: each block's particles (tile_span) reordered
+// by row length, longest first, ties in the order given (the wavefronts of a
+// tile then hold rows of similar length, which need similar numbers of
+// batches); the particle of each slot, the slot of each particle and each
+// slot's row length.
+__global__ __launch_bounds__(kBlock) void k_tile_slots(TileSpans spans, int32_t nblocks,
+                                                       const int32_t* __restrict__ order,
+                                                       const int32_t* __restrict__ nop,
+                                                       int32_t* __restrict__ member,
+                                                       int32_t* __restrict__ slot_of,
+                                                       int32_t* __restrict__ slot_len) {
   __shared__ int32_t mem[kTileRowsMax];
   __shared__ int32_t len[kTileRowsMax];
-  for (int32_t b = blockIdx.x; b < ngroups; b += gridDim.x) {
-    const int32_t i0 = geo[4 * b], ni = geo[4 * b + 1];
-    for (int32_t t = threadIdx.x; t < ni; t += blockDim.x) {
-      const int32_t i = order[i0 + t];
+  for (int32_t b = blockIdx.x; b < nblocks; b += gridDim.x) {
+    const TileSpan g = tile_span(spans, b);
+    for (int32_t t = threadIdx.x; t < g.ni; t += blockDim.x) {
+      const int32_t i = order[g.i0 + t];
       mem[t] = i;
       len[t] = nop[i];
     }
     __syncthreads();
-    for (int32_t t = threadIdx.x; t < ni; t += blockDim.x) {
+    for (int32_t t = threadIdx.x; t < g.ni; t += blockDim.x) {
       const int32_t l = len[t];
-      int32_t r = 0;
-      for (int32_t u = 0; u < ni; u++) r += len[u] > l || (len[u] == l && u < t);
-      order[i0 + r] = mem[t];
+      int32_t r = g.i0;
+      for (int32_t u = 0; u < g.ni; u++) r += len[u] > l || (len[u] == l && u < t);
+      member[r] = mem[t];
+      slot_of[mem[t]] = r;
+      slot_len[r] = l;
     }
     __syncthreads();
   }
-}
-
-// Row length of the particle in each slot.
-__global__ void k_slot_nop(int32_t n, const int32_t* __restrict__ member,
-                           const int32_t* __restrict__ nop, int32_t* __restrict__ out) {
-  for (int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; t < n;
-       t += static_cast<int64_t>(gridDim.x) * blockDim.x)
-    out[t] = nop[member[t]];
 }
 
 }  // namespace
@@ -1796,26 +1911,47 @@ void dev_release(ListWork& w) {
                     &w.tile_geo, &w.rep_of, &w.order, &w.order_grid, &w.slot_of})
     dev_release(*m);
   dev_release(w.part);
+  if (w.results) (void)hipHostFree(w.results);
+  w.results = nullptr;
+}
+
+// The host-visible results (pinned memory that kernels write): a result is
+// valid once the stream has been synchronised after its kernel.
+int results(ListWork& w) {
+  if (!w.results)
+    LTRY(hipHostMalloc(reinterpret_cast<void**>(&w.results), sizeof(ListResults), hipHostMallocDefault),
+         "hipHostMalloc");
+  return LJGPU_OK;
+}
+
+int dev_scan_async(hipStream_t s, const int32_t* in, int32_t* out, int64_t n, ListWork& w,
+                   ScanStats* res) {
+  if (n <= kScanSmall) {
+    k_scan_small<<<1, 1024, 0, s>>>(in, static_cast<int32_t>(n), out, res);
+    LTRY(hipGetLastError(), "scan kernel");
+    return LJGPU_OK;
+  }
+  const int64_t nb = (n + kScanTile - 1) / kScanTile;
+  LCHECK(dev_reserve(w.scan_sums, sizeof(ScanTile) * nb, s));
+  ScanTile* tiles = w.scan_sums.as<ScanTile>();
+  k_scan_reduce<<<static_cast<int>(nb), kBlock, 0, s>>>(in, n, tiles);
+  if (nb > kScanTiles) {
+    k_scan_sums<<<1, kBlock, 0, s>>>(tiles, nb);
+    k_scan_apply<true><<<static_cast<int>(nb), kBlock, 0, s>>>(in, n, tiles, out, res);
+  } else {
+    k_scan_apply<false><<<static_cast<int>(nb), kBlock, 0, s>>>(in, n, tiles, out, res);
+  }
+  LTRY(hipGetLastError(), "scan kernels");
+  return LJGPU_OK;
 }
 
 int dev_scan(hipStream_t s, const int32_t* in, int32_t* out, int64_t n, ListWork& w,
              int64_t* total) {
   *total = 0;
-  if (n <= 0) {
-    LCHECK(fill<int32_t>(s, out, 1, 0));
-    return LJGPU_OK;
-  }
-  const int64_t nb = (n + kScanTile - 1) / kScanTile;
-  LCHECK(dev_reserve(w.scan_sums, sizeof(int64_t) * nb, s));
-  LCHECK(dev_reserve(w.small, sizeof(int64_t) * 8, s));
-  int64_t* sums = w.scan_sums.as<int64_t>();
-  int64_t* tot = w.small.as<int64_t>();
-  k_scan_reduce<<<static_cast<int>(nb), kBlock, 0, s>>>(in, n, sums);
-  k_scan_sums<<<1, kBlock, 0, s>>>(sums, nb, tot);
-  k_scan_apply<<<static_cast<int>(nb), kBlock, 0, s>>>(in, n, sums, tot, out);
-  LTRY(hipGetLastError(), "scan kernels");
-  LTRY(hipMemcpyAsync(total, tot, sizeof(int64_t), hipMemcpyDeviceToHost, s), "hipMemcpyAsync");
+  LCHECK(results(w));
+  LCHECK(dev_scan_async(s, in, out, std::max<int64_t>(n, 0), w, &w.results->scan));
   LTRY(hipStreamSynchronize(s), "hipStreamSynchronize");
+  *total = w.results->scan.total;
   return LJGPU_OK;
 }
 
@@ -1903,6 +2039,7 @@ int dev_makepair(hipStream_t s, const PosIn& q, int32_t n, double box, double se
   out.n = n;
   LCHECK(dev_reserve(out.nop, sizeof(int32_t) * std::max(n, 1), s));
   LCHECK(dev_reserve(out.ptr, sizeof(int32_t) * (static_cast<size_t>(n) + 1), s));
+  w.row_min = w.row_max = 0;
   if (n == 0) {
     out.e = 0;
     LCHECK(dev_reserve(out.list, sizeof(int32_t), s));
@@ -1949,37 +2086,31 @@ int dev_makepair(hipStream_t s, const PosIn& q, int32_t n, double box, double se
   LCHECK(dev_reserve(w.cpos, sizeof(double4) * n, s));
   int32_t* count = w.cell_count.as<int32_t>();
   int32_t* cstart = w.cell_start.as<int32_t>();
-  LCHECK(fill<int32_t>(s, count, ncell, 0));
-  LCHECK(dev_reserve(w.small, sizeof(int64_t) * 8, s));
-  int32_t* outside = w.small.as<int32_t>() + 12;
-  LCHECK(fill<int32_t>(s, outside, 1, 0));
+  int32_t* outside = count + ncell;
+  LCHECK(fill<int32_t>(s, count, ncell + 1, 0));
+  LCHECK(results(w));
   k_cell_assign<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, q, g, count, w.cell_slot.as<int32_t>(),
                                                        w.cell_of.as<int32_t>(), outside);
   LTRY(hipGetLastError(), "cell assign kernel");
-  int64_t total = 0;
-  LCHECK(dev_scan(s, count, cstart, ncell, w, &total));
-  k_cell_scatter<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, q, w.cell_of.as<int32_t>(),
-                                                        w.cell_slot.as<int32_t>(), cstart,
-                                                        w.cpos.as<double4>(),
-                                                        w.cell_sorted.as<int32_t>());
-  LTRY(hipGetLastError(), "cell scatter kernel");
+  LCHECK(dev_scan_async(s, count, cstart, ncell, w, &w.results->cells));
   const bool half = kind == LJGPU_LIST_HALF;
   const int R = cg.brute ? 0 : (fine ? 2 : 1);
   // Unsorted rows need a candidate order fixed by the positions alone: the
   // stencil kernel's run order with each cell's particles by index. The
   // single-cell kernel has no such order, so it always sorts.
   if (R == 0) sort_rows = true;
-  if (!sort_rows) {
-    // The per-cell insertion sort is quadratic in the cell's population:
-    // crowded cells (a collapsed or clustered system) sort rows instead.
-    int32_t cmin = 0, cmax = 0;
-    LCHECK(dev_minmax(s, count, static_cast<int32_t>(ncell), w, &cmin, &cmax));
-    if (cmax > kCellOrderMax) sort_rows = true;
+  if (sort_rows) {
+    k_cell_scatter<<<grid_for(n, kBlock), kBlock, 0, s>>>(
+        n, q, w.cell_of.as<int32_t>(), w.cell_slot.as<int32_t>(), cstart, w.cpos.as<double4>(),
+        w.cell_sorted.as<int32_t>());
+  } else {
+    int32_t* arrival = w.cell_sorted.as<int32_t>();
+    k_bin_index<<<grid_for(n, kBlock), kBlock, 0, s>>>(
+        n, w.cell_of.as<int32_t>(), w.cell_slot.as<int32_t>(), cstart, arrival);
+    k_cell_place<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, q, w.cell_of.as<int32_t>(), cstart,
+                                                        arrival, w.cpos.as<double4>());
   }
-  if (!sort_rows) {
-    k_cell_order<<<grid_for(ncell, kBlock), kBlock, 0, s>>>(ncell, cstart, w.cpos.as<double4>());
-    LTRY(hipGetLastError(), "cell order kernel");
-  }
+  LTRY(hipGetLastError(), "cell scatter kernels");
   const int grid = grid_for(n, kBlock, INT32_MAX);
   const int wave_grid = grid_for(ncell * 64, kBlock);  // one wavefront per cell, grid-stride
   auto pairs = [&](auto mode_tag, int32_t cap, int32_t* nop, const int32_t* ptr, int32_t* outl) {
@@ -2020,19 +2151,22 @@ int dev_makepair(hipStream_t s, const PosIn& q, int32_t n, double box, double se
     cap = (cap + 31) / 32 * 32;
     if (static_cast<double>(n) * cap * 4.0 > 16.0 * (1u << 30)) cap = 0;
   }
-  int32_t mx = 0;
   if (cap > 0) {
     LCHECK(dev_reserve(w.tmp, sizeof(int32_t) * static_cast<size_t>(n) * cap, s));
     pairs(std::integral_constant<int, 2>{}, cap, out.nop.as<int32_t>(), nullptr,
           w.tmp.as<int32_t>());
     LTRY(hipGetLastError(), "pair kernel");
-    int32_t mn = 0;
-    LCHECK(dev_minmax(s, out.nop.as<int32_t>(), n, w, &mn, &mx));
   } else {
     pairs(std::integral_constant<int, 0>{}, 0, out.nop.as<int32_t>(), nullptr, nullptr);
     LTRY(hipGetLastError(), "pair count kernel");
   }
+  int64_t total = 0;
   LCHECK(dev_scan(s, out.nop.as<int32_t>(), out.ptr.as<int32_t>(), n, w, &total));
+  const int32_t mx = w.results->scan.hi;
+  w.row_min = w.results->scan.lo;
+  w.row_max = mx;
+  // Crowded cells (a collapsed or clustered system) are not in index order.
+  if (w.results->cells.hi > kCellOrderMax) sort_rows = true;
   if (total > INT32_MAX) return set_error(LJGPU_ERR_CAPACITY, "list longer than 2^31-1 entries");
   out.e = total;
   LCHECK(dev_reserve(out.list, sizeof(int32_t) * std::max<int64_t>(total, 1), s));
@@ -2106,15 +2240,19 @@ int dev_make_ell(hipStream_t s, const DevCSR& c, int32_t width, DevMem& ell) {
   return LJGPU_OK;
 }
 
-int dev_tile_order(hipStream_t s, const PosIn& q, int32_t n, double box,
-                   const std::vector<int32_t>& replicas, const std::vector<double>& boxes,
-                   int32_t T, ListWork& w, bool* ok) {
-  *ok = false;
+int dev_tile_order_begin(hipStream_t s, const PosIn& q, int32_t n, double box,
+                         const std::vector<int32_t>& replicas, const std::vector<double>& boxes,
+                         int32_t T, ListWork& w, bool* begun) {
+  *begun = false;
   if (n <= 0 || T <= 0) return LJGPU_OK;
   const std::vector<int32_t> single = {0, n};
   const std::vector<int32_t>& off = replicas.empty() ? single : replicas;
   const int32_t nsys = static_cast<int32_t>(off.size()) - 1;
-  std::vector<OrderGrid> grids(nsys);
+  // Kept: the upload below reads it after this returns.
+  std::vector<char>& store = w.order_host;
+  const size_t gbytes = (sizeof(OrderGrid) * nsys + 255) / 256 * 256;
+  store.resize(gbytes + sizeof(int32_t) * off.size());
+  OrderGrid* grids = reinterpret_cast<OrderGrid*>(store.data());
   int64_t keys = 0;
   for (int32_t r = 0; r < nsys; r++) {
     const double L = replicas.empty() ? box : boxes[r];
@@ -2143,15 +2281,16 @@ int dev_tile_order(hipStream_t s, const PosIn& q, int32_t n, double box,
     keys += static_cast<int64_t>(g.nc[0]) * g.nc[1] * g.nc[2];
     if (keys > INT32_MAX - 1) return LJGPU_OK;
   }
-  const size_t gbytes = (sizeof(OrderGrid) * grids.size() + 255) / 256 * 256;
-  LCHECK(dev_reserve(w.order_grid, gbytes + sizeof(int32_t) * off.size(), s));
-  LTRY(hipMemcpyAsync(w.order_grid.p, grids.data(), sizeof(OrderGrid) * grids.size(),
-                      hipMemcpyHostToDevice, s), "hipMemcpyAsync");
   const int32_t* rep_of = nullptr;
+  const OrderGrid* dgrids = nullptr;
   if (!replicas.empty()) {
-    int32_t* doff = reinterpret_cast<int32_t*>(static_cast<char*>(w.order_grid.p) + gbytes);
-    LTRY(hipMemcpyAsync(doff, off.data(), sizeof(int32_t) * off.size(), hipMemcpyHostToDevice, s),
+    std::memcpy(store.data() + gbytes, off.data(), sizeof(int32_t) * off.size());
+    LCHECK(dev_reserve(w.order_grid, store.size(), s));
+    LTRY(hipMemcpyAsync(w.order_grid.p, store.data(), store.size(), hipMemcpyHostToDevice, s),
          "hipMemcpyAsync");
+    dgrids = static_cast<const OrderGrid*>(w.order_grid.p);
+    const int32_t* doff =
+        reinterpret_cast<const int32_t*>(static_cast<const char*>(w.order_grid.p) + gbytes);
     LCHECK(dev_reserve(w.rep_of, sizeof(int32_t) * n, s));
     k_replica_of<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, doff, nsys, w.rep_of.as<int32_t>());
     LTRY(hipGetLastError(), "replica index kernel");
@@ -2161,105 +2300,104 @@ int dev_tile_order(hipStream_t s, const PosIn& q, int32_t n, double box,
   LCHECK(dev_reserve(w.cell_start, sizeof(int32_t) * (keys + 1), s));
   LCHECK(dev_reserve(w.cell_slot, sizeof(int32_t) * n, s));
   LCHECK(dev_reserve(w.cell_of, sizeof(int32_t) * n, s));
+  LCHECK(dev_reserve(w.cell_sorted, sizeof(int32_t) * n, s));
   LCHECK(dev_reserve(w.order, sizeof(int32_t) * n, s));
+  LCHECK(results(w));
   int32_t* count = w.cell_count.as<int32_t>();
+  int32_t* start = w.cell_start.as<int32_t>();
+  int32_t* arrival = w.cell_sorted.as<int32_t>();
+  const int32_t* key_of = w.cell_of.as<int32_t>();
   LCHECK(fill<int32_t>(s, count, keys, 0));
-  k_order_key<<<grid_for(n, kBlock), kBlock, 0, s>>>(
-      n, q, static_cast<const OrderGrid*>(w.order_grid.p), rep_of, count,
-      w.cell_slot.as<int32_t>(), w.cell_of.as<int32_t>());
+  k_order_key<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, q, grids[0], dgrids, rep_of, count,
+                                                     w.cell_slot.as<int32_t>(),
+                                                     w.cell_of.as<int32_t>());
   LTRY(hipGetLastError(), "tile order key kernel");
-  int32_t kmin = 0, kmax = 0;
-  LCHECK(dev_minmax(s, count, static_cast<int32_t>(keys), w, &kmin, &kmax));
-  if (kmax > kCellOrderMax) return LJGPU_OK;  // a crowded bin: keep index order
-  int64_t total = 0;
-  LCHECK(dev_scan(s, count, w.cell_start.as<int32_t>(), keys, w, &total));
-  k_order_scatter<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, w.cell_of.as<int32_t>(),
-                                                         w.cell_slot.as<int32_t>(),
-                                                         w.cell_start.as<int32_t>(),
-                                                         w.order.as<int32_t>());
-  k_order_sort<<<grid_for(keys, kBlock), kBlock, 0, s>>>(keys, w.cell_start.as<int32_t>(),
-                                                         w.order.as<int32_t>());
+  LCHECK(dev_scan_async(s, count, start, keys, w, &w.results->order));
+  k_bin_index<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, key_of, w.cell_slot.as<int32_t>(), start,
+                                                     arrival);
+  k_order_place<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, key_of, start, arrival,
+                                                       w.order.as<int32_t>());
   LTRY(hipGetLastError(), "tile order kernels");
-  *ok = true;
+  *begun = true;
   return LJGPU_OK;
 }
 
-int dev_length_sort(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<int32_t>& reps,
-                    ListWork& w) {
-  if (T <= 0 || T > kTileRowsMax || c.n <= 0) return LJGPU_OK;
-  // The groups are dev_make_tiles's blocks of T consecutive slots.
-  std::vector<int32_t> geo;
-  const std::vector<int32_t> single = {0, c.n};
-  const std::vector<int32_t>& off = reps.empty() ? single : reps;
-  for (size_t r = 0; r + 1 < off.size(); r++)
-    for (int32_t i0 = off[r]; i0 < off[r + 1]; i0 += T)
-      geo.insert(geo.end(), {i0, std::min(T, off[r + 1] - i0), 0, 0});
-  const int32_t ng = static_cast<int32_t>(geo.size() / 4);
-  if (ng == 0) return LJGPU_OK;
-  LCHECK(dev_reserve(w.tile_geo, sizeof(int32_t) * geo.size(), s));
-  LTRY(hipMemcpyAsync(w.tile_geo.p, geo.data(), sizeof(int32_t) * geo.size(),
-                      hipMemcpyHostToDevice, s), "hipMemcpyAsync");
-  k_group_length_sort<<<std::min(ng, 65535), kBlock, 0, s>>>(
-      w.tile_geo.as<int32_t>(), ng, c.nop.as<int32_t>(), w.order.as<int32_t>());
-  LTRY(hipGetLastError(), "tile length sort kernel");
-  // The upload's host vector must outlive the copy.
+bool dev_tile_order_end(const ListWork& w) {
+  return w.results->order.hi <= kCellOrderMax;  // a crowded bin: keep index order
+}
+
+int dev_tile_order(hipStream_t s, const PosIn& q, int32_t n, double box,
+                   const std::vector<int32_t>& replicas, const std::vector<double>& boxes,
+                   int32_t T, ListWork& w, bool* ok) {
+  LCHECK(dev_tile_order_begin(s, q, n, box, replicas, boxes, T, w, ok));
+  if (!*ok) return LJGPU_OK;
   LTRY(hipStreamSynchronize(s), "hipStreamSynchronize");
+  *ok = dev_tile_order_end(w);
   return LJGPU_OK;
+}
+
+// The blocks of T consecutive slots, restarted at every replica boundary.
+int tile_spans(hipStream_t s, int32_t n, int32_t T, const std::vector<int32_t>& reps, ListWork& w,
+               TileSpans* spans, int32_t* nblocks) {
+  *spans = TileSpans{nullptr, T, n};
+  *nblocks = (n + T - 1) / T;
+  if (reps.empty()) return LJGPU_OK;
+  // Kept: the upload reads it after this returns. One not yet read must not
+  // be written over.
+  std::vector<int32_t>& geo = w.geo_host;
+  if (!geo.empty()) LTRY(hipStreamSynchronize(s), "hipStreamSynchronize");
+  geo.clear();
+  for (size_t r = 0; r + 1 < reps.size(); r++)
+    for (int32_t i0 = reps[r]; i0 < reps[r + 1]; i0 += T)
+      geo.insert(geo.end(), {i0, std::min(T, reps[r + 1] - i0), static_cast<int32_t>(r), 0});
+  *nblocks = static_cast<int32_t>(geo.size() / 4);
+  LCHECK(dev_reserve(w.tile_geo, sizeof(int32_t) * std::max<size_t>(geo.size(), 1), s));
+  if (!geo.empty())
+    LTRY(hipMemcpyAsync(w.tile_geo.p, geo.data(), sizeof(int32_t) * geo.size(),
+                        hipMemcpyHostToDevice, s), "hipMemcpyAsync");
+  spans->geo = w.tile_geo.as<int32_t>();
+  return LJGPU_OK;
+}
+
+int dev_tile_slots(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<int32_t>& reps,
+                   ListWork& w, DevTiles& out) {
+  TileSpans spans;
+  int32_t nb = 0;
+  LCHECK(tile_spans(s, c.n, T, reps, w, &spans, &nb));
+  LCHECK(dev_reserve(out.member, sizeof(int32_t) * c.n, s));
+  LCHECK(dev_reserve(out.slot_ptr, sizeof(int32_t) * (static_cast<size_t>(c.n) + 1), s));
+  LCHECK(dev_reserve(w.slot_of, sizeof(int32_t) * c.n, s));
+  LCHECK(dev_reserve(w.counts, sizeof(int32_t) * (static_cast<size_t>(c.n) + 1), s));
+  k_tile_slots<<<std::max(1, std::min(nb, 65535)), kBlock, 0, s>>>(
+      spans, nb, w.order.as<int32_t>(), c.nop.as<int32_t>(), out.member.as<int32_t>(),
+      w.slot_of.as<int32_t>(), w.counts.as<int32_t>());
+  LTRY(hipGetLastError(), "tile slot kernel");
+  return dev_scan_async(s, w.counts.as<int32_t>(), out.slot_ptr.as<int32_t>(), c.n, w, nullptr);
 }
 
 int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<int32_t>& reps,
-                   const int32_t* member, ListWork& w, DevTiles& out) {
+                   bool spatial, ListWork& w, DevTiles& out) {
   out.tile_particles = 0;
   out.blocks = 0;
   if (T <= 0 || T > kTileRowsMax || c.n <= 0) return LJGPU_OK;
   // The slot order and each slot's row start in the slot-ordered rows.
   // Index order: slot = particle and the list's own row starts. Otherwise
-  // the slot order, the slot of each particle (blocks key their particles
-  // by slot) and each slot's row start in the rows stored in slot order.
-  out.order = member ? LJGPU_TILE_ORDER_SPATIAL : LJGPU_TILE_ORDER_INDEX;
-  const int32_t* mem = nullptr;
-  const int32_t* slot_of = nullptr;
-  const int32_t* sptr = c.ptr.as<int32_t>();
-  if (member) {
-    LCHECK(dev_reserve(out.member, sizeof(int32_t) * c.n, s));
-    LCHECK(dev_reserve(out.slot_ptr, sizeof(int32_t) * (static_cast<size_t>(c.n) + 1), s));
-    LCHECK(dev_reserve(w.slot_of, sizeof(int32_t) * c.n, s));
-    LCHECK(dev_reserve(w.counts, sizeof(int32_t) * (static_cast<size_t>(c.n) + 1), s));
-    int32_t* m = out.member.as<int32_t>();
-    LTRY(hipMemcpyAsync(m, member, sizeof(int32_t) * c.n, hipMemcpyDeviceToDevice, s),
-         "hipMemcpyAsync");
-    k_inverse<<<grid_for(c.n, kBlock), kBlock, 0, s>>>(c.n, m, w.slot_of.as<int32_t>());
-    k_slot_nop<<<grid_for(c.n, kBlock), kBlock, 0, s>>>(c.n, m, c.nop.as<int32_t>(),
-                                                         w.counts.as<int32_t>());
-    LTRY(hipGetLastError(), "tile order kernels");
-    int64_t e = 0;
-    LCHECK(dev_scan(s, w.counts.as<int32_t>(), out.slot_ptr.as<int32_t>(), c.n, w, &e));
-    if (e != c.e) return set_error(LJGPU_ERR_HIP, "tile order is not a permutation of the rows");
-    mem = m;
-    slot_of = w.slot_of.as<int32_t>();
-    sptr = out.slot_ptr.as<int32_t>();
-  }
-  // Blocks of T consecutive slots, restarted at every replica boundary.
-  std::vector<int32_t> geo;
-  const std::vector<int32_t> single = {0, c.n};
-  const std::vector<int32_t>& off = reps.empty() ? single : reps;
-  for (size_t r = 0; r + 1 < off.size(); r++)
-    for (int32_t i0 = off[r]; i0 < off[r + 1]; i0 += T)
-      geo.insert(geo.end(), {i0, std::min(T, off[r + 1] - i0), static_cast<int32_t>(r), 0});
-  const int32_t nb = static_cast<int32_t>(geo.size() / 4);
+  // dev_tile_slots's (blocks key their particles by slot).
+  out.order = spatial ? LJGPU_TILE_ORDER_SPATIAL : LJGPU_TILE_ORDER_INDEX;
+  const int32_t* member = spatial ? out.member.as<int32_t>() : nullptr;
+  const int32_t* slot_of = spatial ? w.slot_of.as<int32_t>() : nullptr;
+  const int32_t* sptr = spatial ? out.slot_ptr.as<int32_t>() : c.ptr.as<int32_t>();
+  TileSpans spans;
+  int32_t nb = 0;
+  LCHECK(tile_spans(s, c.n, T, reps, w, &spans, &nb));
   if (nb == 0) return LJGPU_OK;
-  LCHECK(dev_reserve(w.tile_geo, sizeof(int32_t) * geo.size(), s));
-  LTRY(hipMemcpyAsync(w.tile_geo.p, geo.data(), sizeof(int32_t) * geo.size(),
-                      hipMemcpyHostToDevice, s), "hipMemcpyAsync");
-  const int32_t* dgeo = w.tile_geo.as<int32_t>();
-  LCHECK(dev_reserve(w.small, sizeof(int64_t) * 8, s));
+  LCHECK(results(w));
   LCHECK(dev_reserve(w.tile_stats, sizeof(int4) * static_cast<size_t>(nb), s));
   int4* stats = w.tile_stats.as<int4>();
   const int grid = std::min(nb, 65535);
   // The force kernel copies entry offsets in whole 16-byte chunks: pad.
   const int64_t nlocal = c.e + kTileLocalPad;
   LCHECK(dev_reserve(out.local, sizeof(uint16_t) * nlocal, s));
-  LCHECK(fill<uint16_t>(s, out.local.as<uint16_t>() + c.e, kTileLocalPad, 0));
   LCHECK(dev_reserve(out.desc, sizeof(int32_t) * 8 * static_cast<size_t>(nb), s));
   // One pass when every block can own kTileMaxStage staging slots within
   // kTileOnePassBytes (and the offsets fit int32); otherwise count, scan, fill.
@@ -2276,10 +2414,10 @@ int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<
       kTileCodeMax, (c.e / c.n + 1) * T * 5 / 4 + 64));
   const size_t code_bytes = sizeof(uint16_t) * ecap;
   auto read_stats = [&](int32_t (&back)[8]) -> int {
-    k_tile_stats<<<1, 1024, 0, s>>>(nb, stats, w.small.as<int32_t>());
+    k_tile_stats<<<1, 1024, 0, s>>>(nb, stats, out.local.as<uint16_t>() + c.e, w.results->tiles);
     LTRY(hipGetLastError(), "tile stats kernel");
-    LTRY(hipMemcpyAsync(back, w.small.p, sizeof(back), hipMemcpyDeviceToHost, s), "hipMemcpyAsync");
     LTRY(hipStreamSynchronize(s), "hipStreamSynchronize");
+    std::copy(w.results->tiles, w.results->tiles + 8, back);
     return LJGPU_OK;
   };
   if (one_pass) {
@@ -2294,12 +2432,12 @@ int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<
     for (int pass = 0; pass < 2; pass++) {
       if (pass == 0)
         k_tile_pages<<<grid, std::min(512, std::max(256, T * kPageLanes)), (npages + 15) / 16 * 16, s>>>(
-            dgeo, nb, mem, slot_of, sptr, c.ptr.as<int32_t>(), c.list.as<int32_t>(), pshift,
+            spans, nb, member, slot_of, sptr, c.ptr.as<int32_t>(), c.list.as<int32_t>(), pshift,
             npages, out.desc.as<int32_t>(), out.stage.as<int32_t>(),
             member ? out.stage_slot.as<int32_t>() : nullptr, out.local.as<uint16_t>(), stats);
       else
         k_tile_fill<false><<<grid, threads, code_bytes, s>>>(
-            dgeo, nb, mem, slot_of, sptr, c.ptr.as<int32_t>(), c.list.as<int32_t>(), nullptr, ecap,
+            spans, nb, member, slot_of, sptr, c.ptr.as<int32_t>(), c.list.as<int32_t>(), nullptr, ecap,
             nullptr, out.desc.as<int32_t>(), out.stage.as<int32_t>(),
             member ? out.stage_slot.as<int32_t>() : nullptr, out.local.as<uint16_t>(), stats);
       LTRY(hipGetLastError(), "tile fill kernel");
@@ -2316,7 +2454,7 @@ int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<
     LCHECK(dev_reserve(w.tile_ns, sizeof(int32_t) * (static_cast<size_t>(nb) + 1), s));
     LCHECK(dev_reserve(w.tile_soff, sizeof(int32_t) * (static_cast<size_t>(nb) + 1), s));
     k_tile_fill<true><<<grid, threads, 0, s>>>(
-        dgeo, nb, mem, slot_of, sptr, c.ptr.as<int32_t>(), c.list.as<int32_t>(), nullptr, 0,
+        spans, nb, member, slot_of, sptr, c.ptr.as<int32_t>(), c.list.as<int32_t>(), nullptr, 0,
         w.tile_ns.as<int32_t>(), nullptr, nullptr, nullptr, nullptr, stats);
     LTRY(hipGetLastError(), "tile count kernel");
     int32_t back[8];
@@ -2331,7 +2469,7 @@ int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<
     if (member)
       LCHECK(dev_reserve(out.stage_slot, sizeof(int32_t) * std::max<int64_t>(staged, 1), s));
     k_tile_fill<false><<<grid, threads, code_bytes, s>>>(
-        dgeo, nb, mem, slot_of, sptr, c.ptr.as<int32_t>(), c.list.as<int32_t>(),
+        spans, nb, member, slot_of, sptr, c.ptr.as<int32_t>(), c.list.as<int32_t>(),
         w.tile_soff.as<int32_t>(), ecap, nullptr, out.desc.as<int32_t>(),
         out.stage.as<int32_t>(), member ? out.stage_slot.as<int32_t>() : nullptr,
         out.local.as<uint16_t>(), stats);
@@ -2365,13 +2503,18 @@ int dev_slice_tiles(hipStream_t s, const int32_t* slot_ptr, int32_t lanes, int32
                                                         slot_ptr, lanes, unroll,
                                                         w.counts.as<int32_t>());
   LTRY(hipGetLastError(), "slice length kernel");
-  int64_t total = 0;
-  LCHECK(dev_scan(s, w.counts.as<int32_t>(), t.wave_off.as<int32_t>(), nw, w, &total));
+  // The slices' length is at most every wavefront's with the longest row; read
+  // back only where that would be a waste.
+  const int64_t kb = static_cast<int64_t>(lanes) * unroll;
+  int64_t total = nw * 64 * unroll * ((t.longest + kb - 1) / kb);
+  if (total <= int64_t{1} << 26)
+    LCHECK(dev_scan_async(s, w.counts.as<int32_t>(), t.wave_off.as<int32_t>(), nw, w, nullptr));
+  else
+    LCHECK(dev_scan(s, w.counts.as<int32_t>(), t.wave_off.as<int32_t>(), nw, w, &total));
   // The kernel's offset prefetch reads up to two batches past a slice.
-  const int64_t pad = 2 * 64 * static_cast<int64_t>(unroll) + 64;
+  const int32_t pad = 2 * 64 * unroll + 64;
   if (total + pad > INT32_MAX) return LJGPU_OK;
   LCHECK(dev_reserve(t.sliced, sizeof(uint16_t) * (total + pad), s));
-  LCHECK(fill<uint16_t>(s, t.sliced.as<uint16_t>() + total, pad, 0));
   CutDev cd{};
   const bool cut = bank_order && hint && hint->q.x && !t.cut;
   if (cut) {
@@ -2403,7 +2546,7 @@ int dev_slice_tiles(hipStream_t s, const int32_t* slot_ptr, int32_t lanes, int32
   kernel<<<std::min(t.blocks, 65535), 512, rows + std::max(order, pos_lds ? pos : 0), s>>>(
       t.desc.as<int32_t>(), t.blocks, slot_ptr,
       t.cut || cut ? t.inner.as<int32_t>() : nullptr, t.local.as<uint16_t>(), cd, grows, stride,
-      lanes, wpb, scale, t.wave_off.as<int32_t>(), t.sliced.as<uint16_t>());
+      lanes, wpb, scale, pad, t.wave_off.as<int32_t>(), t.sliced.as<uint16_t>());
   LTRY(hipGetLastError(), "tile slice kernel");
   if (cut) t.cut = true;
   t.sliced_lanes = lanes;
@@ -2441,7 +2584,7 @@ int dev_half_tiles(hipStream_t s, int32_t n, ListWork& w, DevTiles& t) {
   LCHECK(fill<int32_t>(s, count, n, 0));
   k_half_fill<<<grid, kBlock, 0, s>>>(nb, desc, keys, w.tile_soff.as<int32_t>(), first, count,
                                       t.half_at.as<int32_t>());
-  k_order_sort<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, first, t.half_at.as<int32_t>());
+  k_half_sort<<<(n + kBlock - 1) / kBlock, kBlock, 0, s>>>(n, first, t.half_at.as<int32_t>());
   LTRY(hipGetLastError(), "half tile fill kernels");
   return LJGPU_OK;
 }

@@ -171,27 +171,38 @@ __global__ __launch_bounds__(kBlock) void k_kinetic(int32_t n, const double* __r
   if (threadIdx.x == 0) partial[blockIdx.x] = t;
 }
 
-// Working copies in slot order: out[s] = in[order[s]] (gather) or
-// out[order[s]] = in[s] (scatter), for 4-double rows and int32 values.
-__global__ void k_gather_rows(int32_t n, const int32_t* __restrict__ order,
-                              const double4* __restrict__ in, double4* __restrict__ out) {
+// The working copies re-sorted: slot s takes old slot order[s]. The positions
+// go to qref, where the displacement check wants them anyway, the momenta to
+// tmp; k_resort_back copies both over the working copies.
+__global__ void k_resort(int32_t n, const int32_t* __restrict__ order,
+                         const double4* __restrict__ q, const double4* __restrict__ p,
+                         const int32_t* __restrict__ perm, double4* __restrict__ qref,
+                         double4* __restrict__ tmp, int32_t* __restrict__ perm_out) {
   for (int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; t < n;
-       t += static_cast<int64_t>(gridDim.x) * blockDim.x)
-    out[t] = in[order[t]];
+       t += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    const int32_t i = order[t];
+    qref[t] = q[i];
+    tmp[t] = p[i];
+    perm_out[t] = perm[i];
+  }
 }
 
+__global__ void k_resort_back(int32_t n, const double4* __restrict__ qref,
+                              const double4* __restrict__ tmp, double4* __restrict__ q,
+                              double4* __restrict__ p) {
+  for (int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; t < n;
+       t += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    q[t] = qref[t];
+    p[t] = tmp[t];
+  }
+}
+
+// Slot order back to the caller's: out[order[s]] = in[s].
 __global__ void k_scatter_rows(int32_t n, const int32_t* __restrict__ order,
                                const double4* __restrict__ in, double4* __restrict__ out) {
   for (int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; t < n;
        t += static_cast<int64_t>(gridDim.x) * blockDim.x)
     out[order[t]] = in[t];
-}
-
-__global__ void k_gather_i32(int32_t n, const int32_t* __restrict__ order,
-                             const int32_t* __restrict__ in, int32_t* __restrict__ out) {
-  for (int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; t < n;
-       t += static_cast<int64_t>(gridDim.x) * blockDim.x)
-    out[t] = in[order[t]];
 }
 
 __global__ void k_iota_i32(int32_t n, int32_t* __restrict__ out) {
@@ -454,28 +465,28 @@ int ljgpu_md_run(ljgpu_ctx* ctx, double* q, double* p, int32_t n, double box,
   TRY(dev_reserve(ctx->md_qref, sizeof(double) * 4 * std::max(n, 1), ctx->stream));
   auto rebuild = [&]() -> int {
     HIP_TRY(hipEventRecord(b0, ctx->stream), "hipEventRecord");
+    bool referenced = false;  // md_qref holds the positions
     if (slots) {
       // Re-sort the working copies: new slot s takes old slot order[s].
       bool ordered = false;
       TRY(dev_tile_order(ctx->stream, in, n, box, {}, {}, order_tile, ctx->work, &ordered));
       if (ordered) {
-        const int32_t* order = ctx->work.order.as<int32_t>();
+        double4* q4 = reinterpret_cast<double4*>(wq);
+        double4* p4 = reinterpret_cast<double4*>(wp);
+        double4* qref = ctx->md_qref.as<double4>();
         double4* tmp = ctx->md_tmp.as<double4>();
-        for (double* w : {wq, wp}) {
-          k_gather_rows<<<grid_n, kBlock, 0, ctx->stream>>>(n, order,
-                                                            reinterpret_cast<double4*>(w), tmp);
-          HIP_TRY(hipMemcpyAsync(w, tmp, row_bytes, hipMemcpyDeviceToDevice, ctx->stream),
-                  "hipMemcpyAsync");
-        }
-        k_gather_i32<<<grid_n, kBlock, 0, ctx->stream>>>(n, order, perm, perm_spare);
+        k_resort<<<grid_n, kBlock, 0, ctx->stream>>>(n, ctx->work.order.as<int32_t>(), q4, p4,
+                                                     perm, qref, tmp, perm_spare);
+        k_resort_back<<<grid_n, kBlock, 0, ctx->stream>>>(n, qref, tmp, q4, p4);
         HIP_TRY(hipGetLastError(), "slot gather kernels");
         std::swap(perm, perm_spare);
+        referenced = true;
       }
     }
     // Rows in the build's own order: the dynamics need the pair set, not
     // the reference's row order, and that order is fixed by the positions.
     TRY(build_list(ctx, in, n, box, search, LJGPU_LIST_FULL, false));
-    if (n > 0)
+    if (n > 0 && !referenced)
       HIP_TRY(hipMemcpyAsync(ctx->md_qref.p, wq, sizeof(double) * 4 * n,
                              hipMemcpyDeviceToDevice, ctx->stream), "hipMemcpyAsync");
     HIP_TRY(hipEventRecord(b1, ctx->stream), "hipEventRecord");
