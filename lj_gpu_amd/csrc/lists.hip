@@ -775,101 +775,92 @@ __device__ __forceinline__ double readlane_d(double v, int lane) {
   return __hiloint2double(hi, lo);
 }
 
-// One wavefront per cell, for cell grids with a stencil (R >= 1). The cell's
-// particles sit one per lane (in groups of 64); the candidates of the
-// (2R+1)^3 cells around it are walked as one flattened sequence, 64 per
-// round, so each candidate is loaded once for all of the cell's particles
-// instead of once per particle. A round's hits for one particle go to
-// consecutive addresses of its row (ballot, then each hit lane's rank among
-// them), so the stores coalesce. The runs of the flattened sequence are the
-// x-rows of the stencil, contiguous in cell order: (2R+1)^2 rows, each split
-// at most once where it wraps around a periodic box (the grid has at least
-// 2R+1 cells per side). Same predicate (within_search, in the same argument
-// order), exclusions and MODEs as k_pairs; a row's entries come out in
-// candidate order and are sorted afterwards.
 // The candidates of one cell (see k_pairs_wave), with the minimum image
 // (IMAGE) or without it: a cell whose stencil does not wrap around the box,
 // with every position inside [0, box), has no pair that the image would
-// shift, so the predicate without it gives the same result.
-template <int MODE, bool HALF, int R, bool IMAGE>
-__device__ __forceinline__ void pairs_cell(int32_t p0, int32_t p1, int32_t total, int32_t pre,
-                                           int32_t rs, int32_t excl,
+// shift, so the predicate without it gives the same result. at(f) is the
+// place in cpos of candidate f < total.
+constexpr int kPairGroup = 5;     // particles of a cell tested together
+constexpr int kPairCand = 1024;   // candidates whose places are kept in LDS
+
+template <int MODE, bool HALF, bool IMAGE, class At>
+__device__ __forceinline__ void pairs_cell(int32_t p0, int32_t p1, int32_t total, At&& at,
                                            const double4* __restrict__ cpos, const GridArgs& g,
                                            double half_box, double sl2, int32_t cap,
                                            int32_t* __restrict__ nop,
                                            const int32_t* __restrict__ ptr,
                                            int32_t* __restrict__ out) {
-  constexpr int kSpan = 2 * R + 1;
-  constexpr int kRuns = 2 * kSpan * kSpan;
   const int lane = threadIdx.x & 63;
-  for (int32_t g0 = p0; g0 < p1; g0 += 64) {
-    const int32_t mg = min(64, p1 - g0);
+  for (int32_t g0 = p0; g0 < p1; g0 += kPairGroup) {
+    const int32_t mg = min(kPairGroup, p1 - g0);
     double4 pi = make_double4(0.0, 0.0, 0.0, 0.0);
     if (lane < mg) pi = cpos[g0 + lane];
     const int32_t iv = static_cast<int32_t>(pi.w);
-    int64_t basev = 0;
-    if (MODE == 1) basev = lane < mg ? ptr[iv] : 0;
-    if (MODE == 2) basev = static_cast<int64_t>(iv) * cap;
-    int32_t cntv = 0;
-    for (int32_t f0 = 0; f0 < total; f0 += 64) {
-      const int32_t f = f0 + lane;
-      const bool live = f < total;
-      // The run holding f: the number of runs ending at or before f.
-      int r = 0;
+    int32_t pv = 0;
+    if (MODE == 1) pv = lane < mg ? ptr[iv] : 0;
+    // The group's particles as scalars.
+    double4 a[kPairGroup];
+    int32_t id[kPairGroup], cnt[kPairGroup];
+    char* row[kPairGroup];
 #pragma unroll
-      for (int bit = 32; bit > 0; bit >>= 1) {
-        const int t = r + bit;
-        const int32_t v = __shfl(pre, min(t, 64) - 1, 64);
-        if (t <= kRuns && v <= f) r = t;
-      }
-      const int rr = min(r, kRuns - 1);
-      const int32_t u = __shfl(rs, rr, 64) + (f - __shfl(excl, rr, 64));
-      // Lanes past the end read candidate 0 (a valid address) and test nothing.
-      const double4 pj = cpos[live ? u : 0];
+    for (int k = 0; k < kPairGroup; k++) {
+      a[k] = make_double4(readlane_d(pi.x, k), readlane_d(pi.y, k), readlane_d(pi.z, k), 0.0);
+      id[k] = __builtin_amdgcn_readlane(iv, k);
+      cnt[k] = 0;
+      if (MODE == 1) row[k] = reinterpret_cast<char*>(out + __builtin_amdgcn_readlane(pv, k));
+      if (MODE == 2) row[k] = reinterpret_cast<char*>(out + static_cast<int64_t>(id[k]) * cap);
+    }
+    for (int32_t f0 = 0; f0 < total; f0 += 64) {
+      const bool live = f0 + lane < total;
+      // Lanes past the end read the last candidate, moved out of reach.
+      double4 pj = cpos[at(min(f0 + lane, total - 1))];
+      pj.x = live ? pj.x : INFINITY;
       const int32_t j = static_cast<int32_t>(pj.w);
-      for (int k = 0; k < mg; k++) {
-        double4 a;
-        a.x = readlane_d(pi.x, k);
-        a.y = readlane_d(pi.y, k);
-        a.z = readlane_d(pi.z, k);
-        a.w = 0.0;
-        const int32_t ik = __builtin_amdgcn_readlane(iv, k);
-        const bool hit = live && (HALF ? j > ik : j != ik) &&
-                         within_search<IMAGE>(a, pj, g.box, half_box, sl2);
-        const uint64_t mask = __ballot(hit);
-        if (mask == 0) continue;
-        const int32_t ck = __builtin_amdgcn_readlane(cntv, k);
-        if (MODE != 0 && hit) {
-          const int32_t rank = static_cast<int32_t>(__builtin_amdgcn_mbcnt_hi(
+#pragma unroll
+      for (int k = 0; k < kPairGroup; k++) {
+        if (k >= mg) break;  // the whole wavefront
+        const uint64_t mask =
+            __builtin_amdgcn_ballot_w64(within_search<IMAGE>(a[k], pj, g.box, half_box, sl2)) &
+            __builtin_amdgcn_ballot_w64(HALF ? j > id[k] : j != id[k]);
+        if (MODE != 0) {
+          // The place after the row's hits so far and the lower lanes' ones.
+          const uint32_t to = __builtin_amdgcn_mbcnt_hi(
               static_cast<uint32_t>(mask >> 32),
-              __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(mask), 0u)));
-          const int64_t bk =
-              (static_cast<int64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(
-                   static_cast<int32_t>(basev >> 32), k)))
-               << 32) |
-              static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int32_t>(basev), k));
-          if (MODE == 1 || ck + rank < cap) out[bk + ck + rank] = j;
+              __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(mask), static_cast<uint32_t>(cnt[k])));
+          const bool hit = __builtin_amdgcn_inverse_ballot_w64(mask);
+          if (hit & (MODE == 1 || to < static_cast<uint32_t>(cap)))
+            *reinterpret_cast<int32_t*>(row[k] + to * 4u) = j;
         }
-        if (lane == k) cntv = ck + __popcll(mask);
+        cnt[k] += __popcll(mask);
       }
     }
-    if (MODE != 1 && lane < mg) nop[iv] = cntv;
+    if (MODE != 1) {
+      int32_t n = 0;
+#pragma unroll
+      for (int k = 0; k < kPairGroup; k++) n = lane == k ? cnt[k] : n;
+      if (lane < mg) nop[iv] = n;
+    }
   }
 }
 
-// One wavefront per cell, for cell grids with a stencil (R >= 1). The cell's
-// particles sit one per lane (in groups of 64); the candidates of the
-// (2R+1)^3 cells around it are walked as one flattened sequence, 64 per
-// round, so each candidate is loaded once for all of the cell's particles
-// instead of once per particle. A round's hits for one particle go to
-// consecutive addresses of its row (ballot, then each hit lane's rank among
-// them), so the stores coalesce. The runs of the flattened sequence are the
-// x-rows of the stencil, contiguous in cell order: (2R+1)^2 rows, each split
-// at most once where it wraps around a periodic box (the grid has at least
-// 2R+1 cells per side). Same predicate (within_search, in the same argument
+// One wavefront per cell, for cell grids with a stencil (R >= 1). The
+// candidates of the (2R+1)^3 cells around it are walked as one flattened
+// sequence, 64 per round, and tested against kPairGroup of the cell's
+// particles at a time (about four to five of a fine cell's, so mostly one
+// group), whose coordinates, counts and row addresses are scalars: a pair costs the
+// eight FP64 operations of the predicate and a handful for the place of a hit. A
+// round's hits for one particle go to consecutive addresses of its row
+// (ballot, then each hit's rank among them), so the stores coalesce. The
+// runs of the flattened sequence are the x-rows of the stencil, contiguous
+// in cell order: (2R+1)^2 rows, each split at most once where it wraps around
+// a periodic box (the grid has at least 2R+1 cells per side); their places
+// are written out in LDS once per cell (found by a search over the runs
+// where a cell has more than kPairCand). Same predicate (within_search, in the same argument
 // order), exclusions and MODEs as k_pairs; a row's entries come out in
 // candidate order and are sorted afterwards. *outside (from k_cell_assign)
-// keeps the minimum image on in every cell.
+// keeps the minimum image on in every cell. Bound by VALU issue: 572 us at
+// 1,048,576 particles (density 0.8, search length 3.3); one particle per
+// step with its coordinates fetched from a lane each round took 1007.
 template <int MODE, bool HALF, int R>
 __global__ __launch_bounds__(kBlock) void k_pairs_wave(int32_t ncell,
                                                        const double4* __restrict__ cpos,
@@ -879,6 +870,8 @@ __global__ __launch_bounds__(kBlock) void k_pairs_wave(int32_t ncell,
                                                        const int32_t* __restrict__ ptr,
                                                        int32_t* __restrict__ out,
                                                        const int32_t* __restrict__ outside) {
+  __shared__ int32_t cand_lds[kBlock / 64][kPairCand];
+  int32_t* cand = cand_lds[threadIdx.x >> 6];
   constexpr int kSpan = 2 * R + 1;
   constexpr int kRuns = 2 * kSpan * kSpan;
   static_assert(kRuns <= 64, "one run per lane");
@@ -887,35 +880,39 @@ __global__ __launch_bounds__(kBlock) void k_pairs_wave(int32_t ncell,
   const bool all_inside = *outside == 0;
   const double half_box = 0.5 * g.box;
   const int64_t waves = static_cast<int64_t>(gridDim.x) * (kBlock / 64);
-  for (int64_t c64 = (blockIdx.x * static_cast<int64_t>(kBlock) + threadIdx.x) >> 6; c64 < ncell;
-       c64 += waves) {
+  // The wavefront's cell and all that follows from it are scalars.
+  const int64_t first = blockIdx.x * static_cast<int64_t>(kBlock / 64) +
+                        __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / 64);
+  for (int64_t c64 = first; c64 < ncell; c64 += waves) {
     const int32_t c = static_cast<int32_t>(c64);
     const int32_t p0 = cell_start[c], p1 = cell_start[c + 1];
     if (p0 == p1) continue;  // the whole wavefront
     const int cx = c % g.nc0, cy = (c / g.nc0) % g.nc1, cz = c / (g.nc0 * g.nc1);
-    // Lane r < kRuns: run r of the stencil as [rs, rs + rl) in cpos.
+    // Lane r < kRuns: run r of the stencil as [rs, rs + rl) in cpos. An x-row's
+    // two runs are its parts before and behind the box's face where it
+    // wraps, else its halves.
     int32_t rs = 0, rl = 0;
     if (lane < kRuns) {
       const int yz = lane >> 1;
       int z = cz + yz / kSpan - R, y = cy + yz % kSpan - R;
       bool ok = true;
       if (periodic) {
-        z = (z + g.nc2) % g.nc2;
-        y = (y + g.nc1) % g.nc1;
+        z += z < 0 ? g.nc2 : z >= g.nc2 ? -g.nc2 : 0;
+        y += y < 0 ? g.nc1 : y >= g.nc1 ? -g.nc1 : 0;
       } else {
         ok = z >= 0 && z < g.nc2 && y >= 0 && y < g.nc1;
       }
       const int x0 = cx - R, x1 = cx + R;
-      int a = 1, b = 0;  // inclusive x range of cells; empty when a > b
-      if ((lane & 1) == 0) {
-        a = max(x0, 0);
-        b = min(x1, g.nc0 - 1);
-      } else if (periodic && x0 < 0) {
-        a = x0 + g.nc0;
-        b = g.nc0 - 1;
+      const bool first = (lane & 1) == 0;
+      int a = max(x0, 0), b = min(x1, g.nc0 - 1);  // inclusive x range of cells
+      if (periodic && x0 < 0) {
+        if (!first) a = x0 + g.nc0, b = g.nc0 - 1;
       } else if (periodic && x1 >= g.nc0) {
-        a = 0;
-        b = x1 - g.nc0;
+        if (!first) a = 0, b = x1 - g.nc0;
+      } else {
+        const int mid = (a + b) >> 1;
+        if (first) b = mid;
+        else a = mid + 1;
       }
       if (ok && a <= b) {
         const int32_t rowc = (z * g.nc1 + y) * g.nc0;
@@ -930,15 +927,35 @@ __global__ __launch_bounds__(kBlock) void k_pairs_wave(int32_t ncell,
       if (lane >= o) pre += v;
     }
     const int32_t excl = pre - rl;
-    const int32_t total = __shfl(pre, 63, 64);
+    const int32_t total = __builtin_amdgcn_readlane(pre, 63);
     const bool wraps = periodic && (!all_inside || cx < R || cx + R >= g.nc0 || cy < R ||
                                     cy + R >= g.nc1 || cz < R || cz + R >= g.nc2);
-    if (wraps)
-      pairs_cell<MODE, HALF, R, true>(p0, p1, total, pre, rs, excl, cpos, g, half_box, sl2, cap,
-                                      nop, ptr, out);
-    else
-      pairs_cell<MODE, HALF, R, false>(p0, p1, total, pre, rs, excl, cpos, g, half_box, sl2, cap,
-                                       nop, ptr, out);
+    auto walk = [&](auto&& at) {
+      if (wraps)
+        pairs_cell<MODE, HALF, true>(p0, p1, total, at, cpos, g, half_box, sl2, cap, nop, ptr, out);
+      else
+        pairs_cell<MODE, HALF, false>(p0, p1, total, at, cpos, g, half_box, sl2, cap, nop, ptr,
+                                      out);
+    };
+    if (total <= kPairCand) {
+      for (int32_t k = 0; k < rl; k++) cand[excl + k] = rs + k;
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // one wavefront's own
+      walk([&](int32_t f) { return cand[f]; });
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    } else {
+      walk([&](int32_t f) {
+        // The run holding f: the number of runs ending at or before f.
+        int r = 0;
+#pragma unroll
+        for (int bit = 32; bit > 0; bit >>= 1) {
+          const int t = r + bit;
+          const int32_t v = __shfl(pre, min(t, 64) - 1, 64);
+          if (t <= kRuns && v <= f) r = t;
+        }
+        const int rr = min(r, kRuns - 1);
+        return __shfl(rs, rr, 64) + (f - __shfl(excl, rr, 64));
+      });
+    }
   }
 }
 
