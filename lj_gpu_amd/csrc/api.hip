@@ -59,6 +59,7 @@ void reset_list(ljgpu_ctx* ctx) {
   ctx->max_np = ctx->min_np = 0;
   ctx->eval.n = 0;
   ctx->eval.e = 0;
+  ctx->eval.slab_stride = 0;
   ctx->eval_half = false;
   ctx->half_mode = 0;
   ctx->ell_ready = false;
@@ -126,8 +127,14 @@ int ensure_tiles(ljgpu_ctx* ctx, const PosIn* q, double box) {
                        ctx->work, &ordered));
   if (ordered)
     TRY(dev_tile_slots(ctx->stream, ctx->eval, want, ctx->rep_off, ctx->work, ctx->tiles));
+  // Rows that keep the list's order (the MD loop's) have their slices made with
+  // the tiles; local is then read by other launch shapes' energy only.
+  const SliceReq req{ctx->lanes, ctx->unroll, ctx->work.row_max,
+                     ctx->tile_offsets_lds || ctx->lanes != 4 || ctx->unroll != 4};
+  const bool with_slices = !ctx->bank_order && ctx->work.row_max > 0;
   for (int32_t tp = want; tp >= 1 && ctx->eval.n > 0; tp /= 2) {
-    TRY(dev_make_tiles(ctx->stream, ctx->eval, tp, ctx->rep_off, ordered, ctx->work, ctx->tiles));
+    TRY(dev_make_tiles(ctx->stream, ctx->eval, tp, ctx->rep_off, ordered,
+                       with_slices ? &req : nullptr, ctx->work, ctx->tiles));
     if (ctx->tiles.tile_particles == 0) continue;
     if (!ctx->eval_half || ctx->tiles.max_stage <= kHalfMaxStage) break;
     ctx->tiles.tile_particles = ctx->tiles.blocks = 0;
@@ -344,7 +351,11 @@ int build_list(ljgpu_ctx* ctx, const PosIn& q, int32_t n, double box, double sea
   ctx->ell_ready = false;
   ctx->tiles_for = -1;
   ctx->tiles_ordered = false;
+  // Unsorted rows (the MD loop's) are tiled from the pair search's slab; the
+  // list itself is filled only where something reads it.
+  if (box <= 0.0 || tile == 0) TRY(dev_copy_slab(ctx->stream, ctx->work, ctx->eval));
   TRY(prepare_layouts(ctx, &q, box));
+  if (ctx->tiles.blocks == 0) TRY(dev_copy_slab(ctx->stream, ctx->work, ctx->eval));
   HIP_TRY(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
   return LJGPU_OK;
 }

@@ -35,6 +35,9 @@ struct DevCSR {
   int32_t n = 0;
   int64_t e = 0;
   DevMem nop, ptr, list;
+  // > 0: the rows are still in the pair search's slab (ListWork::tmp), row i
+  // at i * slab_stride, and `list` is not filled (dev_copy_slab).
+  int32_t slab_stride = 0;
 };
 void dev_release(DevCSR& c);
 
@@ -153,9 +156,13 @@ int dev_expand_half(hipStream_t s, int32_t n, const int32_t* nop, const int32_t*
 // box > 0; rows ascending in i. With sort_rows, partners ascending (the
 // reference's order); without, each row's partners come in an order fixed
 // by the positions (stencil runs, cells, particle index within a cell), the
-// same on every build from the same positions.
+// same on every build from the same positions, and usually stay in the
+// search's slab (out.slab_stride).
 int dev_makepair(hipStream_t s, const PosIn& q, int32_t n, double box, double search_length,
                  int kind, ListWork& w, DevCSR& out, bool sort_rows = true);
+
+// The rows of a list that is still in the slab, copied to its `list`.
+int dev_copy_slab(hipStream_t s, ListWork& w, DevCSR& c);
 
 // Smallest and largest of a[0..n) (synchronises); 0, 0 for n = 0.
 int dev_minmax(hipStream_t s, const int32_t* a, int32_t n, ListWork& w, int32_t* mn, int32_t* mx);
@@ -181,9 +188,18 @@ int dev_tile_slots(hipStream_t s, const DevCSR& c, int32_t tile_particles,
 // block's replica. Returns LJGPU_OK with out.tile_particles = 0 when a block
 // does not fit the LDS budget (the caller then halves the tile size or
 // evaluates untiled). With `spatial` the blocks cover the slots of
-// dev_tile_slots, else particles in index order.
+// dev_tile_slots, else particles in index order. With `slices` (rows in list
+// order, the longest known) the wavefront slices are made in the same pass
+// where they can be (sliced_lanes > 0 afterwards), and local is then written
+// only if wanted.
+struct SliceReq {
+  int32_t lanes, unroll;
+  int32_t longest;  // longest row
+  bool local;
+};
 int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t tile_particles,
-                   const std::vector<int32_t>& replicas, bool spatial, ListWork& w, DevTiles& out);
+                   const std::vector<int32_t>& replicas, bool spatial, const SliceReq* slices,
+                   ListWork& w, DevTiles& out);
 
 // The tiles' entry offsets sliced per wavefront, for a tile kernel in
 // which `lanes` consecutive lanes own one row and take entries in batches

@@ -997,23 +997,38 @@ __device__ __forceinline__ T lds_load(const T* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// The blocks of a tiling: geo (4 ints per block: first slot, count, replica)
-// for replicas, else (null) blocks of T consecutive slots of n.
+// The blocks of a tiling: geo (`step` ints per block: first slot, count, and
+// in replicas' four the replica), else (null) blocks of T consecutive slots
+// of n.
 struct TileSpans {
   const int32_t* geo;
-  int32_t T, n;
+  int32_t T, n, step;
 };
 struct TileSpan {
   int32_t i0, ni, rid;
 };
 __device__ __forceinline__ TileSpan tile_span(const TileSpans& g, int32_t b) {
-  if (g.geo) return TileSpan{g.geo[4 * b], g.geo[4 * b + 1], g.geo[4 * b + 2]};
+  if (g.geo) {
+    const int32_t* d = g.geo + static_cast<int64_t>(g.step) * b;
+    return TileSpan{d[0], d[1], d[2]};
+  }
   return TileSpan{b * g.T, min(g.T, g.n - b * g.T), 0};
 }
 
 struct TileGeom {
   int32_t i0, ni, ne, rid;
   int64_t e0;
+};
+
+// Where a particle's row starts: in a list by row pointers, or (stride > 0) in
+// the pair search's slab.
+struct RowSource {
+  const int32_t* list;
+  const int32_t* ptr;
+  int64_t stride;
+  __device__ __forceinline__ const int32_t* row(int32_t i) const {
+    return list + (stride > 0 ? i * stride : static_cast<int64_t>(ptr[i]));
+  }
 };
 
 // Block b's entries are [slot_ptr[i0], slot_ptr[i0 + ni]) of the slot-ordered
@@ -1065,7 +1080,7 @@ template <bool COUNT>
 __global__ __launch_bounds__(1024) void k_tile_fill(
     TileSpans spans, int32_t nblocks, const int32_t* __restrict__ member,
     const int32_t* __restrict__ slot_of, const int32_t* __restrict__ slot_ptr,
-    const int32_t* __restrict__ ptr, const int32_t* __restrict__ list,
+    RowSource rows,
     const int32_t* __restrict__ soff, int32_t ecap, int32_t* __restrict__ ns_out,
     int32_t* __restrict__ desc, int32_t* __restrict__ stage, int32_t* __restrict__ stage_slot,
     uint16_t* __restrict__ local, int4* __restrict__ stats) {
@@ -1094,7 +1109,7 @@ __global__ __launch_bounds__(1024) void k_tile_fill(
     auto walk = [&](int r, int32_t k0, int32_t step) {
       const int32_t a = slot_ptr[g.i0 + r];
       const int32_t m = slot_ptr[g.i0 + r + 1] - a;
-      const int32_t src = ptr[member ? member[g.i0 + r] : g.i0 + r];
+      const int32_t* src = rows.row(member ? member[g.i0 + r] : g.i0 + r);
       const int32_t eoff = a - static_cast<int32_t>(g.e0);
       if (k0 == 0) atomicMax(&longest, m);
       for (; k0 < m; k0 += step * kWordBatch) {
@@ -1103,7 +1118,7 @@ __global__ __launch_bounds__(1024) void k_tile_fill(
 #pragma unroll
         for (int u = 0; u < kWordBatch; u++) {
           const int32_t k = k0 + u * step;
-          key[u] = k < m ? list[src + k] : -1;
+          key[u] = k < m ? src[k] : -1;
         }
         if (slot_of) {
 #pragma unroll
@@ -1212,11 +1227,11 @@ __global__ __launch_bounds__(1024) void k_tile_fill(
       for (int r = group; r < g.ni; r += groups) {
         const int32_t a = slot_ptr[g.i0 + r];
         const int32_t m = slot_ptr[g.i0 + r + 1] - a;
-        const int32_t src = ptr[member ? member[g.i0 + r] : g.i0 + r];
+        const int32_t* src = rows.row(member ? member[g.i0 + r] : g.i0 + r);
         const int32_t eoff = a - static_cast<int32_t>(g.e0);
         for (int32_t k = lane; k < m; k += kWordLanes) {
           if (eoff + k < ecap) continue;
-          int32_t key = list[src + k];
+          int32_t key = src[k];
           if (slot_of) key = slot_of[key];
           uint32_t h = word_hash(key >> 4);
           while (keys[h] != key >> 4) h = (h + 1) & (kWords - 1);
@@ -1286,8 +1301,15 @@ __global__ __launch_bounds__(1024) void k_tile_stats(int32_t nblocks, const int4
 // more: 87 against 64 us at 119,000 particles, 521 against 364 us at a
 // million). The hashed set of k_tile_fill takes 119 and 742 us there. A tile with more pages
 // than fit kPageBytes says so in stats[b].w, and the caller uses k_tile_fill.
+//   With slices.out the wavefront slices of the rows as they stand (see
+// k_tile_slices) leave from LDS as well, and local may be null.
+struct SliceDev {
+  uint16_t* out;            // null: no slices
+  const int32_t* wave_off;
+  int32_t lanes, wpb, stride, pad;
+};
 constexpr int kPageLanes = 8;
-constexpr int kPageKeys = 20;
+constexpr int kPageKeys = 16;
 constexpr int kPageBytes = 24576;
 constexpr int kPageDir = 32768;  // most pages of a list
 static_assert(kPageBytes / 128 < 255, "a page number fits a byte");
@@ -1295,8 +1317,7 @@ static_assert(kPageBytes / 128 < 255, "a page number fits a byte");
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6))) void k_tile_pages(
     TileSpans spans, int32_t nblocks, const int32_t* __restrict__ member,
     const int32_t* __restrict__ slot_of, const int32_t* __restrict__ slot_ptr,
-    const int32_t* __restrict__ ptr, const int32_t* __restrict__ list, int32_t pshift,
-    int32_t npages, int32_t* __restrict__ desc, int32_t* __restrict__ stage,
+    RowSource rows, int32_t pshift, int32_t npages, SliceDev slices, int32_t* __restrict__ desc, int32_t* __restrict__ stage,
     int32_t* __restrict__ stage_slot, uint16_t* __restrict__ local, int4* __restrict__ stats) {
   extern __shared__ uint32_t page_lds[];
   __shared__ uint32_t table[kPageBytes / 16];  // slots present, base rank << 16
@@ -1310,6 +1331,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6))) void k
   const int lane = tid & (kPageLanes - 1), group = tid / kPageLanes, groups = nt / kPageLanes;
   const int32_t low = (1 << pshift) - 1;
   const int32_t chunk = ((npages + nt - 1) / nt + 3) / 4;  // directory words per thread
+  if (slices.out && blockIdx.x == 0)
+    for (int t = tid; t < slices.pad; t += nt)
+      slices.out[slices.wave_off[static_cast<int64_t>(nblocks) * slices.wpb] + t] = 0;
   for (int32_t b = blockIdx.x; b < nblocks; b += gridDim.x) {
     const TileGeom g = tile_geom(spans, b, slot_ptr);
     for (int t = tid; t < (npages + 3) / 4; t += nt) page_lds[t] = 0;
@@ -1318,13 +1342,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6))) void k
     // first slot, which belongs to the set anyway.
     int32_t key[kPageKeys];
     int32_t mine = 0;  // the row's entries from this lane's first on
-    const int32_t* row = list + lane;
-    uint16_t* out = local + lane;
+    const int32_t* row = rows.list;
+    int32_t a0 = 0;
     if (group < g.ni) {
-      const int32_t a = slot_ptr[g.i0 + group];
-      mine = slot_ptr[g.i0 + group + 1] - a - lane;
-      row += ptr[member ? member[g.i0 + group] : g.i0 + group];
-      out += a;
+      a0 = slot_ptr[g.i0 + group];
+      mine = slot_ptr[g.i0 + group + 1] - a0 - lane;
+      row = rows.row(member ? member[g.i0 + group] : g.i0 + group) + lane;
     }
 #pragma unroll
     for (int u = 0; u < kPageKeys; u++) {
@@ -1336,15 +1359,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6))) void k
       for (int u = 0; u < kPageKeys; u++)
         key[u] = key[u] >= 0 ? slot_of[static_cast<uint32_t>(key[u])] : g.i0;
     }
-    // f(slot, entry) of every other entry of the block.
+    // f(slot, row, its start, place) of every other entry of the block.
     auto others = [&](auto&& f) {
       for (int r = group; r < g.ni; r += groups) {
         const int32_t a = slot_ptr[g.i0 + r];
         const int32_t m = slot_ptr[g.i0 + r + 1] - a;
-        const int32_t src = ptr[member ? member[g.i0 + r] : g.i0 + r];
+        const int32_t* src = rows.row(member ? member[g.i0 + r] : g.i0 + r);
         for (int32_t k = lane + (r == group ? kPageKeys * kPageLanes : 0); k < m; k += kPageLanes) {
-          const int32_t j = list[src + k];
-          f(slot_of ? slot_of[j] : j, a + k);
+          const int32_t j = src[k];
+          f(slot_of ? slot_of[j] : j, r, a, k);
         }
         if (lane == 0) atomicMax(&longest, m);
       }
@@ -1352,7 +1375,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6))) void k
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < kPageKeys; u++) dir[key[u] >> pshift] = 1;
-    others([&](int32_t s, int32_t) { dir[s >> pshift] = 1; });
+    others([&](int32_t s, int, int32_t, int32_t) { dir[s >> pshift] = 1; });
     for (int t = tid; t < g.ni; t += nt) dir[(g.i0 + t) >> pshift] = 1;
     __syncthreads();
     int32_t pages = 0;
@@ -1381,7 +1404,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6))) void k
       key[u] = dir[key[u] >> pshift] << pshift | (key[u] & low);  // its byte from here on
       mark[key[u]] = 1;
     }
-    others([&](int32_t s, int32_t) { mark[dir[s >> pshift] << pshift | (s & low)] = 1; });
+    others([&](int32_t s, int, int32_t, int32_t) { mark[dir[s >> pshift] << pshift | (s & low)] = 1; });
     for (int t = tid; t < g.ni; t += nt) {
       const int32_t s = g.i0 + t;
       mark[dir[s >> pshift] << pshift | (s & low)] = 1;
@@ -1435,13 +1458,38 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6))) void k
       const uint32_t v = table[at >> 4];
       return static_cast<uint16_t>(((v >> 16) + __popc(v & ((1u << (at & 15)) - 1))) * 24);
     };
+    // The rows in LDS too, where the directory's bytes were, if their slices
+    // are made here.
+    uint16_t* lds_rows = reinterpret_cast<uint16_t*>(used);
+    auto put = [&](uint16_t v, int r, int32_t a, int32_t k) {
+      if (local) local[a + k] = v;
+      if (slices.out) lds_rows[r * slices.stride + k] = v;
+    };
 #pragma unroll
     for (int u = 0; u < kPageKeys; u++) {
       const uint16_t v = offset(key[u]);
-      if (u * kPageLanes < mine) out[u * kPageLanes] = v;
+      if (u * kPageLanes < mine) put(v, group, a0, lane + u * kPageLanes);
     }
-    others([&](int32_t s, int32_t e) { local[e] = offset(dir[s >> pshift] << pshift | (s & low)); });
+    others([&](int32_t s, int r, int32_t a, int32_t k) {
+      put(offset(dir[s >> pshift] << pshift | (s & low)), r, a, k);
+    });
     __syncthreads();
+    if (slices.out) {
+      const int lsh = 31 - __clz(slices.lanes);
+      const int rpw = 64 >> lsh;  // rows per wavefront
+      for (int w = tid / 64; w < slices.wpb; w += nt / 64) {
+        const int32_t* wo = slices.wave_off + static_cast<int64_t>(b) * slices.wpb + w;
+        const int32_t p0 = wo[0], n = wo[1] - wo[0];
+        const int r = w * rpw + ((tid & 63) >> lsh);
+        const int32_t m = r < g.ni ? slot_ptr[g.i0 + r + 1] - slot_ptr[g.i0 + r] : 0;
+        const uint16_t* src = lds_rows + (r < g.ni ? r : 0) * slices.stride;
+        int k = tid & (slices.lanes - 1);
+#pragma unroll 4
+        for (int32_t p = tid & 63; p < n; p += 64, k += slices.lanes)
+          slices.out[p0 + p] = k < m ? src[k] : uint16_t{0};
+      }
+      __syncthreads();
+    }
   }
 }
 
@@ -1473,13 +1521,14 @@ __global__ __launch_bounds__(kBankBlock) void k_bank_order(const int32_t* __rest
 
 // Slice lengths: per (block, wavefront slot), 64 * unroll offsets for each
 // batch its longest row needs (0 for slots past the block's rows).
-__global__ void k_wave_slices(const int32_t* __restrict__ desc, int32_t nblocks, int32_t wpb,
+__global__ void k_wave_slices(TileSpans spans, int32_t nblocks, int32_t wpb,
                               const int32_t* __restrict__ slot_ptr, int32_t lanes, int32_t unroll,
                               int32_t* __restrict__ len) {
   const int64_t id = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
   if (id >= static_cast<int64_t>(nblocks) * wpb) return;
   const int32_t b = static_cast<int32_t>(id / wpb), w = static_cast<int32_t>(id % wpb);
-  const int32_t i0 = desc[8 * static_cast<int64_t>(b)], ni = desc[8 * static_cast<int64_t>(b) + 1];
+  const TileSpan g = tile_span(spans, b);
+  const int32_t i0 = g.i0, ni = g.ni;
   const int32_t rpw = 64 / lanes, kb = lanes * unroll;
   int32_t batches = 0;
   for (int32_t r = w * rpw; r < min(ni, (w + 1) * rpw); r++) {
@@ -2057,6 +2106,7 @@ int dev_makepair(hipStream_t s, const PosIn& q, int32_t n, double box, double se
   LCHECK(dev_reserve(out.nop, sizeof(int32_t) * std::max(n, 1), s));
   LCHECK(dev_reserve(out.ptr, sizeof(int32_t) * (static_cast<size_t>(n) + 1), s));
   w.row_min = w.row_max = 0;
+  out.slab_stride = 0;
   if (n == 0) {
     out.e = 0;
     LCHECK(dev_reserve(out.list, sizeof(int32_t), s));
@@ -2186,19 +2236,17 @@ int dev_makepair(hipStream_t s, const PosIn& q, int32_t n, double box, double se
   if (w.results->cells.hi > kCellOrderMax) sort_rows = true;
   if (total > INT32_MAX) return set_error(LJGPU_ERR_CAPACITY, "list longer than 2^31-1 entries");
   out.e = total;
-  LCHECK(dev_reserve(out.list, sizeof(int32_t) * std::max<int64_t>(total, 1), s));
   if (cap > 0 && mx <= cap) {
     w.last_max_row = mx;
     if (!sort_rows) {
-      k_copy_slab<<<grid_for((n + kSlabRows - 1) / kSlabRows, kBlock / 64), kBlock, 0, s>>>(
-          n, out.nop.as<int32_t>(), out.ptr.as<int32_t>(), w.tmp.as<int32_t>(), cap,
-          out.list.as<int32_t>());
-      LTRY(hipGetLastError(), "slab copy kernel");
+      out.slab_stride = cap;  // the rows stay in w.tmp: dev_copy_slab
       return LJGPU_OK;
     }
+    LCHECK(dev_reserve(out.list, sizeof(int32_t) * std::max<int64_t>(total, 1), s));
     return row_sort(s, n, out.nop.as<int32_t>(), out.ptr.as<int32_t>(), w.tmp.as<int32_t>(),
                     out.list.as<int32_t>(), cap);
   }
+  LCHECK(dev_reserve(out.list, sizeof(int32_t) * std::max<int64_t>(total, 1), s));
   if (cap > 0) w.last_max_row = mx;
   if (!sort_rows) {
     pairs(std::integral_constant<int, 1>{}, 0, out.nop.as<int32_t>(), out.ptr.as<int32_t>(),
@@ -2212,6 +2260,17 @@ int dev_makepair(hipStream_t s, const PosIn& q, int32_t n, double box, double se
   LTRY(hipGetLastError(), "pair fill kernel");
   return row_sort(s, n, out.nop.as<int32_t>(), out.ptr.as<int32_t>(), w.tmp.as<int32_t>(),
                   out.list.as<int32_t>());
+}
+
+int dev_copy_slab(hipStream_t s, ListWork& w, DevCSR& c) {
+  if (c.slab_stride == 0) return LJGPU_OK;
+  LCHECK(dev_reserve(c.list, sizeof(int32_t) * std::max<int64_t>(c.e, 1), s));
+  k_copy_slab<<<grid_for((c.n + kSlabRows - 1) / kSlabRows, kBlock / 64), kBlock, 0, s>>>(
+      c.n, c.nop.as<int32_t>(), c.ptr.as<int32_t>(), w.tmp.as<int32_t>(), c.slab_stride,
+      c.list.as<int32_t>());
+  LTRY(hipGetLastError(), "slab copy kernel");
+  c.slab_stride = 0;
+  return LJGPU_OK;
 }
 
 int dev_minmax(hipStream_t s, const int32_t* a, int32_t n, ListWork& w, int32_t* mn,
@@ -2356,7 +2415,7 @@ int dev_tile_order(hipStream_t s, const PosIn& q, int32_t n, double box,
 // The blocks of T consecutive slots, restarted at every replica boundary.
 int tile_spans(hipStream_t s, int32_t n, int32_t T, const std::vector<int32_t>& reps, ListWork& w,
                TileSpans* spans, int32_t* nblocks) {
-  *spans = TileSpans{nullptr, T, n};
+  *spans = TileSpans{nullptr, T, n, 4};
   *nblocks = (n + T - 1) / T;
   if (reps.empty()) return LJGPU_OK;
   // Kept: the upload reads it after this returns. One not yet read must not
@@ -2392,8 +2451,43 @@ int dev_tile_slots(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<
   return dev_scan_async(s, w.counts.as<int32_t>(), out.slot_ptr.as<int32_t>(), c.n, w, nullptr);
 }
 
+// Entries past the last slice that the kernels' offset prefetch reads: two
+// batches.
+int32_t slice_pad(int32_t unroll) { return 2 * 64 * unroll + 64; }
+
+// Lengths and starts of the slices (t.wave_off) and room for them (t.sliced);
+// *wpb: wavefronts per block, 0 where slices cannot be made.
+int plan_slices(hipStream_t s, const TileSpans& spans, int32_t nblocks, int32_t T,
+                const int32_t* slot_ptr, int32_t lanes, int32_t unroll, int32_t longest,
+                ListWork& w, DevTiles& t, int32_t* wpb) {
+  *wpb = 0;
+  if (lanes < 1 || lanes > 64 || (64 % lanes) != 0 || unroll < 1 || (unroll & (unroll - 1)) != 0)
+    return LJGPU_OK;
+  const int32_t waves = (T * lanes + 63) / 64;
+  if (waves > kSliceWavesMax) return LJGPU_OK;
+  const int64_t nw = static_cast<int64_t>(nblocks) * waves;
+  LCHECK(dev_reserve(w.counts, sizeof(int32_t) * (static_cast<size_t>(nw) + 1), s));
+  LCHECK(dev_reserve(t.wave_off, sizeof(int32_t) * (static_cast<size_t>(nw) + 1), s));
+  k_wave_slices<<<grid_for(nw, kBlock), kBlock, 0, s>>>(spans, nblocks, waves, slot_ptr, lanes,
+                                                        unroll, w.counts.as<int32_t>());
+  LTRY(hipGetLastError(), "slice length kernel");
+  // The slices' length is at most every wavefront's with the longest row; read
+  // back only where that would be a waste.
+  const int64_t kb = static_cast<int64_t>(lanes) * unroll;
+  int64_t total = nw * 64 * unroll * ((longest + kb - 1) / kb);
+  if (total <= int64_t{1} << 26)
+    LCHECK(dev_scan_async(s, w.counts.as<int32_t>(), t.wave_off.as<int32_t>(), nw, w, nullptr));
+  else
+    LCHECK(dev_scan(s, w.counts.as<int32_t>(), t.wave_off.as<int32_t>(), nw, w, &total));
+  const int32_t pad = slice_pad(unroll);
+  if (total + pad > INT32_MAX) return LJGPU_OK;
+  LCHECK(dev_reserve(t.sliced, sizeof(uint16_t) * (total + pad), s));
+  *wpb = waves;
+  return LJGPU_OK;
+}
+
 int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<int32_t>& reps,
-                   bool spatial, ListWork& w, DevTiles& out) {
+                   bool spatial, const SliceReq* req, ListWork& w, DevTiles& out) {
   out.tile_particles = 0;
   out.blocks = 0;
   if (T <= 0 || T > kTileRowsMax || c.n <= 0) return LJGPU_OK;
@@ -2408,6 +2502,22 @@ int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<
   int32_t nb = 0;
   LCHECK(tile_spans(s, c.n, T, reps, w, &spans, &nb));
   if (nb == 0) return LJGPU_OK;
+  const RowSource source{c.slab_stride > 0 ? w.tmp.as<int32_t>() : c.list.as<int32_t>(),
+                         c.ptr.as<int32_t>(), c.slab_stride};
+  // Slices of the rows as they stand, where the tiles' rows fit LDS.
+  SliceDev slices{};
+  const int32_t stride = req ? 2 * ((req->longest + 1) / 2 | 1) : 0;
+  if (req && req->lanes > 1 && static_cast<int64_t>(T) * stride * 2 <= kPageBytes) {
+    LCHECK(plan_slices(s, spans, nb, T, sptr, req->lanes, req->unroll, req->longest, w, out,
+                       &slices.wpb));
+    if (slices.wpb > 0) {
+      slices.out = out.sliced.as<uint16_t>();
+      slices.wave_off = out.wave_off.as<int32_t>();
+      slices.lanes = req->lanes;
+      slices.stride = stride;
+      slices.pad = slice_pad(req->unroll);
+    }
+  }
   LCHECK(results(w));
   LCHECK(dev_reserve(w.tile_stats, sizeof(int4) * static_cast<size_t>(nb), s));
   int4* stats = w.tile_stats.as<int4>();
@@ -2449,12 +2559,13 @@ int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<
     for (int pass = 0; pass < 2; pass++) {
       if (pass == 0)
         k_tile_pages<<<grid, std::min(512, std::max(256, T * kPageLanes)), (npages + 15) / 16 * 16, s>>>(
-            spans, nb, member, slot_of, sptr, c.ptr.as<int32_t>(), c.list.as<int32_t>(), pshift,
-            npages, out.desc.as<int32_t>(), out.stage.as<int32_t>(),
-            member ? out.stage_slot.as<int32_t>() : nullptr, out.local.as<uint16_t>(), stats);
+            spans, nb, member, slot_of, sptr, source, pshift,
+            npages, slices, out.desc.as<int32_t>(), out.stage.as<int32_t>(),
+            member ? out.stage_slot.as<int32_t>() : nullptr,
+            slices.out && !req->local ? nullptr : out.local.as<uint16_t>(), stats);
       else
         k_tile_fill<false><<<grid, threads, code_bytes, s>>>(
-            spans, nb, member, slot_of, sptr, c.ptr.as<int32_t>(), c.list.as<int32_t>(), nullptr, ecap,
+            spans, nb, member, slot_of, sptr, source, nullptr, ecap,
             nullptr, out.desc.as<int32_t>(), out.stage.as<int32_t>(),
             member ? out.stage_slot.as<int32_t>() : nullptr, out.local.as<uint16_t>(), stats);
       LTRY(hipGetLastError(), "tile fill kernel");
@@ -2462,7 +2573,14 @@ int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<
       LCHECK(read_stats(back));
       std::copy(back, back + 4, h);
       std::memcpy(&st, back + 6, sizeof(st));
-      if (back[4] == 0) break;  // else partners over too many pages: the hashed set
+      if (back[4] == 0) {
+        if (pass == 0 && slices.out && back[0] == 0) {
+          out.sliced_lanes = req->lanes;
+          out.sliced_unroll = req->unroll;
+          out.waves_per_block = slices.wpb;
+        }
+        break;
+      }  // else partners over too many pages: the hashed set
     }
     if (h[0] != 0) return LJGPU_OK;  // does not fit: caller retries smaller or runs untiled
     staged = static_cast<int64_t>(st);
@@ -2471,7 +2589,7 @@ int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<
     LCHECK(dev_reserve(w.tile_ns, sizeof(int32_t) * (static_cast<size_t>(nb) + 1), s));
     LCHECK(dev_reserve(w.tile_soff, sizeof(int32_t) * (static_cast<size_t>(nb) + 1), s));
     k_tile_fill<true><<<grid, threads, 0, s>>>(
-        spans, nb, member, slot_of, sptr, c.ptr.as<int32_t>(), c.list.as<int32_t>(), nullptr, 0,
+        spans, nb, member, slot_of, sptr, source, nullptr, 0,
         w.tile_ns.as<int32_t>(), nullptr, nullptr, nullptr, nullptr, stats);
     LTRY(hipGetLastError(), "tile count kernel");
     int32_t back[8];
@@ -2486,7 +2604,7 @@ int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<
     if (member)
       LCHECK(dev_reserve(out.stage_slot, sizeof(int32_t) * std::max<int64_t>(staged, 1), s));
     k_tile_fill<false><<<grid, threads, code_bytes, s>>>(
-        spans, nb, member, slot_of, sptr, c.ptr.as<int32_t>(), c.list.as<int32_t>(),
+        spans, nb, member, slot_of, sptr, source,
         w.tile_soff.as<int32_t>(), ecap, nullptr, out.desc.as<int32_t>(),
         out.stage.as<int32_t>(), member ? out.stage_slot.as<int32_t>() : nullptr,
         out.local.as<uint16_t>(), stats);
@@ -2508,30 +2626,12 @@ int dev_slice_tiles(hipStream_t s, const int32_t* slot_ptr, int32_t lanes, int32
                     int32_t scale, bool bank_order, int32_t n, const CutHint* hint, ListWork& w,
                     DevTiles& t) {
   t.sliced_lanes = t.sliced_unroll = t.waves_per_block = 0;
-  if (t.blocks <= 0 || lanes < 1 || lanes > 64 || (64 % lanes) != 0 || unroll < 1 ||
-      (unroll & (unroll - 1)) != 0)
-    return LJGPU_OK;
-  const int32_t wpb = (t.tile_particles * lanes + 63) / 64;
-  if (wpb > kSliceWavesMax) return LJGPU_OK;
-  const int64_t nw = static_cast<int64_t>(t.blocks) * wpb;
-  LCHECK(dev_reserve(w.counts, sizeof(int32_t) * (static_cast<size_t>(nw) + 1), s));
-  LCHECK(dev_reserve(t.wave_off, sizeof(int32_t) * (static_cast<size_t>(nw) + 1), s));
-  k_wave_slices<<<grid_for(nw, kBlock), kBlock, 0, s>>>(t.desc.as<int32_t>(), t.blocks, wpb,
-                                                        slot_ptr, lanes, unroll,
-                                                        w.counts.as<int32_t>());
-  LTRY(hipGetLastError(), "slice length kernel");
-  // The slices' length is at most every wavefront's with the longest row; read
-  // back only where that would be a waste.
-  const int64_t kb = static_cast<int64_t>(lanes) * unroll;
-  int64_t total = nw * 64 * unroll * ((t.longest + kb - 1) / kb);
-  if (total <= int64_t{1} << 26)
-    LCHECK(dev_scan_async(s, w.counts.as<int32_t>(), t.wave_off.as<int32_t>(), nw, w, nullptr));
-  else
-    LCHECK(dev_scan(s, w.counts.as<int32_t>(), t.wave_off.as<int32_t>(), nw, w, &total));
-  // The kernel's offset prefetch reads up to two batches past a slice.
-  const int32_t pad = 2 * 64 * unroll + 64;
-  if (total + pad > INT32_MAX) return LJGPU_OK;
-  LCHECK(dev_reserve(t.sliced, sizeof(uint16_t) * (total + pad), s));
+  if (t.blocks <= 0) return LJGPU_OK;
+  int32_t wpb = 0;
+  LCHECK(plan_slices(s, TileSpans{t.desc.as<int32_t>(), 0, 0, 8}, t.blocks, t.tile_particles,
+                     slot_ptr, lanes, unroll, t.longest, w, t, &wpb));
+  if (wpb == 0) return LJGPU_OK;
+  const int32_t pad = slice_pad(unroll);
   CutDev cd{};
   const bool cut = bank_order && hint && hint->q.x && !t.cut;
   if (cut) {
