@@ -228,14 +228,16 @@ k_ell(P pos, M mom, int32_t n, const int32_t* __restrict__ nop, const int32_t* _
 }
 
 // Shift a position by whole box lengths to the periodic image nearest the
-// reference point c (no-op in an open box).
+// reference point c (no-op in an open box); fx is -c.x / box and so on. Where
+// two images are equally far, to rounding, either is taken: a tile that uses
+// the shifted positions as they are has no partner within the cutoff there.
 template <bool PBC>
-__device__ __forceinline__ void unwrap_near(double& x, double& y, double& z, double cx,
-                                            double cy, double cz, const PairParams& pp) {
+__device__ __forceinline__ void unwrap_near(double& x, double& y, double& z, double fx,
+                                            double fy, double fz, const PairParams& pp) {
   if constexpr (PBC) {
-    x = fma(-pp.box, rint((x - cx) * pp.inv_box), x);
-    y = fma(-pp.box, rint((y - cy) * pp.inv_box), y);
-    z = fma(-pp.box, rint((z - cz) * pp.inv_box), z);
+    x = fma(-pp.box, rint(fma(x, pp.inv_box, fx)), x);
+    y = fma(-pp.box, rint(fma(y, pp.inv_box, fy)), y);
+    z = fma(-pp.box, rint(fma(z, pp.inv_box, fz)), z);
   }
 }
 
@@ -249,14 +251,14 @@ __device__ __forceinline__ T lds_at(uint32_t a) {
 }
 
 // One entry of a tile row: in FP64 the unit force scalar (lj_df_unit_f64,
-// the row's sum is scaled by 24*dt in tile_body), otherwise pair_compute.
+// the row's sum is scaled in tile_body), otherwise pair_compute.
 template <int PREC, bool MI>
 __device__ __forceinline__ void tile_pair(double dx, double dy, double dz, const PairParams& pp,
                                           Accum<PREC>& acc) {
   if constexpr (PREC == kF64) {
     min_image<MI>(dx, dy, dz, pp);
     const double r2 = fma(dz, dz, fma(dy, dy, dx * dx));
-    acc.add(lj_df_unit_f64(rcp_f64(r2), !(r2 > pp.cl2)), 0.0f, dx, dy, dz);
+    acc.add(lj_df_unit_f64(rcp_scaled_f64(r2, kCbrt2), !(r2 > pp.cl2)), 0.0f, dx, dy, dz);
   } else {
     pair_compute<PREC, MI, false>(MomAos{nullptr}, 0, true, dx, dy, dz, pp, acc);
   }
@@ -310,9 +312,9 @@ __device__ __forceinline__ void tile_row(const M& mom, const uint16_t* lrow, int
 // skips the force arithmetic (the wavefront branches as a whole): the
 // reference's `if (r2 > CL2) continue;` for a whole batch. Rows hold their
 // entries in cutoff classes (cut_partition), so the entries beyond the
-// cutoff collect at the rows' ends. In FP64 the force scalar omits the
-// factor 24*dt (lj_df_unit_f64), which tile_body applies to the row's sum,
-// and the batch's U reciprocals come from one (rcp_f64_batch). PBC is the
+// cutoff collect at the rows' ends. In FP64 the force scalar omits a
+// factor (lj_df_unit_f64), which tile_body applies to the row's sum,
+// and the batch's U reciprocals come from one (rcp_scaled_f64_batch). PBC is the
 // kernel's box (periodic or open); MI whether this row needs the minimum
 // image.
 template <int TPI, int U, int PREC, bool PBC, bool MI, bool LIMIT, bool REFILL, int US, class M>
@@ -353,7 +355,7 @@ __device__ __forceinline__ void tile_batch(const M& mom, const uint16_t* __restr
   if constexpr (PREC == kF64) {
 #pragma unroll
     for (int u = 0; u < U; u++) s[u] = LIMIT && !valid[u] ? 1.0 : r2[u];
-    rcp_f64_batch<U>(s);
+    rcp_scaled_f64_batch<U>(s, kCbrt2);
   }
 #pragma unroll
   for (int u = 0; u < U; u++) {
@@ -481,6 +483,7 @@ __device__ __forceinline__ void tile_body(P pos, M mom, const int32_t* __restric
   double cx = 0.0, cy = 0.0, cz = 0.0;
   // The block's middle particle (its slot when the arrays are in slot order).
   if constexpr (PBC) pos.ld(member ? d1.w : i0 + ni / 2, cx, cy, cz);
+  const double ux = -cx * pp.inv_box, uy = -cy * pp.inv_box, uz = -cz * pp.inv_box;
   // The thread's own row, requested before the staging so that its latency
   // overlaps it: first the indices (the first staging pass's particles, own
   // particle, row bounds, offset slice), then what they address (own
@@ -528,7 +531,7 @@ __device__ __forceinline__ void tile_body(P pos, M mom, const int32_t* __restric
     _Pragma("unroll") for (int r = 0; r < kStageR; r++) {                     \
       const int t = (T0) + r * nt + static_cast<int>(threadIdx.x);            \
       if (t < ns) {                                                           \
-        unwrap_near<PBC>(x[r], y[r], z[r], cx, cy, cz, pp);                   \
+        unwrap_near<PBC>(x[r], y[r], z[r], ux, uy, uz, pp);                   \
         lds[3 * t] = x[r];                                                    \
         lds[3 * t + 1] = y[r];                                                \
         lds[3 * t + 2] = z[r];                                                \
@@ -569,7 +572,7 @@ __device__ __forceinline__ void tile_body(P pos, M mom, const int32_t* __restric
   const uint16_t* loff = reinterpret_cast<const uint16_t*>(lb + off_area) + (eoff - e0);
   int far = 0;
   if constexpr (PBC) {
-    unwrap_near<PBC>(xi, yi, zi, cx, cy, cz, pp);
+    unwrap_near<PBC>(xi, yi, zi, ux, uy, uz, pp);
     far = active && (fabs(xi - cx) >= reach || fabs(yi - cy) >= reach || fabs(zi - cz) >= reach);
   }
   // The frame check ORed over the workgroup through one LDS word: threads
@@ -605,9 +608,9 @@ __device__ __forceinline__ void tile_body(P pos, M mom, const int32_t* __restric
     double fy = segment_sum<TPI>(acc.vy());
     double fz = segment_sum<TPI>(acc.vz());
     if constexpr (PREC == kF64) {
-      fx *= pp.c24;
-      fy *= pp.c24;
-      fz *= pp.c24;
+      fx *= pp.c_unit;
+      fy *= pp.c_unit;
+      fz *= pp.c_unit;
     }
     if (active && sub == 0) mom.add(i, fx, fy, fz);
   }
@@ -685,6 +688,7 @@ k_tile_half(P pos, const int32_t* __restrict__ member,
   const int i0 = d0.x, ni = d0.y, soff = d0.z, ns = d0.w;
   double cx = 0.0, cy = 0.0, cz = 0.0;
   if constexpr (PBC) pos.ld(member ? d1.w : i0 + ni / 2, cx, cy, cz);
+  const double ux = -cx * pp.inv_box, uy = -cy * pp.inv_box, uz = -cz * pp.inv_box;
   const int seg = tid / TPI, sub = tid & (TPI - 1);
   const bool active = seg < ni;
   const int slot = i0 + (active ? seg : 0);
@@ -700,7 +704,7 @@ k_tile_half(P pos, const int32_t* __restrict__ member,
   for (int t = tid; t < ns; t += nt) {
     double x, y, z;
     pos.ld(stage[soff + t], x, y, z);
-    unwrap_near<PBC>(x, y, z, cx, cy, cz, pp);
+    unwrap_near<PBC>(x, y, z, ux, uy, uz, pp);
     double* c = cell + kHalfStride / 8 * t;
     c[0] = x;
     c[1] = y;
@@ -708,7 +712,7 @@ k_tile_half(P pos, const int32_t* __restrict__ member,
     c[3] = c[4] = c[5] = 0.0;
   }
   if constexpr (PBC) {
-    unwrap_near<PBC>(xi, yi, zi, cx, cy, cz, pp);
+    unwrap_near<PBC>(xi, yi, zi, ux, uy, uz, pp);
     if (active && (fabs(xi - cx) >= reach || fabs(yi - cy) >= reach || fabs(zi - cz) >= reach))
       *flag = 1;
   }
@@ -1080,6 +1084,7 @@ inline int pair_params(const ForceArgs& fa, const LaunchConfig& lc, PairParams* 
     return set_error(LJGPU_ERR_INVALID_ARGUMENT, "block size must be a multiple of 64 in [64, 1024]");
   pp->c24 = 24.0 * fa.dt;
   pp->c48 = 48.0 * fa.dt;
+  pp->c_unit = pp->c24 * kUnitScale;
   pp->cl2 = fa.cl2;
   pp->box = fa.box > 0.0 ? fa.box : 0.0;
   pp->inv_box = fa.box > 0.0 ? 1.0 / fa.box : 0.0;

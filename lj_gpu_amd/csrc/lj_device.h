@@ -122,6 +122,7 @@ struct MomSoa {
 // square root (computed on the host, so no kernel spends VALU on it).
 struct PairParams {
   double c24, c48, cl2, box, inv_box, rc;
+  double c_unit;  // c24 * kUnitScale (lj_df_unit_f64)
   float c24f, c48f;
 };
 
@@ -149,34 +150,40 @@ __device__ __forceinline__ double rcp_f64(double x) {
   return fma(fma(-x, r, 1.0), r, r);
 }
 
-// The reciprocals of x[0..N) in place (N = 1, 2 or 4) from one refined
-// reciprocal of their product (Montgomery's simultaneous inversion):
-// 1/x0 = x1 / (x0 x1) and so on. A refined reciprocal costs the
-// transcendental unit's quarter rate plus two FMAs; four of them cost
-// 96 cycles per wavefront, one of the product with the nine products
-// around it 60. Each result carries five roundings more than the refined
-// reciprocal's own error (about 11 ulp): about 16 ulp, 4e-15 relative. The
-// factors are squared distances of LJ pairs, so their product stays far
-// from overflow and underflow.
+// c / x in FP64, the refined reciprocal with one more product.
+__device__ __forceinline__ double rcp_scaled_f64(double x, double c) {
+  const double r = __builtin_amdgcn_rcp(x);
+  const double cr = c * r;
+  return fma(fma(-x, r, 1.0), cr, cr);
+}
+
+// c / x of x[0..N) in place (N = 1, 2 or 4) from one refined reciprocal of
+// their product (Montgomery's simultaneous inversion): 1/x0 = x1 / (x0 x1)
+// and so on. A refined reciprocal costs the transcendental unit's quarter
+// rate plus two FMAs; four of them cost 96 cycles per wavefront, one of the
+// product with the ten products around it 64. Each result carries five
+// roundings more than the refined reciprocal's own error (about 11 ulp):
+// about 16 ulp, 4e-15 relative. The factors are squared distances of LJ
+// pairs, so their product stays far from overflow and underflow.
 template <int N>
-__device__ __forceinline__ void rcp_f64_batch(double (&x)[N]) {
+__device__ __forceinline__ void rcp_scaled_f64_batch(double (&x)[N], double c) {
   static_assert(N == 1 || N == 2 || N == 4, "batched reciprocal of 1, 2 or 4 values");
   if constexpr (N == 1) {
-    x[0] = rcp_f64(x[0]);
+    x[0] = rcp_scaled_f64(x[0], c);
   } else if constexpr (N == 2) {
-    const double r = rcp_f64(x[0] * x[1]);
+    const double r = rcp_scaled_f64(x[0] * x[1], c);
     const double a = x[0];
     x[0] = x[1] * r;
     x[1] = a * r;
   } else {
     const double p01 = x[0] * x[1], p23 = x[2] * x[3];
-    const double r = rcp_f64(p01 * p23);
+    const double r = rcp_scaled_f64(p01 * p23, c);
     const double r01 = r * p23, r23 = r * p01;
-    const double a = x[0], c = x[2];
+    const double a = x[0], b = x[2];
     x[0] = x[1] * r01;
     x[1] = a * r01;
     x[2] = x[3] * r23;
-    x[3] = c * r23;
+    x[3] = b * r23;
   }
 }
 
@@ -196,15 +203,20 @@ __device__ __forceinline__ double lj_df_f64(double r2, const PairParams& pp) {
   return lj_df_f64_s(rcp_f64(r2), r2, pp);
 }
 
-// FP64 force scalar without the factor 24*dt: s^4 (1 - 2 s^3) with s = 1/r2,
-// exactly 0 where `inside` is false (only the high word of s is cleared, as
-// in lj_df_f64). The tiled kernels multiply each row's sum by 24*dt once, so
-// the constants here are instruction operands instead of registers.
+// FP64 force scalar up to a factor: with s = kCbrt2 / r2, s^4 - s^7 is
+// kCbrt2^4 times s0^4 (1 - 2 s0^3) for s0 = 1/r2, as kCbrt2^3 = 2 (to 6.2e-17:
+// the nearest double to the cube root happens to lie that close). Folding the 2
+// into s saves a multiplication per pair; the tiled kernels multiply each
+// row's sum by kUnitScale * 24 * dt once. Exactly 0 where `inside` is false
+// (only the high word of s is cleared, as in lj_df_f64).
+constexpr double kCbrt2 = 0x1.428a2f98d728bp+0;
+constexpr double kUnitScale = 0.5 / kCbrt2;
 __device__ __forceinline__ double lj_df_unit_f64(double s, bool inside) {
   const int hi = inside ? __double2hiint(s) : 0;
   s = __hiloint2double(hi, __double2loint(s));
-  const double s3 = s * s * s;
-  return (s3 * s) * fma(-2.0, s3, 1.0);
+  const double s2 = s * s;
+  const double s3 = s2 * s, s4 = s2 * s2;
+  return fma(-s3, s4, s4);
 }
 
 // Mixed-precision force scalar: r2 (computed in FP64) rounded once to FP32,
@@ -238,11 +250,26 @@ struct KahanF32 {
 };
 
 // Sum over the `W` consecutive lanes of a wavefront segment (W a power of two
-// <= 64); every lane of the segment receives the total.
+// <= 64); every lane of the segment receives the total. Steps up to 16 lanes
+// are DPP moves (the quad's neighbour and its other pair; then, with equal
+// values within a quad or an eight, the mirrored lane), which stay out of the
+// LDS pipe that the tile kernels' reads fill: through shuffles a row's three
+// sums took twelve LDS passes.
+template <int CTRL>
+__device__ __forceinline__ double dpp_d(double v) {
+  return __hiloint2double(
+      __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true),
+      __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true));
+}
+
 template <int W>
 __device__ __forceinline__ double segment_sum(double v) {
+  if constexpr (W >= 2) v += dpp_d<0xB1>(v);   // quad_perm [1, 0, 3, 2]
+  if constexpr (W >= 4) v += dpp_d<0x4E>(v);   // quad_perm [2, 3, 0, 1]
+  if constexpr (W >= 8) v += dpp_d<0x141>(v);  // row_half_mirror
+  if constexpr (W >= 16) v += dpp_d<0x140>(v); // row_mirror
 #pragma unroll
-  for (int m = W / 2; m >= 1; m >>= 1) v += __shfl_xor(v, m, W);
+  for (int m = 16; m < W; m <<= 1) v += __shfl_xor(v, m, W);
   return v;
 }
 
