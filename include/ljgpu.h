@@ -411,16 +411,16 @@ int ljgpu_maxwell_boltzmann(int32_t particle_number, double temperature, uint32_
 
 /* Run repeated force evaluations (steps >= 4) and the MD driver's plain steps
  * as replays of captured HIP graphs (1, the default) or as individual
- * launches (0). A force call of `steps` launches replays graphs of 64, 16 and
- * 4 launches (longest first) and launches the remaining 0-3 singly; each
- * graph is captured once per argument set and kept in a cache of 12 (least
+ * launches (0). A force call of `steps` evaluations replays graphs of 64, 16
+ * and 4 evaluations (longest first) and launches the remaining 0-3; a launch
+ * over LDS tiles carries about sqrt of a graph's evaluations. Each graph is captured once per argument set and kept in a cache of 12 (least
  * recently used evicted). */
 int ljgpu_set_graphs(ljgpu_ctx* ctx, int enable);
 
 /* Concurrent chains of a many-step call over LDS tiles (1 to 4, default 2).
  * With c > 1, a call of 4 or more steps over at least 64 * c tiles splits
  * the tiles into c contiguous parts and runs each part's steps as its own
- * chain of launches on its own stream of the context, forked from and joined
+ * chain of launches (about sqrt(steps) of them) on its own stream of the context, forked from and joined
  * back into the context stream within the call (launched directly, not
  * replayed from graphs). The parts update disjoint particles, so the momenta
  * are bitwise those of one chain; one chain's launch ramp and tail overlap

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <functional>
 #include <mutex>
@@ -452,6 +453,33 @@ int launch_one(ljgpu_ctx* ctx, const ListView& lv, const LaunchConfig& lc, const
   return launch_one_on(ctx->stream, lv, lc, fa, mixed, accum);
 }
 
+// Launches that carry `steps` evaluations: about sqrt(steps) of them, up to
+// kMaxLaunchSteps evaluations each, over full-list tiles (a tile updates its
+// own particles only, so its evaluations need no order across tiles), one per
+// evaluation otherwise.
+int32_t launches_of(const ListView& lv, const LaunchConfig& lc, int32_t steps) {
+  if (lv.tile_blocks <= 0 || lc.half_atomic || steps <= 1) return steps;
+  const int32_t per = std::clamp(static_cast<int32_t>(std::lround(std::sqrt(steps))), 1,
+                                 kMaxLaunchSteps);
+  return (steps + per - 1) / per;
+}
+
+// Launch l of `launches` that carry `steps` evaluations together.
+int launch_part(hipStream_t stream, const ListView& lv, LaunchConfig lc, const ForceArgs& fa,
+                bool mixed, int accum, int32_t steps, int32_t launches, int32_t l) {
+  lc.steps = static_cast<int32_t>(int64_t{steps} * (l + 1) / launches -
+                                  int64_t{steps} * l / launches);
+  return launch_one_on(stream, lv, lc, fa, mixed, accum);
+}
+
+int launch_steps(ljgpu_ctx* ctx, const ListView& lv, const LaunchConfig& lc, const ForceArgs& fa,
+                 bool mixed, int accum, int32_t steps) {
+  const int32_t launches = launches_of(lv, lc, steps);
+  for (int32_t l = 0; l < launches; l++)
+    TRY(launch_part(ctx->stream, lv, lc, fa, mixed, accum, steps, launches, l));
+  return LJGPU_OK;
+}
+
 int enqueue_force(ljgpu_ctx* ctx, const ForceArgs& fa, bool mixed, int accum) {
   if (ctx->n == 0) return LJGPU_OK;
   ListView lv;
@@ -731,10 +759,11 @@ int run_steps(ljgpu_ctx* ctx, const ForceArgs& caller, int32_t steps, bool mixed
         HIP_TRY(hipStreamWaitEvent(ctx->chain_stream[c - 1], ctx->ev_fork, 0),
                 "hipStreamWaitEvent");
     }
-    for (int32_t s = 0; s < steps; s++)
+    const int32_t launches = launches_of(lv, lc, steps);
+    for (int32_t l = 0; l < launches; l++)
       for (int c = 0; c < chains; c++)
-        TRY(launch_one_on(c == 0 ? ctx->stream : ctx->chain_stream[c - 1], part[c], lc, fa, mixed,
-                          accum));
+        TRY(launch_part(c == 0 ? ctx->stream : ctx->chain_stream[c - 1], part[c], lc, fa, mixed,
+                        accum, steps, launches, l));
     for (int c = 1; c < chains; c++) {
       HIP_TRY(hipEventRecord(ctx->ev_join[c - 1], ctx->chain_stream[c - 1]), "hipEventRecord");
       HIP_TRY(hipStreamWaitEvent(ctx->stream, ctx->ev_join[c - 1], 0), "hipStreamWaitEvent");
@@ -750,14 +779,13 @@ int run_steps(ljgpu_ctx* ctx, const ForceArgs& caller, int32_t steps, bool mixed
         const StepKey key = step_key(fa, lv, lc, mixed, accum, chunk, 1);
         hipGraphExec_t exec = nullptr;
         TRY(cached_graph(ctx, key, [&]() {
-          for (int32_t s = 0; s < chunk; s++) TRY(launch_one(ctx, lv, lc, fa, mixed, accum));
-          return LJGPU_OK;
+          return launch_steps(ctx, lv, lc, fa, mixed, accum, chunk);
         }, &exec));
         for (; done + chunk <= steps; done += chunk)
           HIP_TRY(hipGraphLaunch(exec, ctx->stream), "hipGraphLaunch");
       }
     }
-    for (; done < steps; done++) TRY(launch_one(ctx, lv, lc, fa, mixed, accum));
+    TRY(launch_steps(ctx, lv, lc, fa, mixed, accum, steps - done));
   }
   if (slots) TRY(slot_scatter(ctx, fa, caller));
   return LJGPU_OK;

@@ -16,9 +16,9 @@
 namespace ljgpu {
 
 // Graph replay of repeated force evaluations. A force call of `steps`
-// launches runs as replays of captured graphs of kGraphChunks[c] launches,
-// taken greedily from the longest (so 20 steps = 16 + 4), then fewer than
-// kGraphMinSteps single launches. A graph is captured once per set of kernel
+// evaluations runs as replays of captured graphs of kGraphChunks[c] evaluations,
+// taken greedily from the longest (so 20 steps = 16 + 4), then launches for
+// fewer than kGraphMinSteps. A graph is captured once per set of kernel
 // arguments and chunk length and kept in a small cache (kGraphCacheSize
 // entries, least recently used evicted), so calls that alternate step counts,
 // precisions or arrays replay their graphs instead of re-capturing them.
@@ -37,6 +37,17 @@ constexpr int32_t kGraphChunk = 100;
 // less overlap on MI355X); single-chain calls replay graphs.
 constexpr int kMaxChains = 4;
 constexpr int32_t kMinChainTiles = 64;  // fewer tiles: one chain
+// A launch over tiles carries several evaluations of a call, each workgroup
+// running its tile that many times (it reads everything again each time). A
+// launch costs about 3 to 4.5 us of host time and a ramp and a tail on the
+// device, so one launch per evaluation left small systems waiting for the
+// host; the last launch's tail grows with the evaluations it carries. About
+// sqrt(steps) per launch balances the two. Measured, one per launch / 4 / 10 /
+// 100: 119,164 particles, 100 evaluations 1530 / 1464 / 1437 / 1602 us, 10
+// evaluations 199 / 194 / 209 us; 62,500 particles in an open box, 100
+// evaluations 850 / 589 / 555 / 586 us; 16,384 particles, 10 evaluations 136 /
+// 104 / 104 us.
+constexpr int32_t kMaxLaunchSteps = 16;
 // Calls with at least kSlotMinSteps steps over spatially ordered tiles run
 // over copies of q and p in slot order (two gathers and a scatter per call).
 constexpr int32_t kSlotMinSteps = 16;

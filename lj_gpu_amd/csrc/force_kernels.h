@@ -445,7 +445,8 @@ __device__ __forceinline__ void tile_row_stream(const M& mom, const uint16_t* __
 // offsets from global memory instead (less LDS per workgroup, so more
 // resident workgroups per CU).
 //
-// A launch covers tiles [first, first + nblocks). They are assigned
+// A launch covers tiles [first, first + nblocks), `steps` evaluations of each
+// (a workgroup reads and stages its tile anew for every one). They are assigned
 // XCD-aware: the workgroups on XCD x (blockIdx % 8 == x) walk the contiguous
 // range [x*per, (x+1)*per) of the launch's tiles with a stride of gridDim/8. With one workgroup per tile each does a single tile; with a
 // smaller (persistent) grid each loops over several, so resident workgroups
@@ -577,7 +578,8 @@ __device__ __forceinline__ void tile_body(P pos, M mom, const int32_t* __restric
   }
   // The frame check ORed over the workgroup through one LDS word: threads
   // that fail it write this tile's index, which no earlier tile of this
-  // workgroup used, so the word needs no reset.
+  // workgroup used (an earlier evaluation of this tile found the same), so the
+  // word needs no reset.
   if (far) *flag = b;
   __syncthreads();  // staging complete
   const bool any_far = PBC && *flag == b;
@@ -630,7 +632,7 @@ k_tile(P pos, M mom, const int32_t* __restrict__ nop, const int32_t* __restrict_
        const int32_t* __restrict__ stage,
        const uint16_t* __restrict__ local, const uint16_t* __restrict__ sliced,
        const int32_t* __restrict__ wave_off, int32_t wpb, int32_t first, int32_t nblocks,
-       PairParams pp, double reach, const double2* __restrict__ rep_box) {
+       int32_t steps, PairParams pp, double reach, const double2* __restrict__ rep_box) {
   // Dynamic LDS only (no static LDS, so its base is address 0 and constant
   // offsets fold into the LDS instructions): a 16-byte header holding the
   // frame-check word, then the tile's positions (and offsets).
@@ -644,10 +646,16 @@ k_tile(P pos, M mom, const int32_t* __restrict__ nop, const int32_t* __restrict_
   const int stride = static_cast<int>(gridDim.x) / kXcds;
   const int t_end = min(nblocks, (xcd + 1) * per);
   for (int b = xcd * per + static_cast<int>(blockIdx.x) / kXcds; b < t_end; b += stride) {
-    tile_body<TPI, U, PREC, P, M, PBC, OFFS_LDS, SL>(pos, mom, nop, member, slot_ptr, desc, stage,
-                                                     local, sliced, wave_off, wpb, first + b, pp,
-                                                     reach, rep_box, lb, flag, nullptr);
-    __syncthreads();  // the next tile overwrites this tile's LDS
+    for (int s = 0; s < steps; s++) {
+      // Opaque, so that each step reads its tile again instead of holding what
+      // the first one read in registers.
+      int tile = first + b;
+      asm volatile("" : "+s"(tile));
+      tile_body<TPI, U, PREC, P, M, PBC, OFFS_LDS, SL>(pos, mom, nop, member, slot_ptr, desc,
+                                                       stage, local, sliced, wave_off, wpb, tile,
+                                                       pp, reach, rep_box, lb, flag, nullptr);
+      __syncthreads();  // the next step or tile overwrites this one's LDS
+    }
   }
 }
 
@@ -943,7 +951,8 @@ int run_tile(hipStream_t s, P pos, M mom, const ListView& lv, const PairParams& 
                      lds_bytes, s, pos, mom, lv.nop, lv.tile_member, lv.tile_slot_ptr,
                      reinterpret_cast<const int4*>(lv.tile_desc), lv.tile_stage, lv.tile_local,
                      lv.tile_sliced, lv.tile_wave_off, lv.tile_waves_per_block, lv.tile_first,
-                     lv.tile_blocks, pp, reach, reinterpret_cast<const double2*>(lv.replica_box));
+                     lv.tile_blocks, lc.steps, pp, reach,
+                     reinterpret_cast<const double2*>(lv.replica_box));
   return launch_status("tiled force kernel launch");
 }
 

@@ -244,6 +244,7 @@ struct LaunchConfig {
   bool tile_offsets_lds = false;  // tile kernel: stage entry offsets in LDS too
   int tile_resident = 0;     // tile kernel: persistent grid of this many workgroups per CU (0: one per tile)
   int cus = 0;               // compute units of the device
+  int steps = 1;             // tile kernel: force evaluations per launch
   bool half_atomic = false;  // list is a half list: scatter to j with atomics
   bool clamp = false;   // clamp every index read into range (unvalidated lists)
 };

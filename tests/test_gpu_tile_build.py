@@ -117,3 +117,30 @@ def test_atomic_half_lists_over_tiles(ctx, name, layout, tile):
         assert normwise(p, f) < FP64_TOL
     assert ctx.list_info().tile_particles == 0 and ctx.get_tiles() is None
     ctx.set_half_mode(G.HALF_AUTO)
+
+
+@pytest.mark.parametrize("tile,resident", [(64, 0), (4, 0), (1, 1)])
+@pytest.mark.parametrize("graphs", [True, False])
+def test_launches_of_several_evaluations(ctx, tile, resident, graphs):
+    """A launch over tiles carries several evaluations of a call (in one chain
+    for 14 tiles, two for 215 or 859, a persistent grid of fewer workgroups than
+    tiles included): bit for bit what as many calls of one give."""
+    q, box, full, _ = system("ragged")
+    n = q.shape[0]
+    print(f"tile={tile} resident={resident} graphs={graphs}", flush=True)
+    ctx.set_kernel_config(4, 256, 4)
+    ctx.set_tiling(tile, resident_per_cu=resident)
+    ctx.set_half_mode(G.HALF_AUTO)
+    ctx.set_graphs(graphs)
+    dq, da, db = ctx.array(q), ctx.zeros(q.shape), ctx.zeros(q.shape)
+    ctx.build_list(dq, n, box, G.LIST_FULL)
+    for steps in (2, 3, 5, 10, 17, 300):
+        da.zero()
+        db.zero()
+        ctx.force_aos_f64(dq, da, 1e-3, G.CL2, box, steps)
+        for _ in range(steps):
+            ctx.force_aos_f64(dq, db, 1e-3, G.CL2, box, 1)
+        ctx.sync()
+        np.testing.assert_array_equal(da.download(), db.download())
+    ctx.set_graphs(True)
+    ctx.set_tiling(64)
