@@ -201,6 +201,8 @@ int build_list(ljgpu_ctx* ctx, const PosIn& q, int32_t n, double box, double sea
                bool sort_rows = true);
 // Enqueue one force evaluation p += F(q) * dt over the installed list.
 int enqueue_force(ljgpu_ctx* ctx, const ForceArgs& fa, bool mixed, int accum);
+int launch_one_on(hipStream_t stream, const ListView& lv, const LaunchConfig& lc,
+                  const ForceArgs& fa, bool mixed, int accum);
 // `steps` force evaluations (graph replays where possible).
 int run_steps(ljgpu_ctx* ctx, const ForceArgs& fa, int32_t steps, bool mixed, int accum);
 void drop_graph(ljgpu_ctx* ctx);

@@ -1117,6 +1117,15 @@ int run_force(void* stream, const ListView& lv, const ForceArgs& fa, const Launc
     return run_layout<PREC>(s, pos, mom, lv, pp, lc);
   }
   PosAos pos{fa.q[0]};
+  if (fa.q_next) {
+    if constexpr (PREC != kMixedKahan) {
+      if (can_drift(lv, lc, fa) && lc.steps == 1) {
+        MomDrift mom{fa.p[0], fa.q[0], fa.q_next, fa.drift_dt, pp.box, pp.inv_box};
+        return run_tile<4, 4, PREC, PosAos, MomDrift, true, false, true>(s, pos, mom, lv, pp, lc);
+      }
+    }
+    return set_error(LJGPU_ERR_INVALID_ARGUMENT, "kick and drift: launch shape");
+  }
   MomAos mom{fa.p[0]};
   return run_layout<PREC>(s, pos, mom, lv, pp, lc);
 }

@@ -84,6 +84,39 @@ struct MomAos {
   }
 };
 
+// x mapped into [0, box): one multiply by 1/box instead of a divide, then
+// the last-bit cases (a result just below 0, or equal to box) folded in.
+__device__ __forceinline__ double wrap_box(double x, double box, double inv_box) {
+  x = fma(-box, floor(x * inv_box), x);
+  if (x < 0.0) x += box;
+  return x >= box ? x - box : x;
+}
+
+// AoS momenta whose kick is followed by the particle's drift: the new
+// positions q + p dt, wrapped into [0, box), go to another array, as other
+// tiles still read the old ones.
+struct MomDrift {
+  double* __restrict__ p;
+  const double* __restrict__ q;
+  double* __restrict__ q_next;
+  double dt, box, inv_box;
+  __device__ __forceinline__ void add(int i, double ax, double ay, double az) const {
+    double* r = p + 4 * static_cast<int64_t>(i);
+    double4 row = reinterpret_cast<const double4*>(q)[i];
+    double2 xy = *reinterpret_cast<double2*>(r);
+    double z = r[2];
+    xy.x += ax;
+    xy.y += ay;
+    z += az;
+    *reinterpret_cast<double2*>(r) = xy;
+    r[2] = z;
+    row.x = wrap_box(fma(xy.x, dt, row.x), box, inv_box);
+    row.y = wrap_box(fma(xy.y, dt, row.y), box, inv_box);
+    row.z = wrap_box(fma(z, dt, row.z), box, inv_box);
+    reinterpret_cast<double4*>(q_next)[i] = row;
+  }
+};
+
 struct MomAos3 {
   double* __restrict__ p;
   __device__ __forceinline__ void add(int i, double ax, double ay, double az) const {

@@ -235,6 +235,10 @@ struct ForceArgs {
   const double* q[3] = {nullptr, nullptr, nullptr};  // AoS: q[0] is double[N][4] (or [3])
   double* p[3] = {nullptr, nullptr, nullptr};
   double dt = 0, cl2 = 0, box = 0;
+  // Not null: the kick is followed by the drift q_next = q + drift_dt * p,
+  // wrapped into the box (tiles that can_drift).
+  double* q_next = nullptr;
+  double drift_dt = 0;
 };
 
 struct LaunchConfig {
@@ -248,6 +252,16 @@ struct LaunchConfig {
   bool half_atomic = false;  // list is a half list: scatter to j with atomics
   bool clamp = false;   // clamp every index read into range (unvalidated lists)
 };
+
+// Whether a launch can end in the particles' drift (ForceArgs::q_next): AoS
+// arrays in slot order in a periodic box, over tiles sliced for the default
+// four lanes and four entries, the one shape that kernel is built for.
+inline bool can_drift(const ListView& lv, const LaunchConfig& lc, const ForceArgs& fa) {
+  return !fa.soa && !fa.aos3 && fa.box > 0.0 && lv.tile_blocks > 0 && !lv.tile_member &&
+         !lv.replica_box && !lc.half_atomic && !lc.tile_offsets_lds && !lc.clamp &&
+         lc.lanes == 4 && lc.unroll == 4 && lv.tile_sliced && lv.tile_sliced_lanes == 4 &&
+         lv.tile_sliced_unroll == 4;
+}
 
 // Enqueue one force evaluation on `stream`. Returns LJGPU_OK or an error.
 int launch_force_f64(void* stream, const ListView& lv, const ForceArgs& fa,
