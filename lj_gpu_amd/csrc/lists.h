@@ -217,7 +217,7 @@ int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t tile_particles,
 // (cut_partition) of the positions in `cut`, if it has any and they have
 // none yet, and the places of a row (its inner ones, then the others) are given out so
 // that the lanes that read LDS together mostly read different banks
-// (slice_part). Without it places follow local.
+// (order_part). Without it places follow local.
 struct CutHint {
   PosIn q;                        // positions in the caller's particle order
   double box = 0.0;               // single system: periodic box (<= 0 open)

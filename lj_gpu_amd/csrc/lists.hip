@@ -1538,53 +1538,126 @@ __global__ void k_wave_slices(TileSpans spans, int32_t nblocks, int32_t wpb,
   len[id] = batches * 64 * unroll;
 }
 
-// The places of one part of a row (its inner entries, or the others), by one
-// lane: n ranks in[0], in[step], ... take the places out[0 .. n), whose first
-// one has target class `phase`. cnt is this lane's column of the class counts
-// (kBankClasses words, kSliceRows apart). The q-th entry of a class takes the
-// q-th place that has the class as its target; the entries beyond those fill,
-// in order, the places whose class ran out. No entry waits for the one
-// before it, unlike bank_class_order's walk over the classes left, and a row
-// that runs out of a class leaves only that place to chance.
-__device__ __forceinline__ void slice_part(uint16_t* in, int step, uint16_t* out, uint32_t* cnt,
-                                           int phase, int n) {
-  constexpr int kB = 8;  // entries in flight
+constexpr int kRowLanes = 8;  // lanes that walk one row together
+constexpr int kRowBatch = 4;  // entries per lane in flight
+
+// LDS of one wavefront's order_part: class counts, a byte each, four classes to
+// a word, a column of words per lane; and the free places of its rows.
+struct OrderLds {
+  uint32_t cnt[kBankClasses / 4][64];
+  uint8_t hole[64 / kRowLanes][kBankRowMax];
+};
+static_assert(kTileMaxStage <= 255 * kBankClasses, "a class of a row fits a byte");
+static_assert(kBankClasses == 4 * kRowLanes, "one lane per word of counts, four steps a level");
+
+// The places of one part of each row (its inner entries, or the others),
+// kRowLanes lanes to a row, a wavefront's rows together: n ranks from[0],
+// from[step], ... (of at most nmax in any of its rows) take the places
+// to[0 .. n), the same memory, whose first one has target class `phase`. Each
+// lane counts its own entries by class; a sum over the row's lanes leaves the
+// number of each lane's first one, from which its entries take their numbers
+// q, and the q-th entry of a class takes the q-th place that has the class as
+// its target. The entries beyond those fill, in order, the places whose class ran out. One lane per row and
+// the seven other wavefronts idle took 182 us with the rest of k_tile_slices at
+// 119,000 particles (density 1), 35 at 2,000; this way 125 and 26.
+__device__ __forceinline__ void order_part(const uint16_t* from, int step, uint16_t* to, int phase,
+                                           int n, int nmax, OrderLds& lds) {
+  constexpr int kSteps = kBankRowMax / kRowLanes, kGroup = 8;
+  const int wl = static_cast<int>(threadIdx.x) & 63;
+  int lane = wl & (kRowLanes - 1);
+  const int seg = wl - lane;
+  asm volatile("" : "+v"(lane));  // places and comparisons again, not held in registers
+  const uint32_t below = (1u << lane) - 1;
+  uint32_t* cnt = &lds.cnt[0][wl];
+  uint8_t* holes = lds.hole[seg / kRowLanes];
+  // This row's lanes for which `c` holds.
+  auto row_bits = [&](bool c) {
+    const uint64_t v = __ballot(c);
+    const uint32_t h = wl < 32 ? static_cast<uint32_t>(v) : static_cast<uint32_t>(v >> 32);
+    return h >> (seg & 31) & ((1u << kRowLanes) - 1);
+  };
 #pragma unroll
-  for (int c = 0; c < kBankClasses; c++) cnt[c * kSliceRows] = 0;
+  for (int w = 0; w < kBankClasses / 4; w++) cnt[w * 64] = 0;
+  uint32_t entry[kSteps / 2];  // two ranks each
+#pragma unroll
+  for (int g = 0; g < kSteps; g += kGroup) {
+    if (g * kRowLanes >= nmax) break;  // the whole wavefront
+#pragma unroll
+    for (int u = g; u < g + kGroup; u++) {
+      const int t = u * kRowLanes + lane;
+      const uint32_t x = from[(t < n ? t : 0) * step];
+      entry[u / 2] = u % 2 ? entry[u / 2] | x << 16 : x;
+    }
+#pragma unroll
+    for (int u = g; u < g + kGroup; u++) {
+      const uint32_t x = entry[u / 2] >> 16 * (u % 2) & 0xffffu;
+      if (u * kRowLanes + lane < n) atomicAdd(&cnt[(x >> 2 & 7) * 64], 1u << (x & 3) * 8);
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the wavefront's own, in order
+  // Lane w sums word w of the row's counts: each lane's first number.
+  uint32_t total = 0;
+  {
+    uint32_t* word = &lds.cnt[lane][seg];
+    uint32_t v[kRowLanes];
+#pragma unroll
+    for (int j = 0; j < kRowLanes; j++) v[j] = word[j];
+#pragma unroll
+    for (int j = 0; j < kRowLanes; j++) {
+      word[j] = total;
+      total += v[j];
+    }
+  }
+  // Place k has the class (phase + k) % 32, and it is the (k / 32)-th of it.
+  uint32_t of_class[4];
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const int c = (phase + j * kRowLanes + lane) & (kBankClasses - 1);
+    of_class[j] = __shfl(total, seg + c / 4, 64) >> (c & 3) * 8 & 255u;
+  }
+  int free = 0;
+  for (int level = 0; level * kBankClasses < nmax; level++) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int k = level * kBankClasses + j * kRowLanes + lane;
+      const bool hole = k < n && level >= static_cast<int>(of_class[j]);
+      const uint32_t bits = row_bits(hole);
+      if (hole) holes[free + __popc(bits & below)] = static_cast<uint8_t>(k);
+      free += __popc(bits);
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   int left = 0;
-  for (int k0 = 0; k0 < n; k0 += kB) {
-    int x[kB];
-    uint32_t q[kB];
+  asm volatile("" : "+v"(n), "+v"(lane));
 #pragma unroll
-    for (int u = 0; u < kB; u++) x[u] = in[min(k0 + u, n - 1) * step];
+  for (int g = 0; g < kSteps; g += kGroup) {
+    if (g * kRowLanes >= nmax) break;
+    uint32_t q[kGroup];
 #pragma unroll
-    for (int u = 0; u < kB; u++)
-      q[u] = atomicAdd(&cnt[(x[u] & (kBankClasses - 1)) * kSliceRows], k0 + u < n ? 1u : 0u);
-#pragma unroll
-    for (int u = 0; u < kB; u++) {
-      if (k0 + u >= n) continue;
-      const int d = ((x[u] - phase) & (kBankClasses - 1)) + kBankClasses * static_cast<int>(q[u]);
-      if (d < n) out[d] = static_cast<uint16_t>(x[u]);
-      else in[left++ * step] = static_cast<uint16_t>(x[u]);  // where it was read already
-    }
-  }
-  int at = 0;
-  for (int k0 = 0; k0 < n; k0 += kB) {
-    uint32_t q[kB];
-    uint16_t x[kB];
-    bool hole[kB];
-#pragma unroll
-    for (int u = 0; u < kB; u++) q[u] = cnt[((phase + k0 + u) & (kBankClasses - 1)) * kSliceRows];
-#pragma unroll
-    for (int u = 0; u < kB; u++) {
-      hole[u] = k0 + u < n && static_cast<uint32_t>(k0 + u) / kBankClasses >= q[u];
-      x[u] = in[min(at, n - 1) * step];
-      at += hole[u] ? 1 : 0;
+    for (int u = g; u < g + kGroup; u++) {
+      const uint32_t x = entry[u / 2] >> 16 * (u % 2) & 0xffffu;
+      q[u - g] = atomicAdd(&cnt[(x >> 2 & 7) * 64],
+                           u * kRowLanes + lane < n ? 1u << (x & 3) * 8 : 0u) >> (x & 3) * 8 & 255u;
     }
 #pragma unroll
-    for (int u = 0; u < kB; u++)
-      if (hole[u]) out[k0 + u] = x[u];
+    for (int u = g; u < g + kGroup; u++) {
+      const uint32_t x = entry[u / 2] >> 16 * (u % 2) & 0xffffu;
+      int d = static_cast<int>(((x - phase) & (kBankClasses - 1)) + kBankClasses * q[u - g]);
+      const bool valid = u * kRowLanes + lane < n, over = valid && d >= n;
+      const uint32_t bits = row_bits(over);
+      if (over) d = holes[left + __popc(bits & below)];
+      left += __popc(bits);
+      if (valid) to[d] = static_cast<uint16_t>(x);
+    }
   }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
+// The wavefront's largest v.
+__device__ __forceinline__ int wave_max(int v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
+  return __builtin_amdgcn_readfirstlane(v);
 }
 
 struct CutDev {
@@ -1595,8 +1668,6 @@ struct CutDev {
   const double* rep_box;
   double cl2;
 };
-constexpr int kRowLanes = 8;  // lanes that read one row together
-constexpr int kRowBatch = 5;  // entries per lane in flight
 
 // The slices of one block per workgroup, rows in groups of `grows` (at most
 // kSliceRows, a multiple of a wavefront's rows): slice position p of
@@ -1609,30 +1680,32 @@ constexpr int kRowBatch = 5;  // entries per lane in flight
 // `local` as well; inner[s] receives the inner count of slot s's row. The
 // partners' positions are staged in LDS (POS_LDS) or, where they do not fit,
 // read from memory.
-//   ORDER gives the places of each class out by slice_part, so that the 32
+//   ORDER gives the places of each class out by order_part, so that the 32
 // lanes that read LDS together mostly read different banks (the row's phase
-// is its first lane's place among them): one lane per row, all of a group in
-// one wavefront, on ranks in LDS, rows `stride` (an odd number of dwords)
-// apart, inner entries forward from the row's start, the others backward from
-// its end. At density 1 a half-wavefront's read then takes 2.3 passes over the
+// is its first lane's place among them), on ranks in LDS, rows `stride` (an odd
+// number of dwords) apart, inner entries forward from the row's start, the
+// others backward from its end. At density 1 a half-wavefront's read then takes 2.3 passes over the
 // banks (modelled on the tiles of 119,164 particles) against 2.6 in the
 // bank-class order: FP64 forces 2.4 %, mixed 4 % faster.
 //   Rows of more than kBankRowMax entries, and all rows without ORDER, keep
-// the order of `local`.
+// the order of `local`. Three workgroups fit a CU's LDS, hence the 80 VGPRs
+// (a dozen spilled in the CUT form; at 167 registers one workgroup fits).
+constexpr int kSliceThreads = 512;
+static_assert(kSliceThreads == kSliceRows * kRowLanes, "order_part takes a group's rows at once");
+
 template <bool CUT, bool POS_LDS, bool ORDER>
-__global__ __launch_bounds__(512) void k_tile_slices(
+__global__ __launch_bounds__(kSliceThreads) __attribute__((amdgpu_waves_per_eu(6))) void k_tile_slices(
     const int32_t* __restrict__ desc, int32_t nblocks, const int32_t* __restrict__ slot_ptr,
     int32_t* __restrict__ inner, uint16_t* __restrict__ local, CutDev cut, int32_t grows,
     int32_t stride, int32_t lanes, int32_t wpb, int32_t scale, int32_t pad,
     const int32_t* __restrict__ wave_off, uint16_t* __restrict__ sliced) {
   extern __shared__ double slice_lds[];
   __shared__ int32_t start[kSliceRows], len[kSliceRows], in_len[kSliceRows];
-  // The rows; then the staged positions, whose place the class counts and the
-  // ordered rows take afterwards.
+  // The rows; then the staged positions, whose place order_part's memory takes
+  // afterwards.
   uint16_t* in = reinterpret_cast<uint16_t*>(slice_lds);
   double* pos = slice_lds + (grows * stride + 3) / 4;
-  uint32_t* cnt = reinterpret_cast<uint32_t*>(pos);
-  uint16_t* out = ORDER ? reinterpret_cast<uint16_t*>(cnt + kBankClasses * kSliceRows) : in;
+  OrderLds* order = reinterpret_cast<OrderLds*>(pos);
   const int tid = static_cast<int>(threadIdx.x), nt = static_cast<int>(blockDim.x);
   const int lane = tid & (kRowLanes - 1), seg = (tid & 63) & ~(kRowLanes - 1);
   const int lsh = 31 - __clz(lanes);
@@ -1744,13 +1817,19 @@ __global__ __launch_bounds__(512) void k_tile_slices(
       }
       __syncthreads();
       if (ORDER) {
-        if (tid < nr && len[tid] <= kBankRowMax) {
-          const int m = len[tid], nin = in_len[tid];
-          const int phase = (g0 + tid) << lsh;
-          uint16_t* row = in + tid * stride;
-          if (nin > 0) slice_part(row, 1, out + tid * stride, cnt + tid, phase, nin);
-          if (m > nin)
-            slice_part(row + m - 1, -1, out + tid * stride + nin, cnt + tid, phase + nin, m - nin);
+        // At least as many threads as the group's rows have lanes.
+        const int r = tid / kRowLanes;
+        const int m = r < nr && len[r] <= kBankRowMax ? len[r] : 0;
+        const int nin = m > 0 ? in_len[r] : 0;
+        const int phase = (g0 + r) << lsh;
+        uint16_t* row = in + min(r, grows - 1) * stride;
+#pragma nounroll
+        for (int part = 0; part < 2; part++) {
+          const int n = part ? m - nin : nin, most = wave_max(n);
+          if (most == 0) continue;  // the whole wavefront
+          const int skip = part ? nin : 0;
+          order_part(part ? row + max(m - 1, 0) : row, part ? -1 : 1, row + skip, phase + skip, n,
+                     most, order[tid / 64]);
         }
         __syncthreads();
       }
@@ -1760,7 +1839,7 @@ __global__ __launch_bounds__(512) void k_tile_slices(
         const int r = w * rpw + ((tid & 63) >> lsh) - g0;
         const int m = r < nr ? len[r] : 0;
         const bool direct = m > kBankRowMax;
-        const uint16_t* src = direct ? local + start[r] : out + min(r, grows - 1) * stride;
+        const uint16_t* src = direct ? local + start[r] : in + min(r, grows - 1) * stride;
         int k = tid & (lanes - 1);
 #pragma unroll 4
         for (int32_t p = tid & 63; p < n; p += 64, k += lanes)
@@ -2651,7 +2730,7 @@ int dev_slice_tiles(hipStream_t s, const int32_t* slot_ptr, int32_t lanes, int32
   size_t rows = 0, order = 0;
   for (;; grows /= 2) {
     rows = (sizeof(uint16_t) * stride * grows + 7) / 8 * 8;
-    order = bank_order ? rows + sizeof(uint32_t) * kBankClasses * kSliceRows : 0;
+    order = bank_order ? sizeof(OrderLds) * kSliceThreads / 64 : 0;
     if (grows == kSliceRows / 2 || rows + order <= kTileLdsMax) break;
   }
   const size_t pos = cut ? sizeof(double) * 3 * static_cast<size_t>(t.max_stage) : 0;
@@ -2660,7 +2739,7 @@ int dev_slice_tiles(hipStream_t s, const int32_t* slot_ptr, int32_t lanes, int32
                 : !cut      ? k_tile_slices<false, false, true>
                 : pos_lds   ? k_tile_slices<true, true, true>
                             : k_tile_slices<true, false, true>;
-  kernel<<<std::min(t.blocks, 65535), 512, rows + std::max(order, pos_lds ? pos : 0), s>>>(
+  kernel<<<std::min(t.blocks, 65535), kSliceThreads, rows + std::max(order, pos_lds ? pos : 0), s>>>(
       t.desc.as<int32_t>(), t.blocks, slot_ptr,
       t.cut || cut ? t.inner.as<int32_t>() : nullptr, t.local.as<uint16_t>(), cd, grows, stride,
       lanes, wpb, scale, pad, t.wave_off.as<int32_t>(), t.sliced.as<uint16_t>());
