@@ -316,39 +316,105 @@ __global__ __launch_bounds__(kBlock) void k_copy_rows(int32_t n, const int32_t* 
 
 // Sort of each segment [start[r], start[r] + len[r]) of src into the same
 // positions of dst, ascending, one wavefront per segment. Segments of up to
-// 64*R elements are sorted in registers by a bitonic network (element
-// e = r*64 + lane in register r of that lane; partners closer than 64 are
-// exchanged across lanes, farther ones between a lane's own registers), padded
-// with INT32_MAX. Longer segments fall back to a rank sort from memory: each
+// 512 elements are sorted in registers by a bitonic network (element e = r*64 +
+// lane in register r of that lane; partners closer than 64 are exchanged
+// across lanes, farther ones between a lane's own registers), padded with
+// INT32_MAX. Longer segments fall back to a rank sort from memory: each
 // element goes to the number of smaller elements plus the equal ones before
 // it.
-template <int R>
-__device__ __forceinline__ void wave_bitonic(int32_t (&v)[R], int lane) {
+//   Exchanges across lanes are DPP moves and permlane swaps; through shuffles
+// the sort was bound by the LDS pipe (132 passes for a row of 150: 175 us at
+// 119,000 particles, density 1). What bounds it now is VALU issue, so a row of
+// 129 to 192 sorts three registers, not four.
+
+// The lanes that keep the smaller value where lanes J apart are exchanged
+// within sorted runs of K (64: all one run).
+constexpr uint64_t keep_min_lanes(int K, int J, bool descending) {
+  uint64_t m = 0;
+  for (int l = 0; l < 64; l++) {
+    const bool up = ((K < 64 && (l & K)) != 0) == descending;
+    if (((l & J) == 0) == up) m |= uint64_t{1} << l;
+  }
+  return m;
+}
+
+template <int CTRL>
+__device__ __forceinline__ int32_t dpp_i32(int32_t v) {
+  return __builtin_amdgcn_mov_dpp(v, CTRL, 0xf, 0xf, true);
+}
+
+// One exchange between the lanes l and l ^ J.
+template <int K, int J, bool DESC>
+__device__ __forceinline__ void exchange(int32_t& v) {
+  int32_t a = v, b;
+  if constexpr (J == 16 || J == 32) {
+    // The swap leaves each pair's two values in a and b of both its lanes.
+    const auto ab = J == 16 ? __builtin_amdgcn_permlane16_swap(v, v, false, false)
+                            : __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    a = static_cast<int32_t>(ab[0]);
+    b = static_cast<int32_t>(ab[1]);
+  } else if constexpr (J == 8) {
+    b = dpp_i32<0x128>(v);  // row_ror:8
+  } else if constexpr (J == 4) {
+    b = dpp_i32<0x1B>(dpp_i32<0x141>(v));  // row_half_mirror, then each quad reversed
+  } else if constexpr (J == 2) {
+    b = dpp_i32<0x4E>(v);  // quad_perm [2, 3, 0, 1]
+  } else {
+    static_assert(J == 1, "lanes up to 32 apart");
+    b = dpp_i32<0xB1>(v);  // quad_perm [1, 0, 3, 2]
+  }
+  const bool low = __builtin_amdgcn_inverse_ballot_w64(keep_min_lanes(K, J, DESC));
+  v = low ? min(a, b) : max(a, b);
+}
+
+// Runs of K in v, each one bitonic, sorted in alternating directions.
+template <int K, int J, bool DESC>
+__device__ __forceinline__ void merge_lanes(int32_t& v) {
+  exchange<K, J, DESC>(v);
+  if constexpr (J > 1) merge_lanes<K, J / 2, DESC>(v);
+}
+
+// v[0..R), bitonic, sorted.
+template <int R, bool DESC>
+__device__ __forceinline__ void merge_regs(int32_t* v) {
+  if constexpr (R == 1) {
+    merge_lanes<64, 32, DESC>(v[0]);
+  } else {
 #pragma unroll
-  for (int k = 2; k <= 64 * R; k <<= 1) {
-#pragma unroll
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      if (j >= 64) {
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-          const int pr = r ^ (j / 64);
-          if (pr > r) {
-            const bool up = ((r * 64 + lane) & k) == 0;
-            const int32_t a = v[r], b = v[pr];
-            v[r] = up ? min(a, b) : max(a, b);
-            v[pr] = up ? max(a, b) : min(a, b);
-          }
-        }
-      } else {
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-          const int32_t other = __shfl_xor(v[r], j, 64);
-          const bool up = ((r * 64 + lane) & k) == 0;
-          const bool keep_min = ((lane & j) == 0) == up;
-          v[r] = keep_min ? min(v[r], other) : max(v[r], other);
-        }
-      }
+    for (int r = 0; r < R / 2; r++) {
+      const int32_t lo = min(v[r], v[r + R / 2]), hi = max(v[r], v[r + R / 2]);
+      v[r] = DESC ? hi : lo;
+      v[r + R / 2] = DESC ? lo : hi;
     }
+    merge_regs<R / 2, DESC>(v);
+    merge_regs<R / 2, DESC>(v + R / 2);
+  }
+}
+
+template <int R, bool DESC>
+__device__ __forceinline__ void sort_regs(int32_t* v) {
+  if constexpr (R == 1) {
+    merge_lanes<2, 1, DESC>(v[0]);
+    merge_lanes<4, 2, DESC>(v[0]);
+    merge_lanes<8, 4, DESC>(v[0]);
+    merge_lanes<16, 8, DESC>(v[0]);
+    merge_lanes<32, 16, DESC>(v[0]);
+    merge_lanes<64, 32, DESC>(v[0]);
+  } else if constexpr (R == 3) {
+    static_assert(!DESC, "ascending only");
+    // As four registers with one of padding after the third: that one stays
+    // where it is, and the steps with it vanish.
+    sort_regs<2, false>(v);
+    sort_regs<1, true>(v + 2);
+    const int32_t lo = min(v[1], v[2]);
+    v[2] = max(v[1], v[2]);
+    v[1] = lo;
+    merge_regs<2, false>(v);
+    merge_regs<1, false>(v + 2);
+  } else {
+    sort_regs<R / 2, false>(v);
+    sort_regs<R / 2, true>(v + R / 2);
+    merge_regs<R, DESC>(v);
   }
 }
 
@@ -361,7 +427,7 @@ __device__ __forceinline__ void sort_segment(const int32_t* __restrict__ src,
     const int e = r * 64 + lane;
     v[r] = e < m ? src[e] : INT32_MAX;
   }
-  wave_bitonic<R>(v, lane);
+  sort_regs<R, false>(v);
 #pragma unroll
   for (int r = 0; r < R; r++) {
     const int e = r * 64 + lane;
@@ -390,6 +456,8 @@ __global__ __launch_bounds__(kBlock) void k_row_sort(int32_t n, const int32_t* _
       sort_segment<1>(in, o, m, lane);
     } else if (m <= 128) {
       sort_segment<2>(in, o, m, lane);
+    } else if (m <= 192) {
+      sort_segment<3>(in, o, m, lane);
     } else if (m <= 256) {
       sort_segment<4>(in, o, m, lane);
     } else if (m <= 512) {

@@ -357,3 +357,23 @@ def test_tile_order_switch_and_untiled(ctx):
     ctx.set_tiling(0)
     assert ctx.get_tile_order() == (-1, None)
     ctx.set_tiling(64)
+
+
+@pytest.mark.parametrize("sizes", [(2, 3, 64, 65, 66), (128, 129, 130, 150), (192, 193, 194),
+                                   (256, 257, 258), (512, 513, 514, 515)])
+def test_rows_of_every_sort_width(ctx, sizes):
+    """Clusters of m particles in a shuffled order, each particle the partner
+    of all others of its cluster: rows of m - 1 entries, ascending, at the
+    lengths where the sort changes its width."""
+    rng = np.random.default_rng(3)
+    n = sum(sizes)
+    q = np.zeros((n, 4))
+    of = rng.permutation(np.repeat(np.arange(len(sizes)), sizes))
+    q[:, :3] = rng.uniform(0.0, 1.0, (n, 3))
+    q[:, 0] += 10.0 * of
+    dq = ctx.array(q)
+    ctx.build_list(dq, n, 0.0, G.LIST_FULL)
+    got = ctx.get_list()
+    rows = [np.setdiff1d(np.flatnonzero(of == of[i]), [i]) for i in range(n)]
+    np.testing.assert_array_equal(got.number_of_partners, [len(r) for r in rows])
+    np.testing.assert_array_equal(got.sorted_list, np.concatenate(rows))
