@@ -1121,7 +1121,9 @@ int run_force(void* stream, const ListView& lv, const ForceArgs& fa, const Launc
     if constexpr (PREC != kMixedKahan) {
       if (can_drift(lv, lc, fa) && lc.steps == 1) {
         MomDrift mom{fa.p[0], fa.q[0], fa.q_next, fa.drift_dt, pp.box, pp.inv_box};
-        return run_tile<4, 4, PREC, PosAos, MomDrift, true, false, true>(s, pos, mom, lv, pp, lc);
+        return lc.lanes == 4
+                   ? run_tile<4, 4, PREC, PosAos, MomDrift, true, false, true>(s, pos, mom, lv, pp, lc)
+                   : run_tile<16, 4, PREC, PosAos, MomDrift, true, false, true>(s, pos, mom, lv, pp, lc);
       }
     }
     return set_error(LJGPU_ERR_INVALID_ARGUMENT, "kick and drift: launch shape");

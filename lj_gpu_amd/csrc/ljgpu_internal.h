@@ -254,13 +254,13 @@ struct LaunchConfig {
 };
 
 // Whether a launch can end in the particles' drift (ForceArgs::q_next): AoS
-// arrays in slot order in a periodic box, over tiles sliced for the default
-// four lanes and four entries, the one shape that kernel is built for.
+// arrays in slot order in a periodic box, over tiles sliced for four or sixteen
+// lanes and four entries, the shapes that kernel is built for.
 inline bool can_drift(const ListView& lv, const LaunchConfig& lc, const ForceArgs& fa) {
   return !fa.soa && !fa.aos3 && fa.box > 0.0 && lv.tile_blocks > 0 && !lv.tile_member &&
          !lv.replica_box && !lc.half_atomic && !lc.tile_offsets_lds && !lc.clamp &&
-         lc.lanes == 4 && lc.unroll == 4 && lv.tile_sliced && lv.tile_sliced_lanes == 4 &&
-         lv.tile_sliced_unroll == 4;
+         (lc.lanes == 4 || lc.lanes == 16) && lc.unroll == 4 && lv.tile_sliced &&
+         lv.tile_sliced_lanes == lc.lanes && lv.tile_sliced_unroll == 4;
 }
 
 // Enqueue one force evaluation on `stream`. Returns LJGPU_OK or an error.

@@ -371,3 +371,28 @@ def test_md_kicks_that_end_in_the_next_drift(ctx, every, prec, accum):
     np.testing.assert_array_equal(out[0][0], out[1][0])
     np.testing.assert_array_equal(out[0][1], out[1][1])
     np.testing.assert_array_equal(out[0][0][:, 3], q0[:, 3])
+
+
+@pytest.mark.parametrize("cells,tile", [(11, 64), (12, 64), (11, 32)])
+@pytest.mark.parametrize("prec", [G.PREC_F64, G.PREC_MIXED])
+def test_md_shapes_on_both_sides_of_the_few_particle_rule(ctx, cells, tile, prec):
+    """5,324 particles run as sixteen lanes over tiles of 16, 6,912 (and any
+    other tile size) as configured, which is what the context reports after the run;
+    graphs and single launches agree bit for bit."""
+    q0, p0, box = liquid(cells)
+    ctx.set_kernel_config(4, 256, 4)
+    ctx.set_tiling(tile)
+    out = []
+    for graphs in (True, False):
+        ctx.set_graphs(graphs)
+        dq, dp = ctx.array(q0), ctx.array(p0)
+        st, _ = ctx.md_run(dq, dp, box, 12, DT, rebuild_every=6, precision=prec)
+        assert st.max_abs_drift < 1e-3 * q0.shape[0]
+        out.append((dq.download(), dp.download()))
+    ctx.set_graphs(True)
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    np.testing.assert_array_equal(out[0][1], out[1][1])
+    ctx.build_list(dq, q0.shape[0], box, G.LIST_FULL)
+    info = ctx.list_info()
+    assert info.tile_particles == tile
+    ctx.set_tiling(64)
