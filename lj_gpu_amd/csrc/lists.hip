@@ -617,29 +617,38 @@ struct GridArgs {
 
 __device__ __forceinline__ int cell_coord(double x, double origin, double width, int m, double box) {
   x -= origin;
-  if (box > 0.0) x -= box * floor(x / box);  // the wrapped image's cell
+  // The wrapped image's cell (no division for the positions inside: their
+  // quotient is below 1).
+  if (box > 0.0 && !(x >= 0.0 && x < box)) x -= box * floor(x / box);
   const int v = static_cast<int>(floor(x / width));
   return min(max(v, 0), m - 1);
 }
 
-// Also sets *outside when a periodic box has a coordinate outside [0, box)
-// (the pair search then applies the minimum image in every cell).
-__global__ void k_cell_assign(int32_t n, PosIn q, GridArgs g, int32_t* __restrict__ count,
+// A particle's cell; sets *outside when a periodic box has a coordinate outside
+// [0, box) (the pair search then applies the minimum image in every cell).
+struct CellKey {
+  PosIn q;
+  GridArgs g;
+  __device__ __forceinline__ int32_t operator()(int64_t t, int32_t* outside) const {
+    const int64_t o = t * q.stride;
+    const double x = q.x[o], y = q.y[o], z = q.z[o];
+    // Written as negations so that NaN counts as outside.
+    if (g.box > 0.0 &&
+        !(x >= 0.0 && x < g.box && y >= 0.0 && y < g.box && z >= 0.0 && z < g.box))
+      atomicOr(outside, 1);
+    const int cx = cell_coord(x, g.o0, g.w0, g.nc0, g.box);
+    const int cy = cell_coord(y, g.o1, g.w1, g.nc1, g.box);
+    const int cz = cell_coord(z, g.o2, g.w2, g.nc2, g.box);
+    return (cz * g.nc1 + cy) * g.nc0 + cx;
+  }
+};
+
+__global__ void k_cell_assign(int32_t n, CellKey key, int32_t* __restrict__ count,
                               int32_t* __restrict__ slot, int32_t* __restrict__ cell_of,
                               int32_t* __restrict__ outside) {
   for (int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; t < n;
        t += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    const int64_t o = t * q.stride;
-    if (g.box > 0.0) {
-      const double x = q.x[o], y = q.y[o], z = q.z[o];
-      // Written as negations so that NaN counts as outside.
-      if (!(x >= 0.0 && x < g.box && y >= 0.0 && y < g.box && z >= 0.0 && z < g.box))
-        atomicOr(outside, 1);
-    }
-    const int cx = cell_coord(q.x[o], g.o0, g.w0, g.nc0, g.box);
-    const int cy = cell_coord(q.y[o], g.o1, g.w1, g.nc1, g.box);
-    const int cz = cell_coord(q.z[o], g.o2, g.w2, g.nc2, g.box);
-    const int32_t c = (cz * g.nc1 + cy) * g.nc0 + cx;
+    const int32_t c = key(t, outside);
     cell_of[t] = c;
     slot[t] = atomicAdd(&count[c], 1);
   }
@@ -705,6 +714,101 @@ __global__ void k_cell_place(int32_t n, PosIn q, const int32_t* __restrict__ cel
     const int64_t o = static_cast<int64_t>(i) * q.stride;
     cpos[bin_place(t, i, cell_of, start, arrival)] =
         make_double4(q.x[o], q.y[o], q.z[o], static_cast<double>(i));
+  }
+}
+
+// What a binned particle leaves at its place: its cell-ordered position and
+// cell, or its index.
+struct CellPut {
+  PosIn q;
+  double4* cpos;
+  int32_t* cell;
+  __device__ __forceinline__ void operator()(int32_t place, int32_t i, int32_t c) const {
+    const int64_t o = static_cast<int64_t>(i) * q.stride;
+    cpos[place] = make_double4(q.x[o], q.y[o], q.z[o], static_cast<double>(i));
+    cell[place] = c;
+  }
+};
+struct OrderPut {
+  int32_t* order;
+  __device__ __forceinline__ void operator()(int32_t place, int32_t i, int32_t) const {
+    order[place] = i;
+  }
+};
+
+// Few particles binned by one workgroup, counts and arrival order in LDS: what
+// k_cell_assign or k_order_key, a scan, k_bin_index and a placing kernel do for
+// more, whose five launches took 16 us and the gaps between them at 2,048
+// particles; this one takes 9 to 11 there and 12 to 15 at 4,000, bound by one
+// compute unit's latencies, and twice as many particles would cost what the
+// launches do. start (null: not wanted) takes the bins' starts, *flag what the
+// keys' flag gathered.
+constexpr int32_t kBinSmall = 4096;   // particles
+constexpr int32_t kBinsSmall = 8192;  // bins
+constexpr int kBinThreads = 1024;
+
+template <class Key, class Put>
+__global__ __launch_bounds__(kBinThreads) void k_bin_small(int32_t n, int32_t nbins, Key key,
+                                                           Put put, int32_t* __restrict__ start,
+                                                           int32_t* __restrict__ flag,
+                                                           ScanStats* __restrict__ res) {
+  __shared__ int32_t bin[kBinsSmall + 1];
+  __shared__ uint16_t arrival[kBinSmall];
+  __shared__ int32_t sh[kBinThreads / 64], slo[kBinThreads / 64], shi[kBinThreads / 64];
+  __shared__ int32_t gathered;
+  constexpr int kPer = kBinSmall / kBinThreads;
+  const int32_t tid = static_cast<int32_t>(threadIdx.x);
+  for (int32_t c = tid; c <= nbins; c += kBinThreads) bin[c] = 0;
+  if (tid == 0) gathered = 0;
+  __syncthreads();
+  int32_t mine[kPer], slot[kPer];
+#pragma unroll
+  for (int u = 0; u < kPer; u++) {
+    const int32_t t = u * kBinThreads + tid;
+    if (t >= n) break;
+    mine[u] = key(t, &gathered);
+    slot[u] = atomicAdd(&bin[mine[u]], 1);
+  }
+  __syncthreads();
+  const int32_t piece = (nbins + kBinThreads - 1) / kBinThreads;
+  const int32_t c0 = min(tid * piece, nbins), c1 = min(c0 + piece, nbins);
+  int32_t v = 0, lo = INT32_MAX, hi = INT32_MIN, total;
+  for (int32_t c = c0; c < c1; c++) {
+    const int32_t x = bin[c];
+    v += x;
+    lo = min(lo, x);
+    hi = max(hi, x);
+  }
+  int32_t run = block_exclusive<int32_t>(v, &total, sh);
+  for (int32_t c = c0; c < c1; c++) {
+    const int32_t x = bin[c];
+    bin[c] = run;
+    if (start) start[c] = run;
+    run += x;
+  }
+  if (tid == 0) {
+    bin[nbins] = n;
+    if (start) start[nbins] = n;
+    if (flag) *flag = gathered;
+  }
+  block_extrema(lo, hi, slo, shi);
+  if (tid == 0) *res = ScanStats{n, lo, hi};
+#pragma unroll
+  for (int u = 0; u < kPer; u++) {
+    const int32_t t = u * kBinThreads + tid;
+    if (t < n) arrival[bin[mine[u]] + slot[u]] = static_cast<uint16_t>(t);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kPer; u++) {
+    const int32_t t = u * kBinThreads + tid;
+    if (t >= n) break;
+    const int32_t a = bin[mine[u]], b = bin[mine[u] + 1];
+    int32_t place = a;
+    if (b - a > kCellOrderMax) place += slot[u];
+    else
+      for (int32_t k = a; k < b; k++) place += arrival[k] < t ? 1 : 0;
+    put(place, t, mine[u]);
   }
 }
 
@@ -2015,17 +2119,26 @@ struct OrderGrid {
   int32_t key0;    // first key of the system
 };
 
-__global__ void k_order_key(int32_t n, PosIn q, OrderGrid one, const OrderGrid* __restrict__ grids,
-                            const int32_t* __restrict__ rep_of, int32_t* __restrict__ count,
-                            int32_t* __restrict__ slot, int32_t* __restrict__ key_of) {
-  for (int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; t < n;
-       t += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+struct OrderKey {
+  PosIn q;
+  OrderGrid one;
+  const OrderGrid* grids;
+  const int32_t* rep_of;
+  __device__ __forceinline__ int32_t operator()(int64_t t, int32_t*) const {
     const OrderGrid g = rep_of ? grids[rep_of[t]] : one;
     const int64_t o = t * q.stride;
     const int cx = cell_coord(q.x[o], 0.0, g.w[0], g.nc[0], g.box);
     const int cy = cell_coord(q.y[o], 0.0, g.w[1], g.nc[1], g.box);
     const int cz = cell_coord(q.z[o], 0.0, g.w[2], g.nc[2], g.box);
-    const int32_t k = g.key0 + (cz * g.nc[1] + cy) * g.nc[0] + cx;
+    return g.key0 + (cz * g.nc[1] + cy) * g.nc[0] + cx;
+  }
+};
+
+__global__ void k_order_key(int32_t n, OrderKey key, int32_t* __restrict__ count,
+                            int32_t* __restrict__ slot, int32_t* __restrict__ key_of) {
+  for (int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; t < n;
+       t += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    const int32_t k = key(t, nullptr);
     key_of[t] = k;
     slot[t] = atomicAdd(&count[k], 1);
   }
@@ -2301,19 +2414,31 @@ int dev_makepair(hipStream_t s, const PosIn& q, int32_t n, double box, double se
   int32_t* count = w.cell_count.as<int32_t>();
   int32_t* cstart = w.cell_start.as<int32_t>();
   int32_t* outside = count + ncell;
-  LCHECK(fill<int32_t>(s, count, ncell + 1, 0));
   LCHECK(results(w));
-  k_cell_assign<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, q, g, count, w.cell_slot.as<int32_t>(),
-                                                       w.cell_of.as<int32_t>(), outside);
-  LTRY(hipGetLastError(), "cell assign kernel");
-  LCHECK(dev_scan_async(s, count, cstart, ncell, w, &w.results->cells));
+  const CellKey key{q, g};
+  const bool few = n <= kBinSmall && ncell <= kBinsSmall;
+  if (few) {
+    k_bin_small<<<1, kBinThreads, 0, s>>>(
+        n, static_cast<int32_t>(ncell), key,
+        CellPut{q, w.cpos.as<double4>(), w.cell_sorted.as<int32_t>()}, cstart, outside,
+        &w.results->cells);
+    LTRY(hipGetLastError(), "cell kernel");
+  } else {
+    LCHECK(fill<int32_t>(s, count, ncell + 1, 0));
+    k_cell_assign<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, key, count, w.cell_slot.as<int32_t>(),
+                                                         w.cell_of.as<int32_t>(), outside);
+    LTRY(hipGetLastError(), "cell assign kernel");
+    LCHECK(dev_scan_async(s, count, cstart, ncell, w, &w.results->cells));
+  }
   const bool half = kind == LJGPU_LIST_HALF;
   const int R = cg.brute ? 0 : (fine ? 2 : 1);
   // Unsorted rows need a candidate order fixed by the positions alone: the
   // stencil kernel's run order with each cell's particles by index. The
   // single-cell kernel has no such order, so it always sorts.
   if (R == 0) sort_rows = true;
-  if (sort_rows) {
+  if (few) {
+    // Placed already, each cell's particles by index.
+  } else if (sort_rows) {
     k_cell_scatter<<<grid_for(n, kBlock), kBlock, 0, s>>>(
         n, q, w.cell_of.as<int32_t>(), w.cell_slot.as<int32_t>(), cstart, w.cpos.as<double4>(),
         w.cell_sorted.as<int32_t>());
@@ -2530,16 +2655,22 @@ int dev_tile_order_begin(hipStream_t s, const PosIn& q, int32_t n, double box,
   int32_t* start = w.cell_start.as<int32_t>();
   int32_t* arrival = w.cell_sorted.as<int32_t>();
   const int32_t* key_of = w.cell_of.as<int32_t>();
-  LCHECK(fill<int32_t>(s, count, keys, 0));
-  k_order_key<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, q, grids[0], dgrids, rep_of, count,
-                                                     w.cell_slot.as<int32_t>(),
-                                                     w.cell_of.as<int32_t>());
-  LTRY(hipGetLastError(), "tile order key kernel");
-  LCHECK(dev_scan_async(s, count, start, keys, w, &w.results->order));
-  k_bin_index<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, key_of, w.cell_slot.as<int32_t>(), start,
-                                                     arrival);
-  k_order_place<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, key_of, start, arrival,
-                                                       w.order.as<int32_t>());
+  const OrderKey key{q, grids[0], dgrids, rep_of};
+  if (n <= kBinSmall && keys <= kBinsSmall) {
+    k_bin_small<<<1, kBinThreads, 0, s>>>(n, static_cast<int32_t>(keys), key,
+                                          OrderPut{w.order.as<int32_t>()}, nullptr, nullptr,
+                                          &w.results->order);
+  } else {
+    LCHECK(fill<int32_t>(s, count, keys, 0));
+    k_order_key<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, key, count, w.cell_slot.as<int32_t>(),
+                                                       w.cell_of.as<int32_t>());
+    LTRY(hipGetLastError(), "tile order key kernel");
+    LCHECK(dev_scan_async(s, count, start, keys, w, &w.results->order));
+    k_bin_index<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, key_of, w.cell_slot.as<int32_t>(), start,
+                                                       arrival);
+    k_order_place<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, key_of, start, arrival,
+                                                         w.order.as<int32_t>());
+  }
   LTRY(hipGetLastError(), "tile order kernels");
   *begun = true;
   return LJGPU_OK;

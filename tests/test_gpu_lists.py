@@ -377,3 +377,27 @@ def test_rows_of_every_sort_width(ctx, sizes):
     rows = [np.setdiff1d(np.flatnonzero(of == of[i]), [i]) for i in range(n)]
     np.testing.assert_array_equal(got.number_of_partners, [len(r) for r in rows])
     np.testing.assert_array_equal(got.sorted_list, np.concatenate(rows))
+
+
+@pytest.mark.parametrize("n", [1, 2, 1023, 1025, 4095, 4096, 4097])
+@pytest.mark.parametrize("kind", ["periodic", "outside", "open", "sparse", "crowded"])
+def test_few_particles_binned_by_one_workgroup(ctx, n, kind):
+    """Both sides of the 4,096-particle rule (and, sparse, of the 8,192-bin
+    one): shuffled lattices in a periodic box (outside: some moved out of it
+    by its length), open ones, a few particles in a large box, and hundreds in one cell."""
+    rng = np.random.default_rng(11)
+    q, box = G.lattice_periodic(11, 0.8, 3)
+    q = np.ascontiguousarray(q[rng.permutation(q.shape[0])[:n]])
+    if kind == "outside":
+        q[q[:, 0] < 0.4 * box, 0] += box
+    elif kind == "open":
+        box = 0.0
+    elif kind == "sparse":
+        q[:, :3] *= 4.0
+        box *= 4.0
+    elif kind == "crowded":
+        q[:min(n, 300), :3] = 5.0 + rng.uniform(0.0, 0.2, (min(n, 300), 3))
+    print(f"n={n} {kind}", flush=True)
+    dq = ctx.array(q)
+    ctx.build_list(dq, n, box, G.LIST_FULL)
+    _same(ctx.get_list(), G.makepair(q, box, G.LIST_FULL))
