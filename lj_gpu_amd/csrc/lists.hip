@@ -1711,7 +1711,7 @@ __global__ void k_wave_slices(TileSpans spans, int32_t nblocks, int32_t wpb,
 }
 
 constexpr int kRowLanes = 8;  // lanes that walk one row together
-constexpr int kRowBatch = 4;  // entries per lane in flight
+constexpr int kRowBatch = 3;  // entries per lane in flight
 
 // LDS of one wavefront's order_part: class counts, a byte each, four classes to
 // a word, a column of words per lane; and the free places of its rows.
@@ -1731,7 +1731,7 @@ static_assert(kBankClasses == 4 * kRowLanes, "one lane per word of counts, four 
 // q, and the q-th entry of a class takes the q-th place that has the class as
 // its target. The entries beyond those fill, in order, the places whose class ran out. One lane per row and
 // the seven other wavefronts idle took 182 us with the rest of k_tile_slices at
-// 119,000 particles (density 1), 35 at 2,000; this way 125 and 26.
+// 119,000 particles (density 1), 35 at 2,000; this way 122 and 25.
 __device__ __forceinline__ void order_part(const uint16_t* from, int step, uint16_t* to, int phase,
                                            int n, int nmax, OrderLds& lds) {
   constexpr int kSteps = kBankRowMax / kRowLanes, kGroup = 8;
@@ -1872,7 +1872,7 @@ __global__ __launch_bounds__(kSliceThreads) __attribute__((amdgpu_waves_per_eu(6
     int32_t stride, int32_t lanes, int32_t wpb, int32_t scale, int32_t pad,
     const int32_t* __restrict__ wave_off, uint16_t* __restrict__ sliced) {
   extern __shared__ double slice_lds[];
-  __shared__ int32_t start[kSliceRows], len[kSliceRows], in_len[kSliceRows];
+  __shared__ int32_t start[kSliceRows], len[kSliceRows];
   // The rows; then the staged positions, whose place order_part's memory takes
   // afterwards.
   uint16_t* in = reinterpret_cast<uint16_t*>(slice_lds);
@@ -1899,9 +1899,35 @@ __global__ __launch_bounds__(kSliceThreads) __attribute__((amdgpu_waves_per_eu(6
         const int32_t m = slot_ptr[i0 + g0 + tid + 1] - a;
         start[tid] = a;
         len[tid] = m;
-        in_len[tid] = !CUT && inner ? inner[i0 + g0 + tid] : m;
       }
+      // The row of these lanes, its particle's position and its first entries,
+      // requested before the staging so that their latencies overlap it.
+      const int r = tid / kRowLanes;
+      const int32_t slot = i0 + g0 + min(r, nr - 1);
+      const int32_t a = slot_ptr[slot];
+      const int all = slot_ptr[slot + 1] - a;
+      const int m = r < nr && all <= kBankRowMax ? all : 0;
+      if (CUT && r < nr && all > kBankRowMax && lane == 0) inner[slot] = all;
+      int nin = CUT || m == 0 ? 0 : inner ? inner[slot] : m, nout = 0;
+      double xi = 0.0, yi = 0.0, zi = 0.0;
+      if (CUT) {
+        const int64_t i = static_cast<int64_t>(cut.member ? cut.member[slot] : slot) * st;
+        xi = cut.q.x[i];
+        yi = cut.q.y[i];
+        zi = cut.q.z[i];
+      }
+      constexpr int kStep = kRowBatch * kRowLanes;
+      int next[kRowBatch];
+      auto load = [&](int k0) {
+#pragma unroll
+        for (int u = 0; u < kRowBatch; u++) {
+          const int k = k0 + u * kRowLanes + lane;
+          next[u] = local[a + (k < m ? k : 0)];
+        }
+      };
+      if (m > 0) load(0);
       if (CUT && POS_LDS) {
+#pragma unroll 2
         for (int t = tid; t < ns; t += nt) {
           const int64_t j = static_cast<int64_t>(cut.stage[soff + t]) * st;
           pos[3 * t] = cut.q.x[j];
@@ -1910,91 +1936,65 @@ __global__ __launch_bounds__(kSliceThreads) __attribute__((amdgpu_waves_per_eu(6
         }
       }
       __syncthreads();
-      for (int r = tid / kRowLanes; r < nr; r += nt / kRowLanes) {
-        const int32_t a = start[r];
-        const int m = len[r];
-        if (m > kBankRowMax) {
-          if (CUT && lane == 0) inner[i0 + g0 + r] = m;
-          continue;
-        }
-        uint16_t* row = in + r * stride;
-        int nin = CUT ? 0 : in_len[r], nout = 0;
-        double xi = 0.0, yi = 0.0, zi = 0.0;
-        if (CUT) {
-          const int32_t slot = i0 + g0 + r;
-          const int64_t i = static_cast<int64_t>(cut.member ? cut.member[slot] : slot) * st;
-          xi = cut.q.x[i];
-          yi = cut.q.y[i];
-          zi = cut.q.z[i];
-        }
-        for (int k0 = 0; k0 < m; k0 += kRowBatch * kRowLanes) {
-          int rank[kRowBatch];
+      uint16_t* row = in + min(r, grows - 1) * stride;
+      for (int k0 = 0; k0 < m; k0 += kStep) {
+        int rank[kRowBatch];
+#pragma unroll
+        for (int u = 0; u < kRowBatch; u++)
+          rank[u] = k0 + u * kRowLanes + lane < m ? next[u] / 24 : -1;
+        if (k0 + kStep < m) load(k0 + kStep);
+        if (!CUT) {
 #pragma unroll
           for (int u = 0; u < kRowBatch; u++) {
             const int k = k0 + u * kRowLanes + lane;
-            rank[u] = k < m ? local[a + k] / 24 : -1;
+            if (rank[u] >= 0)
+              row[ORDER && k >= nin ? m - 1 - (k - nin) : k] = static_cast<uint16_t>(rank[u]);
           }
-          if (!CUT) {
-#pragma unroll
-            for (int u = 0; u < kRowBatch; u++) {
-              const int k = k0 + u * kRowLanes + lane;
-              if (rank[u] >= 0)
-                row[ORDER && k >= nin ? m - 1 - (k - nin) : k] = static_cast<uint16_t>(rank[u]);
-            }
-            continue;
-          }
-          bool in_u[kRowBatch];
-#pragma unroll
-          for (int u = 0; u < kRowBatch; u++) {
-            const int t = max(rank[u], 0);
-            double xj, yj, zj;
-            if (POS_LDS) {
-              xj = pos[3 * t];
-              yj = pos[3 * t + 1];
-              zj = pos[3 * t + 2];
-            } else {
-              const int64_t j = static_cast<int64_t>(cut.stage[soff + t]) * st;
-              xj = cut.q.x[j];
-              yj = cut.q.y[j];
-              zj = cut.q.z[j];
-            }
-            in_u[u] = cut_inner(xi, yi, zi, xj, yj, zj, box, cut.cl2);
-          }
-#pragma unroll
-          for (int u = 0; u < kRowBatch; u++) {
-            const bool valid = rank[u] >= 0;
-            constexpr uint32_t kSeg = (1u << kRowLanes) - 1;
-            const uint32_t vm = kSeg & static_cast<uint32_t>(__ballot(valid) >> seg);
-            const uint32_t im = kSeg & static_cast<uint32_t>(__ballot(valid && in_u[u]) >> seg);
-            const uint32_t below = (1u << lane) - 1;
-            if (valid)
-              row[in_u[u] ? nin + __popc(im & below) : m - 1 - nout - __popc(vm & ~im & below)] =
-                  static_cast<uint16_t>(rank[u]);
-            nin += __popc(im);
-            nout += __popc(vm & ~im);
-          }
+          continue;
         }
-        if (CUT) {
-          if (lane == 0) {
-            inner[i0 + g0 + r] = nin;
-            in_len[r] = nin;
+        bool in_u[kRowBatch];
+#pragma unroll
+        for (int u = 0; u < kRowBatch; u++) {
+          const int t = max(rank[u], 0);
+          double xj, yj, zj;
+          if (POS_LDS) {
+            xj = pos[3 * t];
+            yj = pos[3 * t + 1];
+            zj = pos[3 * t + 2];
+          } else {
+            const int64_t j = static_cast<int64_t>(cut.stage[soff + t]) * st;
+            xj = cut.q.x[j];
+            yj = cut.q.y[j];
+            zj = cut.q.z[j];
           }
-          // The row goes back in its new order (its lanes belong to one
-          // wavefront, so their LDS writes come before these reads).
-          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-          if (nout > 0)
-            for (int k = lane; k < m; k += kRowLanes)
-              local[a + k] = static_cast<uint16_t>(row[k < nin ? k : m - 1 - (k - nin)] * 24);
+          in_u[u] = cut_inner(xi, yi, zi, xj, yj, zj, box, cut.cl2);
         }
+#pragma unroll
+        for (int u = 0; u < kRowBatch; u++) {
+          const bool valid = rank[u] >= 0;
+          constexpr uint32_t kSeg = (1u << kRowLanes) - 1;
+          const uint32_t vm = kSeg & static_cast<uint32_t>(__ballot(valid) >> seg);
+          const uint32_t im = kSeg & static_cast<uint32_t>(__ballot(valid && in_u[u]) >> seg);
+          const uint32_t below = (1u << lane) - 1;
+          if (valid)
+            row[in_u[u] ? nin + __popc(im & below) : m - 1 - nout - __popc(vm & ~im & below)] =
+                static_cast<uint16_t>(rank[u]);
+          nin += __popc(im);
+          nout += __popc(vm & ~im);
+        }
+      }
+      if (CUT && m > 0) {
+        if (lane == 0) inner[slot] = nin;
+        // The row goes back in its new order (its lanes belong to one
+        // wavefront, so their LDS writes come before these reads).
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (nout > 0)
+          for (int k = lane; k < m; k += kRowLanes)
+            local[a + k] = static_cast<uint16_t>(row[k < nin ? k : m - 1 - (k - nin)] * 24);
       }
       __syncthreads();
       if (ORDER) {
-        // At least as many threads as the group's rows have lanes.
-        const int r = tid / kRowLanes;
-        const int m = r < nr && len[r] <= kBankRowMax ? len[r] : 0;
-        const int nin = m > 0 ? in_len[r] : 0;
         const int phase = (g0 + r) << lsh;
-        uint16_t* row = in + min(r, grows - 1) * stride;
 #pragma nounroll
         for (int part = 0; part < 2; part++) {
           const int n = part ? m - nin : nin, most = wave_max(n);
