@@ -16,7 +16,8 @@ Prints ONE JSON line on stdout:
                  untimed call of K steps and a short untimed settling period
   mixed          the same for the mixed-precision kernel, with its force error
                  against the FP64 kernel (max and RMS, normwise)
-  roofline       algorithmic bytes per launch / median launch time, vs 8 TB/s
+  roofline       algorithmic bytes per evaluation / median time of one, vs 8 TB/s
+                 ("launch" in its field names: a launch may carry several)
   cpu_baseline   the reference's force_sorted (half list, j scatter) restated
                  in oracle/cpu_baseline.cpp (-O3, AVX2/FMA), on one host core,
                  a bounded sample of the same list; cpu_baselines_other holds
@@ -28,7 +29,7 @@ Usage: python bench.py [--gpus 1] [--steps K] [--warmup W] [--repeats R]
 The other workloads print one JSON line each in the same format: "large" the
 same evaluation on FCC 4*64^3 = 1,048,576 particles with FP64, mixed and
 Kahan-mixed kernels; "replicas" 256 periodic boxes of uneven size in one
-autotuned launch per step; "md" K velocity-Verlet steps of 8,388,608
+autotuned shape; "md" K velocity-Verlet steps of 8,388,608
 particles at density 0.8 with device list rebuilds whenever a particle has
 moved half the skin.
 """
@@ -67,7 +68,7 @@ TRAFFIC_FILE = os.path.join(ROOT, "profiles", "lj_force_f64_N119164_rho1_traffic
 
 
 def measured_traffic(info, tile_order):
-    """HBM bytes per launch of the FP64 force kernel, from the committed
+    """HBM bytes per evaluation of the FP64 force kernel, from the committed
     rocprofv3 FETCH_SIZE/WRITE_SIZE runs (copy-calibrated) when they were
     taken with the kernel configuration in use; None otherwise."""
     try:
@@ -130,7 +131,7 @@ def cpu_baselines(q, box, half, full, dt, budget_s: float) -> list[dict]:
 
 
 def time_leg(ctx, fn, steps: int, warmup: int, repeats: int, settle_ms: float) -> dict:
-    """Time `fn(steps)` (one force call of `steps` launches) the way the
+    """Time `fn(steps)` (one force call of `steps` evaluations) the way the
     reference's measure() times its launch loop (cuda/force_cuda.cu:330-336):
     only the launches, after every one-time cost. `warmup` untimed steps,
     then one untimed call of exactly `steps` steps (so the graphs and buffers
@@ -219,7 +220,7 @@ def bench_large(args, G, np) -> dict:
 
 def bench_replicas(args, G, np) -> dict:
     """256 periodic replica boxes (FCC 4*k^3, k uniform in 6..20, density
-    uniform in [0.5, 1.0]) in one tiled launch per step, configuration from
+    uniform in [0.5, 1.0]) in tiled launches over all of them, configuration from
     the autotuner, 100-step loops replayed as HIP graphs."""
     dt = 0.01
     q, off, boxes = G.replica_workload(256, seed=4)
@@ -247,7 +248,7 @@ def bench_replicas(args, G, np) -> dict:
         "ms_per_step": round(ms, 6), "higher_is_better": True, "scaling": "weak",
         "vs_baseline": None, "dtype": "f64", "data": "synthetic",
         "config": {"workload": f"256 periodic LJ replicas, FCC 4*k^3 with k in 6..20, density in "
-                               f"[0.5, 1], {n} particles in total, one tiled launch per step, "
+                               f"[0.5, 1], {n} particles in total, tiled launches over all of them, "
                                f"dt {dt}, AoS", "particles": n, "replicas": 256,
                    "list_entries": e, "unique_pairs": e // 2, "autotuned": best},
         "roofline": roofline(4 * e + 104 * n, ms / 1e3),

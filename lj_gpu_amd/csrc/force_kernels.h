@@ -619,11 +619,10 @@ __device__ __forceinline__ void tile_body(P pos, M mom, const int32_t* __restric
 }
 
 // Register budget (measured on MI355X): five waves per SIMD, at most 96
-// VGPRs (the default FP64 kernel takes 90, the mixed one 86, neither
-// spills). With the first staging pass peeled off its loop and the batched
-// reciprocal, FP64 no longer fits six waves' 80 VGPRs without spilling; the
-// mixed kernels run 7 % faster at five waves than at six and 5 % faster
-// than at four.
+// VGPRs. The periodic FP64 kernels take 80, so six waves fit (1.8 % faster
+// at 1,048,576 particles than at 90 registers and five); forcing 80 where the
+// compiler needs more spills (+26 %). The mixed ones take 96: they ran 7 %
+// faster at five waves than at six and 5 % faster than at four.
 template <int TPI, int U, int PREC, class P, class M, bool PBC, bool OFFS_LDS, bool SL>
 __global__ void __launch_bounds__(1024)
 __attribute__((amdgpu_waves_per_eu(5)))
