@@ -145,7 +145,7 @@ int ensure_tiles(ljgpu_ctx* ctx, const PosIn* q, double box) {
   // as many as pairs, and the untiled kernel stays.
   if (ctx->eval_half && 2 * ctx->tiles.staged > ctx->eval.e)
     ctx->tiles.tile_particles = ctx->tiles.blocks = 0;
-  // The slot-order copies that calls of kSlotMinSteps or more steps run over
+  // The slot-order copies that calls of many steps (kSlotMinSteps) run over
   // are reserved with the tiles, so a force call never allocates.
   if (ctx->tiles.blocks > 0 && ctx->tiles.order == LJGPU_TILE_ORDER_SPATIAL &&
       ctx->tiles.staged > 0) {
@@ -453,13 +453,18 @@ int launch_one(ljgpu_ctx* ctx, const ListView& lv, const LaunchConfig& lc, const
   return launch_one_on(ctx->stream, lv, lc, fa, mixed, accum);
 }
 
-// Launches that carry `steps` evaluations: about sqrt(steps) of them, up to
-// kMaxLaunchSteps evaluations each, over full-list tiles (a tile updates its
-// own particles only, so its evaluations need no order across tiles), one per
-// evaluation otherwise.
+// How often the tiles fill the GPU twice over.
+double tile_rounds(const ListView& lv, const LaunchConfig& lc) {
+  return lv.tile_blocks / (kTileRound * std::max(1.0, 1.0 * lc.cus));
+}
+
+// Launches that carry `steps` evaluations (see kMaxLaunchSteps) over full-list
+// tiles (a tile updates its own particles only, so its evaluations need no
+// order across tiles), one per evaluation otherwise.
 int32_t launches_of(const ListView& lv, const LaunchConfig& lc, int32_t steps) {
   if (lv.tile_blocks <= 0 || lc.half_atomic || steps <= 1) return steps;
-  const int32_t per = std::clamp(static_cast<int32_t>(std::lround(std::sqrt(steps))), 1,
+  const double weight = std::max(1.0, tile_rounds(lv, lc));
+  const int32_t per = std::clamp(static_cast<int32_t>(std::lround(std::sqrt(steps * weight))), 1,
                                  kMaxLaunchSteps);
   return (steps + per - 1) / per;
 }
@@ -732,7 +737,9 @@ int run_steps(ljgpu_ctx* ctx, const ForceArgs& caller, int32_t steps, bool mixed
   // and the staging's accesses are then contiguous runs. The arithmetic is
   // the same, so the momenta equal those of per-step evaluations bit for bit.
   ForceArgs fa = caller;
-  const bool slots = steps >= kSlotMinSteps && lv.tile_blocks > 0 && lv.tile_stage_slot;
+  const int32_t slot_min =
+      tile_rounds(lv, lc) >= kSlotLargeRounds ? kSlotMinStepsLarge : kSlotMinSteps;
+  const bool slots = steps >= slot_min && lv.tile_blocks > 0 && lv.tile_stage_slot;
   if (slots) {
     TRY(slot_gather(ctx, caller, &fa));
     lv.tile_member = nullptr;

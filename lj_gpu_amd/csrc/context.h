@@ -41,16 +41,27 @@ constexpr int32_t kMinChainTiles = 64;  // fewer tiles: one chain
 // running its tile that many times (it reads everything again each time). A
 // launch costs about 3 to 4.5 us of host time and a ramp and a tail on the
 // device, so one launch per evaluation left small systems waiting for the
-// host; the last launch's tail grows with the evaluations it carries. About
-// sqrt(steps) per launch balances the two. Measured, one per launch / 4 / 10 /
-// 100: 119,164 particles, 100 evaluations 1530 / 1464 / 1437 / 1602 us, 10
-// evaluations 199 / 194 / 209 us; 62,500 particles in an open box, 100
-// evaluations 850 / 589 / 555 / 586 us; 16,384 particles, 10 evaluations 136 /
-// 104 / 104 us.
+// host, and its evaluations after the first find the tile in L2; the last
+// launch's tail grows with the evaluations it carries. About sqrt(steps) per launch
+// balances these. Measured, one per launch / 4 / 10 / 100: 119,164 particles,
+// 100 evaluations 1530 / 1464 / 1437 / 1602 us, 10 evaluations 199 / 194 / 209
+// us; 62,500 particles in an open box, 100 evaluations 850 / 589 / 555 / 586
+// us; 16,384 particles, 10 evaluations 136 / 104 / 104 us. Where tiles come in many
+// rounds of kTileRound per compute unit (twice the resident ones) the tail weighs
+// less, and a launch carries sqrt(rounds) times as many: 1,048,576 particles,
+// 10 evaluations 1483 / 1399 / 1350, 256 replicas of 3 million together 3732 / 3382 /
+// 3367; at 256,000 (1.3 rounds) 346 / 348 / 361.
 constexpr int32_t kMaxLaunchSteps = 16;
+constexpr double kTileRound = 12.0;
 // Calls with at least kSlotMinSteps steps over spatially ordered tiles run
 // over copies of q and p in slot order (two gathers and a scatter per call).
+// Systems of more than kSlotLargeRounds rounds of tiles, whose rows do not stay
+// in the L2s, do so from kSlotMinStepsLarge steps on: 10 evaluations of 1,048,576
+// particles take 1446 us with copies and 1473 without (AoS), 1500 and 1578
+// (SoA); of 119,164 206 and 202 (AoS), 238 and 240 (SoA).
 constexpr int32_t kSlotMinSteps = 16;
+constexpr int32_t kSlotMinStepsLarge = 10;
+constexpr double kSlotLargeRounds = 4.0;
 // Energy sums: a fixed grid of kEnergyBlocks workgroups (each striding over
 // the rows) writes one partial per workgroup and quantity (potential,
 // kinetic, pairs inside the cutoff), added afterwards in block order, so the

@@ -144,3 +144,34 @@ def test_launches_of_several_evaluations(ctx, tile, resident, graphs):
         np.testing.assert_array_equal(da.download(), db.download())
     ctx.set_graphs(True)
     ctx.set_tiling(64)
+
+
+@pytest.mark.parametrize("cells", [22, 24])
+@pytest.mark.parametrize("soa", [False, True])
+def test_many_rounds_of_tiles(ctx, cells, soa):
+    """Systems of more than four rounds of tiles (55,296 particles in tiles of
+    4: 13,824 tiles) take slot-order copies from ten evaluations on and more
+    of them per launch than smaller ones (42,592): bit for bit what as many
+    calls of one give."""
+    q, box = G.lattice_periodic(cells, 0.5, 3)
+    n = q.shape[0]
+    print(f"cells={cells} soa={soa}", flush=True)
+    ctx.set_kernel_config(4, 256, 4)
+    ctx.set_tiling(4)
+    ctx.set_half_mode(G.HALF_AUTO)
+    if soa:
+        dq = [ctx.array(np.ascontiguousarray(q[:, c])) for c in range(3)]
+        da, db = ([ctx.zeros(n) for _ in range(3)] for _ in range(2))
+        build, force = ctx.build_list_soa, ctx.force_soa_f64
+    else:
+        dq, da, db = ctx.array(q), ctx.zeros(q.shape), ctx.zeros(q.shape)
+        build, force = ctx.build_list, ctx.force_aos_f64
+    build(dq, n, box, G.LIST_FULL)
+    for steps in (9, 10, 11):
+        force(dq, da, 1e-3, G.CL2, box, steps)
+        for _ in range(steps):
+            force(dq, db, 1e-3, G.CL2, box, 1)
+    ctx.sync()
+    for a, b in zip(da if soa else [da], db if soa else [db]):
+        np.testing.assert_array_equal(a.download(), b.download())
+    ctx.set_tiling(64)
