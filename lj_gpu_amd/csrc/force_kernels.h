@@ -298,6 +298,17 @@ __device__ __forceinline__ void tile_row(const M& mom, const uint16_t* lrow, int
   }
 }
 
+// An entry offset. A launch of one evaluation (the MD loop's, MomDrift) reads
+// each once: past the L2, which its positions then keep (40 MD steps of
+// 1,048,576 particles 11.52 -> 11.37 ms). Launches of several evaluations read
+// them again from there (119,164 particles, 100 evaluations: 1464 us, past the
+// L2 1632).
+template <class M>
+__device__ __forceinline__ uint32_t offset_at(const uint16_t* __restrict__ p) {
+  if constexpr (std::is_same<M, MomDrift>::value) return __builtin_nontemporal_load(p);
+  else return *p;
+}
+
 // One batch of a tile row: all U partner positions are read from LDS before
 // any is used, then the U entries are computed; the offsets buffer `o` is
 // refilled in between with the batch two ahead (loads from global memory
@@ -334,7 +345,7 @@ __device__ __forceinline__ void tile_batch(const M& mom, const uint16_t* __restr
   }
   if constexpr (REFILL) {
 #pragma unroll
-    for (int u = 0; u < U; u++) o[u] = lrow[refill + u * US + ls];
+    for (int u = 0; u < U; u++) o[u] = offset_at<M>(lrow + refill + u * US + ls);
   }
   bool in[U];
   bool inside = false;
@@ -378,13 +389,13 @@ __device__ __forceinline__ void tile_batch(const M& mom, const uint16_t* __restr
 
 // The first batch's offsets of a row in either layout of tile_row_stream,
 // loaded before the tile's staging so that their latency hides behind it.
-template <int TPI, int U, bool SL>
+template <int TPI, int U, bool SL, class M>
 __device__ __forceinline__ void row_prefetch(const uint16_t* __restrict__ lrow, int sub,
                                              uint32_t (&oa)[U]) {
   constexpr int US = SL ? 64 : TPI;
   const int ls = SL ? 0 : sub;
 #pragma unroll
-  for (int u = 0; u < U; u++) oa[u] = lrow[u * US + ls];
+  for (int u = 0; u < U; u++) oa[u] = offset_at<M>(lrow + u * US + ls);
 }
 
 // As tile_row, with the row's entry offsets read from global memory through
@@ -407,7 +418,7 @@ __device__ __forceinline__ void tile_row_stream(const M& mom, const uint16_t* __
   const int nfull = np / kB;
   uint32_t ob[U];
 #pragma unroll
-  for (int u = 0; u < U; u++) ob[u] = lrow[JS + u * US + ls];
+  for (int u = 0; u < U; u++) ob[u] = offset_at<M>(lrow + JS + u * US + ls);
   int b = 0;
   for (; b + 2 <= nfull; b += 2) {
     tile_batch<TPI, U, PREC, PBC, MI, false, true, US>(mom, lrow, oa, b * kB, (b + 2) * JS, ls,
@@ -518,7 +529,7 @@ __device__ __forceinline__ void tile_body(P pos, M mom, const int32_t* __restric
     // the U * TPI entries from the block's first, lie inside the padded
     // offset arrays.
     grow = SL ? sliced + wo + (threadIdx.x & 63) : local + eoff + rs;
-    row_prefetch<TPI, U, SL>(grow, sub, oa);
+    row_prefetch<TPI, U, SL, M>(grow, sub, oa);
   }
   // Staging issues all of a thread's loads of a pass before its LDS writes,
   // so each thread has kStageR independent gathers in flight. The first
