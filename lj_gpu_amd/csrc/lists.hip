@@ -954,17 +954,25 @@ __device__ __forceinline__ double readlane_d(double v, int lane) {
 // place in cpos of candidate f < total.
 constexpr int kPairGroup = 5;     // particles of a cell tested together
 constexpr int kPairCand = 1024;   // candidates whose places are kept in LDS
+// Up to this many cells, four or two wavefronts share a cell's particles: so few
+// wavefronts leave the SIMDs idle, and the search takes as long as one cell's
+// rounds. List refresh with one force evaluation, one / two / four: 2,048 particles
+// (343 cells) 157 / 149 / 147 us, 4,000 (1,000) 175 / 167 / 163, 6,912 (1,728) 179 /
+// 174 / 174, 16,384 (4,096) 210 / 206 / 211, 32,000 (8,000) 247 / 246 / 255.
+constexpr int64_t kPairCellsFour = 1024;
+constexpr int64_t kPairCellsTwo = 4096;
 
 template <int MODE, bool HALF, bool IMAGE, class At>
-__device__ __forceinline__ void pairs_cell(int32_t p0, int32_t p1, int32_t total, At&& at,
+__device__ __forceinline__ void pairs_cell(int32_t p0, int32_t p1, int32_t per, int32_t step,
+                                           int32_t total, At&& at,
                                            const double4* __restrict__ cpos, const GridArgs& g,
                                            double half_box, double sl2, int32_t cap,
                                            int32_t* __restrict__ nop,
                                            const int32_t* __restrict__ ptr,
                                            int32_t* __restrict__ out) {
   const int lane = threadIdx.x & 63;
-  for (int32_t g0 = p0; g0 < p1; g0 += kPairGroup) {
-    const int32_t mg = min(kPairGroup, p1 - g0);
+  for (int32_t g0 = p0; g0 < p1; g0 += step) {
+    const int32_t mg = min(per, p1 - g0);
     double4 pi = make_double4(0.0, 0.0, 0.0, 0.0);
     if (lane < mg) pi = cpos[g0 + lane];
     const int32_t iv = static_cast<int32_t>(pi.w);
@@ -1015,7 +1023,7 @@ __device__ __forceinline__ void pairs_cell(int32_t p0, int32_t p1, int32_t total
   }
 }
 
-// One wavefront per cell, for cell grids with a stencil (R >= 1). The
+// One wavefront per cell (2^split of them in small systems), for cell grids with a stencil (R >= 1). The
 // candidates of the (2R+1)^3 cells around it are walked as one flattened
 // sequence, 64 per round, and tested against kPairGroup of the cell's
 // particles at a time (about four to five of a fine cell's, so mostly one
@@ -1042,7 +1050,8 @@ __global__ __launch_bounds__(kBlock) void k_pairs_wave(int32_t ncell,
                                                        int32_t* __restrict__ nop,
                                                        const int32_t* __restrict__ ptr,
                                                        int32_t* __restrict__ out,
-                                                       const int32_t* __restrict__ outside) {
+                                                       const int32_t* __restrict__ outside,
+                                                       int32_t split) {
   __shared__ int32_t cand_lds[kBlock / 64][kPairCand];
   int32_t* cand = cand_lds[threadIdx.x >> 6];
   constexpr int kSpan = 2 * R + 1;
@@ -1056,10 +1065,13 @@ __global__ __launch_bounds__(kBlock) void k_pairs_wave(int32_t ncell,
   // The wavefront's cell and all that follows from it are scalars.
   const int64_t first = blockIdx.x * static_cast<int64_t>(kBlock / 64) +
                         __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / 64);
-  for (int64_t c64 = first; c64 < ncell; c64 += waves) {
-    const int32_t c = static_cast<int32_t>(c64);
-    const int32_t p0 = cell_start[c], p1 = cell_start[c + 1];
-    if (p0 == p1) continue;  // the whole wavefront
+  for (int64_t w64 = first; w64 < int64_t{ncell} << split; w64 += waves) {
+    const int32_t c = static_cast<int32_t>(w64 >> split);
+    const int32_t cell0 = cell_start[c], p1 = cell_start[c + 1];
+    // This wavefront's groups: `per` particles each, from p0 on.
+    const int32_t per = min(kPairGroup, (p1 - cell0 + (1 << split) - 1) >> split);
+    const int32_t p0 = cell0 + per * static_cast<int32_t>(w64 & ((1 << split) - 1));
+    if (p0 >= p1) continue;  // the whole wavefront
     const int cx = c % g.nc0, cy = (c / g.nc0) % g.nc1, cz = c / (g.nc0 * g.nc1);
     // Lane r < kRuns: run r of the stencil as [rs, rs + rl) in cpos. An x-row's
     // two runs are its parts before and behind the box's face where it
@@ -1105,10 +1117,11 @@ __global__ __launch_bounds__(kBlock) void k_pairs_wave(int32_t ncell,
                                     cy + R >= g.nc1 || cz < R || cz + R >= g.nc2);
     auto walk = [&](auto&& at) {
       if (wraps)
-        pairs_cell<MODE, HALF, true>(p0, p1, total, at, cpos, g, half_box, sl2, cap, nop, ptr, out);
+        pairs_cell<MODE, HALF, true>(p0, p1, per, per << split, total, at, cpos, g, half_box, sl2,
+                                     cap, nop, ptr, out);
       else
-        pairs_cell<MODE, HALF, false>(p0, p1, total, at, cpos, g, half_box, sl2, cap, nop, ptr,
-                                      out);
+        pairs_cell<MODE, HALF, false>(p0, p1, per, per << split, total, at, cpos, g, half_box, sl2,
+                                      cap, nop, ptr, out);
     };
     if (total <= kPairCand) {
       for (int32_t k = 0; k < rl; k++) cand[excl + k] = rs + k;
@@ -2452,7 +2465,10 @@ int dev_makepair(hipStream_t s, const PosIn& q, int32_t n, double box, double se
   }
   LTRY(hipGetLastError(), "cell scatter kernels");
   const int grid = grid_for(n, kBlock, INT32_MAX);
-  const int wave_grid = grid_for(ncell * 64, kBlock);  // one wavefront per cell, grid-stride
+  // One wavefront per cell, grid-stride; in small systems several, which share
+  // its particles.
+  const int split = ncell <= kPairCellsFour ? 2 : ncell <= kPairCellsTwo ? 1 : 0;
+  const int wave_grid = grid_for((ncell << split) * 64, kBlock);
   auto pairs = [&](auto mode_tag, int32_t cap, int32_t* nop, const int32_t* ptr, int32_t* outl) {
     constexpr int M = decltype(mode_tag)::value;
     const double4* cp = w.cpos.as<double4>();
@@ -2463,7 +2479,7 @@ int dev_makepair(hipStream_t s, const PosIn& q, int32_t n, double box, double se
   k_pairs<M, H, 0><<<grid, kBlock, 0, s>>>(n, cp, cs, cstart, g, sl2, cap, nop, ptr, outl)
 #define LJ_PAIRS_WAVE(H, RR)                                                                     \
   k_pairs_wave<M, H, RR><<<wave_grid, kBlock, 0, s>>>(static_cast<int32_t>(ncell), cp, cstart, g, \
-                                                      sl2, cap, nop, ptr, outl, outside)
+                                                      sl2, cap, nop, ptr, outl, outside, split)
     if (half) {
       if (R == 0) LJ_PAIRS(true);
       else if (R == 1) LJ_PAIRS_WAVE(true, 1);
