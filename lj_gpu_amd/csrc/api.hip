@@ -319,13 +319,16 @@ int build_list(ljgpu_ctx* ctx, const PosIn& q, int32_t n, double box, double sea
   // decided by the pair search's synchronisation.
   struct OrderBegun {
     ljgpu_ctx* c;
-    ~OrderBegun() { c->order_begun = false; }
+    ~OrderBegun() {
+      c->order_begun = false;
+      c->work.order_job.clear();
+    }
   } order_begun_guard{ctx};
   const int32_t tile = effective_tile(ctx);
   if (tile > 0 && n > 0 && ctx->tile_order == LJGPU_TILE_ORDER_SPATIAL &&
       (expand || ctx->rep_off.empty()))
     TRY(dev_tile_order_begin(ctx->stream, q, n, box, ctx->rep_off, ctx->rep_boxes, tile, ctx->work,
-                             &ctx->order_begun));
+                             &ctx->order_begun, ctx->rep_off.empty()));
   // A full list is the symmetric closure of the half list (the pair
   // predicate is exactly symmetric), so an expanded half list is built
   // directly as the full list.

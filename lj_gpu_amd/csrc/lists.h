@@ -120,6 +120,7 @@ struct ListWork {
   ListResults* results = nullptr;    // pinned
   std::vector<int32_t> geo_host;     // blocks of a replicas' tiling, as uploaded
   std::vector<char> order_host;      // bins and offsets of a replicas' tile order, as uploaded
+  std::vector<char> order_job;       // a tile order left for dev_makepair (else empty)
 };
 void dev_release(ListWork& w);
 
@@ -250,10 +251,12 @@ int dev_tile_order(hipStream_t s, const PosIn& q, int32_t n, double box,
                    int32_t tile_particles, ListWork& w, bool* ok);
 // The same in two steps, so that a caller's next synchronisation serves it
 // too: begin enqueues it (*begun = false: no order for this box), end tells
-// after that synchronisation whether the order holds.
+// after that synchronisation whether the order holds. With `defer` a few
+// particles' order is left in w.order_job for the dev_makepair that follows,
+// which runs it beside its own binning.
 int dev_tile_order_begin(hipStream_t s, const PosIn& q, int32_t n, double box,
                          const std::vector<int32_t>& replicas, const std::vector<double>& boxes,
-                         int32_t tile_particles, ListWork& w, bool* begun);
+                         int32_t tile_particles, ListWork& w, bool* begun, bool defer = false);
 bool dev_tile_order_end(const ListWork& w);
 
 // Batched replicas: lists of every replica (particles [off[r], off[r+1]),

@@ -736,6 +736,29 @@ struct OrderPut {
   }
 };
 
+// Spatial tile order: bins of one system (dev_tile_order).
+struct OrderGrid {
+  double w[3];     // bin widths: x bins, y and z columns
+  double box;      // period
+  int32_t nc[3];   // x bins, y columns, z columns
+  int32_t key0;    // first key of the system
+};
+
+struct OrderKey {
+  PosIn q;
+  OrderGrid one;
+  const OrderGrid* grids;
+  const int32_t* rep_of;
+  __device__ __forceinline__ int32_t operator()(int64_t t, int32_t*) const {
+    const OrderGrid g = rep_of ? grids[rep_of[t]] : one;
+    const int64_t o = t * q.stride;
+    const int cx = cell_coord(q.x[o], 0.0, g.w[0], g.nc[0], g.box);
+    const int cy = cell_coord(q.y[o], 0.0, g.w[1], g.nc[1], g.box);
+    const int cz = cell_coord(q.z[o], 0.0, g.w[2], g.nc[2], g.box);
+    return g.key0 + (cz * g.nc[1] + cy) * g.nc[0] + cx;
+  }
+};
+
 // Few particles binned by one workgroup, counts and arrival order in LDS: what
 // k_cell_assign or k_order_key, a scan, k_bin_index and a placing kernel do for
 // more, whose five launches took 16 us and the gaps between them at 2,048
@@ -748,12 +771,27 @@ constexpr int32_t kBinsSmall = 8192;  // bins
 constexpr int kBinThreads = 1024;
 
 template <class Key, class Put>
-__global__ __launch_bounds__(kBinThreads) void k_bin_small(int32_t n, int32_t nbins, Key key,
-                                                           Put put, int32_t* __restrict__ start,
-                                                           int32_t* __restrict__ flag,
-                                                           ScanStats* __restrict__ res) {
-  __shared__ int32_t bin[kBinsSmall + 1];
-  __shared__ uint16_t arrival[kBinSmall];
+struct BinJob {
+  int32_t n, nbins;
+  Key key;
+  Put put;
+  int32_t* start;
+  int32_t* flag;
+  ScanStats* res;
+};
+struct NoBinJob {};
+using CellJob = BinJob<CellKey, CellPut>;
+using OrderJob = BinJob<OrderKey, OrderPut>;
+
+template <class Key, class Put>
+__device__ __forceinline__ void bin_small(const BinJob<Key, Put>& job, int32_t* bin,
+                                          uint16_t* arrival) {
+  const int32_t n = job.n, nbins = job.nbins;
+  const Key& key = job.key;
+  const Put& put = job.put;
+  int32_t* const start = job.start;
+  int32_t* const flag = job.flag;
+  ScanStats* const res = job.res;
   __shared__ int32_t sh[kBinThreads / 64], slo[kBinThreads / 64], shi[kBinThreads / 64];
   __shared__ int32_t gathered;
   constexpr int kPer = kBinSmall / kBinThreads;
@@ -809,6 +847,18 @@ __global__ __launch_bounds__(kBinThreads) void k_bin_small(int32_t n, int32_t nb
     else
       for (int32_t k = a; k < b; k++) place += arrival[k] < t ? 1 : 0;
     put(place, t, mine[u]);
+  }
+}
+
+// A second job runs beside the first, on a workgroup of its own.
+template <class A, class B>
+__global__ __launch_bounds__(kBinThreads) void k_bin_small(A a, B b) {
+  __shared__ int32_t bin[kBinsSmall + 1];
+  __shared__ uint16_t arrival[kBinSmall];
+  if (std::is_same<B, NoBinJob>::value || blockIdx.x == 0) {
+    bin_small(a, bin, arrival);
+  } else if constexpr (!std::is_same<B, NoBinJob>::value) {
+    bin_small(b, bin, arrival);
   }
 }
 
@@ -2125,29 +2175,6 @@ __global__ void k_half_sort(int32_t n, const int32_t* __restrict__ first,
   }
 }
 
-// Spatial tile order: bins of one system (dev_tile_order).
-struct OrderGrid {
-  double w[3];     // bin widths: x bins, y and z columns
-  double box;      // period
-  int32_t nc[3];   // x bins, y columns, z columns
-  int32_t key0;    // first key of the system
-};
-
-struct OrderKey {
-  PosIn q;
-  OrderGrid one;
-  const OrderGrid* grids;
-  const int32_t* rep_of;
-  __device__ __forceinline__ int32_t operator()(int64_t t, int32_t*) const {
-    const OrderGrid g = rep_of ? grids[rep_of[t]] : one;
-    const int64_t o = t * q.stride;
-    const int cx = cell_coord(q.x[o], 0.0, g.w[0], g.nc[0], g.box);
-    const int cy = cell_coord(q.y[o], 0.0, g.w[1], g.nc[1], g.box);
-    const int cz = cell_coord(q.z[o], 0.0, g.w[2], g.nc[2], g.box);
-    return g.key0 + (cz * g.nc[1] + cy) * g.nc[0] + cx;
-  }
-};
-
 __global__ void k_order_key(int32_t n, OrderKey key, int32_t* __restrict__ count,
                             int32_t* __restrict__ slot, int32_t* __restrict__ key_of) {
   for (int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; t < n;
@@ -2373,6 +2400,15 @@ int dev_expand_half(hipStream_t s, int32_t n, const int32_t* hnop, const int32_t
   return LJGPU_OK;
 }
 
+// The tile order's job that dev_tile_order_begin left for this list build.
+bool take_order_job(ListWork& w, OrderJob* job) {
+  static_assert(std::is_trivially_copyable<OrderJob>::value, "kept as bytes");
+  if (w.order_job.size() != sizeof(*job)) return false;
+  std::memcpy(static_cast<void*>(job), w.order_job.data(), sizeof(*job));
+  w.order_job.clear();
+  return true;
+}
+
 int dev_makepair(hipStream_t s, const PosIn& q, int32_t n, double box, double search_length,
                  int kind, ListWork& w, DevCSR& out, bool sort_rows) {
   const double sl2 = search_length * search_length;
@@ -2432,12 +2468,17 @@ int dev_makepair(hipStream_t s, const PosIn& q, int32_t n, double box, double se
   const CellKey key{q, g};
   const bool few = n <= kBinSmall && ncell <= kBinsSmall;
   if (few) {
-    k_bin_small<<<1, kBinThreads, 0, s>>>(
-        n, static_cast<int32_t>(ncell), key,
-        CellPut{q, w.cpos.as<double4>(), w.cell_sorted.as<int32_t>()}, cstart, outside,
-        &w.results->cells);
+    const CellJob job{n, static_cast<int32_t>(ncell), key,
+                      CellPut{q, w.cpos.as<double4>(), w.cell_sorted.as<int32_t>()}, cstart, outside,
+                      &w.results->cells};
+    OrderJob order;
+    if (take_order_job(w, &order)) k_bin_small<<<2, kBinThreads, 0, s>>>(job, order);
+    else k_bin_small<<<1, kBinThreads, 0, s>>>(job, NoBinJob{});
     LTRY(hipGetLastError(), "cell kernel");
   } else {
+    OrderJob order;
+    if (take_order_job(w, &order)) k_bin_small<<<1, kBinThreads, 0, s>>>(order, NoBinJob{});
+    LTRY(hipGetLastError(), "tile order kernel");
     LCHECK(fill<int32_t>(s, count, ncell + 1, 0));
     k_cell_assign<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, key, count, w.cell_slot.as<int32_t>(),
                                                          w.cell_of.as<int32_t>(), outside);
@@ -2607,8 +2648,9 @@ int dev_make_ell(hipStream_t s, const DevCSR& c, int32_t width, DevMem& ell) {
 
 int dev_tile_order_begin(hipStream_t s, const PosIn& q, int32_t n, double box,
                          const std::vector<int32_t>& replicas, const std::vector<double>& boxes,
-                         int32_t T, ListWork& w, bool* begun) {
+                         int32_t T, ListWork& w, bool* begun, bool defer) {
   *begun = false;
+  w.order_job.clear();
   if (n <= 0 || T <= 0) return LJGPU_OK;
   const std::vector<int32_t> single = {0, n};
   const std::vector<int32_t>& off = replicas.empty() ? single : replicas;
@@ -2674,9 +2716,14 @@ int dev_tile_order_begin(hipStream_t s, const PosIn& q, int32_t n, double box,
   const int32_t* key_of = w.cell_of.as<int32_t>();
   const OrderKey key{q, grids[0], dgrids, rep_of};
   if (n <= kBinSmall && keys <= kBinsSmall) {
-    k_bin_small<<<1, kBinThreads, 0, s>>>(n, static_cast<int32_t>(keys), key,
-                                          OrderPut{w.order.as<int32_t>()}, nullptr, nullptr,
-                                          &w.results->order);
+    const OrderJob job{n, static_cast<int32_t>(keys), key, OrderPut{w.order.as<int32_t>()}, nullptr,
+                       nullptr, &w.results->order};
+    if (defer) {
+      w.order_job.resize(sizeof(job));
+      std::memcpy(w.order_job.data(), &job, sizeof(job));
+    } else {
+      k_bin_small<<<1, kBinThreads, 0, s>>>(job, NoBinJob{});
+    }
   } else {
     LCHECK(fill<int32_t>(s, count, keys, 0));
     k_order_key<<<grid_for(n, kBlock), kBlock, 0, s>>>(n, key, count, w.cell_slot.as<int32_t>(),
