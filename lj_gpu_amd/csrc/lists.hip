@@ -1783,7 +1783,8 @@ struct OrderLds {
   uint32_t cnt[kBankClasses / 4][64];
   uint8_t hole[64 / kRowLanes][kBankRowMax];
 };
-static_assert(kTileMaxStage <= 255 * kBankClasses, "a class of a row fits a byte");
+static_assert(kBankRowMax / kRowLanes * (kRowLanes - 1) <= 255 && kBankRowMax / kRowLanes <= 128,
+              "numbers within a class fit a byte");
 static_assert(kBankClasses == 4 * kRowLanes, "one lane per word of counts, four steps a level");
 
 // The places of one part of each row (its inner entries, or the others),
@@ -1831,7 +1832,10 @@ __device__ __forceinline__ void order_part(const uint16_t* from, int step, uint1
     }
   }
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the wavefront's own, in order
-  // Lane w sums word w of the row's counts: each lane's first number.
+  // Lane w sums word w of the row's counts: each lane's first number. A list
+  // may repeat a partner, so a class can hold all of a row's 256 entries, one
+  // more than a byte: counts of the first seven lanes stop at 127 in the total,
+  // of which only whether it exceeds a level (at most 7) matters.
   uint32_t total = 0;
   {
     uint32_t* word = &lds.cnt[lane][seg];
@@ -1841,6 +1845,8 @@ __device__ __forceinline__ void order_part(const uint16_t* from, int step, uint1
 #pragma unroll
     for (int j = 0; j < kRowLanes; j++) {
       word[j] = total;
+      if (j == kRowLanes - 1)
+        total = (total | (total >> 7 & 0x01010101u) * 0x7fu) & 0x7f7f7f7fu;
       total += v[j];
     }
   }

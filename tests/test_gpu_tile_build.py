@@ -175,3 +175,36 @@ def test_many_rounds_of_tiles(ctx, cells, soa):
     for a, b in zip(da if soa else [da], db if soa else [db]):
         np.testing.assert_array_equal(a.download(), b.download())
     ctx.set_tiling(64)
+
+
+@pytest.mark.parametrize("copies", [1, 7, 255, 256])
+@pytest.mark.parametrize("others", [0, 1, 40])
+def test_rows_that_repeat_a_partner(ctx, copies, others):
+    """A caller's list may name a partner many times: up to all 256 entries of
+    a row that is put in order are then in one class. The untiled kernel's
+    momenta."""
+    n = 400
+    q, box = G.lattice_periodic(5, 0.8, 3)
+    q = np.ascontiguousarray(q[:n])
+    rows = [np.zeros(0, np.int32) for _ in range(n)]
+    others = min(others, 256 - copies)
+    for i in range(0, n, 3):
+        rows[i] = np.concatenate([np.full(copies, (i + 1) % n, np.int32),
+                                  np.array([(i + 2 + k) % n for k in range(others)], np.int32)])
+    nop = np.array([len(r) for r in rows], np.int32)
+    ptr = np.concatenate([[0], np.cumsum(nop)[:-1]]).astype(np.int32)
+    csr = G.CSR(nop, ptr, np.concatenate(rows).astype(np.int32), G.LIST_FULL)
+    print(f"copies={copies} others={others}", flush=True)
+    ctx.set_kernel_config(4, 256, 4)
+    ctx.set_half_mode(G.HALF_AUTO)
+    out = []
+    for tile in (64, 0):
+        ctx.set_tiling(tile)
+        ctx.set_list(csr)
+        dq, dp = ctx.array(q), ctx.zeros(q.shape)
+        ctx.force_aos_f64(dq, dp, 1e-3, G.CL2, box, 1)
+        ctx.sync()
+        out.append(dp.download())
+    ctx.set_tiling(64)
+    assert np.abs(out[1]).max() > 0
+    assert normwise(out[0], out[1]) < FP64_TOL
