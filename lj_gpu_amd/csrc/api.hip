@@ -70,6 +70,7 @@ void reset_list(ljgpu_ctx* ctx) {
   ctx->tiles.tile_particles = 0;
   ctx->tiles.blocks = 0;
   ctx->tiles.sliced_lanes = ctx->tiles.sliced_unroll = 0;
+  ctx->tiles.bank_lanes = ctx->tiles.bank_unroll = 0;
 }
 
 void release_all(ljgpu_ctx* ctx) {
@@ -120,6 +121,7 @@ int ensure_tiles(ljgpu_ctx* ctx, const PosIn* q, double box) {
   ctx->tiles.tile_particles = 0;
   ctx->tiles.blocks = 0;
   ctx->tiles.sliced_lanes = ctx->tiles.sliced_unroll = 0;
+  ctx->tiles.bank_lanes = ctx->tiles.bank_unroll = 0;
   bool ordered = false;
   if (ctx->order_begun)
     ordered = dev_tile_order_end(ctx->work);  // the list build has synchronised since
@@ -194,6 +196,28 @@ int ensure_bank_order(ljgpu_ctx* ctx) {
   if (t.blocks <= 0 || t.bank_done || !ctx->bank_order) return LJGPU_OK;
   TRY(dev_bank_order(ctx->stream, tile_row_starts(ctx), t, t.local.as<uint16_t>()));
   t.bank_done = true;
+  return LJGPU_OK;
+}
+
+// Slices of the rows in the bank-class order (once per tiling and
+// configuration), for the FP32 Kahan sums: their last bits follow the order of
+// the entries (2e-7 of the momenta between orders), and this is the order that
+// the host model of the tiles defines.
+int ensure_bank_slices(ljgpu_ctx* ctx) {
+  DevTiles& t = ctx->tiles;
+  const int32_t lanes = t.sliced_lanes, unroll = t.sliced_unroll;
+  if (t.blocks <= 0 || lanes == 0 || !ctx->bank_order ||
+      (t.bank_lanes == lanes && t.bank_unroll == unroll))
+    return LJGPU_OK;
+  TRY(ensure_bank_order(ctx));
+  t.bank_lanes = t.bank_unroll = 0;
+  std::swap(t.sliced, t.sliced_bank);
+  const int rc = dev_slice_tiles(ctx->stream, tile_row_starts(ctx), lanes, unroll, 24, false,
+                                 ctx->eval.n, nullptr, ctx->work, t);
+  std::swap(t.sliced, t.sliced_bank);
+  if (rc) return rc;
+  t.bank_lanes = t.sliced_lanes;
+  t.bank_unroll = t.sliced_unroll;
   return LJGPU_OK;
 }
 
@@ -380,7 +404,7 @@ int check_force_args(ljgpu_ctx* ctx, double dt, double cl2, int32_t steps, doubl
 }
 
 // Kernel arguments of one force evaluation over the installed list.
-int force_view(ljgpu_ctx* ctx, const ForceArgs& fa, ListView* lv, LaunchConfig* lc) {
+int force_view(ljgpu_ctx* ctx, const ForceArgs& fa, bool kahan, ListView* lv, LaunchConfig* lc) {
   const PosIn in = positions_of(fa);
   TRY(prepare_layouts(ctx, &in, fa.box, fa.cl2));
   *lv = ListView();
@@ -403,7 +427,13 @@ int force_view(ljgpu_ctx* ctx, const ForceArgs& fa, ListView* lv, LaunchConfig* 
     lv->ell_width = ctx->ell_width;
   } else {
     lv->list = ctx->eval.list.as<int32_t>();
-    if (ctx->tiles.blocks > 0) tile_fields(ctx, lv);
+    // Kahan sums of half lists keep the untiled kernel's order of entries.
+    if (ctx->tiles.blocks > 0 && !(kahan && ctx->eval_half)) {
+      if (kahan) TRY(ensure_bank_slices(ctx));
+      tile_fields(ctx, lv);
+      if (kahan && lv->tile_sliced && ctx->tiles.bank_lanes > 0)
+        lv->tile_sliced = ctx->tiles.sliced_bank.as<uint16_t>();
+    }
   }
   return LJGPU_OK;
 }
@@ -492,7 +522,7 @@ int enqueue_force(ljgpu_ctx* ctx, const ForceArgs& fa, bool mixed, int accum) {
   if (ctx->n == 0) return LJGPU_OK;
   ListView lv;
   LaunchConfig lc;
-  TRY(force_view(ctx, fa, &lv, &lc));
+  TRY(force_view(ctx, fa, mixed && accum == LJGPU_ACCUM_KAHAN_F32, &lv, &lc));
   return launch_one(ctx, lv, lc, fa, mixed, accum);
 }
 
@@ -734,7 +764,7 @@ int run_steps(ljgpu_ctx* ctx, const ForceArgs& caller, int32_t steps, bool mixed
   if (ctx->n == 0 || steps == 0) return LJGPU_OK;
   ListView lv;
   LaunchConfig lc;
-  TRY(force_view(ctx, caller, &lv, &lc));
+  TRY(force_view(ctx, caller, mixed && accum == LJGPU_ACCUM_KAHAN_F32, &lv, &lc));
   // With spatially ordered tiles, a call of many steps runs over copies of
   // q and p in slot order (q does not change between its steps): the rows'
   // and the staging's accesses are then contiguous runs. The arithmetic is

@@ -66,6 +66,10 @@ struct DevTiles {
   // sliced_lanes lanes per particle and sliced_unroll entries per lane per
   // batch (see dev_slice_tiles); sliced_lanes = 0: not built.
   DevMem sliced;      // uint16
+  // The slices of rows in the bank-class order (made on first use, for sums
+  // that depend on the order), for bank_lanes and bank_unroll; 0: none.
+  DevMem sliced_bank;
+  int32_t bank_lanes = 0, bank_unroll = 0;
   DevMem wave_off;    // int32 per (block, wavefront slot): start of its slice
   int32_t sliced_lanes = 0, sliced_unroll = 0, waves_per_block = 0;
 

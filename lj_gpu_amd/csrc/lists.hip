@@ -2263,6 +2263,8 @@ void dev_release(DevTiles& t) {
   dev_release(t.stage);
   dev_release(t.local);
   dev_release(t.sliced);
+  dev_release(t.sliced_bank);
+  t.bank_lanes = t.bank_unroll = 0;
   dev_release(t.wave_off);
   t.sliced_lanes = t.sliced_unroll = t.waves_per_block = 0;
   dev_release(t.member);

@@ -36,7 +36,8 @@ constexpr int kBlock = 256;
 // and sixteen lanes: the larger tiles are too few to fill the chip, and a kick
 // takes as long as one tile's chain of loads and batches, which this shortens
 // (7.0 -> 4.9 us at 4,000 particles, 6.4 -> 5.8 at 6,912; even at 8,788, slower
-// beyond).
+// beyond). Kahan sums keep the default shape, on whose lanes their last bits
+// depend.
 constexpr int kFewParticles = 24;
 
 __device__ __forceinline__ double image(double d, double box, double inv_box) {
@@ -395,7 +396,8 @@ int ljgpu_md_run(ljgpu_ctx* ctx, double* q, double* p, int32_t n, double box,
   ctx->tile_order = LJGPU_TILE_ORDER_INDEX;
   ctx->bank_order = false;
   if (box > 0.0 && n > 0 && n <= kFewParticles * ctx->cus && ctx->lanes == 4 && ctx->unroll == 4 &&
-      ctx->tile_particles == 64 && !ctx->tile_offsets_lds) {
+      ctx->tile_particles == 64 && !ctx->tile_offsets_lds &&
+      !(cfg->precision == LJGPU_PREC_MIXED && cfg->accum == LJGPU_ACCUM_KAHAN_F32)) {
     ctx->lanes = 16;
     ctx->tile_particles = 16;
   }
@@ -634,7 +636,7 @@ int ljgpu_md_run(ljgpu_ctx* ctx, double* q, double* p, int32_t n, double box,
     fa.dt = dt;
     ListView klv;
     LaunchConfig klc;
-    TRY(force_view(ctx, fa, &klv, &klc));
+    TRY(force_view(ctx, fa, mixed && accum == LJGPU_ACCUM_KAHAN_F32, &klv, &klc));
     // len (drift, kick) pairs. Where the tiles allow it, every kick but the
     // last one ends in the next drift, positions going back and forth
     // between the working copy and md_tmp (free between rebuilds); the first

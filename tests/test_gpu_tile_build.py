@@ -208,3 +208,36 @@ def test_rows_that_repeat_a_partner(ctx, copies, others):
     ctx.set_tiling(64)
     assert np.abs(out[1]).max() > 0
     assert normwise(out[0], out[1]) < FP64_TOL
+
+
+@pytest.mark.parametrize("name", ["ragged", "long_rows", "open"])
+@pytest.mark.parametrize("lanes,unroll", [(4, 4), (8, 2)])
+def test_kahan_sums_have_slices_of_their_own(ctx, name, lanes, unroll):
+    """Kahan sums run over rows in the bank-class order, made on first use,
+    beside the other kernels' slices: neither changes the other's momenta."""
+    q, box, full, _ = system(name)
+    ctx.set_kernel_config(lanes, 256, unroll)
+    ctx.set_tiling(64)
+    ctx.set_half_mode(G.HALF_AUTO)
+    dq = ctx.array(q)
+
+    def momenta(accum):
+        dp = ctx.zeros(q.shape)
+        if accum is None:
+            ctx.force_aos_f64(dq, dp, 1e-3, G.CL2, box, 3)
+        else:
+            ctx.force_aos_mixed(dq, dp, 1e-3, G.CL2, box, 3, accum)
+        ctx.sync()
+        return dp.download()
+
+    out = []
+    for order in ([None, G.ACCUM_KAHAN_F32, None, G.ACCUM_F64], [G.ACCUM_KAHAN_F32, None, None,
+                                                                 G.ACCUM_F64]):
+        ctx.build_list(dq, q.shape[0], box, G.LIST_FULL)
+        got = [momenta(a) for a in order]
+        out.append({a: g for a, g in zip(order, got)})
+        f64 = [g for a, g in zip(order, got) if a is None]
+        np.testing.assert_array_equal(f64[0], f64[1])
+    for a in out[0]:
+        np.testing.assert_array_equal(out[0][a], out[1][a])
+    ctx.set_kernel_config(4, 256, 4)
