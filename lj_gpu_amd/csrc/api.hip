@@ -380,10 +380,12 @@ int build_list(ljgpu_ctx* ctx, const PosIn& q, int32_t n, double box, double sea
   ctx->tiles_for = -1;
   ctx->tiles_ordered = false;
   // Unsorted rows (the MD loop's) are tiled from the pair search's slab; the
-  // list itself is filled only where something reads it.
+  // list itself is filled only where something reads it: the untiled kernels,
+  // energies that do not run over the tiles, and whoever uses an open box's
+  // list after the run.
   if (box <= 0.0 || tile == 0) TRY(dev_copy_slab(ctx->stream, ctx->work, ctx->eval));
   TRY(prepare_layouts(ctx, &q, box));
-  if (ctx->tiles.blocks == 0) TRY(dev_copy_slab(ctx->stream, ctx->work, ctx->eval));
+  if (!energy_on_tiles(ctx)) TRY(dev_copy_slab(ctx->stream, ctx->work, ctx->eval));
   HIP_TRY(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
   return LJGPU_OK;
 }

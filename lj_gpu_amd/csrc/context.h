@@ -222,6 +222,13 @@ void drop_graph(ljgpu_ctx* ctx);
 int force_view(ljgpu_ctx* ctx, const ForceArgs& fa, bool kahan, ListView* lv, LaunchConfig* lc);
 // The installed tiling's fields of a ListView, as they stand.
 void tile_fields(const ljgpu_ctx* ctx, ListView* lv);
+// Whether energies run over the installed tiles as they stand (four lanes a
+// row, one workgroup a tile: at most 256 particles). Elsewhere they read the
+// list's rows, which a build must have filled then.
+inline bool energy_on_tiles(const ljgpu_ctx* ctx) {
+  return ctx->tiles.blocks > 0 && !ctx->eval_half && ctx->rep_off.empty() &&
+         ctx->tiles.tile_particles * 4 <= 1024;
+}
 // Record the launches `body` enqueues on the context stream into an
 // executable graph.
 int capture(ljgpu_ctx* ctx, const std::function<int()>& body, hipGraphExec_t* out);

@@ -237,17 +237,15 @@ __global__ void k_energy_total(int grid_q, int grid_p, int with_q, int with_p,
 // Launch the energy kernels of the current state into `part` (3 *
 // kEnergyBlocks doubles: potential, kinetic and pair-count partials). Over
 // an installed tiling (the force kernels' layout, used as it stands) the
-// potential runs on the tiles (k_tile_energy), otherwise over the CSR rows
-// (k_potential). *grid_q / *grid_p: the partials of U and pairs / of K.
+// potential runs on the tiles (k_tile_energy, energy_on_tiles), otherwise
+// over the CSR rows (k_potential). *grid_q / *grid_p: the partials of U and pairs / of K.
 int launch_energy(ljgpu_ctx* ctx, const double* q, const double* p, double box, double cl2,
                   double* part, int* grid_q, int* grid_p) {
   const int grid = std::min(kEnergyBlocks, grid_for(ctx->n));
   *grid_q = *grid_p = grid;
   if (q) {
     const double weight = ctx->eval_half ? 1.0 : 0.5;
-    const bool tiled = ctx->tiles.blocks > 0 && !ctx->eval_half && ctx->rep_off.empty() &&
-                       ctx->tiles.tile_particles * 4 <= 1024;
-    if (tiled) {
+    if (energy_on_tiles(ctx)) {
       ListView lv;
       tile_fields(ctx, &lv);
       *grid_q = std::min(kEnergyBlocks, (ctx->tiles.blocks + 7) / 8 * 8);

@@ -396,3 +396,34 @@ def test_md_shapes_on_both_sides_of_the_few_particle_rule(ctx, cells, tile, prec
     info = ctx.list_info()
     assert info.tile_particles == tile
     ctx.set_tiling(64)
+
+
+@pytest.mark.parametrize("lanes,tile", [(2, 512), (2, 257), (2, 256)])
+def test_md_energies_with_tiles_the_energy_kernel_does_not_take(lanes, tile):
+    """A dilute periodic gas in tiles of more than 256 particles: its energies
+    run over the list's rows, which the MD loop's builds otherwise leave in the
+    pair search's slab. Energies and states of the default shape, in a context
+    that never held a list and in one that holds another system's."""
+    q0, p0, box = liquid(6, rho=0.1)
+    dense, _, dense_box = liquid(5)
+    runs = []
+    for shape, used in (((4, 64), False), ((lanes, tile), False), ((lanes, tile), True)):
+        c = G.Context(0)
+        try:
+            c.set_kernel_config(shape[0], 256, 4)
+            c.set_tiling(shape[1])
+            if used:
+                c.set_list(G.makepair(dense, dense_box, G.LIST_FULL))
+            dq, dp = c.array(q0), c.array(p0)
+            _, samples = c.md_run(dq, dp, box, 12, DT, rebuild_every=4, sample_every=3)
+            runs.append((samples, dq.download(), dp.download()))
+            c.build_list(dq, q0.shape[0], box, G.LIST_FULL)
+            assert c.list_info().tile_particles == shape[1]  # such tiles fit
+        finally:
+            c.close()
+    for samples, q, p in runs[1:]:
+        np.testing.assert_allclose(samples, runs[0][0], rtol=1e-11, atol=1e-9)
+        d = (q - runs[0][1])[:, :3]
+        d -= box * np.rint(d / box)
+        assert np.abs(d).max() < 1e-10
+        assert np.abs(p - runs[0][2])[:, :3].max() < 1e-9
