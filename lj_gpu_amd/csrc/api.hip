@@ -341,13 +341,17 @@ int build_list(ljgpu_ctx* ctx, const PosIn& q, int32_t n, double box, double sea
   const bool expand = kind == LJGPU_LIST_FULL || ctx->half_mode_req != LJGPU_HALF_ATOMIC;
   // The spatial tile order needs the positions only: enqueued first, it is
   // decided by the pair search's synchronisation.
-  struct OrderBegun {
+  struct BuildGuard {
     ljgpu_ctx* c;
-    ~OrderBegun() {
+    bool done = false;
+    ~BuildGuard() {
       c->order_begun = false;
       c->work.order_job.clear();
+      // A build that fails with its rows still in the slab installs nothing:
+      // whoever reads the list next would find it unfilled.
+      if (!done && c->eval.slab_stride > 0) reset_list(c);
     }
-  } order_begun_guard{ctx};
+  } guard{ctx};
   const int32_t tile = effective_tile(ctx);
   if (tile > 0 && n > 0 && ctx->tile_order == LJGPU_TILE_ORDER_SPATIAL &&
       (expand || ctx->rep_off.empty()))
@@ -387,6 +391,7 @@ int build_list(ljgpu_ctx* ctx, const PosIn& q, int32_t n, double box, double sea
   TRY(prepare_layouts(ctx, &q, box));
   if (!energy_on_tiles(ctx)) TRY(dev_copy_slab(ctx->stream, ctx->work, ctx->eval));
   HIP_TRY(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
+  guard.done = true;
   return LJGPU_OK;
 }
 
@@ -1389,6 +1394,15 @@ int ljgpu_force_soa_mixed(ljgpu_ctx* ctx, const double* qx, const double* qy, co
   fa.cl2 = cl2;
   fa.box = box;
   return run_steps(ctx, fa, steps, true, accum);
+}
+
+// Not in the header: the most bytes that a buffer of the context may take from
+// now on, as if the device had no more (the tests' way into the paths behind a
+// failed allocation). 0: the evaluated list.
+int ljgpu_internal_limit(ljgpu_ctx* ctx, int buffer, size_t bytes) {
+  if (!ctx || buffer != 0) return set_error(LJGPU_ERR_INVALID_ARGUMENT, "internal_limit");
+  ctx->eval.list.limit = bytes;
+  return LJGPU_OK;
 }
 
 int ljgpu_force_kernel_csr_f64(ljgpu_ctx* ctx, const double* q, double* p, int32_t n, double dt,

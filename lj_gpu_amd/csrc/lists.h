@@ -21,6 +21,7 @@ namespace ljgpu {
 struct DevMem {
   void* p = nullptr;
   size_t bytes = 0;
+  size_t limit = SIZE_MAX;  // most bytes to take (ljgpu_internal_limit)
   template <class T>
   T* as() const {
     return static_cast<T*>(p);

@@ -2239,6 +2239,7 @@ int dev_reserve(DevMem& m, size_t bytes, hipStream_t stream) {
     m.bytes = 0;
   }
   const size_t grow = bytes + bytes / 8;  // headroom for the next, slightly larger build
+  if (grow > m.limit) return hip_err(hipErrorOutOfMemory, "hipMalloc (list buffer)");
   LTRY(hipMalloc(&m.p, grow), "hipMalloc (list buffer)");
   m.bytes = grow;
   return LJGPU_OK;

@@ -7,6 +7,8 @@ pinned to the oracle); the integrator by a numpy velocity-Verlet loop driven
 by the oracle's forces and lists, by time reversibility and by energy
 conservation; graph replay by bitwise equality with individual launches.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -427,3 +429,34 @@ def test_md_energies_with_tiles_the_energy_kernel_does_not_take(lanes, tile):
         d -= box * np.rint(d / box)
         assert np.abs(d).max() < 1e-10
         assert np.abs(p - runs[0][2])[:, :3].max() < 1e-9
+
+
+def test_md_build_without_room_for_the_list_installs_none():
+    """An open box's run whose list cannot be allocated: an error, and no list
+    afterwards (its rows stayed in the pair search's slab, so the list would
+    be read unfilled). With room again the same context runs as a new one."""
+    q0, p0, _ = liquid(6, rho=0.5)
+    c, new = G.Context(0), G.Context(0)
+    try:
+        limit = G.lib().ljgpu_internal_limit
+        limit.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t]
+        dq, dp = c.array(q0), c.array(p0)
+        assert limit(c.handle, 0, 64) == G.OK
+        with pytest.raises(G.LJGPUError) as e:
+            c.md_run(dq, dp, 0.0, 4, DT)
+        assert e.value.code == G.ERR_OUT_OF_MEMORY
+        with pytest.raises(G.LJGPUError) as e:
+            c.energy(dq, dp, 0.0)
+        assert e.value.code == G.ERR_NO_LIST
+        assert limit(c.handle, 0, 2**64 - 1) == G.OK
+        got = []
+        for x in (c, new):
+            dq, dp = x.array(q0), x.array(p0)
+            x.md_run(dq, dp, 0.0, 4, DT)
+            got.append((dq.download(), dp.download(), x.energy(dq, dp, 0.0)))
+        np.testing.assert_array_equal(got[0][0], got[1][0])
+        np.testing.assert_array_equal(got[0][1], got[1][1])
+        assert got[0][2] == got[1][2]
+    finally:
+        c.close()
+        new.close()
