@@ -1405,6 +1405,14 @@ int ljgpu_internal_limit(ljgpu_ctx* ctx, int buffer, size_t bytes) {
   return LJGPU_OK;
 }
 
+// Not in the header (lists of LJGPU_HALF_ATOMIC are reported as untiled): the
+// particles per tile that such a list is evaluated with, 0 for the untiled kernel.
+int ljgpu_internal_half_tile(ljgpu_ctx* ctx, int32_t* tile_particles) {
+  if (!ctx || !tile_particles) return set_error(LJGPU_ERR_INVALID_ARGUMENT, "null argument");
+  *tile_particles = ctx->eval_half && ctx->tiles.blocks > 0 ? ctx->tiles.tile_particles : 0;
+  return LJGPU_OK;
+}
+
 int ljgpu_force_kernel_csr_f64(ljgpu_ctx* ctx, const double* q, double* p, int32_t n, double dt,
                                double cl2, const int32_t* list, const int32_t* nop,
                                const int32_t* ptr, int64_t n_entries, int kind) {

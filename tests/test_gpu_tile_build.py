@@ -5,6 +5,7 @@ in a few runs of slots (the paged one), rows of very different lengths, open
 and periodic boxes. The tiles must equal the host model's (ljgpu_make_tiles_*)
 and the forces over them, whose entry order is the slices' own, the oracle's.
 """
+import ctypes
 import functools
 
 import numpy as np
@@ -13,6 +14,8 @@ import pytest
 import lj_gpu_amd as G
 import oracle as O
 from helpers import FP64_TOL, normwise
+
+MIXED_TOL = 2.0e-6  # normwise, FP32 force scalars with FP64 sums
 
 pytestmark = pytest.mark.gpu
 
@@ -241,3 +244,47 @@ def test_kahan_sums_have_slices_of_their_own(ctx, name, lanes, unroll):
     for a in out[0]:
         np.testing.assert_array_equal(out[0][a], out[1][a])
     ctx.set_kernel_config(4, 256, 4)
+
+
+def half_tile(ctx):
+    """Particles per tile of the installed atomic half list; 0: untiled kernel."""
+    query = G.lib().ljgpu_internal_half_tile
+    query.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int32)]
+    t = ctypes.c_int32(-1)
+    assert query(ctx.handle, ctypes.byref(t)) == G.OK
+    return t.value
+
+
+@pytest.mark.parametrize("name", ["ragged", "mixed_rows", "scattered", "open"])
+@pytest.mark.parametrize("tile", [64, 16, 1])
+def test_which_kernel_an_atomic_half_list_takes(ctx, name, tile):
+    """Tiles where they stage at most half as many partners as the list has
+    entries, the untiled kernel elsewhere (scattered particles, tiles of one);
+    Kahan sums always take the untiled kernel's order of entries."""
+    q, box, _, f = system(name)
+    n = q.shape[0]
+    ctx.set_kernel_config(4, 256, 4)
+    ctx.set_half_mode(G.HALF_ATOMIC)
+    dq, dp = ctx.array(q), ctx.zeros(q.shape)
+    kahan = []
+    for t in (tile, 0):
+        ctx.set_tiling(t)
+        ctx.build_list(dq, n, box, G.LIST_HALF)
+        used = half_tile(ctx)
+        print(f"{name} tile={t} used={used}", flush=True)
+        assert used == (t if name != "scattered" and t > 1 else 0)
+        for accum, tol in ((None, FP64_TOL), (G.ACCUM_F64, MIXED_TOL), (G.ACCUM_KAHAN_F32, None)):
+            dp.zero()
+            if accum is None:
+                ctx.force_aos_f64(dq, dp, 1.0, G.CL2, box, 1)
+            else:
+                ctx.force_aos_mixed(dq, dp, 1.0, G.CL2, box, 1, accum)
+            ctx.sync()
+            if tol is None:
+                kahan.append(dp.download())
+            else:
+                assert normwise(dp.download(), f) < tol
+    # FP32 sums in another order differ by about 1e-7, the additions to memory by rounding.
+    assert normwise(kahan[0], kahan[1]) < FP64_TOL
+    ctx.set_tiling(64)
+    ctx.set_half_mode(G.HALF_AUTO)
