@@ -71,6 +71,7 @@ void reset_list(ljgpu_ctx* ctx) {
   ctx->tiles.blocks = 0;
   ctx->tiles.sliced_lanes = ctx->tiles.sliced_unroll = 0;
   ctx->tiles.bank_lanes = ctx->tiles.bank_unroll = 0;
+  ctx->tiles.half_ready = false;
 }
 
 void release_all(ljgpu_ctx* ctx) {
@@ -105,7 +106,13 @@ int ensure_ell(ljgpu_ctx* ctx) {
   return LJGPU_OK;
 }
 
-// Derive the LDS tiling of the evaluated full list for the current
+// The tile size to derive for the evaluated list (half lists of replicas are
+// not evaluated at all).
+int32_t tile_target(const ljgpu_ctx* ctx) {
+  return ctx->eval_half && !ctx->rep_off.empty() ? 0 : effective_tile(ctx);
+}
+
+// Derive the LDS tiling of the evaluated list for the current
 // configuration. Where a block does not fit the LDS budget the tile size is
 // halved; a list whose single rows do not fit keeps the untiled kernels.
 // With the spatial tile order the blocks take the particles in the order of
@@ -115,7 +122,7 @@ int ensure_ell(ljgpu_ctx* ctx) {
 // order. A tiling derived without positions is derived again, once, when
 // positions first come.
 int ensure_tiles(ljgpu_ctx* ctx, const PosIn* q, double box) {
-  const int32_t want = ctx->eval_half && !ctx->rep_off.empty() ? 0 : effective_tile(ctx);
+  const int32_t want = tile_target(ctx);
   const bool spatial = ctx->tile_order == LJGPU_TILE_ORDER_SPATIAL && want > 0;
   if (want == ctx->tiles_for && (ctx->tiles_ordered || !q || want == 0)) return LJGPU_OK;
   ctx->tiles.tile_particles = 0;
@@ -172,7 +179,9 @@ int ensure_sliced(ljgpu_ctx* ctx, const PosIn* q, double box, double cl2) {
   DevTiles& t = ctx->tiles;
   const int lanes = ctx->eval_half ? kHalfLanes : ctx->lanes;
   const int unroll = ctx->eval_half ? 4 : ctx->unroll;
-  if (t.blocks <= 0 || (t.sliced_lanes == lanes && t.sliced_unroll == unroll)) return LJGPU_OK;
+  if (t.blocks <= 0 || (t.sliced_lanes == lanes && t.sliced_unroll == unroll &&
+                        (!ctx->eval_half || t.half_ready)))
+    return LJGPU_OK;
   CutHint cut;
   if (q) {
     cut.q = *q;
@@ -221,11 +230,33 @@ int ensure_bank_slices(ljgpu_ctx* ctx) {
   return LJGPU_OK;
 }
 
+// Tiles and slices of a half list evaluated with atomics. The untiled kernel
+// needs neither, so a list whose tiles find no room (their force sums alone
+// take 24 bytes per staged partner) or are too many is evaluated with it, and
+// what they took is given back.
+int ensure_half_layouts(ljgpu_ctx* ctx, const PosIn* q, double box, double cl2) {
+  int rc = ensure_tiles(ctx, q, box);
+  if (rc == LJGPU_OK) rc = ensure_sliced(ctx, q, box, cl2);
+  if (rc == LJGPU_OK) return LJGPU_OK;
+  if (rc != LJGPU_ERR_OUT_OF_MEMORY && rc != LJGPU_ERR_CAPACITY) {
+    ctx->tiles_for = -1;  // derived anew at the next use
+    ctx->tiles.blocks = ctx->tiles.tile_particles = 0;
+    return rc;
+  }
+  HIP_TRY(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
+  (void)hipGetLastError();  // the failed allocation's
+  clear_error();
+  dev_release(ctx->tiles);
+  ctx->tiles_for = tile_target(ctx);
+  ctx->tiles_ordered = q != nullptr;
+  return LJGPU_OK;
+}
+
 int prepare_layouts(ljgpu_ctx* ctx, const PosIn* q, double box, double cl2) {
   if (ctx->lanes == 1) return ensure_ell(ctx);
+  if (ctx->eval_half) return ensure_half_layouts(ctx, q, box, cl2);
   TRY(ensure_tiles(ctx, q, box));
   TRY(ensure_sliced(ctx, q, box, cl2));
-  if (ctx->eval_half) return LJGPU_OK;
   return ctx->tile_offsets_lds || ctx->tiles.sliced_lanes == 0 ? ensure_bank_order(ctx) : LJGPU_OK;
 }
 
@@ -1398,10 +1429,13 @@ int ljgpu_force_soa_mixed(ljgpu_ctx* ctx, const double* qx, const double* qy, co
 
 // Not in the header: the most bytes that a buffer of the context may take from
 // now on, as if the device had no more (the tests' way into the paths behind a
-// failed allocation). 0: the evaluated list.
+// failed allocation). 0: the evaluated list, 1: the force sums of a half list's
+// tiles, 2: the tiles' staged particles.
 int ljgpu_internal_limit(ljgpu_ctx* ctx, int buffer, size_t bytes) {
-  if (!ctx || buffer != 0) return set_error(LJGPU_ERR_INVALID_ARGUMENT, "internal_limit");
-  ctx->eval.list.limit = bytes;
+  if (!ctx || buffer < 0 || buffer > 2)
+    return set_error(LJGPU_ERR_INVALID_ARGUMENT, "internal_limit");
+  DevMem* m[] = {&ctx->eval.list, &ctx->tiles.half_part, &ctx->tiles.stage};
+  m[buffer]->limit = bytes;
   return LJGPU_OK;
 }
 

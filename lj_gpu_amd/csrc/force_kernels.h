@@ -970,7 +970,8 @@ template <int PREC, class P, class M, bool PBC>
 int run_tile_half(hipStream_t s, P pos, M mom, const ListView& lv, const PairParams& pp) {
   const int threads = (lv.tile_particles * kHalfLanes + 63) / 64 * 64;
   if (threads > 1024 || lv.tile_sliced_lanes != kHalfLanes ||
-      lv.tile_sliced_unroll != kHalfUnroll || !lv.half_tile || lv.tile_first != 0)
+      lv.tile_sliced_unroll != kHalfUnroll || !lv.half_tile || !lv.half_first || !lv.half_at ||
+      !lv.half_part || lv.tile_first != 0)
     return set_error(LJGPU_ERR_INVALID_ARGUMENT, "tiled half list: launch shape");
   const int grid = (lv.tile_blocks + kXcds - 1) / kXcds * kXcds;
   const size_t lds_bytes = kTileLdsHeader + static_cast<size_t>(lv.tile_max_stage) * kHalfStride;

@@ -81,8 +81,10 @@ struct DevTiles {
   DevMem inner;          // int32 per slot
   int32_t longest = 0;   // longest row
 
-  // Half lists (dev_half_tiles): see ListView.
+  // Half lists (dev_half_tiles): see ListView. half_ready: all four belong to
+  // this tiling.
   DevMem half_tile, half_first, half_at, half_part;
+  bool half_ready = false;
 };
 void dev_release(DevTiles& t);
 

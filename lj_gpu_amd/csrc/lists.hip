@@ -2273,6 +2273,7 @@ void dev_release(DevTiles& t) {
   dev_release(t.stage_slot);
   dev_release(t.inner);
   for (DevMem* m : {&t.half_tile, &t.half_first, &t.half_at, &t.half_part}) dev_release(*m);
+  t.half_ready = false;
   t.cut = t.bank_done = false;
   t.tile_particles = 0;
   t.blocks = 0;
@@ -2841,6 +2842,7 @@ int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<
                    bool spatial, const SliceReq* req, ListWork& w, DevTiles& out) {
   out.tile_particles = 0;
   out.blocks = 0;
+  out.half_ready = false;
   if (T <= 0 || T > kTileRowsMax || c.n <= 0) return LJGPU_OK;
   // The slot order and each slot's row start in the slot-ordered rows.
   // Index order: slot = particle and the list's own row starts. Otherwise
@@ -3024,6 +3026,7 @@ int dev_slice_tiles(hipStream_t s, const int32_t* slot_ptr, int32_t lanes, int32
 }
 
 int dev_half_tiles(hipStream_t s, int32_t n, ListWork& w, DevTiles& t) {
+  t.half_ready = false;
   if (t.blocks <= 0) return LJGPU_OK;
   const int32_t nb = t.blocks;
   LCHECK(dev_reserve(w.tile_ns, sizeof(int32_t) * (static_cast<size_t>(nb) + 1), s));
@@ -3054,6 +3057,7 @@ int dev_half_tiles(hipStream_t s, int32_t n, ListWork& w, DevTiles& t) {
                                       t.half_at.as<int32_t>());
   k_half_sort<<<(n + kBlock - 1) / kBlock, kBlock, 0, s>>>(n, first, t.half_at.as<int32_t>());
   LTRY(hipGetLastError(), "half tile fill kernels");
+  t.half_ready = true;
   return LJGPU_OK;
 }
 

@@ -288,3 +288,50 @@ def test_which_kernel_an_atomic_half_list_takes(ctx, name, tile):
     assert normwise(kahan[0], kahan[1]) < FP64_TOL
     ctx.set_tiling(64)
     ctx.set_half_mode(G.HALF_AUTO)
+
+
+@pytest.mark.parametrize("buffer", [1, 2])
+@pytest.mark.parametrize("device_list", [True, False])
+def test_half_list_whose_tiles_find_no_room(buffer, device_list):
+    """Where the tiles' force sums (or their staged particles) cannot be
+    allocated, the list is installed all the same and takes the untiled kernel,
+    call after call; after a smaller list that is tiled, too. With room again, a
+    new list is tiled."""
+    q, box, _, f = system("ragged")
+    small, small_box = G.lattice_periodic(5, 0.5, 3)
+    c = G.Context(0)
+    try:
+        limit = G.lib().ljgpu_internal_limit
+        limit.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t]
+        c.set_half_mode(G.HALF_ATOMIC)
+        half = G.makepair(q, box, G.LIST_HALF)
+        dq, dp = c.array(q), c.zeros(q.shape)
+
+        def install():
+            if device_list:
+                c.build_list(dq, q.shape[0], box, G.LIST_HALF)
+            else:
+                c.set_list(half)
+
+        def check(tile):
+            for steps in (1, 5, 20):
+                dp.zero()
+                c.force_aos_f64(dq, dp, 1.0 / steps, G.CL2, box, steps)
+                c.sync()
+                assert half_tile(c) == tile
+                assert normwise(dp.download(), f) < FP64_TOL
+
+        assert limit(c.handle, buffer, 64) == G.OK
+        install()
+        check(0)
+        assert limit(c.handle, buffer, 2**64 - 1) == G.OK
+        c.build_list(c.array(small), small.shape[0], small_box, G.LIST_HALF)
+        assert half_tile(c) == 64
+        assert limit(c.handle, buffer, 64) == G.OK
+        install()
+        check(0)
+        assert limit(c.handle, buffer, 2**64 - 1) == G.OK
+        install()
+        check(64)
+    finally:
+        c.close()
