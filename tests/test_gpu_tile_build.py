@@ -335,3 +335,62 @@ def test_half_list_whose_tiles_find_no_room(buffer, device_list):
         check(64)
     finally:
         c.close()
+
+
+def exact_force(q, box, half):
+    """Force of every pair of a half list inside the cutoff in extended
+    precision, and per particle sum(|24 s^4| + |48 s^7|) r, s = 1 / r^2."""
+    i = np.repeat(np.arange(q.shape[0]), half.number_of_partners)
+    j = half.sorted_list
+    x = q[:, :3].astype(np.longdouble)
+    d = x[j] - x[i]
+    d -= np.longdouble(box) * np.rint(d / np.longdouble(box))
+    r2 = (d * d).sum(1)
+    i, j, d, r2 = (a[r2 <= G.CL2] for a in (i, j, d, r2))
+    s = 1 / r2
+    df = 24 * s ** 4 - 48 * s ** 7
+    weight = (24 * s ** 4 + 48 * s ** 7) * np.sqrt(r2)
+    f = np.zeros_like(x)
+    scale = np.zeros(q.shape[0], np.longdouble)
+    for c in range(3):
+        np.add.at(f[:, c], i, df * d[:, c])
+        np.add.at(f[:, c], j, -df * d[:, c])
+    np.add.at(scale, i, weight)
+    np.add.at(scale, j, weight)
+    return f, scale
+
+
+@pytest.mark.parametrize("corner", [0.0, 0.5])
+@pytest.mark.parametrize("tile", [64, 16, 0])
+def test_half_list_forces_lose_nothing_at_a_face(ctx, corner, tile):
+    """A dense block of particles across the corner of a box 30 times its size
+    (or in the middle of it): positions shifted into a tile's frame must not be
+    rounded at the box's magnitude, which moves every pair by 256 u (u = 2^-53) and
+    its force by 14 * 256 u / r. Rounded once each: differences u, r^2 4 u, its
+    reciprocal 6 u, the seventh power and products 45 u; a row's additions 80 u."""
+    q, side = G.lattice_periodic(6, 1.0, 3)
+    box = 300.0
+    # Positions on the grid of the largest ones: wrapping them is exact.
+    x = np.rint((q[:, :3] - side / 2 + corner * box) * 2.0**44) / 2.0**44
+    rng = np.random.default_rng(11)
+    q = np.zeros_like(q)
+    q[:, :3] = np.where(x < 0, x + box, x)
+    # and, below that grid, bits of their own
+    low = q[:, :3] < 16.0
+    q[:, :3] += np.where(low, rng.uniform(0, 2.0**-45, low.shape), 0.0)
+    half = G.makepair(q, box, G.LIST_HALF)
+    f, scale = exact_force(q, box, half)
+    ctx.set_kernel_config(4, 256, 4)
+    ctx.set_tiling(tile)
+    ctx.set_half_mode(G.HALF_ATOMIC)
+    dq, dp = ctx.array(q), ctx.zeros(q.shape)
+    ctx.build_list(dq, q.shape[0], box, G.LIST_HALF)
+    assert half_tile(ctx) == tile
+    ctx.force_aos_f64(dq, dp, 1.0, G.CL2, box, 1)
+    ctx.sync()
+    off = np.abs(dp.download()[:, :3] - f).max(1) / (scale * 2.0**-53)
+    print(f"corner={corner} tile={tile} error {float(off.max()):.1f} u", flush=True)
+    # The untiled kernel rounds differences across a face, up to the box's ulp / 2.
+    assert off.max() < (125 if tile or corner else 125 + 14 * 256)
+    ctx.set_tiling(64)
+    ctx.set_half_mode(G.HALF_AUTO)
