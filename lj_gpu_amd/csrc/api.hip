@@ -70,6 +70,7 @@ void reset_list(ljgpu_ctx* ctx) {
   ctx->tiles.tile_particles = 0;
   ctx->tiles.blocks = 0;
   ctx->tiles.sliced_lanes = ctx->tiles.sliced_unroll = 0;
+  ctx->tiles.bank_rows = false;
   ctx->tiles.bank_lanes = ctx->tiles.bank_unroll = 0;
   ctx->tiles.half_ready = false;
 }
@@ -128,6 +129,7 @@ int ensure_tiles(ljgpu_ctx* ctx, const PosIn* q, double box) {
   ctx->tiles.tile_particles = 0;
   ctx->tiles.blocks = 0;
   ctx->tiles.sliced_lanes = ctx->tiles.sliced_unroll = 0;
+  ctx->tiles.bank_rows = false;
   ctx->tiles.bank_lanes = ctx->tiles.bank_unroll = 0;
   bool ordered = false;
   if (ctx->order_begun)
@@ -190,44 +192,22 @@ int ensure_sliced(ljgpu_ctx* ctx, const PosIn* q, double box, double cl2) {
     cut.cl2 = cl2;
   }
   TRY(dev_slice_tiles(ctx->stream, tile_row_starts(ctx), lanes, unroll,
-                      ctx->eval_half ? kHalfStride : 24, ctx->bank_order && !t.bank_done,
-                      ctx->eval.n, &cut, ctx->work, t));
-  if (!ctx->eval_half) return LJGPU_OK;
+                      ctx->eval_half ? kHalfStride : 24, ctx->bank_order, ctx->eval.n, &cut,
+                      ctx->work, t));
+  // Room for what Kahan sums read, where they would read slices: they come with
+  // a force call, which does not allocate.
+  if (!ctx->eval_half)
+    return ctx->bank_order && !ctx->tile_offsets_lds && t.sliced_lanes > 0
+               ? dev_bank_reserve(ctx->stream, ctx->eval.e, ctx->work, t)
+               : LJGPU_OK;
   // The half-list kernel reads the slices only.
   if (t.sliced_lanes == 0) t.tile_particles = t.blocks = 0;
   return dev_half_tiles(ctx->stream, ctx->eval.n, ctx->work, t);
 }
 
-// The bank-class order of the tiles' rows in `local`, for the kernels that
-// read it instead of the slices (once per tiling).
-int ensure_bank_order(ljgpu_ctx* ctx) {
-  DevTiles& t = ctx->tiles;
-  if (t.blocks <= 0 || t.bank_done || !ctx->bank_order) return LJGPU_OK;
-  TRY(dev_bank_order(ctx->stream, tile_row_starts(ctx), t, t.local.as<uint16_t>()));
-  t.bank_done = true;
-  return LJGPU_OK;
-}
-
-// Slices of the rows in the bank-class order (once per tiling and
-// configuration), for the FP32 Kahan sums: their last bits follow the order of
-// the entries (2e-7 of the momenta between orders), and this is the order that
-// the host model of the tiles defines.
-int ensure_bank_slices(ljgpu_ctx* ctx) {
-  DevTiles& t = ctx->tiles;
-  const int32_t lanes = t.sliced_lanes, unroll = t.sliced_unroll;
-  if (t.blocks <= 0 || lanes == 0 || !ctx->bank_order ||
-      (t.bank_lanes == lanes && t.bank_unroll == unroll))
-    return LJGPU_OK;
-  TRY(ensure_bank_order(ctx));
-  t.bank_lanes = t.bank_unroll = 0;
-  std::swap(t.sliced, t.sliced_bank);
-  const int rc = dev_slice_tiles(ctx->stream, tile_row_starts(ctx), lanes, unroll, 24, false,
-                                 ctx->eval.n, nullptr, ctx->work, t);
-  std::swap(t.sliced, t.sliced_bank);
-  if (rc) return rc;
-  t.bank_lanes = t.sliced_lanes;
-  t.bank_unroll = t.sliced_unroll;
-  return LJGPU_OK;
+// Whether the force kernels read rows of entry offsets, not slices.
+bool reads_rows(const ljgpu_ctx* ctx) {
+  return ctx->tile_offsets_lds || ctx->tiles.sliced_lanes == 0;
 }
 
 // Tiles and slices of a half list evaluated with atomics. The untiled kernel
@@ -257,7 +237,8 @@ int prepare_layouts(ljgpu_ctx* ctx, const PosIn* q, double box, double cl2) {
   if (ctx->eval_half) return ensure_half_layouts(ctx, q, box, cl2);
   TRY(ensure_tiles(ctx, q, box));
   TRY(ensure_sliced(ctx, q, box, cl2));
-  return ctx->tile_offsets_lds || ctx->tiles.sliced_lanes == 0 ? ensure_bank_order(ctx) : LJGPU_OK;
+  if (!ctx->bank_order || !reads_rows(ctx)) return LJGPU_OK;
+  return dev_bank_rows(ctx->stream, tile_row_starts(ctx), ctx->eval.e, ctx->work, ctx->tiles);
 }
 
 PosIn positions_of(const ForceArgs& fa) {
@@ -467,10 +448,17 @@ int force_view(ljgpu_ctx* ctx, const ForceArgs& fa, bool kahan, ListView* lv, La
     lv->list = ctx->eval.list.as<int32_t>();
     // Kahan sums of half lists keep the untiled kernel's order of entries.
     if (ctx->tiles.blocks > 0 && !(kahan && ctx->eval_half)) {
-      if (kahan) TRY(ensure_bank_slices(ctx));
       tile_fields(ctx, lv);
-      if (kahan && lv->tile_sliced && ctx->tiles.bank_lanes > 0)
-        lv->tile_sliced = ctx->tiles.sliced_bank.as<uint16_t>();
+      // FP32 Kahan sums follow the order of the entries in their last bits (2e-7
+      // of the momenta between orders), so theirs is the order that the host
+      // model of the tiles defines; rows that are read as such are in it too.
+      if (ctx->bank_order && !ctx->eval_half && reads_rows(ctx)) {
+        lv->tile_local = bank_rows(ctx->work);
+      } else if (ctx->bank_order && kahan) {
+        TRY(dev_bank_slices(ctx->stream, tile_row_starts(ctx), ctx->eval.e, ctx->work,
+                            ctx->tiles));
+        lv->tile_sliced = bank_slices(ctx->work, ctx->eval.e);
+      }
     }
   }
   return LJGPU_OK;
@@ -1216,19 +1204,10 @@ int ljgpu_get_tiles(ljgpu_ctx* ctx, int32_t* desc, int64_t desc_capacity, int32_
   HIP_TRY(hipMemcpyAsync(desc, t.desc.p, sizeof(int32_t) * 8 * t.blocks, hipMemcpyDeviceToHost,
                          ctx->stream), "hipMemcpyAsync");
   if (ctx->eval.e > 0) {
-    // The rows in the bank-class order, made in a copy: the evaluated
-    // offsets stay as they are.
-    const size_t bytes = sizeof(uint16_t) * ctx->eval.e;
-    const void* src = t.local.p;
-    if (ctx->bank_order && !t.bank_done) {
-      TRY(dev_reserve(ctx->work.tmp, bytes, ctx->stream));
-      HIP_TRY(hipMemcpyAsync(ctx->work.tmp.p, src, bytes, hipMemcpyDeviceToDevice, ctx->stream),
-              "hipMemcpyAsync");
-      TRY(dev_bank_order(ctx->stream, tile_row_starts(ctx), t, ctx->work.tmp.as<uint16_t>()));
-      src = ctx->work.tmp.p;
-    }
-    HIP_TRY(hipMemcpyAsync(local, src, bytes, hipMemcpyDeviceToHost, ctx->stream),
-            "hipMemcpyAsync");
+    // The rows in the bank-class order: the evaluated offsets stay as they are.
+    TRY(dev_bank_rows(ctx->stream, tile_row_starts(ctx), ctx->eval.e, ctx->work, ctx->tiles));
+    HIP_TRY(hipMemcpyAsync(local, bank_rows(ctx->work), sizeof(uint16_t) * ctx->eval.e,
+                           hipMemcpyDeviceToHost, ctx->stream), "hipMemcpyAsync");
   }
   if (t.stage_stride == 0) {
     if (t.staged > 0)

@@ -67,18 +67,19 @@ struct DevTiles {
   // sliced_lanes lanes per particle and sliced_unroll entries per lane per
   // batch (see dev_slice_tiles); sliced_lanes = 0: not built.
   DevMem sliced;      // uint16
-  // The slices of rows in the bank-class order (made on first use, for sums
-  // that depend on the order), for bank_lanes and bank_unroll; 0: none.
-  DevMem sliced_bank;
-  int32_t bank_lanes = 0, bank_unroll = 0;
   DevMem wave_off;    // int32 per (block, wavefront slot): start of its slice
   int32_t sliced_lanes = 0, sliced_unroll = 0, waves_per_block = 0;
+  int64_t slice_elems = 0;  // entries that `sliced` has room for
 
   // Cutoff classes (cut): the rows of local hold their inner entries first,
-  // inner[s] of them in slot s's row. bank_done: local's rows are in the
-  // bank-class order as well (dev_bank_order).
-  bool cut = false, bank_done = false;
+  // inner[s] of them in slot s's row.
+  bool cut = false;
   DevMem inner;          // int32 per slot
+  // The rows in the bank-class order, and slices of them for bank_lanes and
+  // bank_unroll (0: none), made on first use (dev_bank_rows, dev_bank_slices)
+  // in ListWork::tmp: local itself keeps its order.
+  bool bank_rows = false;
+  int32_t bank_lanes = 0, bank_unroll = 0;
   int32_t longest = 0;   // longest row
 
   // Half lists (dev_half_tiles): see ListView. half_ready: all four belong to
@@ -103,7 +104,7 @@ struct ListResults {
 
 // Scratch buffers reused across builds.
 struct ListWork {
-  DevMem scan_sums;   // int64 per scan tile
+  DevMem scan_sums;   // a 16-byte record (sum, extrema) per scan tile
   DevMem small;       // a few int64 results (totals, flags, extrema)
   DevMem cell_count;  // int32 per cell (+1)
   DevMem cell_start;  // int32 per cell (+1)
@@ -112,7 +113,7 @@ struct ListWork {
   DevMem cell_sorted; // int32 per particle, cell order: cell index
   DevMem cpos;        // double4 per particle, cell order: x, y, z, index
   DevMem counts;      // int32 per row (+1)
-  DevMem tmp;         // int32 per list entry
+  DevMem tmp;         // int32 per list entry; between builds see DevTiles::bank_rows
   DevMem tile_ns;     // int32 per tile (+1)
   DevMem tile_soff;   // int32 per tile (+1)
   DevMem tile_stats;  // int4 per tile
@@ -241,9 +242,16 @@ int dev_slice_tiles(hipStream_t s, const int32_t* slot_ptr, int32_t lanes, int32
 // to each slot (in ascending order).
 int dev_half_tiles(hipStream_t s, int32_t n, ListWork& w, DevTiles& t);
 
-// The bank-class order (bank_class_order) of a tiling's rows, in place in
-// `local` (t.local or a copy of it); nothing when t.bank_done.
-int dev_bank_order(hipStream_t s, const int32_t* slot_ptr, const DevTiles& t, uint16_t* local);
+// The bank-class order (bank_class_order) of a tiling's rows, e entries, for what
+// reads rows rather than slices; and slices of those rows, cut as the tiling's
+// (t.sliced), for sums that depend on the order. Nothing where they are made
+// already. Enqueued only, and without allocating after dev_bank_reserve, which
+// leaves them without room where there is none.
+int dev_bank_rows(hipStream_t s, const int32_t* slot_ptr, int64_t e, ListWork& w, DevTiles& t);
+int dev_bank_slices(hipStream_t s, const int32_t* slot_ptr, int64_t e, ListWork& w, DevTiles& t);
+int dev_bank_reserve(hipStream_t s, int64_t e, ListWork& w, DevTiles& t);
+const uint16_t* bank_rows(const ListWork& w);
+const uint16_t* bank_slices(const ListWork& w, int64_t e);
 
 // Spatial particle order for LDS tiles, into w.order: each periodic system
 // (the whole set, or every replica of `replicas` with its box) is cut into

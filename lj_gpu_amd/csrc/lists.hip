@@ -2264,8 +2264,9 @@ void dev_release(DevTiles& t) {
   dev_release(t.stage);
   dev_release(t.local);
   dev_release(t.sliced);
-  dev_release(t.sliced_bank);
+  t.bank_rows = false;
   t.bank_lanes = t.bank_unroll = 0;
+  t.slice_elems = 0;
   dev_release(t.wave_off);
   t.sliced_lanes = t.sliced_unroll = t.waves_per_block = 0;
   dev_release(t.member);
@@ -2274,7 +2275,7 @@ void dev_release(DevTiles& t) {
   dev_release(t.inner);
   for (DevMem* m : {&t.half_tile, &t.half_first, &t.half_at, &t.half_part}) dev_release(*m);
   t.half_ready = false;
-  t.cut = t.bank_done = false;
+  t.cut = false;
   t.tile_particles = 0;
   t.blocks = 0;
   t.staged = 0;
@@ -2834,6 +2835,7 @@ int plan_slices(hipStream_t s, const TileSpans& spans, int32_t nblocks, int32_t 
   const int32_t pad = slice_pad(unroll);
   if (total + pad > INT32_MAX) return LJGPU_OK;
   LCHECK(dev_reserve(t.sliced, sizeof(uint16_t) * (total + pad), s));
+  t.slice_elems = total + pad;
   *wpb = waves;
   return LJGPU_OK;
 }
@@ -2965,7 +2967,8 @@ int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<
     out.stage_stride = 0;
   }
   out.cut = false;
-  out.bank_done = false;
+  out.bank_rows = false;
+  out.bank_lanes = out.bank_unroll = 0;
   out.longest = h[3];
   out.tile_particles = T;
   out.blocks = nb;
@@ -2975,27 +2978,11 @@ int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<
   return LJGPU_OK;
 }
 
-int dev_slice_tiles(hipStream_t s, const int32_t* slot_ptr, int32_t lanes, int32_t unroll,
-                    int32_t scale, bool bank_order, int32_t n, const CutHint* hint, ListWork& w,
-                    DevTiles& t) {
-  t.sliced_lanes = t.sliced_unroll = t.waves_per_block = 0;
-  if (t.blocks <= 0) return LJGPU_OK;
-  int32_t wpb = 0;
-  LCHECK(plan_slices(s, TileSpans{t.desc.as<int32_t>(), 0, 0, 8}, t.blocks, t.tile_particles,
-                     slot_ptr, lanes, unroll, t.longest, w, t, &wpb));
-  if (wpb == 0) return LJGPU_OK;
-  const int32_t pad = slice_pad(unroll);
-  CutDev cd{};
-  const bool cut = bank_order && hint && hint->q.x && !t.cut;
-  if (cut) {
-    cd.q = hint->q;
-    cd.stage = t.stage.as<int32_t>();
-    cd.member = t.order == LJGPU_TILE_ORDER_SPATIAL ? t.member.as<int32_t>() : nullptr;
-    cd.box = hint->box;
-    cd.rep_box = hint->rep_box;
-    cd.cl2 = hint->cl2;
-    LCHECK(dev_reserve(t.inner, sizeof(int32_t) * n, s));
-  }
+// The slices of `local` in `sliced` (k_tile_slices), lengths and starts from
+// plan_slices.
+int fill_slices(hipStream_t s, const int32_t* slot_ptr, int32_t lanes, int32_t unroll,
+                int32_t scale, bool bank_order, const CutDev* cut, uint16_t* local,
+                const DevTiles& t, int32_t wpb, uint16_t* sliced) {
   // Rows an odd number of dwords apart, so that lanes walking one row each
   // read different banks; fewer rows at a time where long ones would not fit.
   const int32_t longest = std::min(std::max(t.longest, 2), kBankRowMax);
@@ -3014,10 +3001,36 @@ int dev_slice_tiles(hipStream_t s, const int32_t* slot_ptr, int32_t lanes, int32
                 : pos_lds   ? k_tile_slices<true, true, true>
                             : k_tile_slices<true, false, true>;
   kernel<<<std::min(t.blocks, 65535), kSliceThreads, rows + std::max(order, pos_lds ? pos : 0), s>>>(
-      t.desc.as<int32_t>(), t.blocks, slot_ptr,
-      t.cut || cut ? t.inner.as<int32_t>() : nullptr, t.local.as<uint16_t>(), cd, grows, stride,
-      lanes, wpb, scale, pad, t.wave_off.as<int32_t>(), t.sliced.as<uint16_t>());
+      t.desc.as<int32_t>(), t.blocks, slot_ptr, t.cut || cut ? t.inner.as<int32_t>() : nullptr,
+      local, cut ? *cut : CutDev{}, grows, stride, lanes, wpb, scale, slice_pad(unroll),
+      t.wave_off.as<int32_t>(), sliced);
   LTRY(hipGetLastError(), "tile slice kernel");
+  return LJGPU_OK;
+}
+
+int dev_slice_tiles(hipStream_t s, const int32_t* slot_ptr, int32_t lanes, int32_t unroll,
+                    int32_t scale, bool bank_order, int32_t n, const CutHint* hint, ListWork& w,
+                    DevTiles& t) {
+  t.sliced_lanes = t.sliced_unroll = t.waves_per_block = 0;
+  t.bank_lanes = t.bank_unroll = 0;
+  if (t.blocks <= 0) return LJGPU_OK;
+  int32_t wpb = 0;
+  LCHECK(plan_slices(s, TileSpans{t.desc.as<int32_t>(), 0, 0, 8}, t.blocks, t.tile_particles,
+                     slot_ptr, lanes, unroll, t.longest, w, t, &wpb));
+  if (wpb == 0) return LJGPU_OK;
+  CutDev cd{};
+  const bool cut = bank_order && hint && hint->q.x && !t.cut;
+  if (cut) {
+    cd.q = hint->q;
+    cd.stage = t.stage.as<int32_t>();
+    cd.member = t.order == LJGPU_TILE_ORDER_SPATIAL ? t.member.as<int32_t>() : nullptr;
+    cd.box = hint->box;
+    cd.rep_box = hint->rep_box;
+    cd.cl2 = hint->cl2;
+    LCHECK(dev_reserve(t.inner, sizeof(int32_t) * n, s));
+  }
+  LCHECK(fill_slices(s, slot_ptr, lanes, unroll, scale, bank_order, cut ? &cd : nullptr,
+                     t.local.as<uint16_t>(), t, wpb, t.sliced.as<uint16_t>()));
   if (cut) t.cut = true;
   t.sliced_lanes = lanes;
   t.sliced_unroll = unroll;
@@ -3061,11 +3074,56 @@ int dev_half_tiles(hipStream_t s, int32_t n, ListWork& w, DevTiles& t) {
   return LJGPU_OK;
 }
 
-int dev_bank_order(hipStream_t s, const int32_t* slot_ptr, const DevTiles& t, uint16_t* local) {
-  if (t.blocks <= 0 || t.bank_done) return LJGPU_OK;
+// ListWork::tmp between builds: the rows with their padding, then the slices.
+size_t bank_rows_bytes(int64_t e) {
+  return sizeof(uint16_t) * static_cast<size_t>((e + kTileLocalPad + 7) / 8 * 8);
+}
+const uint16_t* bank_rows(const ListWork& w) { return w.tmp.as<uint16_t>(); }
+const uint16_t* bank_slices(const ListWork& w, int64_t e) {
+  return w.tmp.as<uint16_t>() + bank_rows_bytes(e) / sizeof(uint16_t);
+}
+
+int bank_room(hipStream_t s, int64_t e, bool slices, ListWork& w, DevTiles& t) {
+  const size_t need = bank_rows_bytes(e) + (slices ? sizeof(uint16_t) * t.slice_elems : 0);
+  if (w.tmp.p && w.tmp.bytes >= need) return LJGPU_OK;
+  t.bank_rows = false;  // the buffer is replaced
+  t.bank_lanes = t.bank_unroll = 0;
+  return dev_reserve(w.tmp, need, s);
+}
+
+int dev_bank_reserve(hipStream_t s, int64_t e, ListWork& w, DevTiles& t) {
+  const int rc = bank_room(s, e, true, w, t);
+  if (rc != LJGPU_ERR_OUT_OF_MEMORY) return rc;
+  (void)hipGetLastError();
+  clear_error();
+  return LJGPU_OK;
+}
+
+int dev_bank_rows(hipStream_t s, const int32_t* slot_ptr, int64_t e, ListWork& w, DevTiles& t) {
+  if (t.blocks <= 0 || t.bank_rows) return LJGPU_OK;
+  LCHECK(bank_room(s, e, false, w, t));
+  uint16_t* rows = w.tmp.as<uint16_t>();
+  LTRY(hipMemcpyAsync(rows, t.local.p, sizeof(uint16_t) * (e + kTileLocalPad),
+                      hipMemcpyDeviceToDevice, s), "hipMemcpyAsync");
   k_bank_order<<<std::min(t.blocks, 65535), kBankBlock, 0, s>>>(
-      t.desc.as<int32_t>(), t.blocks, slot_ptr, t.cut ? t.inner.as<int32_t>() : nullptr, local);
+      t.desc.as<int32_t>(), t.blocks, slot_ptr, t.cut ? t.inner.as<int32_t>() : nullptr, rows);
   LTRY(hipGetLastError(), "tile bank order kernel");
+  t.bank_rows = true;
+  return LJGPU_OK;
+}
+
+int dev_bank_slices(hipStream_t s, const int32_t* slot_ptr, int64_t e, ListWork& w, DevTiles& t) {
+  if (t.blocks <= 0 || t.sliced_lanes == 0 ||
+      (t.bank_lanes == t.sliced_lanes && t.bank_unroll == t.sliced_unroll))
+    return LJGPU_OK;
+  LCHECK(bank_room(s, e, true, w, t));
+  LCHECK(dev_bank_rows(s, slot_ptr, e, w, t));
+  // Lengths and starts of the slices do not depend on the order of a row.
+  uint16_t* rows = w.tmp.as<uint16_t>();
+  LCHECK(fill_slices(s, slot_ptr, t.sliced_lanes, t.sliced_unroll, 24, false, nullptr, rows, t,
+                     t.waves_per_block, rows + bank_rows_bytes(e) / sizeof(uint16_t)));
+  t.bank_lanes = t.sliced_lanes;
+  t.bank_unroll = t.sliced_unroll;
   return LJGPU_OK;
 }
 

@@ -394,3 +394,89 @@ def test_half_list_forces_lose_nothing_at_a_face(ctx, corner, tile):
     assert off.max() < (125 if tile or corner else 125 + 14 * 256)
     ctx.set_tiling(64)
     ctx.set_half_mode(G.HALF_AUTO)
+
+
+def momenta_of(c, q, box, kind, steps=1):
+    dq, dp = c.array(q), c.zeros(q.shape)
+    if kind == "f64":
+        c.force_aos_f64(dq, dp, 1e-3, G.CL2, box, steps)
+    else:
+        accum = G.ACCUM_F64 if kind == "mixed" else G.ACCUM_KAHAN_F32
+        c.force_aos_mixed(dq, dp, 1e-3, G.CL2, box, steps, accum)
+    c.sync()
+    return dp.download()
+
+
+@pytest.mark.parametrize("before", ["kahan", "stage_offsets", "get_tiles"])
+@pytest.mark.parametrize("lanes,unroll", [(8, 2), (4, 4), (64, 1)])
+def test_rows_keep_their_order_whatever_ran_before(before, lanes, unroll):
+    """Kahan sums, offsets staged in LDS and tile inspection take the rows in the
+    bank-class order; the launches that follow over the same list, in another
+    shape, give what they give in a context that did none of these."""
+    q, box, _, _ = system("mixed_rows")
+    out = []
+    for disturbed in (False, True):
+        c = G.Context(0)
+        try:
+            dq = c.array(q)
+            c.build_list(dq, q.shape[0], box, G.LIST_FULL)
+            if disturbed:
+                if before == "kahan":
+                    momenta_of(c, q, box, "kahan")
+                elif before == "get_tiles":
+                    c.get_tiles()
+                else:
+                    c.set_tiling(64, stage_offsets=True)
+                    momenta_of(c, q, box, "f64")
+                    c.set_tiling(64)
+            c.set_kernel_config(lanes, 256, unroll)
+            print(f"{before} lanes={lanes} disturbed={disturbed}", flush=True)
+            got = [momenta_of(c, q, box, k) for k in ("f64", "mixed", "kahan", "f64")]
+            got.append(c.get_tiles().local)
+            out.append(got + [momenta_of(c, q, box, k) for k in ("kahan", "f64")])
+        finally:
+            c.close()
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
+    np.testing.assert_array_equal(out[0][0], out[0][3])
+    np.testing.assert_array_equal(out[0][2], out[0][5])
+
+
+@pytest.mark.parametrize("installed", [False, True])
+def test_force_calls_do_not_allocate(installed):
+    """Once a list is built on the device (or, installed from the host, has had
+    its first force call), force calls of any precision take no more device
+    memory: what a list of 4.6 million entries needs for Kahan sums comes with
+    the list."""
+    info = G.lib().hipMemGetInfo  # of the HIP runtime that the library is linked with
+    info.argtypes = [ctypes.POINTER(ctypes.c_size_t)] * 2
+
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert info(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    q, box = G.lattice_periodic(20, 1.0, 3)
+    full = G.makepair(q, box, G.LIST_FULL) if installed else None
+    warm, c = G.Context(0), G.Context(0)
+    try:
+        for x in (warm, c):  # the first round loads the kernels
+            dq, dp = x.array(q), x.zeros(q.shape)
+            if installed:
+                x.set_list(full)
+                x.force_aos_f64(dq, dp, 1e-3, G.CL2, box, 1)
+            else:
+                x.build_list(dq, q.shape[0], box, G.LIST_FULL)
+            x.sync()
+            was = free()
+            for steps in (1, 3, 20):
+                x.force_aos_f64(dq, dp, 1e-3, G.CL2, box, steps)
+                x.force_aos_mixed(dq, dp, 1e-3, G.CL2, box, steps, G.ACCUM_F64)
+                x.force_aos_mixed(dq, dp, 1e-3, G.CL2, box, steps, G.ACCUM_KAHAN_F32)
+            x.sync()
+            taken = was - free()
+            print(f"installed={installed} taken {taken}", flush=True)
+        assert taken == 0
+    finally:
+        warm.close()
+        c.close()
