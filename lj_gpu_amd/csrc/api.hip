@@ -107,11 +107,14 @@ int ensure_ell(ljgpu_ctx* ctx) {
   return LJGPU_OK;
 }
 
-// The tile size to derive for the evaluated list (half lists of replicas are
-// not evaluated at all).
-int32_t tile_target(const ljgpu_ctx* ctx) {
-  return ctx->eval_half && !ctx->rep_off.empty() ? 0 : effective_tile(ctx);
+// The tile size to derive for the evaluated list, or for a half list evaluated
+// with atomics: those have kHalfLanes lanes a row in a workgroup of at most 1024
+// threads (half lists of replicas are not evaluated at all).
+int32_t tile_target(const ljgpu_ctx* ctx, bool half) {
+  if (!half) return effective_tile(ctx);
+  return ctx->rep_off.empty() ? std::min(effective_tile(ctx), 1024 / kHalfLanes) : 0;
 }
+int32_t tile_target(const ljgpu_ctx* ctx) { return tile_target(ctx, ctx->eval_half); }
 
 // Derive the LDS tiling of the evaluated list for the current
 // configuration. Where a block does not fit the LDS budget the tile size is
@@ -145,17 +148,13 @@ int ensure_tiles(ljgpu_ctx* ctx, const PosIn* q, double box) {
                      ctx->tile_offsets_lds || ctx->lanes != 4 || ctx->unroll != 4};
   const bool with_slices = !ctx->bank_order && ctx->work.row_max > 0;
   for (int32_t tp = want; tp >= 1 && ctx->eval.n > 0; tp /= 2) {
-    TRY(dev_make_tiles(ctx->stream, ctx->eval, tp, ctx->rep_off, ordered,
+    TRY(dev_make_tiles(ctx->stream, ctx->eval, tp, ctx->rep_off, ordered, ctx->eval_half,
                        with_slices ? &req : nullptr, ctx->work, ctx->tiles));
+    if (ctx->eval_half && !ctx->tiles.shared) break;  // smaller tiles share even less
     if (ctx->tiles.tile_particles == 0) continue;
     if (!ctx->eval_half || ctx->tiles.max_stage <= kHalfMaxStage) break;
     ctx->tiles.tile_particles = ctx->tiles.blocks = 0;
   }
-  // A half list's tile writes a force sum per staged partner. Where partners
-  // are hardly shared (scattered particles of an open box) there are nearly
-  // as many as pairs, and the untiled kernel stays.
-  if (ctx->eval_half && 2 * ctx->tiles.staged > ctx->eval.e)
-    ctx->tiles.tile_particles = ctx->tiles.blocks = 0;
   // The slot-order copies that calls of many steps (kSlotMinSteps) run over
   // are reserved with the tiles, so a force call never allocates.
   if (ctx->tiles.blocks > 0 && ctx->tiles.order == LJGPU_TILE_ORDER_SPATIAL &&
@@ -364,9 +363,8 @@ int build_list(ljgpu_ctx* ctx, const PosIn& q, int32_t n, double box, double sea
       if (!done && c->eval.slab_stride > 0) reset_list(c);
     }
   } guard{ctx};
-  const int32_t tile = effective_tile(ctx);
-  if (tile > 0 && n > 0 && ctx->tile_order == LJGPU_TILE_ORDER_SPATIAL &&
-      (expand || ctx->rep_off.empty()))
+  const int32_t tile = tile_target(ctx, !expand);
+  if (tile > 0 && n > 0 && ctx->tile_order == LJGPU_TILE_ORDER_SPATIAL)
     TRY(dev_tile_order_begin(ctx->stream, q, n, box, ctx->rep_off, ctx->rep_boxes, tile, ctx->work,
                              &ctx->order_begun, ctx->rep_off.empty()));
   // A full list is the symmetric closure of the half list (the pair

@@ -1481,8 +1481,8 @@ __global__ __launch_bounds__(1024) void k_tile_fill(
 }
 
 // The tiles' stats in one: out[0] a tile over the LDS budget, [1] most staged,
-// [2] most LDS bytes, [3] longest row, [4] a tile with too many pages, [6..7]
-// the total staged (64 bits). One workgroup.
+// [2] most LDS bytes, [3] longest row, [4] tiles with too many pages, [6..7]
+// the total staged (64 bits), as far as counted. One workgroup.
 __global__ __launch_bounds__(1024) void k_tile_stats(int32_t nblocks, const int4* __restrict__ stats,
                                                      uint16_t* __restrict__ pad,
                                                      int32_t* __restrict__ out) {
@@ -1497,22 +1497,23 @@ __global__ __launch_bounds__(1024) void k_tile_stats(int32_t nblocks, const int4
   unsigned long long n = 0;
   for (int32_t b = threadIdx.x; b < nblocks; b += blockDim.x) {
     const int4 t = stats[b];
-    const bool over = t.y > kTileLdsBudget;
-    v[0] |= over;
+    v[0] |= t.y > kTileLdsBudget;
     v[1] = max(v[1], t.x);
     v[2] = max(v[2], t.y);
     v[3] = max(v[3], t.z);
-    v[4] |= t.w;
-    n += over ? 0 : max(t.x, 0);
+    v[4] += t.w;
+    n += max(t.x, 0);
   }
   for (int d = 32; d > 0; d >>= 1) {
 #pragma unroll
-    for (int k = 0; k < 5; k++) v[k] = max(v[k], __shfl_xor(v[k], d, 64));
+    for (int k = 0; k < 4; k++) v[k] = max(v[k], __shfl_xor(v[k], d, 64));
+    v[4] += __shfl_xor(v[4], d, 64);
     n += __shfl_xor(n, d, 64);
   }
   if ((threadIdx.x & 63) == 0) {
 #pragma unroll
-    for (int k = 0; k < 5; k++) atomicMax(&mx[k], v[k]);
+    for (int k = 0; k < 4; k++) atomicMax(&mx[k], v[k]);
+    atomicAdd(&mx[4], v[4]);
     atomicAdd(&sum, n);
   }
   __syncthreads();
@@ -2841,9 +2842,10 @@ int plan_slices(hipStream_t s, const TileSpans& spans, int32_t nblocks, int32_t 
 }
 
 int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<int32_t>& reps,
-                   bool spatial, const SliceReq* req, ListWork& w, DevTiles& out) {
+                   bool spatial, bool half, const SliceReq* req, ListWork& w, DevTiles& out) {
   out.tile_particles = 0;
   out.blocks = 0;
+  out.shared = true;
   out.half_ready = false;
   if (T <= 0 || T > kTileRowsMax || c.n <= 0) return LJGPU_OK;
   // The slot order and each slot's row start in the slot-ordered rows.
@@ -2928,6 +2930,10 @@ int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<
       LCHECK(read_stats(back));
       std::copy(back, back + 4, h);
       std::memcpy(&st, back + 6, sizeof(st));
+      if (half && (back[4] > nb / 8 || 2 * static_cast<int64_t>(st) > c.e)) {
+        out.shared = false;
+        return LJGPU_OK;
+      }
       if (back[4] == 0) {
         if (pass == 0 && slices.out && back[0] == 0) {
           out.sliced_lanes = req->lanes;
@@ -2950,6 +2956,12 @@ int dev_make_tiles(hipStream_t s, const DevCSR& c, int32_t T, const std::vector<
     int32_t back[8];
     LCHECK(read_stats(back));
     std::copy(back, back + 4, h);
+    unsigned long long st = 0;
+    std::memcpy(&st, back + 6, sizeof(st));
+    if (half && 2 * static_cast<int64_t>(st) > c.e) {
+      out.shared = false;
+      return LJGPU_OK;
+    }
     if (h[0] != 0) return LJGPU_OK;  // does not fit: caller retries smaller or runs untiled
     LCHECK(dev_scan(s, w.tile_ns.as<int32_t>(), w.tile_soff.as<int32_t>(), nb, w, &staged));
     if (staged > INT32_MAX) return LJGPU_OK;

@@ -480,3 +480,63 @@ def test_force_calls_do_not_allocate(installed):
     finally:
         warm.close()
         c.close()
+
+
+@pytest.mark.parametrize("lanes,tile,used", [(2, 512, 256), (2, 257, 256), (2, 256, 256),
+                                             (4, 1000, 256)])
+@pytest.mark.parametrize("installed", [False, True])
+def test_half_lists_in_tiles_of_more_rows_than_their_kernel_takes(ctx, lanes, tile, used, installed):
+    """The half-list kernel has four lanes a row, whatever the configured
+    number: tiles of more than 256 rows become tiles of 256 where those fit (a
+    gas; dense tiles are halved until they do)."""
+    q, box = G.lattice_periodic(6, 0.1, 2)
+    half = G.makepair(q, box, G.LIST_HALF)
+    f, _ = exact_force(q, box, half)
+    ctx.set_kernel_config(lanes, 256, 4)
+    ctx.set_tiling(tile)
+    ctx.set_half_mode(G.HALF_ATOMIC)
+    dq, dp = ctx.array(q), ctx.zeros(q.shape)
+    if installed:
+        ctx.set_list(half)
+    else:
+        ctx.build_list(dq, q.shape[0], box, G.LIST_HALF)
+    for steps in (1, 20):
+        dp.zero()
+        ctx.force_aos_f64(dq, dp, 1.0 / steps, G.CL2, box, steps)
+        ctx.sync()
+        assert half_tile(ctx) == used
+        assert normwise(dp.download(), f.astype(float)) < FP64_TOL
+    ctx.set_kernel_config(4, 256, 4)
+    ctx.set_tiling(64)
+    ctx.set_half_mode(G.HALF_AUTO)
+
+
+@pytest.mark.parametrize("tiles,tiled", [(0, True), (25, True), (150, False)])
+def test_half_lists_with_some_scattered_tiles(ctx, tiles, tiled):
+    """Of the 500 tiles of an open lattice in its own order, some hold
+    particles from all over it: up to an eighth of them the list is tiled (their
+    sets hashed), beyond it takes the untiled kernel."""
+    q = G.lattice_reference(0.5, 40.0)
+    n = q.shape[0]
+    rng = np.random.default_rng(2)
+    at = np.arange(64 * tiles)
+    to = rng.choice(np.arange(64 * tiles, n), at.size, replace=False)
+    order = np.arange(n)
+    order[at], order[to] = to, at
+    q = np.ascontiguousarray(q[order])
+    half = G.makepair(q, 0.0, G.LIST_HALF)
+    f, _ = exact_force(q, 1e9, half)
+    ctx.set_kernel_config(4, 256, 4)
+    ctx.set_tiling(64)
+    ctx.set_half_mode(G.HALF_ATOMIC)
+    dq, dp = ctx.array(q), ctx.zeros(q.shape)
+    ctx.build_list(dq, n, 0.0, G.LIST_HALF)
+    used = half_tile(ctx)
+    print(f"n={n} scattered tiles={tiles}: tile {used}", flush=True)
+    assert (used > 0) == tiled and (tiles > 0 or used == 64)
+    for steps in (1, 20):
+        dp.zero()
+        ctx.force_aos_f64(dq, dp, 1.0 / steps, G.CL2, 0.0, steps)
+        ctx.sync()
+        assert normwise(dp.download(), f.astype(float)) < FP64_TOL
+    ctx.set_half_mode(G.HALF_AUTO)
