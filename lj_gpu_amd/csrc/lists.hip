@@ -1220,9 +1220,31 @@ constexpr int kWordLimit = 3000;
 constexpr int kWordLanes = 16;  // lanes that walk one row together
 constexpr int kWordBatch = 4;   // entries per lane in flight
 constexpr int kSeedRows = 8;    // one row in so many fills the set first
-constexpr int32_t kTileCodeMax = 12288;  // entry codes kept in LDS
+constexpr int kWordPairs = 192;  // more words are ranked by a sort
+constexpr int32_t kTileCodeMax = 12160;  // entry codes kept in LDS, 64 KB with the set
 static_assert(kTileMaxStage <= kWordLimit, "the word limit must cover every tile that fits");
 static_assert(kWordLimit + 1024 < kWords, "probing must always find a free entry");
+
+// The table entries words[0, nw) by ascending key, the others of words[0, p) (p
+// the power of two from nw on) as 0xffff behind them.
+__device__ __forceinline__ void sort_words(uint16_t* words, int nw, int p, const int32_t* keys) {
+  const int tid = static_cast<int>(threadIdx.x), nt = static_cast<int>(blockDim.x);
+  for (int t = nw + tid; t < p; t += nt) words[t] = 0xffff;
+  __syncthreads();
+  auto key = [&](uint16_t x) { return x == 0xffff ? INT32_MAX : keys[x]; };
+  for (int k = 2; k <= p; k <<= 1)
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      for (int t = tid; t < p / 2; t += nt) {
+        const int a = 2 * t - (t & (j - 1)), b = a + j;
+        const uint16_t x = words[a], y = words[b];
+        if ((key(x) > key(y)) == ((a & k) == 0)) {
+          words[a] = y;
+          words[b] = x;
+        }
+      }
+      __syncthreads();
+    }
+}
 
 __device__ __forceinline__ uint32_t word_hash(int32_t w) {
   return (static_cast<uint32_t>(w) * 2654435761u) >> (32 - kWordBits);
@@ -1304,7 +1326,12 @@ __device__ __forceinline__ uint32_t word_add(int32_t w, uint32_t h, uint32_t bit
 // slots; the staged particles are written in that order and each entry's LDS
 // offset 24 * rank in row order. What an entry needs to find its rank (table
 // entry and bit, 16 bits) stays in LDS between the two, so the list and
-// slot_of are read once; entries beyond `ecap` are looked up again.
+// slot_of are read once; entries beyond `ecap` are looked up again. The words of
+// a compact tile are ranked against each other, up to kWordPairs of them; those of
+// scattered partners (hardly two to a word) are sorted. List builds by pairs / by
+// sort: 135 words 2840 / 2836 us, 184 words 819 / 817, 270 words 3401 / 2634, 540
+// words 3458 / 1507, 2145 words 7258 / 1028; compact tiles (100 to 200
+// words, on this kernel) 513 / 561 us at 119,164 particles.
 //   Sixteen lanes share a row (no search for the row of an entry), four
 // entries per lane in flight, with every first probe of a batch issued
 // before any is used. soff null: tile b stages at b * kTileMaxStage, and
@@ -1322,8 +1349,9 @@ __global__ __launch_bounds__(1024) void k_tile_fill(
     uint16_t* __restrict__ local, int4* __restrict__ stats) {
   __shared__ int32_t keys[kWords];
   __shared__ uint32_t masks[kWords];  // slots present, then also the base rank << 16
-  __shared__ uint16_t words[kWordLimit];  // table entries in use
+  __shared__ uint16_t words[kWords];  // table entries in use
   __shared__ int32_t counter, nwords, total, longest;
+  __shared__ int32_t sh[16];
   extern __shared__ uint16_t code[];  // ecap: table entry << 4 | bit of each entry
   const int nt = static_cast<int>(blockDim.x), tid = static_cast<int>(threadIdx.x);
   const int lane = tid & (kWordLanes - 1), group = tid / kWordLanes, groups = nt / kWordLanes;
@@ -1412,9 +1440,22 @@ __global__ __launch_bounds__(1024) void k_tile_fill(
       __syncthreads();
       continue;
     }
-    // Base rank of each word: the slots of all smaller words, eight lanes to
-    // a word.
-    for (int t0 = 0; t0 < nw; t0 += nt / 8) {
+    // Base rank of each word: the slots of all smaller words, a scan over the
+    // sorted words or eight lanes to a word.
+    if (nw > kWordPairs) {
+      sort_words(words, nw, 1 << (32 - __clz(nw - 1)), keys);
+      const int piece = (nw + nt - 1) / nt;
+      const int t0 = min(tid * piece, nw), t1 = min(t0 + piece, nw);
+      int32_t n = 0, all;
+      for (int t = t0; t < t1; t++) n += __popc(masks[words[t]]);
+      int32_t base = block_exclusive<int32_t>(n, &all, sh);
+      for (int t = t0; t < t1; t++) {
+        const int x = words[t];
+        const uint32_t v = masks[x];
+        masks[x] = v | static_cast<uint32_t>(base) << 16;
+        base += __popc(v);
+      }
+    } else for (int t0 = 0; t0 < nw; t0 += nt / 8) {
       const int t = t0 + tid / 8;
       int32_t base = 0;
       if (t < nw) {

@@ -540,3 +540,46 @@ def test_half_lists_with_some_scattered_tiles(ctx, tiles, tiled):
         ctx.sync()
         assert normwise(dp.download(), f.astype(float)) < FP64_TOL
     ctx.set_half_mode(G.HALF_AUTO)
+
+
+@functools.lru_cache(maxsize=None)
+def scattered_system():
+    """27,436 particles of an open box in a shuffled order, and the first one's
+    row over all 215 pages of slots: sets of every tile size are hashed."""
+    q = G.lattice_reference(0.5, 38.0)
+    n = q.shape[0]
+    q = np.ascontiguousarray(q[np.random.default_rng(7).permutation(n)])
+    full = G.makepair(q, 0.0, G.LIST_FULL)
+    row = np.arange(1, n, n // 250).astype(np.int32)
+    lst = np.concatenate([row, full.sorted_list[full.number_of_partners[0]:]]).astype(np.int32)
+    nop = full.number_of_partners.copy()
+    nop[0] = row.size
+    ptr = np.concatenate([[0], np.cumsum(nop)[:-1]]).astype(np.int32)
+    return q, G.CSR(nop, ptr, lst, G.LIST_FULL)
+
+
+@pytest.mark.parametrize("tile,used", [(64, 32), (16, 16), (5, 5), (4, 4), (3, 3), (2, 2), (1, 1)])
+def test_tiles_of_scattered_partners(ctx, tile, used):
+    """Hashed sets of 20 words (ranked against each other) to 1,300 (sorted), on
+    both sides of the change at 192: the host model's tiles, the untiled kernel's
+    forces. Tiles of 64 have too many words and become 32."""
+    q, csr = scattered_system()
+    ctx.set_kernel_config(4, 256, 4)
+    ctx.set_half_mode(G.HALF_AUTO)
+    dq, p = ctx.array(q), []
+    for t in (0, tile):
+        ctx.set_tiling(t)
+        ctx.set_list(csr)
+        dp = ctx.zeros(q.shape)
+        ctx.force_aos_f64(dq, dp, 1.0, G.CL2, 0.0, 1)
+        ctx.sync()
+        p.append(dp.download())
+    print(f"tile={tile} used={ctx.list_info().tile_particles} "
+          f"staged {ctx.list_info().tile_max_stage}", flush=True)
+    assert ctx.list_info().tile_particles == used
+    assert normwise(p[1], p[0]) < FP64_TOL
+    t, h = ctx.get_tiles(), G.make_tiles(csr, used, q=q, box=0.0, cl2=G.CL2)
+    np.testing.assert_array_equal(t.desc, h.desc)
+    np.testing.assert_array_equal(t.stage, h.stage)
+    np.testing.assert_array_equal(t.local, h.local)
+    ctx.set_tiling(64)
