@@ -583,3 +583,24 @@ def test_tiles_of_scattered_partners(ctx, tile, used):
     np.testing.assert_array_equal(t.stage, h.stage)
     np.testing.assert_array_equal(t.local, h.local)
     ctx.set_tiling(64)
+
+
+@pytest.mark.parametrize("accum", [G.ACCUM_F64, G.ACCUM_KAHAN_F32])
+@pytest.mark.parametrize("name", ["ragged", "open"])
+@pytest.mark.parametrize("tile,resident", [(64, 0), (4, 1)])
+def test_mixed_launches_of_several_evaluations(ctx, accum, name, tile, resident):
+    """As test_launches_of_several_evaluations for mixed precision with either
+    kind of sum, whose kernels keep their own form of the loop over evaluations."""
+    q, box, _, _ = system(name)
+    ctx.set_kernel_config(4, 256, 4)
+    ctx.set_tiling(tile, resident_per_cu=resident)
+    ctx.set_half_mode(G.HALF_AUTO)
+    dq, da, db = ctx.array(q), ctx.zeros(q.shape), ctx.zeros(q.shape)
+    ctx.build_list(dq, q.shape[0], box, G.LIST_FULL)
+    for steps in (2, 5, 17, 100):
+        ctx.force_aos_mixed(dq, da, 1e-3, G.CL2, box, steps, accum)
+        for _ in range(steps):
+            ctx.force_aos_mixed(dq, db, 1e-3, G.CL2, box, 1, accum)
+        ctx.sync()
+        np.testing.assert_array_equal(da.download(), db.download())
+    ctx.set_tiling(64)
