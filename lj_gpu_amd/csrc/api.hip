@@ -515,6 +515,13 @@ double tile_rounds(const ListView& lv, const LaunchConfig& lc) {
   return lv.tile_blocks / (kTileRound * std::max(1.0, 1.0 * lc.cus));
 }
 
+// The steps from which a call runs over copies in slot order (see kSlotMinSteps).
+int32_t slot_min_steps(const ForceArgs& fa, double rounds) {
+  if (fa.aos3) return rounds >= kSlotAos3Rounds ? kSlotMinStepsAos3 : kSlotMinSteps;
+  if (rounds < 1.0) return kSlotMinSteps;
+  return fa.soa ? kSlotMinStepsSoa : kSlotMinStepsAos;
+}
+
 // Launches that carry `steps` evaluations (see kMaxLaunchSteps) over full-list
 // tiles (a tile updates its own particles only, so its evaluations need no
 // order across tiles), one per evaluation otherwise.
@@ -794,9 +801,8 @@ int run_steps(ljgpu_ctx* ctx, const ForceArgs& caller, int32_t steps, bool mixed
   // and the staging's accesses are then contiguous runs. The arithmetic is
   // the same, so the momenta equal those of per-step evaluations bit for bit.
   ForceArgs fa = caller;
-  const int32_t slot_min =
-      tile_rounds(lv, lc) >= kSlotLargeRounds ? kSlotMinStepsLarge : kSlotMinSteps;
-  const bool slots = steps >= slot_min && lv.tile_blocks > 0 && lv.tile_stage_slot;
+  const bool slots = steps >= slot_min_steps(caller, tile_rounds(lv, lc)) && lv.tile_blocks > 0 &&
+                     lv.tile_stage_slot;
   if (slots) {
     TRY(slot_gather(ctx, caller, &fa));
     lv.tile_member = nullptr;

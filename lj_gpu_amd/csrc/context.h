@@ -53,15 +53,24 @@ constexpr int32_t kMinChainTiles = 64;  // fewer tiles: one chain
 // 3367; at 256,000 (1.3 rounds) 346 / 348 / 361.
 constexpr int32_t kMaxLaunchSteps = 16;
 constexpr double kTileRound = 12.0;
-// Calls with at least kSlotMinSteps steps over spatially ordered tiles run
-// over copies of q and p in slot order (two gathers and a scatter per call).
-// Systems of more than kSlotLargeRounds rounds of tiles, whose rows do not stay
-// in the L2s, do so from kSlotMinStepsLarge steps on: 10 evaluations of 1,048,576
-// particles take 1446 us with copies and 1473 without (AoS), 1500 and 1578
-// (SoA); of 119,164 206 and 202 (AoS), 238 and 240 (SoA).
+// Calls of at least this many steps over spatially ordered tiles run over copies
+// of q and p in slot order (a gather and a scatter per call, two gathers for SoA
+// and double3 arrays). What the copies save grows with the system, whose
+// arrays do not stay in the L2s, and with the disorder of its particles, which
+// the caller's order alone tells: the lines lie where particles in lattice order
+// break even. Times with copies over times without, lattice order / shuffled:
+//   AoS    172 tiles 8 steps 1.01 / 1.00, 16 steps 1.00 / 0.98 (14 tiles 1.04 / 1.03);
+//          one round (kTileRound) 8 steps 1.00; 1.3 rounds 4 steps 1.02 / 0.89, 8 steps
+//          0.99 / 0.84; 2.3 rounds 8 steps 0.99 / 0.81; 5.3 rounds 8 steps 0.99 / 0.79
+//   SoA    0.3 rounds 8 steps 1.04 / 0.75; 0.6 rounds 8 steps 1.02 / 0.59; 1.3 rounds
+//          4 steps 1.01 / 0.55; 5.3 rounds 4 steps 0.98 / 0.33
+//   double3  1.3 rounds 8 steps 1.03 / 0.82, 12 steps 1.02 / 0.79; 5.3 rounds 8 steps
+//          1.02 / 0.73, 10 steps 1.00 / 0.71
 constexpr int32_t kSlotMinSteps = 16;
-constexpr int32_t kSlotMinStepsLarge = 10;
-constexpr double kSlotLargeRounds = 4.0;
+constexpr int32_t kSlotMinStepsAos = 8;     // from one round of tiles on
+constexpr int32_t kSlotMinStepsSoa = 4;     // from one round of tiles on
+constexpr int32_t kSlotMinStepsAos3 = 10;   // from kSlotAos3Rounds on
+constexpr double kSlotAos3Rounds = 4.0;
 // Energy sums: a fixed grid of kEnergyBlocks workgroups (each striding over
 // the rows) writes one partial per workgroup and quantity (potential,
 // kinetic, pairs inside the cutoff), added afterwards in block order, so the

@@ -604,3 +604,36 @@ def test_mixed_launches_of_several_evaluations(ctx, accum, name, tile, resident)
         ctx.sync()
         np.testing.assert_array_equal(da.download(), db.download())
     ctx.set_tiling(64)
+
+
+@pytest.mark.parametrize("cells", [14, 15])
+@pytest.mark.parametrize("layout", ["aos", "soa", "aos3"])
+@pytest.mark.parametrize("kind", [G.LIST_FULL, G.LIST_HALF])
+def test_copies_in_slot_order_around_one_round_of_tiles(ctx, cells, layout, kind):
+    """10,976 and 13,500 particles in tiles of 4 are 0.9 and 1.1 rounds of tiles of
+    256 compute units; from one round on shorter calls run over copies of the
+    arrays in slot order: bit for bit what as many calls of one step give."""
+    q, box = G.lattice_periodic(cells, 0.5, 3)
+    q = np.ascontiguousarray(q[np.random.default_rng(cells).permutation(q.shape[0])])
+    n = q.shape[0]
+    ctx.set_kernel_config(4, 256, 4)
+    ctx.set_tiling(4)
+    ctx.set_half_mode(G.HALF_AUTO)
+    if layout == "soa":
+        dq = [ctx.array(np.ascontiguousarray(q[:, c])) for c in range(3)]
+        da, db = ([ctx.zeros(n) for _ in range(3)] for _ in range(2))
+        build, force = ctx.build_list_soa, ctx.force_soa_f64
+    else:
+        w = 4 if layout == "aos" else 3
+        dq, da, db = ctx.array(np.ascontiguousarray(q[:, :w])), ctx.zeros((n, w)), ctx.zeros((n, w))
+        build = ctx.build_list if w == 4 else ctx.build_list_aos3
+        force = ctx.force_aos_f64 if w == 4 else ctx.force_aos3_f64
+    build(dq, n, box, kind)
+    for steps in (3, 4, 7, 8, 9, 10, 15, 16):
+        force(dq, da, 1e-3, G.CL2, box, steps)
+        for _ in range(steps):
+            force(dq, db, 1e-3, G.CL2, box, 1)
+        ctx.sync()
+        for a, b in zip(*(([x] if layout != "soa" else x) for x in (da, db))):
+            np.testing.assert_array_equal(a.download(), b.download())
+    ctx.set_tiling(64)
