@@ -60,14 +60,14 @@ constexpr double kTileRound = 12.0;
 // the caller's order alone tells: the lines lie where particles in lattice order
 // break even. Times with copies over times without, lattice order / shuffled:
 //   AoS    172 tiles 8 steps 1.01 / 1.00, 16 steps 1.00 / 0.98 (14 tiles 1.04 / 1.03);
-//          one round (kTileRound) 8 steps 1.00; 1.3 rounds 4 steps 1.02 / 0.89, 8 steps
-//          0.99 / 0.84; 2.3 rounds 8 steps 0.99 / 0.81; 5.3 rounds 8 steps 0.99 / 0.79
+//          one round (kTileRound) 6 steps 1.02; 1.3 rounds 4 steps 1.02 / 0.89, 6 steps
+//          0.99 / 0.85; 2.3 rounds 6 steps 0.99 / 0.82; 5.3 rounds 6 steps 1.00 / 0.80
 //   SoA    0.3 rounds 8 steps 1.04 / 0.75; 0.6 rounds 8 steps 1.02 / 0.59; 1.3 rounds
 //          4 steps 1.01 / 0.55; 5.3 rounds 4 steps 0.98 / 0.33
 //   double3  1.3 rounds 8 steps 1.03 / 0.82, 12 steps 1.02 / 0.79; 5.3 rounds 8 steps
 //          1.02 / 0.73, 10 steps 1.00 / 0.71
 constexpr int32_t kSlotMinSteps = 16;
-constexpr int32_t kSlotMinStepsAos = 8;     // from one round of tiles on
+constexpr int32_t kSlotMinStepsAos = 6;     // from one round of tiles on
 constexpr int32_t kSlotMinStepsSoa = 4;     // from one round of tiles on
 constexpr int32_t kSlotMinStepsAos3 = 10;   // from kSlotAos3Rounds on
 constexpr double kSlotAos3Rounds = 4.0;
