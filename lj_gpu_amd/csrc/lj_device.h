@@ -236,20 +236,20 @@ __device__ __forceinline__ double lj_df_f64(double r2, const PairParams& pp) {
   return lj_df_f64_s(rcp_f64(r2), r2, pp);
 }
 
-// FP64 force scalar up to a factor: with s = kCbrt2 / r2, s^4 - s^7 is
+// FP64 force scalar up to a factor: with s = kCbrt2 / r2, s^4 (1 - s^3) is
 // kCbrt2^4 times s0^4 (1 - 2 s0^3) for s0 = 1/r2, as kCbrt2^3 = 2 (to 6.2e-17:
 // the nearest double to the cube root happens to lie that close). Folding the 2
 // into s saves a multiplication per pair; the tiled kernels multiply each
 // row's sum by kUnitScale * 24 * dt once. Exactly 0 where `inside` is false
-// (only the high word of s is cleared, as in lj_df_f64).
+// (only the high word of s is cleared, as in lj_df_f64). As a product, so that a
+// pair too close for s^4 gives an infinite force: s^4 - s^7 would be NaN.
 constexpr double kCbrt2 = 0x1.428a2f98d728bp+0;
 constexpr double kUnitScale = 0.5 / kCbrt2;
 __device__ __forceinline__ double lj_df_unit_f64(double s, bool inside) {
   const int hi = inside ? __double2hiint(s) : 0;
   s = __hiloint2double(hi, __double2loint(s));
   const double s2 = s * s;
-  const double s3 = s2 * s, s4 = s2 * s2;
-  return fma(-s3, s4, s4);
+  return (s2 * s2) * fma(-s2, s, 1.0);
 }
 
 // Mixed-precision force scalar: r2 (computed in FP64) rounded once to FP32,

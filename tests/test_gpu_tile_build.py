@@ -637,3 +637,36 @@ def test_copies_in_slot_order_around_one_round_of_tiles(ctx, cells, layout, kind
         for a, b in zip(*(([x] if layout != "soa" else x) for x in (da, db))):
             np.testing.assert_array_equal(a.download(), b.download())
     ctx.set_tiling(64)
+
+
+@pytest.mark.parametrize("unroll", [1, 2, 4])
+@pytest.mark.parametrize("gap", [1e-30, 1e-40, 1e-50])
+def test_particles_that_all_but_coincide(ctx, gap, unroll):
+    """Two particles so close that s = 1 / r^2 overflows in the fourth power: the
+    tiled kernel's momenta are the untiled one's, infinite in the pair's
+    directions, and finite for the others."""
+    q, box = G.lattice_periodic(6, 0.5, 3)
+    q = q.copy()
+    # a pair at the origin, nobody else within reach of the overflow
+    q[0, :3] = 0.0
+    q[1, :3] = gap * np.array([1.0, 2.0, 3.0])
+    full = G.makepair(q, box, G.LIST_FULL)
+    ctx.set_half_mode(G.HALF_AUTO)
+    ctx.set_kernel_config(4, 256, unroll)
+    p = []
+    for tile in (0, 64):
+        ctx.set_tiling(tile)
+        ctx.set_list(full)
+        dq, dp = ctx.array(q), ctx.zeros(q.shape)
+        ctx.force_aos_f64(dq, dp, 1e-3, G.CL2, box, 1)
+        ctx.sync()
+        p.append(dp.download()[:, :3])
+    print(f"gap {gap}: {p[0][0]} {p[1][0]}", flush=True)
+    assert not np.isnan(p[0]).any() and not np.isnan(p[1]).any()
+    big = np.abs(p[0]) > 1e100
+    np.testing.assert_array_equal(np.isinf(p[0]), np.isinf(p[1]))
+    np.testing.assert_array_equal(np.sign(p[0][big]), np.sign(p[1][big]))
+    assert big[:2].all() and not big[2:].any()
+    assert normwise(p[1][2:], p[0][2:]) < FP64_TOL
+    ctx.set_kernel_config(4, 256, 4)
+    ctx.set_tiling(64)
