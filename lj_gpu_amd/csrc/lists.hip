@@ -2708,8 +2708,10 @@ int dev_tile_order_begin(hipStream_t s, const PosIn& q, int32_t n, double box,
   const std::vector<int32_t> single = {0, n};
   const std::vector<int32_t>& off = replicas.empty() ? single : replicas;
   const int32_t nsys = static_cast<int32_t>(off.size()) - 1;
-  // Kept: the upload below reads it after this returns.
+  // Kept: the upload below reads it after this returns. One not yet read (of a
+  // build that failed before it synchronised) must not be written over.
   std::vector<char>& store = w.order_host;
+  if (!replicas.empty() && !store.empty()) LTRY(hipStreamSynchronize(s), "hipStreamSynchronize");
   const size_t gbytes = (sizeof(OrderGrid) * nsys + 255) / 256 * 256;
   store.resize(gbytes + sizeof(int32_t) * off.size());
   OrderGrid* grids = reinterpret_cast<OrderGrid*>(store.data());
