@@ -3109,9 +3109,9 @@ int dev_half_tiles(hipStream_t s, int32_t n, ListWork& w, DevTiles& t) {
   int32_t* first = t.half_first.as<int32_t>();
   k_half_counts<<<grid_for(nb, kBlock), kBlock, 0, s>>>(nb, desc, w.tile_ns.as<int32_t>());
   LTRY(hipGetLastError(), "half tile count kernel");
-  int64_t total = 0;
-  LCHECK(dev_scan(s, w.tile_ns.as<int32_t>(), w.tile_soff.as<int32_t>(), nb, w, &total));
+  const int64_t total = t.staged;
   if (total > INT32_MAX) return set_error(LJGPU_ERR_CAPACITY, "half list: too many staged partners");
+  LCHECK(dev_scan_async(s, w.tile_ns.as<int32_t>(), w.tile_soff.as<int32_t>(), nb, w, nullptr));
   LCHECK(dev_reserve(t.half_at, sizeof(int32_t) * std::max<int64_t>(total, 1), s));
   LCHECK(dev_reserve(t.half_part, sizeof(double) * 3 * std::max<int64_t>(total, 1), s));
   const int grid = std::min(nb, 65535);
@@ -3119,7 +3119,7 @@ int dev_half_tiles(hipStream_t s, int32_t n, ListWork& w, DevTiles& t) {
   k_half_places<<<grid, kBlock, 0, s>>>(nb, desc, keys, w.tile_soff.as<int32_t>(),
                                         t.half_tile.as<int2>(), count);
   LTRY(hipGetLastError(), "half tile place kernel");
-  LCHECK(dev_scan(s, count, first, n, w, &total));
+  LCHECK(dev_scan_async(s, count, first, n, w, nullptr));
   LCHECK(fill<int32_t>(s, count, n, 0));
   k_half_fill<<<grid, kBlock, 0, s>>>(nb, desc, keys, w.tile_soff.as<int32_t>(), first, count,
                                       t.half_at.as<int32_t>());
