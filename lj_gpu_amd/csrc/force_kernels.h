@@ -473,8 +473,8 @@ __device__ __forceinline__ void tile_row_stream(const M& mom, const uint16_t* __
 // particle, and (b) the block's ne per-entry LDS offsets (one contiguous,
 // coalesced range of `local`, which holds the rows in slot order: slot s's
 // row starts at slot_ptr[s]). A null member means that positions, momenta
-// and `stage` are given in slot order (particle index = slot). Rows then run entirely out of LDS: the random
-// gathers of the CSR kernel become LDS reads and the list costs 2 bytes per
+// and `stage` are given in slot order (particle index = slot). Rows then run
+// entirely out of LDS: the random gathers of the CSR kernel become LDS reads and the list costs 2 bytes per
 // entry. In the unwrapped frame a pair difference equals its minimum image
 // whenever every particle of the block lies within box/2 - rc of the
 // reference point (rc = cutoff); blocks where that fails apply the minimum
@@ -485,8 +485,9 @@ __device__ __forceinline__ void tile_row_stream(const M& mom, const uint16_t* __
 // A launch covers tiles [first, first + nblocks), `steps` evaluations of each
 // (a workgroup reads and stages its tile anew for every one). They are assigned
 // XCD-aware: the workgroups on XCD x (blockIdx % 8 == x) walk the contiguous
-// range [x*per, (x+1)*per) of the launch's tiles with a stride of gridDim/8. With one workgroup per tile each does a single tile; with a
-// smaller (persistent) grid each loops over several, so resident workgroups
+// range [x*per, (x+1)*per) of the launch's tiles with a stride of gridDim/8.
+// With one workgroup per tile each does a single tile; with a smaller
+// (persistent) grid each loops over several, so resident workgroups
 // drift out of phase and one's staging and memory stalls overlap another's
 // arithmetic.
 template <int TPI, int U, int PREC, class P, class M, bool PBC, bool OFFS_LDS, bool SL>
@@ -659,7 +660,8 @@ __device__ __forceinline__ void tile_body(P pos, M mom, const int32_t* __restric
 // VGPRs. The periodic FP64 kernels take 80, so six waves fit (1.8 % faster
 // at 1,048,576 particles than at 90 registers and five); forcing 80 where the
 // compiler needs more spills (+26 %). The mixed ones take 96: they ran 7 %
-// faster at five waves than at six and 5 % faster than at four.
+// faster at five waves than at six and 5 % faster than at four. The Kahan
+// ones take 88.
 template <int TPI, int U, int PREC, class P, class M, bool PBC, bool OFFS_LDS, bool SL>
 __global__ void __launch_bounds__(1024)
 __attribute__((amdgpu_waves_per_eu(5)))
@@ -693,7 +695,7 @@ k_tile(P pos, M mom, const int32_t* __restrict__ nop, const int32_t* __restrict_
                                                      local, sliced, wave_off, wpb, tile, pp, reach,
                                                      rep_box, lb, flag, nullptr);
     __syncthreads();  // the next step or tile overwrites this one's LDS
-    if (++s == steps) {
+    if (++s >= steps) {
       s = 0;
       b += stride;
     }
