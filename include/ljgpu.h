@@ -291,9 +291,10 @@ int ljgpu_force_soa_f64(ljgpu_ctx* ctx, const double* qx, const double* qy, cons
 /* The same over packed double[N][3] arrays (x, y, z; 24 B per particle,
  * 8-byte aligned): the reference's double3 instantiation of every kernel
  * (cuda/force_cuda.cu:26-27 buffers, :354-375 MEASURE_FOR_ALLTYPES). Same
- * arithmetic and results as the double4 calls. A call of 16 or more steps
- * over spatially ordered tiles runs on internal 4-double copies in slot
- * order, like the double4 calls, and writes p back in the caller's rows. */
+ * arithmetic and results as the double4 calls. A call of many steps (16, or
+ * 10 for large systems) over spatially ordered tiles runs on internal
+ * 4-double copies in slot order, as the double4 calls (6 steps) and SoA calls
+ * (4) of large systems do, and writes p back in the caller's rows. */
 int ljgpu_force_aos3_f64(ljgpu_ctx* ctx, const double* q, double* p, double dt, double cl2,
                          double box, int32_t steps);
 
@@ -413,18 +414,19 @@ int ljgpu_maxwell_boltzmann(int32_t particle_number, double temperature, uint32_
  * as replays of captured HIP graphs (1, the default) or as individual
  * launches (0). A force call of `steps` evaluations replays graphs of 64, 16
  * and 4 evaluations (longest first) and launches the remaining 0-3; a launch
- * over LDS tiles carries about sqrt of a graph's evaluations. Each graph is captured once per argument set and kept in a cache of 12 (least
- * recently used evicted). */
+ * over LDS tiles carries about sqrt of a graph's evaluations. Each graph is
+ * captured once per argument set and kept in a cache of 12 (least recently
+ * used evicted). */
 int ljgpu_set_graphs(ljgpu_ctx* ctx, int enable);
 
 /* Concurrent chains of a many-step call over LDS tiles (1 to 4, default 2).
  * With c > 1, a call of 4 or more steps over at least 64 * c tiles splits
  * the tiles into c contiguous parts and runs each part's steps as its own
- * chain of launches (about sqrt(steps) of them) on its own stream of the context, forked from and joined
- * back into the context stream within the call (launched directly, not
- * replayed from graphs). The parts update disjoint particles, so the momenta
- * are bitwise those of one chain; one chain's launch ramp and tail overlap
- * the others' work. No counterpart in the reference (which launches on the
+ * chain of launches (about sqrt(steps) of them) on its own stream of the
+ * context, forked from and joined back into the context stream within the
+ * call (launched directly, not replayed from graphs). The parts update
+ * disjoint particles, so the momenta are bitwise those of one chain; one
+ * chain's launch ramp and tail overlap the others' work. No counterpart in the reference (which launches on the
  * default stream). */
 int ljgpu_set_chains(ljgpu_ctx* ctx, int chains);
 

@@ -1073,13 +1073,13 @@ __device__ __forceinline__ void pairs_cell(int32_t p0, int32_t p1, int32_t per, 
   }
 }
 
-// One wavefront per cell (2^split of them in small systems), for cell grids with a stencil (R >= 1). The
-// candidates of the (2R+1)^3 cells around it are walked as one flattened
-// sequence, 64 per round, and tested against kPairGroup of the cell's
-// particles at a time (about four to five of a fine cell's, so mostly one
-// group), whose coordinates, counts and row addresses are scalars: a pair costs the
-// eight FP64 operations of the predicate and a handful for the place of a hit. A
-// round's hits for one particle go to consecutive addresses of its row
+// One wavefront per cell (2^split of them in small systems), for cell grids
+// with a stencil (R >= 1). The candidates of the (2R+1)^3 cells around it are
+// walked as one flattened sequence, 64 per round, and tested against kPairGroup
+// of the cell's particles at a time (about four to five of a fine cell's, so
+// mostly one group), whose coordinates, counts and row addresses are scalars: a
+// pair costs the eight FP64 operations of the predicate and a handful for the
+// place of a hit. A round's hits for one particle go to consecutive addresses of its row
 // (ballot, then each hit's rank among them), so the stores coalesce; they are
 // read much later, hence non-temporal (580 -> 570 us at 1,048,576 particles). The
 // runs of the flattened sequence are the x-rows of the stencil, contiguous
@@ -1595,8 +1595,8 @@ static_assert(kPageBytes / 128 < 255, "a page number fits a byte");
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6))) void k_tile_pages(
     TileSpans spans, int32_t nblocks, const int32_t* __restrict__ member,
     const int32_t* __restrict__ slot_of, const int32_t* __restrict__ slot_ptr,
-    RowSource rows, int32_t pshift, int32_t npages, SliceDev slices, int32_t* __restrict__ desc, int32_t* __restrict__ stage,
-    int32_t* __restrict__ stage_slot, uint16_t* __restrict__ local, int4* __restrict__ stats) {
+    RowSource rows, int32_t pshift, int32_t npages, SliceDev slices,
+    int32_t* __restrict__ desc, int32_t* __restrict__ stage, int32_t* __restrict__ stage_slot, uint16_t* __restrict__ local, int4* __restrict__ stats) {
   extern __shared__ uint32_t page_lds[];
   __shared__ uint32_t table[kPageBytes / 16];  // slots present, base rank << 16
   __shared__ uint32_t used[kPageBytes / 4];    // a byte per slot of the pages in use
@@ -1836,8 +1836,8 @@ static_assert(kBankClasses == 4 * kRowLanes, "one lane per word of counts, four 
 // lane counts its own entries by class; a sum over the row's lanes leaves the
 // number of each lane's first one, from which its entries take their numbers
 // q, and the q-th entry of a class takes the q-th place that has the class as
-// its target. The entries beyond those fill, in order, the places whose class ran out. One lane per row and
-// the seven other wavefronts idle took 182 us with the rest of k_tile_slices at
+// its target. The entries beyond those fill, in order, the places whose class
+// ran out. One lane per row and the seven other wavefronts idle took 182 us with the rest of k_tile_slices at
 // 119,000 particles (density 1), 35 at 2,000; this way 122 and 25.
 __device__ __forceinline__ void order_part(const uint16_t* from, int step, uint16_t* to, int phase,
                                            int n, int nmax, OrderLds& lds) {

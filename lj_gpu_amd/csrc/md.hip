@@ -238,7 +238,8 @@ __global__ void k_energy_total(int grid_q, int grid_p, int with_q, int with_p,
 // kEnergyBlocks doubles: potential, kinetic and pair-count partials). Over
 // an installed tiling (the force kernels' layout, used as it stands) the
 // potential runs on the tiles (k_tile_energy, energy_on_tiles), otherwise
-// over the CSR rows (k_potential). *grid_q / *grid_p: the partials of U and pairs / of K.
+// over the CSR rows (k_potential). *grid_q / *grid_p: the partials of U and
+// pairs / of K.
 int launch_energy(ljgpu_ctx* ctx, const double* q, const double* p, double box, double cl2,
                   double* part, int* grid_q, int* grid_p) {
   const int grid = std::min(kEnergyBlocks, grid_for(ctx->n));
