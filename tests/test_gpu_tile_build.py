@@ -460,7 +460,7 @@ def test_force_calls_do_not_allocate(installed):
     full = G.makepair(q, box, G.LIST_FULL) if installed else None
     warm, c = G.Context(0), G.Context(0)
     try:
-        for x in (warm, c):  # the first round loads the kernels
+        for x in (warm, c):  # the first context loads the kernels
             dq, dp = x.array(q), x.zeros(q.shape)
             if installed:
                 x.set_list(full)
