@@ -683,21 +683,34 @@ k_tile(P pos, M mom, const int32_t* __restrict__ nop, const int32_t* __restrict_
   const int per = (nblocks + kXcds - 1) / kXcds;
   const int stride = static_cast<int>(gridDim.x) / kXcds;
   const int t_end = min(nblocks, (xcd + 1) * per);
-  int s = 0;
-  for (int b = xcd * per + static_cast<int>(blockIdx.x) / kXcds; b < t_end;) {
-    // Opaque, so that each step reads its tile again instead of holding what the
-    // last one read in registers. Not for Kahan sums: their kernel spilled 12
-    // registers with it (4 to 12 % slower at 256,000 particles and in replicas) and
-    // has none to spare without.
-    int tile = first + b;
-    if constexpr (PREC != kMixedKahan) asm volatile("" : "+s"(tile));
+  const int b0 = xcd * per + static_cast<int>(blockIdx.x) / kXcds;
+  auto evaluate = [&](int tile) {
     tile_body<TPI, U, PREC, P, M, PBC, OFFS_LDS, SL>(pos, mom, nop, member, slot_ptr, desc, stage,
                                                      local, sliced, wave_off, wpb, tile, pp, reach,
                                                      rep_box, lb, flag, nullptr);
     __syncthreads();  // the next step or tile overwrites this one's LDS
-    if (++s >= steps) {
-      s = 0;
-      b += stride;
+  };
+  if constexpr (PREC == kMixedKahan) {
+    // Evaluations and tiles in one loop: with the loops below the Kahan kernel
+    // spilled 12 registers (4 to 12 % slower at 256,000 particles and in replicas);
+    // the others are up to 1 % faster with them.
+    int s = 0;
+    for (int b = b0; b < t_end;) {
+      evaluate(first + b);
+      if (++s >= steps) {
+        s = 0;
+        b += stride;
+      }
+    }
+  } else {
+    for (int b = b0; b < t_end; b += stride) {
+      for (int s = 0; s < steps; s++) {
+        // Opaque, so that each step reads its tile again instead of holding what
+        // the first one read in registers.
+        int tile = first + b;
+        asm volatile("" : "+s"(tile));
+        evaluate(tile);
+      }
     }
   }
 }
